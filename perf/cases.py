@@ -131,9 +131,20 @@ def _check(rc):
         raise RuntimeError(ffi.last_error())
 
 
+def _attention_layer(s):
+    """Norm weights [2, d] (bf16) of a full-attention layer and the keys and values its cache holds, [2, length, hkv * d]
+    in the cache's type (None where it is empty): keys of unit variance per channel, as a per-head norm leaves them, and
+    values of unit variance."""
+    c = s.case
+    norm = (1.0 + 0.1 * torch.randn(2, c["d"], device="cuda", generator=s.gen)).to(torch.bfloat16)
+    if not c["length"]:
+        return norm, None
+    kv = torch.randn(2, c["length"], c["hkv"] * c["d"], device="cuda", generator=s.gen)
+    return norm, kv.to(torch.bfloat16) if c["bf16"] else kv
+
+
 def _attention(s, layers, length, capacity, interval=1):
-    """A context of `layers` layers whose full-attention caches hold `length` positions: keys of unit variance per
-    channel, as a per-head norm leaves them, and values of unit variance."""
+    """A context of `layers` layers whose full-attention caches hold `length` positions."""
     c = s.case
     lin = {} if interval == 1 else dict(linear_num_k_heads=c["hk"], linear_num_v_heads=c["hv"])
     s.ctx = Ctx(Config(num_layers=layers, full_attn_interval=interval, num_attn_heads=c["hq"], num_kv_heads=c["hkv"],
@@ -141,40 +152,46 @@ def _attention(s, layers, length, capacity, interval=1):
     for layer in range(layers):
         if (layer + 1) % interval:
             continue
-        norm = _bits(1.0 + 0.1 * torch.randn(2, c["d"], device="cuda", generator=s.gen))
+        norm, kv = _attention_layer(s)
+        norm = _bits(norm)
         s.ctx.set_full_weights(layer, norm[0], norm[1])
         if length:
-            kv = torch.randn(2, length, c["hkv"] * c["d"], device="cuda", generator=s.gen)
             kv = _bits(kv) if c["bf16"] else kv.cpu().numpy()
             s.ctx.kv_import(layer, kv[0], kv[1])
 
 
-def _deltanet(s, layers, zero_state=False):
+def _deltanet_layer(s):
+    """conv weights, A_log, dt bias, norm weights, conv history and recurrent state of a DeltaNet layer."""
+    hv, conv = s.case["hv"], (2 * s.case["hk"] + s.case["hv"]) * 128
+    rnd = lambda *n: torch.randn(*n, device="cuda", generator=s.gen)  # noqa: E731
+    bf = torch.bfloat16
+    return ((0.5 * rnd(conv, 4)).to(bf), 0.5 * rnd(hv), (0.5 * rnd(hv)).to(bf), (1.0 + 0.2 * rnd(128)).to(bf),
+            rnd(3, conv), 0.02 * rnd(hv * 128 * 128))
+
+
+def _deltanet(s, layers):
     """Weights and states of the DeltaNet layers `layers` of the state's context."""
-    cfg = s.ctx.cfg
     for layer in layers:
-        rnd = lambda *n: torch.randn(*n, device="cuda", generator=s.gen)  # noqa: E731
-        s.ctx.set_linear_weights(layer, _bits(0.5 * rnd(cfg.conv_dim, cfg.conv_kernel_size)),
-                                 (0.5 * rnd(cfg.linear_num_v_heads)).cpu().numpy(), _bits(0.5 * rnd(cfg.linear_num_v_heads)),
-                                 _bits(1.0 + 0.2 * rnd(cfg.linear_value_dim)))
-        if not zero_state:
-            s.ctx.linear_state_import(layer, rnd(cfg.conv_kernel_size - 1, cfg.conv_dim).cpu().numpy(),
-                                      (0.02 * rnd(cfg.ssm_elems)).cpu().numpy())
+        conv_w, a_log, dt_bias, norm, history, state = _deltanet_layer(s)
+        s.ctx.set_linear_weights(layer, _bits(conv_w), a_log.cpu().numpy(), _bits(dt_bias), _bits(norm))
+        s.ctx.linear_state_import(layer, history.cpu().numpy(), state.cpu().numpy())
 
 
 def _deltanet_inputs(s, layers, tokens):
-    cfg = s.ctx.cfg
-    n = layers * tokens
-    return (s.randn(n, cfg.conv_dim), s.randn(n, cfg.v_total), s.randn(n, cfg.linear_num_v_heads),
-            s.randn(n, cfg.linear_num_v_heads), s.empty(n, cfg.v_total))
+    hv, n = s.case["hv"], layers * tokens
+    return (s.randn(n, (2 * s.case["hk"] + hv) * 128), s.randn(n, hv * 128), s.randn(n, hv), s.randn(n, hv), s.empty(n, hv * 128))
+
+
+def _weights(s, out_dim, in_dim):
+    """4-bit weights: nibbles of all values, group scales and biases (bf16) that give weights of about 1 / sqrt(in_dim)."""
+    w = torch.randint(-2 ** 31, 2 ** 31, (out_dim, in_dim // 8), device="cuda", generator=s.gen, dtype=torch.int64).to(torch.int32)
+    scale = 0.2 / math.sqrt(in_dim) * (0.5 + torch.rand(out_dim, in_dim // 64, device="cuda", generator=s.gen))
+    return w, scale.to(torch.bfloat16), (-7.5 * scale).to(torch.bfloat16)
 
 
 def _projection(s, out_dim, in_dim, x, out):
-    """A spec of one 4-bit product: nibbles of all values, scales that give weights of about 1 / sqrt(in_dim)."""
-    w = torch.randint(-2 ** 31, 2 ** 31, (out_dim, in_dim // 8), device="cuda", generator=s.gen, dtype=torch.int64).to(torch.int32)
-    scale = 0.2 / math.sqrt(in_dim) * (0.5 + torch.rand(out_dim, in_dim // 64, device="cuda", generator=s.gen))
-    bias = (-7.5 * scale).to(torch.bfloat16)
-    scale = scale.to(torch.bfloat16)
+    """A spec of one 4-bit product."""
+    w, scale, bias = _weights(s, out_dim, in_dim)
     if s.case["tiled"]:
         t = torch.empty(int(s.lib.mfa_matvec_tiled_words(out_dim, in_dim)), device="cuda", dtype=torch.int32)
         _check(s.lib.mfa_matvec_tile_weights_dev(s.ctx.h, out_dim, in_dim, w.data_ptr(), scale.data_ptr(), bias.data_ptr(),
@@ -299,6 +316,122 @@ def run(s):
     for a in s.args:
         _check(call(*a))
     return s.out
+
+
+# ---- the same outputs in 64 bits ------------------------------------------------------------------------------------
+# The inputs are drawn again, in prepare's order.  A cache holds keys and values in its own type, so appended rows are
+# rounded to it here too; all else is float64.
+
+def _rotate(x, pos):
+    """Rotation of the first quarter of the channels of [tokens, heads, d] at positions pos (base 1e7)."""
+    half = x.shape[2] // 8
+    angle = pos.double()[:, None] * 1e7 ** (-torch.arange(half, device="cuda", dtype=torch.float64) / half)
+    cos, sin = angle.cos()[:, None], angle.sin()[:, None]
+    a, b = x[..., :half], x[..., half:2 * half]
+    return torch.cat([a * cos - b * sin, b * cos + a * sin, x[..., 2 * half:]], 2)
+
+
+def _rms(x, eps=1e-6):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + eps)
+
+
+def _attend(q, k, v, gate, length):
+    """Causal attention of tokens [t, hq, d] at positions length .. over keys and values [length + t, hkv, d]."""
+    t, hq, d = q.shape
+    hpk, out = hq // k.shape[1], torch.empty_like(q)
+    hidden = torch.arange(k.shape[0], device="cuda")[None, :] > length + torch.arange(t, device="cuda")[:, None]
+    for h in range(hq):
+        scores = q[:, h] @ k[:, h // hpk].T / math.sqrt(d)
+        out[:, h] = scores.masked_fill_(hidden, -math.inf).softmax(1) @ v[:, h // hpk]
+    return (out * gate.sigmoid()).reshape(t, hq * d)
+
+
+def _exact_layers(s, cached, qp, k, v):
+    """Attention layers from the raw projections: [layers, tokens, hq * d]."""
+    c, kept = s.case, torch.bfloat16 if s.case["bf16"] else torch.float32
+    t, outs = qp.shape[1], []
+    for layer, (norm, kv) in enumerate(cached):
+        pos, norm = c["length"] + torch.arange(t, device="cuda"), norm.double()
+        split = qp[layer].double().view(t, c["hq"], 2, c["d"])
+        q = _rotate(_rms(split[:, :, 0]) * norm[0], pos)
+        rows = (_rotate(_rms(k[layer].double().view(t, c["hkv"], c["d"])) * norm[1], pos), v[layer].view(t, c["hkv"], c["d"]))
+        keys, values = (torch.cat(([kv[i].double().view(-1, c["hkv"], c["d"])] if kv is not None else []) + [r.to(kept).double()])
+                        for i, r in enumerate(rows))
+        outs.append(_attend(q, keys, values, split[:, :, 1], c["length"]))
+    return torch.stack(outs)
+
+
+def _exact_deltanet(s, layers, *chunks):
+    """Chunks of inputs, one after the other, through DeltaNet layers `layers` = [_deltanet_layer(s), ...] together:
+    outputs [layers * tokens, hv * 128] of each chunk."""
+    n, hk, hv = len(layers), s.case["hk"], s.case["hv"]
+    conv_w, a_log, dt_bias, norm, history, state = (torch.stack([x[i].double() for x in layers]) for i in range(6))
+    state, outs = state.view(n, hv, 128, 128), []   # [layer, head, value channel, key channel]
+    for qkv, z, alpha, beta, _ in chunks:
+        t = qkv.shape[0] // n
+        seen = torch.cat([history, qkv.double().view(n, t, -1)], 1)
+        history = seen[:, -3:]
+        y = sum(seen[:, i:i + t] * conv_w[:, None, :, i] for i in range(4))
+        y = y * y.sigmoid()
+        q, k = (_rms(y[..., i * hk * 128:(i + 1) * hk * 128].view(n, t, hk, 128)).repeat_interleave(hv // hk, 2) for i in range(2))
+        q, k, v = q / 128.0, k / math.sqrt(128.0), y[..., 2 * hk * 128:].view(n, t, hv, 128)
+        keep = (-a_log.exp()[:, None] * torch.log1p((alpha.double().view(n, t, hv) + dt_bias[:, None]).exp())).exp()
+        rate = beta.double().view(n, t, hv).sigmoid()
+        o = torch.empty_like(v)
+        for i in range(t):
+            state = state * keep[:, i, :, None, None]
+            off = rate[:, i, :, None] * (v[:, i] - (state * k[:, i, :, None]).sum(-1))
+            state = state + off[..., None] * k[:, i, :, None]
+            o[:, i] = (state * q[:, i, :, None]).sum(-1)
+        z = z.double().view(n, t, hv, 128)
+        outs.append((_rms(o) * norm[:, None, None] * z * z.sigmoid()).reshape(n * t, hv * 128))
+    return outs
+
+
+def _exact_weights(s, out_dim, in_dim):
+    w, scale, bias = _weights(s, out_dim, in_dim)
+    nibbles = torch.stack([(w >> (4 * i)) & 15 for i in range(8)], -1).view(out_dim, in_dim // 64, 64)
+    return (nibbles.double() * scale.double()[..., None] + bias.double()[..., None]).view(out_dim, in_dim)
+
+
+def exact(case, seed):
+    s = _State(case, seed)
+    kind, n = case["kind"], case["layers"]
+    if kind in ("step", "decode", "prompt_attn"):
+        qd, kd, t = case["hq"] * case["d"], case["hkv"] * case["d"], case.get("tokens", 1)
+        cached = [_attention_layer(s) for _ in range(n)]
+        if kind != "decode":
+            return _exact_layers(s, cached, s.randn(n, t, 2 * qd), s.randn(n, t, kd), s.randn(n, t, kd))
+        return _exact_decode(s, cached, s.randn(n, qd), s.randn(n, qd))
+    if kind in ("gdn_step", "prompt_gdn"):
+        layers = [_deltanet_layer(s) for _ in range(n)]
+        chunks = [_deltanet_inputs(s, n, case.get("tokens", 1))]
+        if kind == "gdn_step":
+            return _exact_deltanet(s, layers, *chunks)[0]
+        return tuple(_exact_deltanet(s, layers, *chunks, _deltanet_inputs(s, n, 1)))
+    if kind == "sweep":
+        full, qd = n // 4, case["hq"] * case["d"]
+        cached = [_attention_layer(s) for _ in range(full)]
+        layers = [_deltanet_layer(s) for _ in range(n - full)]
+        out = _exact_decode(s, cached, s.randn(full, qd), s.randn(full, qd))
+        return out, _exact_deltanet(s, layers, _deltanet_inputs(s, n - full, 1))[0]
+    if kind == "latent":
+        h, length = case["heads"], case["length"]
+        q, qe, latent, rope = s.randn(n, h, 512), s.randn(n, h, 64), s.randn(n, length, 512), s.randn(n, length, 64)
+        return torch.stack([((q[i].double() @ latent[i].double().T + qe[i].double() @ rope[i].double().T) / math.sqrt(576.0))
+                            .softmax(1) @ latent[i].double() for i in range(n)])
+    qd, kd, hidden, out = case["hq"] * case["d"], case["hkv"] * case["d"], case["hidden"], []
+    for _ in range(n):
+        x, core = s.randn(hidden), s.randn(qd)
+        out.append([_exact_weights(s, m, hidden) @ x.double() for m in (2 * qd, kd, kd)] + [_exact_weights(s, hidden, qd) @ core.double()])
+    return out
+
+
+def _exact_decode(s, cached, q, gate):
+    c = s.case
+    heads = lambda x, n: x.double().view(-1, n, c["d"])  # noqa: E731
+    return torch.cat([_attend(heads(q[i], c["hq"]), heads(kv[0], c["hkv"]), heads(kv[1], c["hkv"]), heads(gate[i], c["hq"]),
+                              c["length"] - 1) for i, (_, kv) in enumerate(cached)])
 
 
 # ---- what a pass cannot do without ---------------------------------------------------------------------------------
