@@ -92,6 +92,7 @@ static void destroy(Ctx *c) {
     for (void *p : c->slabs)
         if (p) (void)hipFree(p);
     if (c->part_o) (void)hipFree(c->part_o);
+    if (c->chunk_part) (void)hipFree(c->chunk_part);
     if (c->part_ml) (void)hipFree(c->part_ml);
     if (c->stage) (void)hipFree(c->stage);
     if (c->gdn_scratch) (void)hipFree(c->gdn_scratch);
@@ -309,10 +310,33 @@ static int ensure_workspace(Ctx *c, int n_tok, int64_t kv_len, int layers = 1) {
                                   sdpa_workspace_ml_elems(Hq, Hkv, splits, n_tok));
 }
 
+// The plan of a prompt chunk on 32x32 tiles (not with a forced split count, which is the decode kernel's).  The first
+// plan that splits the cache allocates the workspace, whose size never changes; while the stream is being captured,
+// or without memory for it, the plan is one that needs none.
+static ChunkPlan chunk_plan(Ctx *c, int n_tok, int64_t kv_len) {
+    const mfa_config &g = c->cfg;
+    if (c->forced_splits || c->partial_only) return ChunkPlan{};
+    const auto plan = [&](size_t ws_elems) {
+        return sdpa_chunk_plan(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, kv_len, c->num_cus, ws_elems);
+    };
+    const ChunkPlan p = plan(kChunkPartElems);
+    if (p.splits <= 1 || c->chunk_part) return p;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return plan(0);
+    if (hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        c->chunk_part = nullptr;
+        return plan(0);
+    }
+    c->chunk_part_elems = kChunkPartElems;
+    return p;
+}
+
 // What sdpa_dev could still refuse for n_tok tokens over a cache of kv_len positions, checked
 // (and the split-K workspace grown) while the cache is as the caller left it.
 static int sdpa_prepare(Ctx *c, int n_tok, int64_t kv_len) {
     const mfa_config &g = c->cfg;
+    if (chunk_plan(c, n_tok, kv_len).applies) return MFA_OK;
     if (!c->forced_splits && !c->partial_only &&
         sdpa_prefill_applies(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, n_tok, kv_len, c->num_cus))
         return MFA_OK;   // one launch, no workspace
@@ -325,6 +349,10 @@ static int sdpa_prepare(Ctx *c, int n_tok, int64_t kv_len) {
 // n_tok tokens whose K/V rows are already in the cache (the last n_tok positions).
 static int sdpa_dev(Ctx *c, FullLayer *f, int n_tok, const float *q, const float *gate, float *out) {
     if (f->len <= 0) return fail(MFA_ERR_INVALID, "kv_len must be > 0 (got %d)", f->len);
+    const ChunkPlan p = chunk_plan(c, n_tok, f->len);
+    if (p.applies)
+        return launch_sdpa_chunk(c->stream, p, c->cfg.num_attn_heads, c->cfg.num_kv_heads, c->cfg.head_dim, n_tok, f->len,
+                                 c->plane_elems, f->k, f->v, q, gate, out, c->chunk_part, c->chunk_part_elems);
     if (!c->forced_splits && !c->partial_only &&
         sdpa_prefill_applies(c->cfg.kv_dtype, c->cfg.num_attn_heads, c->cfg.num_kv_heads, n_tok, f->len,
                              c->num_cus))
@@ -1214,6 +1242,8 @@ int mfa_debug_fill_workspace(mfa_ctx *ctx, uint32_t pattern) {
     if (!c) return fail(MFA_ERR_INVALID, "NULL context");
     if (c->part_o) MFA_HIP(hipMemsetD32Async((hipDeviceptr_t)c->part_o, (int)pattern, c->part_o_elems, c->stream));
     if (c->part_ml) MFA_HIP(hipMemsetD32Async((hipDeviceptr_t)c->part_ml, (int)pattern, c->part_ml_elems, c->stream));
+    if (c->chunk_part)
+        MFA_HIP(hipMemsetD32Async((hipDeviceptr_t)c->chunk_part, (int)pattern, c->chunk_part_elems + c->chunk_part_elems / 32, c->stream));
     MFA_HIP(hipStreamSynchronize(c->stream));
     return MFA_OK;
 }

@@ -163,6 +163,9 @@ struct Ctx {
     size_t part_o_elems = 0, part_ml_elems = 0;
     int32_t forced_splits = 0;
     int32_t partial_only = 0;
+    // partials of a split prompt chunk (sdpa_chunk.hip), allocated by the first one, of a size that never changes
+    float *chunk_part = nullptr;
+    size_t chunk_part_elems = 0;
     // scratch of the Gated-DeltaNet chunk kernels (grown on demand)
     float *gdn_scratch = nullptr;
     size_t gdn_scratch_elems = 0;
@@ -277,6 +280,21 @@ bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_l
 int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                         size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                         const float *gate, float *out, int num_cus);
+// sdpa_chunk.hip: the same for a bf16 cache on 32x32 matrix tiles; `splits` > 1 leaves partials in a
+// workspace and merges them in a second launch.
+struct ChunkPlan {
+    bool applies;     // false: the split-K decode kernel serves the chunk
+    int rw, ks;       // row waves (32 rows each) and wave sets of a workgroup
+    int nrt;          // row tiles of 32 * rw rows per kv head
+    int splits, bps;  // splits of the cache, blocks of 32 positions per split
+};
+// Workspace of a context: the partial rows of a split chunk are at most kChunkPartElems floats (33.5 MB, two
+// workgroups per CU of 128 rows x 128 channels), their maxima and sums a 32nd of that.
+static constexpr size_t kChunkPartElems = (size_t)512 * 128 * 128;
+ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, size_t ws_elems);
+int launch_sdpa_chunk(hipStream_t stream, const ChunkPlan &plan, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
+                      size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
+                      const float *gate, float *out, float *ws, size_t ws_elems);
 // Scatter `n_rows` row-major rows ([n_rows, Hkv*D], f32 or bf16 source) into the
 // tiled planes starting at position pos0.
 int launch_kv_scatter(hipStream_t stream, int kv_dtype, int src_is_bf16, int Hkv, int D,

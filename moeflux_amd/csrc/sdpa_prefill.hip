@@ -1,5 +1,5 @@
-// Causal attention of a prompt chunk over the tiled KV cache, for chunks large enough
-// that the query rows alone fill the machine.
+// Causal attention of a prompt chunk over a tiled f32 KV cache, for chunks large enough
+// that the query rows alone fill the machine (a bf16 cache: sdpa_chunk.hip).
 //
 // The reference has no batched prefill: eval_prompt is a token loop
 // (crates/moeflux/src/riir/mod.rs:1196-1214) whose every token runs the decode chain of
@@ -9,7 +9,7 @@
 // A workgroup is 4 waves; every wave owns RG groups of 16 query rows (rows of one kv
 // head: token-major, then the hpk query heads that share it) from start to end: its
 // query operands and its output tiles stay in registers and its soft-max needs no other
-// wave.  The workgroup walks the cache blocks (of V: 32 or 16 positions) that its rows may see; each
+// wave.  The workgroup walks the cache blocks (of V: 16 positions) that its rows may see; each
 // block's K and V (already in MFMA operand order in memory) is copied into LDS once by all 256 threads,
 // double buffered, and every wave takes its operands from there.  With RG = 2 an operand
 // read from LDS feeds two row groups.  Nothing is split along the cache, so the gated,
@@ -17,16 +17,6 @@
 #include "sdpa_wave.h"
 
 namespace mfa {
-
-// 1 / (1 + e^-x) from the hardware exp2 and reciprocal (each good to 1 ulp)
-__device__ inline float fast_sigmoid(float x) {
-    return __builtin_amdgcn_rcpf(1.0f + fast_exp2(-x * kLog2e));
-}
-
-// How far (in log2 units) a row's running maximum may rise above the reference its
-// exponentials are taken against before the accumulators are rescaled: probabilities
-// stay below 2^8, which costs nothing in f32 and spares most rescaling passes.
-static constexpr float kLazyRescale = 8.0f;
 
 // grid (workgroups of RW*RG row groups, Hkv), 64*RW*KS threads.  Waves RW*ks .. RW*ks+RW-1
 // form set ks: all sets serve the same RW*RG row groups, set ks taking blocks ks, ks + KS, ...
@@ -105,18 +95,14 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         fetch(std::integral_constant<int, 2>{}, 2);
         fetch(std::integral_constant<int, 3>{}, 3);
     }
-    // A bf16 cache's scores are products of the raw query, split into a bf16 high and low part, and are
-    // scaled as they leave the matrix core: a query that is exact in bf16 (what a bf16 model hands
-    // over) then has no low parts, and a wave all of whose rows are such leaves their products out.
     uint4 qr[RG][W::QREGS];
-    bool q_exact = true;
     int64_t limit[RG], limit_min[RG], limit_max[RG];
     bool full[RG];
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         const RowGroup rows{kvh, hg0 + r, hpk, Hq, n_tok, kv_len0};
         if (KS == 1 || ks == 0) {   // uniform over the wave
-            W::load_q_regs(qr[r], q, lane, rows, W::kScaleAfter ? 1.0f : qscale);
+            W::load_q_regs(qr[r], q, lane, rows, qscale);
             if constexpr (KS > 1) {
 #pragma unroll
                 for (int i = 0; i < W::QREGS; i++) s_q[(rw * RG + r) * W::QREGS + i][lane] = qr[r][i];
@@ -137,9 +123,6 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
                 for (int i = 0; i < W::QREGS; i++) qr[r][i] = s_q[(rw * RG + r) * W::QREGS + i][lane];
         }
     }
-#pragma unroll
-    for (int r = 0; r < RG; r++) q_exact = q_exact && W::q_low_parts_zero(qr[r]);
-    q_exact = __all(q_exact);
     int64_t wave_max = limit_max[0];
 #pragma unroll
     for (int r = 1; r < RG; r++) wave_max = limit_max[r] > wave_max ? limit_max[r] : wave_max;
@@ -162,13 +145,8 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         uint4 kreg[NLOAD];
 #pragma unroll
         for (int i = 0; i < NLOAD; i++) kreg[i] = cur[i * 64 + lane];
-        if (q_exact) {
 #pragma unroll
-            for (int r = 0; r < RG; r++) W::template scores_reg<true>(kreg, qr[r], sc[r]);
-        } else {
-#pragma unroll
-            for (int r = 0; r < RG; r++) W::template scores_reg<false>(kreg, qr[r], sc[r]);
-        }
+        for (int r = 0; r < RG; r++) W::scores_reg(kreg, qr[r], sc[r]);
     };
     auto finish = [&](int64_t b, const uint4 *cur, const typename W::Scores (&sc)[RG]) __attribute__((always_inline)) {
         uint4 p[RG][W::P_U4];
@@ -176,9 +154,6 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         for (int r = 0; r < RG; r++) {
             float x[NX];
             W::unpack(sc[r], x);
-            // kScaleAfter: x is unscaled; the scale (positive) enters the row maximum once and the
-            // exponentials' arguments as a fused multiply-add
-            const float xs = W::kScaleAfter ? qscale : 1.0f;
             if (!full[r] || (b + 1) * W::BLK > limit_min[r]) {  // a block some row must not see in full
 #pragma unroll
                 for (int e = 0; e < NX; e++)
@@ -188,7 +163,6 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
 #pragma unroll
             for (int e = 1; e < NX; e++) m_loc = fmaxf(m_loc, x[e]);
             m_loc = rows_max(m_loc);
-            if constexpr (W::kScaleAfter) m_loc *= xs;
             // m_loc > -inf + 8 is false while the row has seen nothing, so m_ref stays
             // -inf; the exponent's reference is then 0 and every probability is 0.
             const bool move = m_loc > m_ref[r] + kLazyRescale;
@@ -201,7 +175,7 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
             float e[NX], psum = 0.f;
 #pragma unroll
             for (int i = 0; i < NX; i++) {
-                e[i] = fast_exp2(W::kScaleAfter ? fmaf(x[i], xs, -ref) : x[i] - ref);  // 0 for masked positions
+                e[i] = fast_exp2(x[i] - ref);  // 0 for masked positions
                 psum += e[i];
             }
             l_run[r] = l_run[r] * alpha + psum;
@@ -361,9 +335,8 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
 // row-group path: either the cache is short (nothing to gain from splitting it) or the
 // rows alone give at least half the CUs a workgroup.
 bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_len, int num_cus) {
-    if (n_tok < 2) return false;
-    const int blk = kv_dtype == MFA_KV_BF16 ? 32 : 16;
-    const int64_t nblk = (kv_len + blk - 1) / blk;
+    if (kv_dtype != MFA_KV_F32 || n_tok < 2) return false;
+    const int64_t nblk = (kv_len + 15) / 16;
     const int64_t nhg = ((int64_t)n_tok * (Hq / Hkv) + 15) / 16;
     const int64_t nwg = (nhg + 3) / 4 * Hkv;
     return nblk <= 64 || nwg >= num_cus / 2;
@@ -372,7 +345,7 @@ bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_l
 int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                         size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                         const float *gate, float *out, int num_cus) {
-    if (!sdpa_shape_supported(kv_dtype, D))
+    if (kv_dtype != MFA_KV_F32 || !sdpa_shape_supported(kv_dtype, D))
         return fail(MFA_ERR_SHAPE, "sdpa: head_dim %d / kv dtype %d not supported", D, kv_dtype);
     if (n_tok <= 0 || kv_len < n_tok)
         return fail(MFA_ERR_INVALID, "sdpa: kv_len must be > 0 (got %lld for %d tokens)", (long long)kv_len, n_tok);
@@ -393,23 +366,20 @@ int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     const int64_t kv_len0 = kv_len - n_tok;
     const dim3 grid((unsigned)nwg, Hkv);
-#define MFA_LAUNCH(KV, DD, RGG, DEP, KSS, RWW)                                                                 \
-    hipLaunchKernelGGL((sdpa_prefill_kernel<KV, DD, RGG, DEP, KSS, RWW>), grid, dim3(64 * RWW * KSS), 0, stream, \
-                       (const KV *)k_tiled, (const KV *)v_tiled, plane_elems, q, gate, hpk, Hq, n_tok, kv_len0,   \
+#define MFA_LAUNCH(DD, RGG, DEP, KSS, RWW)                                                                          \
+    hipLaunchKernelGGL((sdpa_prefill_kernel<float, DD, RGG, DEP, KSS, RWW>), grid, dim3(64 * RWW * KSS), 0, stream, \
+                       (const float *)k_tiled, (const float *)v_tiled, plane_elems, q, gate, hpk, Hq, n_tok, kv_len0, \
                        qscale, out)
-#define MFA_LAUNCH_D(KV)                                         \
-    if (D == 256) MFA_LAUNCH(KV, 256, 1, 2, 1, 4);               \
-    else if (D == 128) {                                         \
-        if (big) MFA_LAUNCH(KV, 128, 2, 2, 1, 4);                \
-        else if (small) MFA_LAUNCH(KV, 128, 1, 4, 2, 4);         \
-        else MFA_LAUNCH(KV, 128, 1, 4, 1, 4);                    \
-    } else {                                                     \
-        if (big) MFA_LAUNCH(KV, 64, 2, 2, 1, 4);                 \
-        else if (small) MFA_LAUNCH(KV, 64, 1, 4, 2, 4);          \
-        else MFA_LAUNCH(KV, 64, 1, 4, 1, 4);                     \
+    if (D == 256) MFA_LAUNCH(256, 1, 2, 1, 4);
+    else if (D == 128) {
+        if (big) MFA_LAUNCH(128, 2, 2, 1, 4);
+        else if (small) MFA_LAUNCH(128, 1, 4, 2, 4);
+        else MFA_LAUNCH(128, 1, 4, 1, 4);
+    } else {
+        if (big) MFA_LAUNCH(64, 2, 2, 1, 4);
+        else if (small) MFA_LAUNCH(64, 1, 4, 2, 4);
+        else MFA_LAUNCH(64, 1, 4, 1, 4);
     }
-    if (kv_dtype == MFA_KV_BF16) { MFA_LAUNCH_D(uint16_t) } else { MFA_LAUNCH_D(float) }
-#undef MFA_LAUNCH_D
 #undef MFA_LAUNCH
     MFA_HIP(hipGetLastError());
     return MFA_OK;

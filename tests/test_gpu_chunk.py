@@ -1,0 +1,62 @@
+"""The prompt-chunk attention kernel over bf16 caches: tile edges, splits of the cache, their workspace."""
+import numpy as np
+import pytest
+
+from tests.util import rel_err, rel_err_rows
+
+pytestmark = pytest.mark.gpu
+
+# The query and the probabilities enter as two bf16 parts: 2^-17 of an operand each, on scores of a few units.
+TOL = 1e-4
+
+
+def _inputs(oracle, Hq, Hkv, d, T, L0, seed):
+    rng = np.random.default_rng(seed)
+    k, v = (oracle.bf16_to_f32(oracle.f32_to_bf16(rng.standard_normal((L0 + T, Hkv * d)).astype(np.float32))) for _ in range(2))
+    q = rng.standard_normal((T, Hq * d)).astype(np.float32)
+    return q, rng.standard_normal((T, Hq * d)).astype(np.float32), k, v
+
+
+def _ctx(mfa, Hq, Hkv, d, cap):
+    from moeflux_amd import Config
+    return mfa.Ctx(Config(num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d,
+                          kv_capacity=cap, kv_dtype=1))
+
+
+# Rows of a workgroup are 128 or 64, of a wave 32, blocks 32 positions, chunks of K 64; long caches are split.
+@pytest.mark.parametrize("Hq,Hkv,d,T,L0", [
+    (8, 2, 128, 8, 0), (8, 2, 128, 9, 23), (4, 1, 64, 31, 1), (4, 1, 256, 33, 31),     # a row either side of a tile
+    (16, 1, 128, 2, 62), (16, 1, 256, 3, 61), (6, 2, 64, 65, 64),                      # positions either side of a chunk of K
+    (32, 4, 128, 40, 2500), (16, 2, 256, 50, 1990), (16, 2, 256, 130, 600), (16, 4, 64, 70, 2047),   # splits
+    (3, 3, 128, 129, 4000), (24, 1, 256, 11, 2303),
+])
+def test_chunk_against_the_oracle(mfa, oracle, Hq, Hkv, d, T, L0):
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, T + L0)
+    ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, q, g, k, v).reshape(T, Hq * d)
+    with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+        if L0:
+            c.kv_import(0, k[:L0], v[:L0])
+        out = c.prefill_attn(0, q, g, k[L0:], v[L0:])
+        # once more over a workspace of NaN: a split whose positions a tile cannot see leaves its part unwritten
+        c.memory_seq_rm(L0)
+        if L0:
+            c.kv_import(0, k[:L0], v[:L0])
+        assert c.lib.mfa_debug_fill_workspace(c.h, 0x7FC00000) == 0
+        again = c.prefill_attn(0, q, g, k[L0:], v[L0:])
+    assert rel_err(out, ref) <= TOL
+    assert rel_err_rows(out, ref, d) <= 5 * TOL
+    assert np.array_equal(out, again)
+
+
+def test_chunk_split_with_peaked_scores(mfa, oracle):
+    """Scores of +-130: the running maximum rises by far more than the lazy rescaling's 2^8, in some splits only."""
+    Hq, Hkv, d, T, L0 = 16, 2, 256, 130, 600
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, 3)
+    q *= 8.0
+    k[::97] *= 4.0
+    ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, q, g, k, v).reshape(T, Hq * d)
+    with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+        c.kv_import(0, k[:L0], v[:L0])
+        out = c.prefill_attn(0, q, g, k[L0:], v[L0:])
+    # a score s carries up to 2^-17 |s| from the query's two parts: 1e-3 of a probability at |s| = 130
+    assert rel_err(out, ref) <= 2e-3
