@@ -352,7 +352,8 @@ static int sdpa_dev(Ctx *c, FullLayer *f, int n_tok, const float *q, const float
     const ChunkPlan p = chunk_plan(c, n_tok, f->len);
     if (p.applies)
         return launch_sdpa_chunk(c->stream, p, c->cfg.num_attn_heads, c->cfg.num_kv_heads, c->cfg.head_dim, n_tok, f->len,
-                                 c->plane_elems, f->k, f->v, q, gate, out, c->chunk_part, c->chunk_part_elems);
+                                 c->plane_elems, f->k, f->v, ChunkQuery{q, gate, c->cfg.head_dim}, out, c->chunk_part,
+                                 c->chunk_part_elems);
     if (!c->forced_splits && !c->partial_only &&
         sdpa_prefill_applies(c->cfg.kv_dtype, c->cfg.num_attn_heads, c->cfg.num_kv_heads, n_tok, f->len,
                              c->num_cus))
@@ -743,26 +744,44 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
     if ((int64_t)f->len + T > c->cfg.kv_capacity)
         return fail(MFA_ERR_OVERFLOW, "kv cache overflow: len %d + %d > capacity %d", f->len, T, c->cfg.kv_capacity);
     const size_t qd = (size_t)c->q_dim() * T;
-    if (2 * qd > c->qg_chunk_elems) {
+    MFA_TRY(sdpa_prepare(c, T, (int64_t)f->len + T));
+    // The chunk kernel takes the query and its gate from the projection itself (unless the caller's result would
+    // overwrite rows it has yet to read): all the launch ahead of it leaves is the tokens' rotation table.
+    const ChunkPlan plan = chunk_plan(c, T, (int64_t)f->len + T);
+    const bool raw = plan.applies && sdpa_chunk_takes_raw(c->cfg.head_dim, c->rotary_dim) &&
+                     (out_dev + qd <= q_proj_out_dev || q_proj_out_dev + 2 * qd <= out_dev);
+    const size_t need = raw ? (size_t)T * c->rotary_dim : 2 * qd;
+    if (need > c->qg_chunk_elems) {
         MFA_HIP(hipStreamSynchronize(c->stream));
         if (c->qg_chunk) MFA_HIP(hipFree(c->qg_chunk));
         c->qg_chunk = nullptr;
         c->qg_chunk_elems = 0;
-        MFA_HIP(hipMalloc((void **)&c->qg_chunk, 2 * qd * sizeof(float)));
-        c->qg_chunk_elems = 2 * qd;
+        MFA_HIP(hipMalloc((void **)&c->qg_chunk, need * sizeof(float)));
+        c->qg_chunk_elems = need;
     }
-    MFA_TRY(sdpa_prepare(c, T, (int64_t)f->len + T));
     // the whole chunk is normed, rotated and appended, then one causal pass: row t sees positions [0, len0 + t]
     const int32_t len0 = f->len;
-    const int kSeg = 32768;   // tokens per prologue launch (the grid's second dimension holds 65535)
     int rc = MFA_OK;
-    for (int32_t off = 0; off < T && rc == MFA_OK; off += kSeg) {
-        const int32_t n = T - off < kSeg ? T - off : kSeg;
-        rc = prologue_dev(c, f, pos0 + off, q_proj_out_dev + (size_t)off * 2 * c->q_dim(),
-                          k_dev + (size_t)off * c->kv_dim(), v_dev + (size_t)off * c->kv_dim(),
-                          c->qg_chunk + (size_t)off * c->q_dim(), c->qg_chunk + qd + (size_t)off * c->q_dim(), n);
+    if (raw) {
+        const int D = c->cfg.head_dim;
+        rc = launch_attn_prologue_kv(c->stream, c->cfg.kv_dtype, c->cfg.num_kv_heads, D, c->rotary_dim, c->cfg.rms_norm_eps, T, pos0,
+                                     len0, c->plane_elems, f->k_norm, c->inv_freq, k_dev, v_dev, (float2 *)c->qg_chunk, f->k, f->v);
+        if (rc == MFA_OK) {
+            f->len += T;
+            const ChunkQuery in{q_proj_out_dev, q_proj_out_dev + D, 2 * D, f->q_norm, (const float2 *)c->qg_chunk, c->cfg.rms_norm_eps};
+            rc = launch_sdpa_chunk(c->stream, plan, c->cfg.num_attn_heads, c->cfg.num_kv_heads, D, T, f->len, c->plane_elems, f->k,
+                                   f->v, in, out_dev, c->chunk_part, c->chunk_part_elems);
+        }
+    } else {
+        const int kSeg = 32768;   // tokens per prologue launch (the grid's second dimension holds 65535)
+        for (int32_t off = 0; off < T && rc == MFA_OK; off += kSeg) {
+            const int32_t n = T - off < kSeg ? T - off : kSeg;
+            rc = prologue_dev(c, f, pos0 + off, q_proj_out_dev + (size_t)off * 2 * c->q_dim(),
+                              k_dev + (size_t)off * c->kv_dim(), v_dev + (size_t)off * c->kv_dim(),
+                              c->qg_chunk + (size_t)off * c->q_dim(), c->qg_chunk + qd + (size_t)off * c->q_dim(), n);
+        }
+        if (rc == MFA_OK) rc = sdpa_dev(c, f, T, c->qg_chunk, c->qg_chunk + qd, out_dev);
     }
-    if (rc == MFA_OK) rc = sdpa_dev(c, f, T, c->qg_chunk, c->qg_chunk + qd, out_dev);
     if (rc != MFA_OK) rollback_append(c, f, len0);   // a launch refused after all: the cache is as before the call
     return rc;
 }

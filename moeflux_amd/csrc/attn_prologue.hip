@@ -144,6 +144,90 @@ __global__ void attn_prologue_kernel(int Hq, int Hkv, int D, int rotary_dim, flo
     else k_tiled[(size_t)h * plane_elems + KvTile<KV>::k_off(cache_pos, x, D)] = to_kv<KV>(r);
 }
 
+// The k and v heads of a chunk's tokens on their own, D / EPS lanes per head as above, several tokens to a workgroup
+// (a token's Hkv heads fill a quarter of one at head_dim 128), and the tokens' (cos, sin) into a table for the
+// attention launch.  With the q heads the chunk's prologue moved 8 D bytes more per q head in and out: 512 tokens of 32 + 2 x 4
+// heads of 128 channels took 12 us, of which the q heads' copy was two thirds.
+template <typename KV, int D>
+__global__ __launch_bounds__(256) void attn_prologue_kv_kernel(
+    int Hkv, int rotary_dim, float eps, int n_tok, int tpw, int32_t pos, int64_t cache_pos, size_t plane_elems,
+    const uint16_t *__restrict__ k_norm, const float *__restrict__ inv_freq, const float *__restrict__ k_in,
+    const float *__restrict__ v_in, float2 *__restrict__ table, KV *__restrict__ k_tiled, KV *__restrict__ v_tiled) {
+    constexpr int EPS = sizeof(KV) == 2 ? 8 : 4;
+    constexpr int LPH = D / EPS, HEADS = 256 / LPH;   // heads of a workgroup's pass
+    const int half = rotary_dim >> 1, t0 = blockIdx.x * tpw;
+    const int nt = n_tok - t0 < tpw ? n_tok - t0 : tpw;
+    extern __shared__ float2 s_table[];   // [tpw][half]
+    const int j = threadIdx.x % LPH, c0 = EPS * j, n = nt * Hkv;
+    // a head's rows; the first pass's are asked for ahead of the table, whose sines take as long as they do to arrive
+    float x[EPS], v[EPS];
+    auto rows_at = [&](int b) { return ((size_t)(t0 + b / Hkv) * Hkv + b % Hkv) * D + c0; };
+    auto request = [&](int b) {
+        const size_t at = rows_at(b < n ? b : 0);
+#pragma unroll
+        for (int e = 0; e < EPS; e += 4) {
+            const float4 p = load_f4(k_in + at + e), q = load_f4(v_in + at + e);
+            x[e] = p.x; x[e + 1] = p.y; x[e + 2] = p.z; x[e + 3] = p.w;
+            v[e] = q.x; v[e + 1] = q.y; v[e + 2] = q.z; v[e + 3] = q.w;
+        }
+    };
+    float w[EPS];
+#pragma unroll
+    for (int e = 0; e < EPS; e++) w[e] = bf16_bits_to_f32(k_norm[c0 + e]);
+    request(threadIdx.x / LPH);
+    for (int i = threadIdx.x; i < nt * half; i += 256) {
+        const float2 cs = head_cos_sin((float)(pos + t0 + i / half) * inv_freq[i % half]);
+        s_table[i] = cs;
+        table[(size_t)t0 * half + i] = cs;
+    }
+    __syncthreads();
+    for (int base = 0; base < n; base += HEADS) {   // uniform: the norm's sums run over whole lane groups
+        const int b = base + threadIdx.x / LPH;
+        const bool live = b < n;
+        const int tok = live ? b / Hkv : 0, h = live ? b % Hkv : 0;
+        if (base > 0) request(b);
+        HeadRotor<EPS, D> hr;
+        hr.init(j, rotary_dim, s_table + tok * half);
+        hr.apply(x, w, eps);
+        if (live) {
+            KV *kp = k_tiled + (size_t)h * plane_elems, *vp = v_tiled + (size_t)h * plane_elems;
+            const int64_t p = cache_pos + t0 + tok;
+            // a lane's EPS channels are one operand slot of the key's tile: 16 bytes side by side
+            typedef KV __attribute__((ext_vector_type(EPS))) slot;
+            slot kv;
+#pragma unroll
+            for (int e = 0; e < EPS; e++) {
+                kv[e] = to_kv<KV>(x[e]);
+                vp[KvTile<KV>::v_off(p, c0 + e, D)] = to_kv<KV>(v[e]);
+            }
+            *reinterpret_cast<slot *>(kp + KvTile<KV>::k_off(p, c0, D)) = kv;
+        }
+    }
+}
+
+int launch_attn_prologue_kv(hipStream_t s, int kv_dtype, int Hkv, int D, int rotary_dim, float eps, int n_tok, int32_t pos,
+                            int64_t cache_pos, size_t plane_elems, const uint16_t *k_norm, const float *inv_freq,
+                            const float *k_in, const float *v_in, float2 *table, void *k_tiled, void *v_tiled) {
+    if (kv_dtype != MFA_KV_BF16 || (D != 128 && D != 256) || !head_rotor_applies(kv_dtype, D, rotary_dim))
+        return fail(MFA_ERR_SHAPE, "attention prologue: shape not supported by the k/v form");
+    if (pos < 0 || n_tok <= 0 || (int64_t)pos + n_tok - 1 > INT32_MAX)
+        return fail(MFA_ERR_INVALID, "attention prologue: positions %d .. %lld out of range", pos, (long long)pos + n_tok - 1);
+    // tokens of a workgroup: as many as fill its lanes once
+    const int heads = 256 / (D / 8);
+    int tpw = heads / Hkv;
+    if (tpw < 1) tpw = 1;
+    const dim3 grid((n_tok + tpw - 1) / tpw);
+    const size_t lds = (size_t)tpw * (rotary_dim / 2) * sizeof(float2);
+    if (D == 128)
+        hipLaunchKernelGGL((attn_prologue_kv_kernel<uint16_t, 128>), grid, dim3(256), lds, s, Hkv, rotary_dim, eps, n_tok, tpw, pos,
+                           cache_pos, plane_elems, k_norm, inv_freq, k_in, v_in, table, (uint16_t *)k_tiled, (uint16_t *)v_tiled);
+    else
+        hipLaunchKernelGGL((attn_prologue_kv_kernel<uint16_t, 256>), grid, dim3(256), lds, s, Hkv, rotary_dim, eps, n_tok, tpw, pos,
+                           cache_pos, plane_elems, k_norm, inv_freq, k_in, v_in, table, (uint16_t *)k_tiled, (uint16_t *)v_tiled);
+    MFA_HIP(hipGetLastError());
+    return MFA_OK;
+}
+
 int launch_attn_prologue(hipStream_t s, int kv_dtype, int Hq, int Hkv, int D, int rotary_dim, float eps, int n_tok,
                          int32_t pos, int64_t cache_pos, size_t plane_elems, const uint16_t *q_norm,
                          const uint16_t *k_norm, const float *inv_freq, const float *q_proj, const float *k_in,

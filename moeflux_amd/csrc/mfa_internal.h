@@ -274,6 +274,11 @@ int launch_attn_prologue(hipStream_t s, int kv_dtype, int Hq, int Hkv, int D, in
                          int32_t pos, int64_t cache_pos, size_t plane_elems, const uint16_t *q_norm,
                          const uint16_t *k_norm, const float *inv_freq, const float *q_proj, const float *k_in,
                          const float *v_in, float *q_out, float *gate_out, void *k_tiled, void *v_tiled);
+// The k and v heads alone, and the tokens' rotations table [n_tok, rotary_dim / 2] of (cos, sin) for a launch that norms
+// and rotates the query itself (shapes of head_rotor_applies).
+int launch_attn_prologue_kv(hipStream_t s, int kv_dtype, int Hkv, int D, int rotary_dim, float eps, int n_tok, int32_t pos,
+                            int64_t cache_pos, size_t plane_elems, const uint16_t *k_norm, const float *inv_freq,
+                            const float *k_in, const float *v_in, float2 *table, void *k_tiled, void *v_tiled);
 // sdpa_prefill.hip: the same contract for a chunk whose rows fill the machine without
 // splitting the cache (no workspace, one launch).
 bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_len, int num_cus);
@@ -291,10 +296,20 @@ struct ChunkPlan {
 // Workspace of a context: the partial rows of a split chunk are at most kChunkPartElems floats (33.5 MB, two
 // workgroups per CU of 128 rows x 128 channels), their maxima and sums a 32nd of that.
 static constexpr size_t kChunkPartElems = (size_t)512 * 128 * 128;
+// The chunk's query and gate rows, `stride` floats from one (token, head) to the next.  With q_norm they are the raw q
+// projection [n_tok, Hq, 2, D], to be normed and rotated with table [n_tok, D / 8] of (cos, sin).
+struct ChunkQuery {
+    const float *q, *gate;
+    int stride;
+    const uint16_t *q_norm = nullptr;
+    const float2 *table = nullptr;
+    float eps = 0.f;
+};
+bool sdpa_chunk_takes_raw(int D, int rotary_dim);
 ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, size_t ws_elems);
 int launch_sdpa_chunk(hipStream_t stream, const ChunkPlan &plan, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
-                      size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
-                      const float *gate, float *out, float *ws, size_t ws_elems);
+                      size_t plane_elems, const void *k_tiled, const void *v_tiled, const ChunkQuery &in, float *out,
+                      float *ws, size_t ws_elems);
 // Scatter `n_rows` row-major rows ([n_rows, Hkv*D], f32 or bf16 source) into the
 // tiled planes starting at position pos0.
 int launch_kv_scatter(hipStream_t stream, int kv_dtype, int src_is_bf16, int Hkv, int D,

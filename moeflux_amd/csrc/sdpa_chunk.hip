@@ -33,7 +33,7 @@ static constexpr int kMaxChunkSplits = 16;
 struct ChunkArgs {
     const uint16_t *k, *v;
     size_t plane_elems;
-    const float *q, *gate;
+    ChunkQuery in;
     int hpk, Hq, n_tok;
     int64_t kv_len0;
     float qscale;
@@ -45,7 +45,60 @@ struct ChunkArgs {
     int contiguous;      // 1: an XCD takes whole (kv head, split) pairs
 };
 
-template <int D, int RW, int KS, int G, bool SPLIT>
+// The query rows from their raw projection: RMS norm over the head and the rotation of its first quarter
+// (full_attn_forward.rs:238-323), the arithmetic of attn_prologue.h.  Lane (n, h) holds channels 16 s + 8 h .. + 3 of
+// its row in x[s] and the next four in y[s], lane (n, 1 - h) the rest of the row; the rotated quarter's pairs
+// (i, i + D / 8) are D / 128 k-steps apart and so a lane's own.
+template <int D> struct RowNorm {
+    static constexpr int NS = D / 16, ROT = D / 128;   // k-steps of the row, and of one half of its rotated channels
+    uint4 w[NS], cs[ROT][4];
+
+    // asked for with the rows themselves: behind them they were 3 us of a 20 us launch
+    __device__ __attribute__((always_inline)) inline void request(const ChunkQuery &in, int token, int h) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) w[s] = vec_load((const uint4 *)(in.q_norm + 16 * s + 8 * h));
+#pragma unroll
+        for (int s = 0; s < ROT; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) cs[s][i] = vec_load((const uint4 *)(in.table + ((size_t)token * (D / 8) + 16 * s + 8 * h + 2 * i)));
+    }
+    __device__ __attribute__((always_inline)) inline void apply(uint4 (&x)[NS], uint4 (&y)[NS], float eps) const {
+        auto at = [&](int s, int e) -> unsigned & { return e < 4 ? (e == 0 ? x[s].x : e == 1 ? x[s].y : e == 2 ? x[s].z : x[s].w)
+                                                                 : (e == 4 ? y[s].x : e == 5 ? y[s].y : e == 6 ? y[s].z : y[s].w); };
+        auto part = [](const uint4 &u, int i) { return i == 0 ? u.x : i == 1 ? u.y : i == 2 ? u.z : u.w; };
+        float ss = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = __builtin_bit_cast(float, at(s, e));
+                ss += v * v;
+            }
+        float other = ss;
+        rows_swap32(ss, other);
+        ss += other;
+        const float inv_rms = 1.0f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const unsigned pair = part(w[s], e / 2);
+                const float wt = __builtin_bit_cast(float, e % 2 ? pair & 0xffff0000u : pair << 16);
+                at(s, e) = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, at(s, e)) * inv_rms * wt);
+            }
+#pragma unroll
+        for (int s = 0; s < ROT; s++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float c = __builtin_bit_cast(float, part(cs[s][e / 2], e % 2 * 2)), sn = __builtin_bit_cast(float, part(cs[s][e / 2], e % 2 * 2 + 1));
+                const float a = __builtin_bit_cast(float, at(s, e)), b = __builtin_bit_cast(float, at(s + ROT, e));
+                at(s, e) = __builtin_bit_cast(unsigned, a * c - b * sn);
+                at(s + ROT, e) = __builtin_bit_cast(unsigned, a * sn + b * c);
+            }
+    }
+};
+
+template <int D, int RW, int KS, int G, bool SPLIT, bool RAW>
 __global__ __launch_bounds__(64 * RW * KS, D == 256 ? 1 : 2) void sdpa_chunk_kernel(const ChunkArgs a) {
     constexpr int NS = D / 16;          // k-steps of the scores, 1 KiB pieces of a block's K and of its V
     constexpr int NT = D / 32;          // 32-wide output tiles
@@ -142,10 +195,12 @@ __global__ __launch_bounds__(64 * RW * KS, D == 256 ? 1 : 2) void sdpa_chunk_ker
     uint4 qh[NS], ql[NS];
     {
         uint4 raw[NT][4];
+        std::conditional_t<RAW, RowNorm<D>, int> norm;
+        if constexpr (RAW) norm.request(a.in, ok ? rr / a.hpk : 0, h);
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) raw[t][j] = vec_load((const uint4 *)(a.q + tr_q[j] * D + 32 * t + 4 * tr_chunk));
+            for (int j = 0; j < 4; j++) raw[t][j] = vec_load((const uint4 *)(a.in.q + tr_q[j] * a.in.stride + 32 * t + 4 * tr_chunk));
 #pragma unroll
         for (int g = 0; g < G; g++) request(g);
 #pragma unroll
@@ -154,13 +209,18 @@ __global__ __launch_bounds__(64 * RW * KS, D == 256 ? 1 : 2) void sdpa_chunk_ker
             for (int j = 0; j < 4; j++) tr[tr_at(tr_row + 8 * j, tr_chunk)] = raw[t][j];
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                const int s = 2 * t + u;
-                const float4 x = __builtin_bit_cast(float4, tr[tr_at(n, 4 * u + 2 * h)]), y = __builtin_bit_cast(float4, tr[tr_at(n, 4 * u + 2 * h + 1)]);
-                split_pair(x.x, x.y, qh[s].x, ql[s].x);
-                split_pair(x.z, x.w, qh[s].y, ql[s].y);
-                split_pair(y.x, y.y, qh[s].z, ql[s].z);
-                split_pair(y.z, y.w, qh[s].w, ql[s].w);
+                qh[2 * t + u] = tr[tr_at(n, 4 * u + 2 * h)];
+                ql[2 * t + u] = tr[tr_at(n, 4 * u + 2 * h + 1)];
             }
+        }
+        if constexpr (RAW) norm.apply(qh, ql, a.in.eps);
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const float4 x = __builtin_bit_cast(float4, qh[s]), y = __builtin_bit_cast(float4, ql[s]);
+            split_pair(x.x, x.y, qh[s].x, ql[s].x);
+            split_pair(x.z, x.w, qh[s].y, ql[s].y);
+            split_pair(y.x, y.y, qh[s].z, ql[s].z);
+            split_pair(y.z, y.w, qh[s].w, ql[s].w);
         }
         const unsigned keep = ok ? 0xffffffffu : 0u;   // a row past the chunk's last is all zero
 #pragma unroll
@@ -383,7 +443,7 @@ __global__ __launch_bounds__(64 * RW * KS, D == 256 ? 1 : 2) void sdpa_chunk_ker
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) gt[t][j] = vec_load((const uint4 *)(a.gate + tr_q[j] * D + 32 * t + 4 * tr_chunk));
+            for (int j = 0; j < 4; j++) gt[t][j] = vec_load((const uint4 *)(a.in.gate + tr_q[j] * a.in.stride + 32 * t + 4 * tr_chunk));
 #pragma unroll
         for (int t = 0; t < NT; t++) {
 #pragma unroll
@@ -431,8 +491,9 @@ __global__ __launch_bounds__(256) void sdpa_chunk_merge_kernel(const ChunkArgs a
     for (int j = 0; j < 4; j++) {
         const int r = wt * 32 + tr_row + 8 * j;
         ok[j] = r < nrows;
-        at[j] = (ok[j] ? (size_t)(r / a.hpk) * a.Hq + kvh * a.hpk + r % a.hpk : 0) * D + 32 * t + 4 * tr_chunk;
-        gt[j] = vec_load((const uint4 *)(a.gate + at[j]));
+        const size_t row = ok[j] ? (size_t)(r / a.hpk) * a.Hq + kvh * a.hpk + r % a.hpk : 0;
+        at[j] = row * D + 32 * t + 4 * tr_chunk;
+        gt[j] = vec_load((const uint4 *)(a.in.gate + row * a.in.stride + 32 * t + 4 * tr_chunk));
     }
     float M = neg_inf();
 #pragma unroll
@@ -477,10 +538,13 @@ __global__ __launch_bounds__(256) void sdpa_chunk_merge_kernel(const ChunkArgs a
     }
 }
 
+// Whether the kernel can norm and rotate the query rows itself (RowNorm).
+bool sdpa_chunk_takes_raw(int D, int rotary_dim) { return D >= 128 && rotary_dim * 4 == D; }
+
 // How a chunk is cut up: the shape of a workgroup and the splits of the cache of the smallest estimated cost, or no
 // plan at all where the split-K decode kernel (16-row groups, each streaming the cache by itself) is estimated
-// cheaper, which is where a chunk's rows are few and its cache is long.  The cost is the call's own time and twice the
-// time of the whole device that it takes: a chunk's layers follow each other, but other sequences run beside them
+// cheaper, which is where a chunk's rows are few and its cache is long.  The cost is the call's own time and one and a half
+// times the time of the whole device that it takes: a chunk's layers follow each other, but other sequences run beside them
 // (one estimate alone costs 7 to 12 % of the other over 38 chunks of 6 .. 1500 tokens behind 0 .. 12000 positions, the sum
 // 3 %).  Times in microseconds, fitted to launches measured over those chunks, 10 to 15 % off:
 //   workgroup  kFixed (launch, query, first block, epilogue) + blocks per wave set * kBlock; a CU that holds two
@@ -491,7 +555,7 @@ __global__ __launch_bounds__(256) void sdpa_chunk_merge_kernel(const ChunkArgs a
 ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, size_t ws_elems) {
     ChunkPlan best{};
     if (kv_dtype != MFA_KV_BF16 || n_tok < 2 || !sdpa_shape_supported(kv_dtype, D)) return best;
-    static constexpr double kFixed[2][3] = {{6.0, 6.5, 9.5}, {7.0, 7.6, 13.0}}, kBlock[2][3] = {{0.5, 0.8, 1.58}, {0.55, 0.85, 1.85}};
+    static constexpr double kFixed[2][3] = {{6.0, 9.0, 12.0}, {7.0, 9.0, 14.0}}, kBlock[2][3] = {{0.5, 0.8, 1.58}, {0.55, 0.85, 1.85}};
     static constexpr double kStream[3] = {0.007, 0.0108, 0.0175};
     static constexpr double kLaunch = 12.0, kEmpty = 2.5;   // of a workgroup's fixed time, what its CU is free in
     const int w = D == 64 ? 0 : D == 128 ? 1 : 2, slots = D <= 128 ? 2 : 1;
@@ -518,8 +582,8 @@ ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64
                 t += moved + kLaunch;
                 busy += moved;
             }
-            if (!best.applies || t + 2 * busy < best_cost) {
-                best_cost = t + 2 * busy;
+            if (!best.applies || t + 1.5 * busy < best_cost) {
+                best_cost = t + 1.5 * busy;
                 best = ChunkPlan{true, rw, ks, (int)nrt, (int)want, (int)bps};
             }
         }
@@ -531,36 +595,45 @@ ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64
         if (splits > nblk / 4) splits = nblk / 4;
         if (splits < 1) splits = 1;
         const double load = (double)(groups * splits) / num_cus, stream = (double)kv_len / (double)splits * kStream[w], merge = out_bytes / 8 * 6.9e-6;
-        if (3.0 + ceil(load) * stream + kLaunch + merge + 2 * (load * (stream + 1.0) + merge) < best_cost) return ChunkPlan{};
+        if (3.0 + ceil(load) * stream + kLaunch + merge + 1.5 * (load * (stream + 1.0) + merge) < best_cost) return ChunkPlan{};
     }
     return best;
 }
 
 int launch_sdpa_chunk(hipStream_t stream, const ChunkPlan &p, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
-                      size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q, const float *gate,
+                      size_t plane_elems, const void *k_tiled, const void *v_tiled, const ChunkQuery &in,
                       float *out, float *ws, size_t ws_elems) {
     const size_t elems = p.splits > 1 ? (size_t)Hkv * p.nrt * p.splits * 32 * p.rw * D : 0;
     if (!p.applies || elems > ws_elems) return fail(MFA_ERR_INVALID, "sdpa: chunk plan without its workspace");
     const int hpk = Hq / Hkv;
-    ChunkArgs a{(const uint16_t *)k_tiled, (const uint16_t *)v_tiled, plane_elems, q, gate, hpk, Hq, n_tok, kv_len - n_tok,
+    ChunkArgs a{(const uint16_t *)k_tiled, (const uint16_t *)v_tiled, plane_elems, in, hpk, Hq, n_tok, kv_len - n_tok,
                 (1.0f / sqrtf((float)D)) * kLog2e, out, ws, ws + elems, p.nrt, p.splits, p.bps, Hkv * p.splits,
                 kv_len - n_tok >= n_tok};
     const dim3 grid((unsigned)(p.nrt * Hkv * p.splits));
-#define MFA_CHUNK_L(DD, RWW, KSS, GG)                                                                             \
-    do {                                                                                                          \
-        if (p.splits > 1) hipLaunchKernelGGL((sdpa_chunk_kernel<DD, RWW, KSS, GG, true>), grid, dim3(64 * RWW * KSS), 0, stream, a); \
-        else hipLaunchKernelGGL((sdpa_chunk_kernel<DD, RWW, KSS, GG, false>), grid, dim3(64 * RWW * KSS), 0, stream, a); \
+    const bool raw = in.q_norm != nullptr;
+    if (raw && D < 128) return fail(MFA_ERR_SHAPE, "sdpa: raw query rows of %d channels", D);
+#define MFA_CHUNK(DD, RWW, KSS, GG, SP, RAWW) \
+    hipLaunchKernelGGL((sdpa_chunk_kernel<DD, RWW, KSS, GG, SP, RAWW>), grid, dim3(64 * RWW * KSS), 0, stream, a)
+#define MFA_CHUNK_R(DD, RWW, KSS, GG)                                    \
+    do {                                                                 \
+        if (p.splits > 1 && raw) MFA_CHUNK(DD, RWW, KSS, GG, true, (DD >= 128)); \
+        else if (p.splits > 1) MFA_CHUNK(DD, RWW, KSS, GG, true, false); \
+        else if (raw) MFA_CHUNK(DD, RWW, KSS, GG, false, (DD >= 128));   \
+        else MFA_CHUNK(DD, RWW, KSS, GG, false, false);                  \
     } while (0)
+    // (two wave sets at head_dim >= 128 leave room for one block of each in use and one on its way)
     if (D == 256) {
-        if (p.ks == 1) MFA_CHUNK_L(256, 4, 1, 2);
-        else MFA_CHUNK_L(256, 2, 2, 1);
+        if (p.ks == 1) MFA_CHUNK_R(256, 4, 1, 2);
+        else MFA_CHUNK_R(256, 2, 2, 1);
     } else if (D == 128) {
-        if (p.ks == 1 && p.rw == 4) MFA_CHUNK_L(128, 4, 1, 2);
-        else MFA_CHUNK_L(128, 2, 2, 1);
+        if (p.ks == 1) MFA_CHUNK_R(128, 4, 1, 2);
+        else MFA_CHUNK_R(128, 2, 2, 1);
     } else {
-        if (p.ks == 1) MFA_CHUNK_L(64, 4, 1, 2);
-        else MFA_CHUNK_L(64, 2, 2, 2);
+        if (p.ks == 1) MFA_CHUNK_R(64, 4, 1, 2);
+        else MFA_CHUNK_R(64, 2, 2, 2);
     }
+#undef MFA_CHUNK_R
+#undef MFA_CHUNK
     MFA_HIP(hipGetLastError());
     if (p.splits > 1) {
         const int n_units = Hkv * p.nrt * p.rw * (D / 32);

@@ -27,8 +27,8 @@ def _ctx(mfa, Hq, Hkv, d, cap):
 @pytest.mark.parametrize("Hq,Hkv,d,T,L0", [
     (8, 2, 128, 8, 0), (8, 2, 128, 9, 23), (4, 1, 64, 31, 1), (4, 1, 256, 33, 31),     # a row either side of a tile
     (16, 1, 128, 2, 62), (16, 1, 256, 3, 61), (6, 2, 64, 65, 64),                      # positions either side of a chunk of K
-    (32, 4, 128, 40, 2500), (16, 2, 256, 50, 1990), (16, 2, 256, 130, 600), (16, 4, 64, 70, 2047),   # splits
-    (3, 3, 128, 129, 4000), (24, 1, 256, 11, 2303),
+    (32, 4, 128, 40, 2500), (16, 2, 256, 50, 1990), (16, 2, 64, 40, 5000), (4, 1, 64, 70, 1900),   # splits
+    (16, 2, 256, 130, 600), (3, 3, 128, 129, 4000), (24, 1, 256, 11, 2303),                             # two wave sets; few rows
 ])
 def test_chunk_against_the_oracle(mfa, oracle, Hq, Hkv, d, T, L0):
     q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, T + L0)
@@ -50,7 +50,7 @@ def test_chunk_against_the_oracle(mfa, oracle, Hq, Hkv, d, T, L0):
 
 def test_chunk_split_with_peaked_scores(mfa, oracle):
     """Scores of +-130: the running maximum rises by far more than the lazy rescaling's 2^8, in some splits only."""
-    Hq, Hkv, d, T, L0 = 16, 2, 256, 130, 600
+    Hq, Hkv, d, T, L0 = 16, 2, 256, 50, 1990
     q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, 3)
     q *= 8.0
     k[::97] *= 4.0
@@ -60,3 +60,42 @@ def test_chunk_split_with_peaked_scores(mfa, oracle):
         out = c.prefill_attn(0, q, g, k[L0:], v[L0:])
     # a score s carries up to 2^-17 |s| from the query's two parts: 1e-3 of a probability at |s| = 130
     assert rel_err(out, ref) <= 2e-3
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,T,L0,rotary", [
+    (32, 4, 128, 70, 0, 32), (16, 2, 256, 70, 41, 64), (32, 4, 128, 40, 2500, 32), (16, 2, 256, 50, 1990, 64),
+    (16, 2, 256, 50, 1990, 32), (8, 2, 64, 70, 41, 16),     # not a quarter of the head, head_dim 64: a prologue of its own
+    (6, 3, 128, 77, 10, 32),
+])
+def test_raw_projections_against_the_separate_prologue(mfa, oracle, Hq, Hkv, d, T, L0, rotary):
+    """The chunk kernel's own norm and rotation of the query against the prologue launch, the decode kernel (a forced
+    split count) and the prologue's cache rows; and with the result written over the projection, which sends the call
+    down the prologue's path too."""
+    from moeflux_amd.hip import DeviceArray
+    rng = np.random.default_rng(T + L0 + d)
+    norm = [oracle.f32_to_bf16(1.0 + 0.3 * rng.standard_normal(d)) for _ in range(2)]
+    qp = rng.standard_normal((T, Hq * 2 * d)).astype(np.float32)
+    k, v = (rng.standard_normal((L0 + T, Hkv * d)).astype(np.float32) for _ in range(2))
+
+    def run(how):
+        with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+            c.set_rope(1.0e7, rotary)
+            c.set_full_weights(0, *norm)
+            if L0:
+                c.kv_import(0, k[:L0], v[:L0])
+            if how == "decode":
+                c.set_num_splits(1)
+            if how == "in place":
+                dq, dk, dv = (DeviceArray.from_host(x) for x in (qp, k[L0:], v[L0:]))
+                assert c.lib.mfa_prefill_full_attn_dev(c.h, 0, L0, T, dq.ptr, dk.ptr, dv.ptr, dq.ptr) == 0
+                c.sync()
+                out = dq.to_host().reshape(-1)[:T * Hq * d].reshape(T, Hq * d)
+            else:
+                out = c.prefill_full_attn(0, L0, qp, k[L0:], v[L0:])
+            return out, c.kv_export(0)
+
+    out, cache = run("raw")
+    for how in ("decode", "in place"):
+        other, other_cache = run(how)
+        assert rel_err(out, other) <= TOL, how
+        assert all(np.array_equal(a, b) for a, b in zip(cache, other_cache)), how
