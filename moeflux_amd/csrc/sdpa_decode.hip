@@ -139,7 +139,9 @@ template <typename KV, int D, int NT> struct StepQuery {
 #pragma unroll
                 for (int e = 0; e < EPS; e++) d = fmaf(qraw[i][e], knew[e], d);
                 d = lanes_sum<LPH>(d);
-                if (ok && j == 0) sp.new_score[((size_t)rows.kvh * nhg + rows.hg) * 16 + n] = d * qscale;
+                if (ok && j == 0)   // (at device scope, as the partials: a workgroup of another XCD may merge)
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, d * qscale), buffer_of(sp.new_score),
+                                                          (((rows.kvh * nhg + rows.hg) * 16 + n) * 4), 0, kThrough);
             }
             if (in) {
                 float4 raw[W::QRAW_F4];
@@ -215,12 +217,114 @@ template <int N, int END, int STEP, typename F> __device__ __attribute__((always
     }
 }
 
+// A decode launch that merges its partials itself: every workgroup of a row group draws a ticket when its partial is
+// out, and the one that draws the last combines them all and writes the group's rows (nobody waits for anybody).  The
+// counter goes back to 0 with the last ticket.  For short caches: the merge as a launch of its own costs 3 us of host time,
+// which is what bounds layers this small, and 4 us of the device's; the hop through memory and the last workgroup's reading
+// cost about as long on the device (one_launch_plan).
+struct OneLaunch {
+    const float *gate;
+    float *out;
+    int gate_stride;
+    unsigned *tickets;   // [kv head][row group], 0 between launches
+};
+static constexpr int kOneSplits = 16;
+
+// Partials are stored and loaded at device scope (sc1), past the L2s of the XCDs, so that waiting for the stores ahead of the
+// ticket is all the ordering there is to do: with the fences of the memory model instead (the whole L2 written back and
+// invalidated by every workgroup) a call of 100 positions took 4 us longer and one of 3000 up to 6.
 template <typename KV, int D, bool STEP>
+__device__ inline void one_launch_merge(const OneLaunch &one, const float *part_o, const float *part_ml, int nsplit, int nhg, int hpk,
+                                        int Hq, int kvh, int hg, const std::conditional_t<STEP, StepPrologue, NoPrologue> &sp, int *s_last,
+                                        float (*s_stat)[32]) {
+    constexpr int NT = kWaves * 64, Q = D / 4;   // 16-byte pieces of a row
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's share of the partial is out
+    __syncthreads();
+    if (nsplit > 1) {
+        if (threadIdx.x == 0) {
+            unsigned *ticket = one.tickets + kvh * nhg + hg;
+            const bool last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nsplit - 1;
+            if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *s_last = last;
+        }
+        __syncthreads();
+        if (!*s_last) return;
+    }
+    const size_t pid0 = ((size_t)kvh * nhg + hg) * nsplit;
+    const __amdgpu_buffer_rsrc_t ob = buffer_of(part_o + pid0 * 16 * D), mlb = buffer_of(part_ml + pid0 * 32);
+    const int rows = hpk - 16 * hg < 16 ? hpk - 16 * hg : 16, items = rows * Q;
+    unsigned stat[kOneSplits * 32 / NT];
+#pragma unroll
+    for (int i = 0; i < kOneSplits * 32 / NT; i++) {
+        const int at = i * NT + threadIdx.x;
+        stat[i] = __builtin_amdgcn_raw_buffer_load_b32(mlb, (at < nsplit * 32 ? at : 0) * 4, 0, kThrough);
+    }
+    // NS: splits at most; PER: pieces a thread has in flight (all of their rows, gates and values requested at once)
+    auto combine = [&](auto ns_tag, auto per_tag) __attribute__((always_inline)) {
+        constexpr int NS = decltype(ns_tag)::value, PER = decltype(per_tag)::value;
+        for (int base = 0; base < items; base += PER * NT) {
+            u32x4 row[PER][NS];
+            float4 gate[PER], tok[PER];
+            float tok_score[PER];
+            auto piece = [&](int p) { const int i = base + p * NT + (int)threadIdx.x; return i < items ? i : items - 1; };
+#pragma unroll
+            for (int p = 0; p < PER; p++) {
+                const int item = piece(p), n = item / Q, c = 4 * (item % Q);
+#pragma unroll
+                for (int s = 0; s < NS; s++)
+                    row[p][s] = __builtin_amdgcn_raw_buffer_load_b128(ob, (((s < nsplit ? s : nsplit - 1) * 16 + n) * D + c) * 4, 0, kThrough);
+                gate[p] = load_f4(one.gate + ((size_t)kvh * hpk + 16 * hg + n) * one.gate_stride + c);
+                tok_score[p] = neg_inf();
+                tok[p] = float4{0.f, 0.f, 0.f, 0.f};
+                if constexpr (STEP) {
+                    tok_score[p] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(sp.new_score), ((kvh * nhg + hg) * 16 + n) * 4, 0, kThrough));
+                    const float4 v = load_f4(sp.v_in + (size_t)kvh * D + c);   // as the cache holds it
+                    tok[p] = float4{from_kv(to_kv<KV>(v.x)), from_kv(to_kv<KV>(v.y)), from_kv(to_kv<KV>(v.z)), from_kv(to_kv<KV>(v.w))};
+                }
+            }
+            if (base == 0) {
+#pragma unroll
+                for (int i = 0; i < kOneSplits * 32 / NT; i++) s_stat[(i * NT + threadIdx.x) / 32][threadIdx.x % 32] = __builtin_bit_cast(float, stat[i]);
+                __syncthreads();
+            }
+#pragma unroll
+            for (int p = 0; p < PER; p++) {
+                const int item = piece(p), n = item / Q, c = 4 * (item % Q);
+                float M = tok_score[p];
+#pragma unroll
+                for (int s = 0; s < NS; s++) M = fmaxf(M, s < nsplit ? s_stat[s][n] : neg_inf());
+                const float wt = tok_score[p] == neg_inf() ? 0.f : fast_exp2(tok_score[p] - M);
+                float den = wt;
+                float4 acc = {wt * tok[p].x, wt * tok[p].y, wt * tok[p].z, wt * tok[p].w};
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    const float m = s < nsplit ? s_stat[s][n] : neg_inf(), w = m == neg_inf() ? 0.f : fast_exp2(m - M);
+                    if (w != 0.f) {   // (a split without positions left its rows unwritten)
+                        const float4 x = __builtin_bit_cast(float4, row[p][s]);
+                        den += w * s_stat[s][16 + n];
+                        acc.x += w * x.x; acc.y += w * x.y; acc.z += w * x.z; acc.w += w * x.w;
+                    }
+                }
+                if (base + p * NT + (int)threadIdx.x < items)
+                    *(float4 *)(one.out + ((size_t)kvh * hpk + 16 * hg + n) * D + c) =
+                        float4{(acc.x / den) * merge_gate(one.gate, gate[p].x), (acc.y / den) * merge_gate(one.gate, gate[p].y),
+                               (acc.z / den) * merge_gate(one.gate, gate[p].z), (acc.w / den) * merge_gate(one.gate, gate[p].w)};
+            }
+        }
+    };
+    using std::integral_constant;
+    if (nsplit == 1) combine(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else if (nsplit <= 4) combine(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    else if (nsplit <= 8) combine(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+    else combine(integral_constant<int, kOneSplits>{}, integral_constant<int, 2>{});
+}
+
+template <typename KV, int D, bool STEP, bool ONE>
 __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     const KV *__restrict__ k_tiled, const KV *__restrict__ v_tiled, size_t plane_elems,
     const float *__restrict__ q, int hpk, int Hq, int n_tok, int64_t kv_len0,
     int units_base, int units_rem, float qscale, float *__restrict__ part_o, float *__restrict__ part_ml,
-    std::conditional_t<STEP, StepPrologue, NoPrologue> sp) {
+    std::conditional_t<STEP, StepPrologue, NoPrologue> sp, OneLaunch one) {
     using W = Wave<KV, D>;
     using S = Stream<KV, D, STEP>;
     constexpr int NK = S::NK, NV = S::NV, TPW = S::TPW, VB = S::VB, kRing = S::R;
@@ -231,6 +335,8 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     __shared__ float sm[kWaves][16];
     __shared__ float sl[kWaves][16];
     __shared__ float2 s_tab[STEP ? 128 : 1];
+    __shared__ int s_last;
+    __shared__ float s_stat[ONE ? kOneSplits : 1][32];
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
@@ -266,6 +372,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
             HeadRotor<sq.EPS, D>::table(sq.freq, sp.pos, sp.rotary_dim, s_tab);
             __syncthreads();
             sq.finish(sp, rows, qscale, plane_elems, true, qlds, nhg, s_tab);
+            if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
             return;
         }
     }
@@ -277,6 +384,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, neg_inf()), mlb, n * 4, 0, kThrough);
             __builtin_amdgcn_raw_buffer_store_b32(0u, mlb, (16 + n) * 4, 0, kThrough);
         }
+        if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
         return;
     }
 
@@ -481,6 +589,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, m_run), mlb, n * 4, 0, kThrough);
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, lsum), mlb, (16 + n) * 4, 0, kThrough);
     }
+    if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
 }
 
 // The token a decode step has just appended, as one more split of the merge (MergeOut), and
@@ -653,18 +762,22 @@ size_t sdpa_workspace_ml_elems(int Hq, int Hkv, int splits, int n_tok) {
 template <typename KV, int D, bool STEP, typename SP>
 static void launch_partial(hipStream_t stream, dim3 grid, const void *k, const void *v, size_t plane_elems,
                            const float *q, int hpk, int Hq, int n_tok, int64_t kv_len0, const SplitPlan &plan,
-                           float qscale, float *po, float *pml, const SP &sp) {
-    hipLaunchKernelGGL((sdpa_partial_kernel<KV, D, STEP>), grid, dim3(kWaves * 64), 0, stream, (const KV *)k,
-                       (const KV *)v, plane_elems, q, hpk, Hq, n_tok, kv_len0, plan.base, plan.rem, qscale, po, pml, sp);
+                           float qscale, float *po, float *pml, const SP &sp, const OneLaunch *one) {
+    if (one)
+        hipLaunchKernelGGL((sdpa_partial_kernel<KV, D, STEP, true>), grid, dim3(kWaves * 64), 0, stream, (const KV *)k, (const KV *)v,
+                           plane_elems, q, hpk, Hq, n_tok, kv_len0, plan.base, plan.rem, qscale, po, pml, sp, *one);
+    else
+        hipLaunchKernelGGL((sdpa_partial_kernel<KV, D, STEP, false>), grid, dim3(kWaves * 64), 0, stream, (const KV *)k, (const KV *)v,
+                           plane_elems, q, hpk, Hq, n_tok, kv_len0, plan.base, plan.rem, qscale, po, pml, sp, OneLaunch{});
 }
 
 // dtype and width dispatch of the split-K launch
 template <bool STEP, typename SP>
 static void launch_partial_any(int kv_dtype, int D, hipStream_t stream, dim3 grid, const void *k, const void *v,
                                size_t plane_elems, const float *q, int hpk, int Hq, int n_tok, int64_t kv_len0,
-                               const SplitPlan &plan, float qscale, float *po, float *pml, const SP &sp) {
+                               const SplitPlan &plan, float qscale, float *po, float *pml, const SP &sp, const OneLaunch *one = nullptr) {
 #define MFA_LAUNCH(KV, DD) \
-    launch_partial<KV, DD, STEP>(stream, grid, k, v, plane_elems, q, hpk, Hq, n_tok, kv_len0, plan, qscale, po, pml, sp)
+    launch_partial<KV, DD, STEP>(stream, grid, k, v, plane_elems, q, hpk, Hq, n_tok, kv_len0, plan, qscale, po, pml, sp, one)
     if (kv_dtype == MFA_KV_BF16) {
         if (D == 64) MFA_LAUNCH(uint16_t, 64);
         else if (D == 128) MFA_LAUNCH(uint16_t, 128);
@@ -698,6 +811,28 @@ static int fit_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int n
     return MFA_OK;
 }
 
+// Whether one launch serves a decode call (OneLaunch), and its plan: up to 1024 positions and 768 KiB of K and V per kv head,
+// in at most kOneSplits splits of a pass each.  Measured per layer, three sequences side by side: 7.4 -> 3.6 us at 20 .. 1000
+// positions (16 or 32 heads over 2 of 256, 32 over 4 of 128); one sequence after itself 7.6 -> 6.1 at 20, 8.8 -> 9.8 at 515, 8.5 -> 8.8
+// at 1000.  Past the limits the last workgroup's share of the merge, and the shares of the fewer splits, cost a single sequence
+// more than the launch they save (3000 positions: 9.8 -> 12 to 16.5 us).
+static constexpr int64_t kOnePositions = 1024, kOneBytes = 768 << 10;
+static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int64_t kv_len, int forced_splits, const SdpaWorkspace &ws) {
+    if (!ws.tickets || forced_splits > 0 || kv_len > kOnePositions) return false;
+    if (kv_len * D * (kv_dtype == MFA_KV_BF16 ? 4 : 8) > kOneBytes) return false;
+    const int U = unit_chunks(kv_dtype, D);
+    const int64_t nchunk = (kv_len + kKvChunk - 1) / kKvChunk, nunits = nchunk > U ? (nchunk + U - 1) / U : 1;
+    const int64_t min_units = (min_pass_chunks(kv_dtype, D) + U - 1) / U;
+    int64_t splits = nunits / min_units;
+    if (splits > kOneSplits) splits = kOneSplits;
+    if (splits < 1) splits = 1;
+    plan.nhg = (Hq / Hkv + 15) / 16;
+    plan.splits = (int)splits;
+    plan.base = (int)(nunits / splits);
+    plan.rem = (int)(nunits % splits);
+    return sdpa_workspace_o_elems(Hq, Hkv, D, plan.splits) <= ws.part_o_elems && sdpa_workspace_ml_elems(Hq, Hkv, plan.splits) <= ws.part_ml_elems;
+}
+
 // One decode token of a full-attention layer from its raw projections in two launches: the
 // split-K launch norms and rotates the query heads itself, attends to the len0 positions the
 // cache holds, and the workgroup of the last split (the one with the fewest positions) also scores
@@ -712,14 +847,17 @@ int launch_sdpa_step(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, i
     if (len0 < 0 || pos < 0) return fail(MFA_ERR_INVALID, "attention step: negative position");
     const int hpk = Hq / Hkv;
     SplitPlan plan;
-    MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, 1, len0 > 0 ? len0 : 1, num_cus, forced_splits, ws));
+    const bool one = one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, ws);
+    if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, 1, len0 > 0 ? len0 : 1, num_cus, forced_splits, ws));
+    const OneLaunch ol{q_proj + D, out, 2 * D, ws.tickets};
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     const StepPrologue sp{q_proj, k_in, v_in, q_norm, k_norm, inv_freq, rotary_dim, eps, pos, len0, new_score,
                           k_tiled, v_tiled, plan.splits - 1};
     // rows see positions [0, len0): one token whose own position is not in the cache yet
     launch_partial_any<true>(kv_dtype, D, stream, dim3(plan.splits, plan.nhg, Hkv), k_tiled, v_tiled, plane_elems,
-                             nullptr, hpk, Hq, 1, len0 - 1, plan, qscale, ws.part_o, ws.part_ml, sp);
+                             nullptr, hpk, Hq, 1, len0 - 1, plan, qscale, ws.part_o, ws.part_ml, sp, one ? &ol : nullptr);
     MFA_HIP(hipGetLastError());
+    if (one) return MFA_OK;
     const MergeExtra ex{2 * D, new_score, v_in, kv_dtype == MFA_KV_BF16 ? 1 : 0};
     launch_merge_kernels(stream, ws.part_o, ws.part_ml, plan.splits, hpk, Hq, plan.nhg, D, 1, q_proj + D, out, &ex);
     MFA_HIP(hipGetLastError());
@@ -740,13 +878,15 @@ int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_
         return fail(MFA_ERR_INVALID, "sdpa: kv_len must be > 0 (got %lld for %d tokens)", (long long)kv_len, n_tok);
     const int hpk = Hq / Hkv;
     SplitPlan plan;
-    MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, forced_splits, ws));
+    const bool one = n_tok == 1 && gate && !partial_only && !defer_merge && one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, ws);
+    if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, forced_splits, ws));
+    const OneLaunch ol{gate, out, D, ws.tickets};
     // scores are produced in log2 units: q is pre-multiplied by (1/sqrt(D)) * log2(e)
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     launch_partial_any<false>(kv_dtype, D, stream, dim3(plan.splits, plan.nhg, Hkv), k_tiled, v_tiled, plane_elems, q,
-                              hpk, Hq, n_tok, kv_len - n_tok, plan, qscale, ws.part_o, ws.part_ml, NoPrologue{});
+                              hpk, Hq, n_tok, kv_len - n_tok, plan, qscale, ws.part_o, ws.part_ml, NoPrologue{}, one ? &ol : nullptr);
     MFA_HIP(hipGetLastError());
-    if (partial_only) return MFA_OK;
+    if (partial_only || one) return MFA_OK;
     if (defer_merge && plan.splits <= 16) {
         *defer_merge = SdpaMergeTask{ws.part_o, ws.part_ml, gate, out, plan.splits, hpk, Hq, plan.nhg, D, n_tok * Hq * (D / 64)};
         return MFA_OK;

@@ -215,3 +215,29 @@ def test_shares_of_a_single_unit(mfa, oracle, Hq, Hkv, d, bf16):
             one = c.sdpa_decode(0, q, g)
         assert rel_err(out, ref) <= tol, (L, splits)
         assert rel_err(out, one) <= tol, (L, splits)
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,bf16,lens", [
+    (16, 2, 256, True, (1, 127, 129, 515, 768, 769)), (32, 2, 256, True, (64, 640)), (40, 2, 128, True, (1023, 1024, 1025)),
+    (32, 4, 128, False, (1, 63, 65, 767, 768, 769)), (4, 2, 64, True, (130, 1024)), (3, 1, 64, False, (500, 1024)),
+    (18, 1, 256, False, (384, 385)),
+])
+def test_short_caches_merge_in_the_attention_launch(mfa, oracle, Hq, Hkv, d, bf16, lens):
+    """Either side of the limits of the launch that merges its own partials (up to 1024 positions and 768 KiB per kv head;
+    more than 16 heads per kv head are two row groups): against the oracle, three calls in a row the same to the bit (the
+    counters are back at 0), over a workspace of NaN, and the merge launch (a forced split count) within rounding."""
+    from moeflux_amd import Config
+    top = max(lens)
+    q, g, k, v = sdpa_random_inputs(top + d, Hq, Hkv, d, top, bf16=bf16)
+    tol = 1e-4 if bf16 else TOL_F32   # bf16: the query and the probabilities in two parts of 2^-17
+    with mfa.Ctx(Config(num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d, kv_capacity=top,
+                        kv_dtype=1 if bf16 else 0)) as c:
+        for n in sorted(lens):
+            c.kv_import(0, k[:n], v[:n])
+            assert c.lib.mfa_debug_fill_workspace(c.h, 0x7FC00000) == 0
+            outs = [c.sdpa_decode(0, q, g) for _ in range(3)]
+            assert rel_err(outs[0], oracle.sdpa(n, Hq, Hkv, d, q, g, k[:n], v[:n])) <= tol, n
+            assert all(np.array_equal(outs[0], o) for o in outs[1:]), n
+            c.set_num_splits(2)
+            assert rel_err(outs[0], c.sdpa_decode(0, q, g)) <= tol, n
+            c.set_num_splits(0)
