@@ -279,6 +279,24 @@ static int truncate_full(Ctx *c, FullLayer &f, int32_t new_len) {
     return MFA_OK;
 }
 
+// Every layer's truncation to [0, min(new_len, end)), end = p1 (negative: all), neighbouring layers that drop the same
+// positions in one launch.
+static int truncate_layers(Ctx *c, int32_t new_len, int32_t p1) {
+    const auto target = [&](const FullLayer &f) {
+        const int32_t end = (p1 < 0 || p1 > f.len) ? f.len : p1;
+        return new_len < end ? new_len : end;
+    };
+    for (size_t i = 0, j; i < c->full.size(); i = j) {
+        const int32_t len = c->full[i].len, to = target(c->full[i]);
+        for (j = i + 1; j < c->full.size() && c->full[j].len == len; j++) {}
+        if (to < 0 || to >= len) continue;
+        MFA_TRY(launch_kv_zero(c->stream, c->cfg.kv_dtype, c->cfg.num_kv_heads * (int)(j - i), c->cfg.head_dim, c->plane_elems, to, len,
+                               c->full[i].k, c->full[i].v));
+        for (size_t l = i; l < j; l++) c->full[l].len = to;
+    }
+    return MFA_OK;
+}
+
 // Grows the split-K workspace to at least the given element counts (never shrinks it).
 static int ensure_workspace_elems(Ctx *c, size_t need_o, size_t need_ml) {
     if (need_o <= c->part_o_elems && need_ml <= c->part_ml_elems) return MFA_OK;
@@ -1093,7 +1111,7 @@ int mfa_dequant_matvec_4bit(int32_t out_dim, int32_t in_dim, int32_t group_size,
 int mfa_reset(mfa_ctx *ctx) {
     Ctx *c = as_ctx(ctx);
     if (!c) return fail(MFA_ERR_INVALID, "NULL context");
-    for (auto &f : c->full) MFA_TRY(truncate_full(c, f, 0));
+    MFA_TRY(truncate_layers(c, 0, -1));
     for (auto &l : c->lin) MFA_TRY(reset_linear(c, l));
     MFA_HIP(hipStreamSynchronize(c->stream));
     drop_checkpoints(c);  // keyed by position: a full clear invalidates every key (riir/mod.rs:1965-1968)
@@ -1104,10 +1122,7 @@ int mfa_truncate(mfa_ctx *ctx, int32_t p0, int32_t p1) {
     Ctx *c = as_ctx(ctx);
     if (!c) return fail(MFA_ERR_INVALID, "NULL context");
     const int32_t new_len = p0 < 0 ? 0 : p0;
-    for (auto &f : c->full) {
-        const int32_t end = (p1 < 0 || p1 > f.len) ? f.len : p1;
-        MFA_TRY(truncate_full(c, f, new_len < end ? new_len : end));
-    }
+    MFA_TRY(truncate_layers(c, new_len, p1));
     for (auto &l : c->lin) MFA_TRY(reset_linear(c, l));
     MFA_HIP(hipStreamSynchronize(c->stream));
     return MFA_OK;

@@ -322,9 +322,9 @@ int launch_kv_scatter(hipStream_t stream, int kv_dtype, int src_is_bf16, int Hkv
 int launch_kv_gather(hipStream_t stream, int kv_dtype, int Hkv, int D, size_t plane_elems,
                      int64_t n_rows, const void *k_tiled, const void *v_tiled, float *k_rows,
                      float *v_rows);
-// Zero positions [pos0, pos1) of every plane.
-int launch_kv_zero(hipStream_t stream, int kv_dtype, int Hkv, int D, size_t plane_elems,
-                   int64_t pos0, int64_t pos1, void *k_tiled, void *v_tiled);
+// Zero positions [pos0, pos1) of n_planes planes side by side (a layer's Hkv, or several layers').
+int launch_kv_zero(hipStream_t stream, int kv_dtype, int n_planes, int D, size_t plane_elems, int64_t pos0, int64_t pos1,
+                   void *k_tiled, void *v_tiled);
 
 int launch_plain_copy(hipStream_t stream, void *dst, const void *src, size_t nbytes);
 // A launch that only reads nbytes (sink: 16 bytes per workgroup, never written in practice).
