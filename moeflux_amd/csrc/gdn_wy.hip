@@ -422,8 +422,11 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 // layout of a D tile per 16 columns (lane (n, g): S[row0+n][16c+4g+i]), which is also the B
 // operand of a contraction over the columns.  Wave w serves tokens 16w .. 16w+15 of each
 // block and the column tiles (DK/64)*w .. of the state update.
+// 256 registers a wave (it took 260): a CU then holds two workgroups, of 64 heads' 512 or of two sequences' launches, and
+// one computes while the other waits at a block's barriers (512 tokens, six layers of 32 heads 275 -> 261 us a pass with
+// three sequences side by side).
 template <int DK>
-__global__ __launch_bounds__(256) void gdn_wy_recur_kernel(
+__global__ __launch_bounds__(256, 2) void gdn_wy_recur_kernel(
     int Hk, int Hv, int T, const float *__restrict__ Wt, const float *__restrict__ Qt,
     const float *__restrict__ Ut, const float *__restrict__ Mt, const float *__restrict__ Kt,
     const float *__restrict__ eLc, float *__restrict__ ssm, float *__restrict__ o_raw) {
