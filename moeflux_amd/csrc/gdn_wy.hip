@@ -88,11 +88,17 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     constexpr int NW = NK;        // waves
     constexpr int NTHR = 64 * NW;
     constexpr int NCT = 1;        // 16-wide column tiles of W (and of U) per wave
+    static_assert(!FUSED || NCT == 1, "a wave's v is one column tile");
     __shared__ __align__(16) float sK[kC][LDK];
-    __shared__ __align__(16) float sQ[kC][LDK];  // q^, later v (FUSED: q^ only)
-    __shared__ __align__(16) float sV[FUSED ? kC : 1][LDK];
-    __shared__ __align__(16) float sA[kC][LDC];
-    __shared__ __align__(16) float sT[kC][LDC];
+    // FUSED keeps to half a CU's LDS (81664 bytes of 163840; it was 137472), so that a CU holds two workgroups, of one launch or
+    // of two sequences': v stays in the registers of the wave that multiplies it, A is its ten lower tiles, and T lies
+    // where q^ was.  The kernel waits on memory, LDS and its substitution chain far more than on its products (512 tokens,
+    // six layers 261 -> 237 us a pass with three sequences side by side; 2000 tokens of one layer 176 -> 154).
+    __shared__ __align__(16) float sQ[kC][LDK];  // q^, later v (FUSED: later T)
+    __shared__ __align__(16) float sA[10][16][20];   // tile (I, J <= I) at I (I + 1) / 2 + J
+    __shared__ __align__(16) float sTown[FUSED ? 1 : kC][LDC];
+    static_assert(LDC <= LDK, "T fits where q^ was");
+    float(*sT)[LDC] = FUSED ? reinterpret_cast<float(*)[LDC]>(&sQ[0][0]) : sTown;
     __shared__ __align__(16) float sL[kC], sB[kC], sCw[kC], sKd[kC];
     __shared__ int sR[kC];
 
@@ -111,8 +117,9 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     float lg_in = 0.f, bg_in = 0.f;
     constexpr int NLV = kC * (DV / 4) / NTHR;
     float4 va[FUSED ? 1 : NLV];
+    float vreg[4][4];   // FUSED: v of tokens 16 s + 4 g + i, channel 16 wave + m, phase 3's operand
     if constexpr (FUSED) {
-        constexpr int NCONV = 2 * DK + DV, TT = 16;          // channels of the head; tokens per run
+        constexpr int NCONV = 2 * DK, TT = 16;               // q and k channels of the head; tokens per run
         constexpr int NU = NCONV * (kC / TT) / NTHR;          // (channel, run) units per thread
         static_assert(NCONV * (kC / TT) % NTHR == 0, "whole units per thread");
         const int C = 2 * Hk * DK + Hv * DV;
@@ -136,7 +143,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 #pragma unroll
         for (int u = 0; u < NU; u++) {
             const int unit = tid + u * NTHR, c = unit % NCONV, run = unit / NCONV;
-            const int ch = c < DK ? kh * DK + c : c < 2 * DK ? Hk * DK + kh * DK + (c - DK) : 2 * Hk * DK + vh * DV + (c - 2 * DK);
+            const int ch = c < DK ? kh * DK + c : Hk * DK + kh * DK + (c - DK);
             wbits[u] = *(const uint2 *)(in.conv_w + (unsigned)ch * 4u);
 #pragma unroll
             for (int j = 0; j < TT + 3; j++) {
@@ -151,6 +158,22 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 }
             }
         }
+        // v the same way, in runs of four tokens (seven inputs each)
+        const int vch = 2 * Hk * DK + vh * DV + 16 * wave + m;
+        const uint2 vw = *(const uint2 *)(in.conv_w + (unsigned)vch * 4u);
+        float xv[4][7];
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < 7; j++) {
+                const int rel = 16 * s + 4 * g + j - 3, idx = t0 + rel, last = T - 1 - t0;
+                if (s == 0 && j < 3) {   // the block's first tokens look back before it
+                    const int off = (idx < 0 ? ((in.step_mod + idx + 4) & 3) : rel > last ? last : rel) * C + vch;
+                    xv[s][j] = (idx < 0 ? in.ring : blk_rows)[off];
+                } else {
+                    xv[s][j] = blk_rows[(rel > last ? last : rel) * C + vch];
+                }
+            }
 #pragma unroll
         for (int u = 0; u < NU; u++) {
             const int unit = tid + u * NTHR, c = unit % NCONV, run = unit / NCONV;
@@ -159,8 +182,8 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             ntr = ntr < 0 ? 0 : ntr > TT ? TT : ntr;
             const float wt[4] = {bf16_bits_to_f32((uint16_t)(wbits[u].x & 0xffffu)), bf16_bits_to_f32((uint16_t)(wbits[u].x >> 16)),
                                  bf16_bits_to_f32((uint16_t)(wbits[u].y & 0xffffu)), bf16_bits_to_f32((uint16_t)(wbits[u].y >> 16))};
-            float(*dst)[LDK] = c < DK ? sQ : c < 2 * DK ? sK : sV;
-            const int cc = c < DK ? c : c < 2 * DK ? c - DK : c - 2 * DK;
+            float(*dst)[LDK] = c < DK ? sQ : sK;
+            const int cc = c < DK ? c : c - DK;
 #pragma unroll
             for (int i = 0; i < TT; i++) {
                 float acc = 0.f;
@@ -168,6 +191,19 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 for (int k = 0; k < 4; k++) acc = fmaf(xs[u][i + k], wt[k], acc);
                 dst[TT * run + i][cc] = i < ntr ? silu_f(acc) : 0.f;
             }
+        }
+        {
+            const float wt[4] = {bf16_bits_to_f32((uint16_t)(vw.x & 0xffffu)), bf16_bits_to_f32((uint16_t)(vw.x >> 16)),
+                                 bf16_bits_to_f32((uint16_t)(vw.y & 0xffffu)), bf16_bits_to_f32((uint16_t)(vw.y >> 16))};
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    float acc = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) acc = fmaf(xv[s][i + k], wt[k], acc);
+                    vreg[s][i] = 16 * s + 4 * g + i < nt ? silu_f(acc) : 0.f;
+                }
         }
         if (wave == 0 && lane < nt) {
             // shaders.metal:1321-1326; the decay enters as its logarithm
@@ -285,7 +321,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 const int row = 16 * I + 4 * g + i;
                 const float dl = sL[row] - sL[col];
                 const float d = sR[row] > col ? 0.f : __builtin_amdgcn_exp2f((dl < 0.f ? dl : 0.f) * 1.4426950408889634f);  // v_exp_f32: 1 ulp
-                sA[row][col] = (col < row) ? sB[row] * d * acc[i] : 0.f;
+                sA[idx][4 * g + i][m] = (col < row) ? sB[row] * d * acc[i] : 0.f;
             }
         } else {
             // the tile transposed (k^ as the A side): lane (n = m, g) then holds columns 16J + 4g + i of
@@ -342,7 +378,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             float acc = (i == m) ? 1.f : 0.f;
 #pragma unroll
             for (int j4 = 0; j4 < i; j4 += 4) {
-                const float4 a = lds_f4(&sA[r0 + i][r0 + j4]);  // the same address in every lane
+                const float4 a = lds_f4(&sA[wave * (wave + 1) / 2 + wave][i][j4]);  // the same address in every lane
                 acc = fmaf(-a.x, t[j4], acc);
                 if (j4 + 1 < i) acc = fmaf(-a.y, t[j4 + 1], acc);
                 if (j4 + 2 < i) acc = fmaf(-a.z, t[j4 + 2], acc);
@@ -364,7 +400,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 bt.y = sT[16 * K + 4 * g + 1][16 * J + m];
                 bt.z = sT[16 * K + 4 * g + 2][16 * J + m];
                 bt.w = sT[16 * K + 4 * g + 3][16 * J + m];
-                x = mfma4(lds_f4(&sA[16 * I + m][16 * K + 4 * g]), bt, x);
+                x = mfma4(lds_f4(&sA[I * (I + 1) / 2 + K][m][4 * g]), bt, x);
             }
             // x is held as rows 4g+i of column m: already the B operand of T_II x
             wy_f32x4 r = {0.f, 0.f, 0.f, 0.f};
@@ -386,7 +422,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 bK[s][ct][i] = sK[16 * s + 4 * g + i][16 * (NCT * wave + ct) + m];
-                bV[s][ct][i] = (FUSED ? sV : sQ)[16 * s + 4 * g + i][16 * (NCT * wave + ct) + m];
+                bV[s][ct][i] = FUSED ? vreg[s][i] : sQ[16 * s + 4 * g + i][16 * (NCT * wave + ct) + m];
             }
 #pragma unroll
     for (int tau = 0; tau < 4; tau++) {
