@@ -17,7 +17,7 @@ fn main() {
     // every .hip file under csrc/, in sorted order (a test holds this list to the directory)
     for f in [
         "api.hip", "attn_kernels.hip", "attn_prologue.hip", "checkpoint.hip", "dequant_matvec.hip", "gdn.hip",
-        "gdn_chunk.hip", "gdn_wy.hip", "kv_cache.hip", "mla_sdpa.hip", "sdpa_decode.hip", "sdpa_prefill.hip",
+        "gdn_chunk.hip", "gdn_wy.hip", "kv_cache.hip", "mla_sdpa.hip", "sdpa_chunk.hip", "sdpa_decode.hip", "sdpa_prefill.hip",
         "sdpa_static.hip", "snapshot.hip",
     ] {
         println!("cargo:rerun-if-changed=csrc/{f}");
