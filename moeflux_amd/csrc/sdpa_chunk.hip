@@ -9,7 +9,17 @@
 // it); its query operands (a bf16 high and low part) and its output tiles stay in registers.  The
 // cache is walked in blocks of 32 positions, copied to LDS by asynchronous loads (K and V lie in
 // operand order in memory already, and the pieces of the 16-wide tiles are operands of the 32-wide
-// ones as they are).
+// ones as they are: a 16-byte unit is 8 channels of a key, or 8 positions of a value channel that are
+// the score tile's own).  A KiB of LDS operand feeds two 32x32x16 products, 64 clocks of the matrix core; of
+// 16-row groups it fed half as much, and the four SIMDs asked for all the LDS could give.  The scores of a
+// block are formed beside the soft-max of the one before, two blocks to a barrier where LDS allows.
+// Rows that leave CUs idle split the cache (sdpa_chunk_plan).
+//
+// What bounds it: behind a long cache the matrix cores at the rate they sustain.  512 tokens of 32 heads
+// of 128 behind 32768 positions: 580 us with 16-row groups, 429 with this kernel, 384 with its soft-max
+// left out (both parts of query and probabilities are products, so 2.75e11 operations are 5.5e11 executed: 1.4 PFLOP/s).
+// Over short caches launch, query, first block and epilogue: 512 tokens from an empty cache 17 us,
+// of which the longest workgroup's eight blocks are 7.
 #include <cmath>
 
 #include "sdpa_wave.h"
@@ -544,9 +554,10 @@ bool sdpa_chunk_takes_raw(int D, int rotary_dim) { return D >= 128 && rotary_dim
 // How a chunk is cut up: the shape of a workgroup and the splits of the cache of the smallest estimated cost, or no
 // plan at all where the split-K decode kernel (16-row groups, each streaming the cache by itself) is estimated
 // cheaper, which is where a chunk's rows are few and its cache is long.  The cost is the call's own time and one and a half
-// times the time of the whole device that it takes: a chunk's layers follow each other, but other sequences run beside them
-// (one estimate alone costs 7 to 12 % of the other over 38 chunks of 6 .. 1500 tokens behind 0 .. 12000 positions, the sum
-// 3 %).  Times in microseconds, fitted to launches measured over those chunks, 10 to 15 % off:
+// times the time of the whole device that it takes: a chunk's layers follow each other, but other sequences run beside them.
+// (34 chunks of 6 .. 1500 tokens behind 0 .. 12000 positions, every plan measured: this cost is on average 4 % behind the best
+// with three sequences side by side and 8 % in a call's own time; own time alone 7 and 5 %, three times the device's 2 and 15 %.)
+// Times in microseconds, fitted to launches measured over those chunks:
 //   workgroup  kFixed (launch, query, first block, epilogue) + blocks per wave set * kBlock; a CU that holds two
 //              workgroups (head_dim <= 128) runs them 5 % faster than one after the other
 //   partials   written at 4.5 TB/s, merged at 7.5 TB/s with the gate and the result; 12 for the second launch

@@ -4,7 +4,7 @@
 // attn_softmax_batched / attn_values_batched / sigmoid_gate
 // (crates/moeflux/shaders/shaders.metal:976-1134, encoded at
 // crates/moeflux/src/riir/linear_attn_forward.rs:850-902) and its CPU fallback
-// sdpa_cpu (crates/moeflux/src/riir/sdpa.rs:63-172) with two launches:
+// sdpa_cpu (crates/moeflux/src/riir/sdpa.rs:63-172) with two launches, or one for a short cache (OneLaunch):
 //
 //   sdpa_partial_kernel  grid (splits, 16-row groups, kv heads), 4 waves.
 //     A workgroup streams its share of the cache: K and V pass through a ring of 1 KiB loads
