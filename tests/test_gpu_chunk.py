@@ -99,3 +99,43 @@ def test_raw_projections_against_the_separate_prologue(mfa, oracle, Hq, Hkv, d, 
         other, other_cache = run(how)
         assert rel_err(out, other) <= TOL, how
         assert all(np.array_equal(a, b) for a, b in zip(cache, other_cache)), how
+
+
+def test_chunk_and_short_decode_in_a_captured_graph(mfa, oracle):
+    """Captured on a context that has no chunk workspace yet (the plan then needs none), replayed between eager calls: a
+    chunk whose eager plan splits the cache, and a decode call that draws tickets."""
+    import ctypes as C
+
+    from moeflux_amd.hip import DeviceArray, rt
+    Hq, Hkv, d, T, L0, short = 16, 2, 256, 50, 1990, 515
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, 9)
+    with _ctx(mfa, Hq, Hkv, d, L0 + T) as e:
+        e.kv_import(0, k[:L0], v[:L0])
+        want = e.prefill_attn(0, q, g, k[L0:], v[L0:])
+        e.memory_clear()
+        e.kv_import(0, k[:short], v[:short])
+        want_short = e.sdpa_decode(0, q[0], g[0])
+    dq, dg, dk, dv = (DeviceArray.from_host(x) for x in (q, g, k[L0:], v[L0:]))
+    for what in ("chunk", "decode"):
+        n = L0 if what == "chunk" else short
+        with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+            c.kv_import(0, k[:n], v[:n])
+            out = DeviceArray((T, Hq * d), zero=True)
+            stream, graph, run = C.c_void_p(c.lib.mfa_stream(c.h)), C.c_void_p(), C.c_void_p()
+            assert rt().hipStreamBeginCapture(stream, C.c_int(2)) == 0   # relaxed: other streams are not held up
+            if what == "chunk":
+                rc = c.lib.mfa_prefill_attn_dev(c.h, 0, T, dq.ptr, dg.ptr, dk.ptr, dv.ptr, out.ptr)
+            else:
+                rc = c.lib.mfa_sdpa_decode_dev(c.h, 0, dq.ptr, dg.ptr, out.ptr)
+            assert rt().hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == 0
+            assert rt().hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+            for _ in range(3):
+                assert rt().hipGraphLaunch(run, stream) == 0
+                c.sync()
+                got = out.to_host()
+                if what == "chunk":
+                    assert rel_err(got, want) <= TOL
+                else:
+                    assert np.array_equal(got[0], want_short)
+                    assert np.array_equal(c.sdpa_decode(0, q[0], g[0]), want_short)   # eager work in between
+            assert rt().hipGraphExecDestroy(run) == 0 and rt().hipGraphDestroy(graph) == 0
