@@ -524,8 +524,10 @@ __global__ __launch_bounds__(256) void sdpa_chunk_merge_kernel(const ChunkArgs a
                 v[s][i] = vec_load((const uint4 *)(po + (size_t)(s0 + s < a.nsplit ? s0 + s : a.nsplit - 1) * rw_count * (NT * 4 * 64) + i * 64));
 #pragma unroll
         for (int s = 0; s < 4; s++) {
-            // a split that saw nothing of the row weighs nothing, whatever its part of the workspace holds
-            const float w = (s0 + s < a.nsplit && m[s0 + s] != neg_inf()) ? fast_exp2(m[s0 + s] - M) : 0.f;
+            // a split that saw nothing of the row (sum 0) weighs nothing, whatever its part of the workspace holds; one
+            // that saw nothing but NaN has no maximum either, and its sum carries them into the result
+            const float none = l[s0 + s] == 0.f ? 0.f : l[s0 + s];
+            const float w = s0 + s < a.nsplit ? (m[s0 + s] != neg_inf() ? fast_exp2(m[s0 + s] - M) : none) : 0.f;
             if (w != 0.f) {
                 den += w * l[s0 + s];
 #pragma unroll

@@ -62,6 +62,23 @@ def test_chunk_split_with_peaked_scores(mfa, oracle):
     assert rel_err(out, ref) <= 2e-3
 
 
+@pytest.mark.parametrize("Hq,Hkv,d,T,L0", [(16, 2, 256, 203, 3001), (32, 4, 128, 128, 4000), (16, 2, 64, 40, 5000)])
+def test_chunk_split_of_nothing_but_nan(mfa, oracle, Hq, Hkv, d, T, L0):
+    """The first n keys of a kv head are NaN, for every n that a split of the cache may end at: the rows of its query heads
+    are NaN, as in the token loop, and the other heads' are what they were."""
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, 5)
+    ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, q, g, k, v).reshape(T, Hkv, -1)
+    with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+        for n in range(32, 1600, 32):
+            bad = k.copy()
+            bad[:n, :d] = np.nan
+            c.memory_clear()
+            c.kv_import(0, bad[:L0], v[:L0])
+            out = c.prefill_attn(0, q, g, bad[L0:], v[L0:]).reshape(T, Hkv, -1)
+            assert np.isnan(out[:, 0]).all(), n
+            assert rel_err(out[:, 1:], ref[:, 1:]) <= TOL
+
+
 @pytest.mark.parametrize("Hq,Hkv,d,T,L0,rotary", [
     (32, 4, 128, 70, 0, 32), (16, 2, 256, 70, 41, 64), (32, 4, 128, 40, 2500, 32), (16, 2, 256, 50, 1990, 64),
     (16, 2, 256, 50, 1990, 32), (8, 2, 64, 70, 41, 16),     # not a quarter of the head, head_dim 64: a prologue of its own
