@@ -31,9 +31,14 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 // One 1 KiB piece from memory to LDS without passing through registers: lane l's 16 bytes land at
 // lds + 16 l.  As assembly, because the compiler waits for every such load in flight ahead of every LDS
 // read; the kernel's own wait (wait_pieces) counts them.
+// m0 is a clobber: a builtin that needs it then sets it again behind this.  (The compiler's warning is that it does
+// not keep a reserved register's value across the statement, which is what is wanted.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ inline void copy_piece(const uint4 *src, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 template <int N> __device__ inline void wait_pieces_and_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }

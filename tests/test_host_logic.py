@@ -125,3 +125,20 @@ def test_split_partitioning():
         prev = got
     assert ns(ffi.KV_BF16, 30, 4, 128, 64, 256, 0) == -1          # 30 % 4 != 0
     assert ns(ffi.KV_BF16, 32, 2, 256, 0, 256, 0) == -1
+
+
+def test_inline_assembly_declares_m0():
+    """m0 written by an assembly statement and not among its clobbers is m0 taken from whatever the compiler keeps there."""
+    import os
+    import re
+
+    from moeflux_amd import build
+    files = [f for f in os.listdir(build.CSRC) if f.endswith((".hip", ".h"))]
+    writes = 0
+    for f in files:
+        src = open(os.path.join(build.CSRC, f)).read()
+        for stmt in re.findall(r"\basm\b[^;]*?\((.*?)\)\s*;", src, re.S):
+            if re.search(r"\bm0\s*,", stmt.split(":")[0]):
+                writes += 1
+                assert '"m0"' in stmt, (f, stmt)
+    assert writes > 0
