@@ -771,7 +771,9 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
     const ChunkPlan plan = chunk_plan(c, T, (int64_t)f->len + T);
     const bool raw = plan.applies && sdpa_chunk_takes_raw(c->cfg.head_dim, c->rotary_dim) &&
                      (out_dev + qd <= q_proj_out_dev || q_proj_out_dev + 2 * qd <= out_dev);
-    const size_t need = raw ? (size_t)T * c->rotary_dim : 2 * qd;
+    // Sized for either route (the table is T * rotary_dim floats, less than a head's rows), so that no later chunk of as
+    // many tokens moves it: not one under capture, and none from under a graph that was captured.
+    const size_t need = 2 * qd;
     if (need > c->qg_chunk_elems) {
         MFA_HIP(hipStreamSynchronize(c->stream));
         if (c->qg_chunk) MFA_HIP(hipFree(c->qg_chunk));

@@ -156,3 +156,69 @@ def test_chunk_and_short_decode_in_a_captured_graph(mfa, oracle):
                     assert np.array_equal(got[0], want_short)
                     assert np.array_equal(c.sdpa_decode(0, q[0], g[0]), want_short)   # eager work in between
             assert rt().hipGraphExecDestroy(run) == 0 and rt().hipGraphDestroy(graph) == 0
+
+
+class _Graph:
+    """What `call` puts on a context's stream, captured (relaxed: other streams are not held up)."""
+
+    def __init__(self, c, call):
+        import ctypes as C
+
+        from moeflux_amd.hip import rt
+        self.c, self.rt, self.stream, self.graph, self.run = c, rt(), C.c_void_p(c.lib.mfa_stream(c.h)), C.c_void_p(), C.c_void_p()
+        assert self.rt.hipStreamBeginCapture(self.stream, C.c_int(2)) == 0
+        rc = call()
+        end = self.rt.hipStreamEndCapture(self.stream, C.byref(self.graph))
+        assert rc == 0, c.lib.mfa_last_error_string()
+        assert end == 0
+        assert self.rt.hipGraphInstantiate(C.byref(self.run), self.graph, None, None, C.c_size_t(0)) == 0
+
+    def __call__(self):
+        assert self.rt.hipGraphLaunch(self.run, self.stream) == 0
+        self.c.sync()
+
+    def close(self):
+        assert self.rt.hipGraphExecDestroy(self.run) == 0 and self.rt.hipGraphDestroy(self.graph) == 0
+
+
+@pytest.mark.parametrize("first", ["over the projection", "apart"])
+def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first):
+    """A chunk whose result lies over its projection (a prologue of its own) captured behind one of as many tokens whose
+    result lies apart (query normed in the attention launch), and the other way round; then the first route again, eagerly,
+    and replays."""
+    from moeflux_amd.hip import H2D, DeviceArray, rt
+    Hq, Hkv, d, T = 16, 2, 256, 300
+    rng = np.random.default_rng(4)
+    norm = [oracle.f32_to_bf16(1.0 + 0.3 * rng.standard_normal(d)) for _ in range(2)]
+    qp = rng.standard_normal((T, Hq * 2 * d)).astype(np.float32)
+    k, v = (rng.standard_normal((T, Hkv * d)).astype(np.float32) for _ in range(2))
+    dk, dv = (DeviceArray.from_host(x) for x in (k, v))
+    with _ctx(mfa, Hq, Hkv, d, T) as c:
+        c.set_full_weights(0, *norm)
+        want = c.prefill_full_attn(0, 0, qp, k, v)
+        bufs = {"apart": (DeviceArray.from_host(qp), DeviceArray((T, Hq * d), zero=True)), "over the projection": (DeviceArray.from_host(qp),) * 2}
+
+        def call(where):
+            q, out = bufs[where]
+            return c.lib.mfa_prefill_full_attn_dev(c.h, 0, 0, T, q.ptr, dk.ptr, dv.ptr, out.ptr)
+
+        def check(where):
+            assert rel_err(bufs[where][1].to_host().reshape(-1)[:T * Hq * d].reshape(T, Hq * d), want) <= TOL
+            assert rt().hipMemcpy(bufs[where][0].ptr, qp.ctypes.data, qp.nbytes, H2D) == 0
+
+        second = next(w for w in bufs if w != first)
+    with _ctx(mfa, Hq, Hkv, d, T) as c:   # its scratch is of its own first chunk
+        c.set_full_weights(0, *norm)
+        assert call(first) == 0
+        c.sync()
+        check(first)
+        c.memory_clear()
+        graph = _Graph(c, lambda: call(second))
+        for _ in range(3):
+            graph()
+            check(second)
+            c.memory_clear()
+            assert call(first) == 0
+            c.sync()
+            check(first)
+        graph.close()
