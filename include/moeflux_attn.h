@@ -465,6 +465,18 @@ int32_t mfa_debug_num_splits(int32_t kv_dtype, int32_t num_attn_heads, int32_t n
 int32_t mfa_debug_max_splits(int32_t kv_dtype, int32_t num_attn_heads, int32_t num_kv_heads,
                              int32_t head_dim, int64_t max_len, int32_t num_cus,
                              int32_t forced_splits);
+/* No counterpart in the reference.  The kernel that takes a prompt chunk of n_tok tokens at the
+ * end of a cache of kv_len positions (raw: from raw projections): 0 split-K, 1 16-row groups
+ * over the whole cache, 1000 * row waves of a workgroup (2 or 4) + splits of the cache for
+ * 32x32 tiles; -1 on a bad argument. */
+int32_t mfa_debug_chunk_route(int32_t kv_dtype, int32_t num_attn_heads, int32_t num_kv_heads,
+                              int32_t head_dim, int32_t n_tok, int64_t kv_len, int32_t num_cus,
+                              int32_t raw);
+/* Prompt chunks of a context over a bf16 cache take the given kernel (1 or 1000 * row waves +
+ * splits, as above; the splits at most the cache's blocks of 32 positions), -1 (default): by their
+ * sizes.  A measurement and test switch; no result depends on it beyond rounding.  A chunk whose
+ * partials would not fit the workspace is refused. */
+int mfa_debug_set_chunk_route(mfa_ctx *ctx, int32_t route);
 
 /* A plain device-to-device copy kernel on the context's stream (nbytes read, nbytes
  * written, nbytes a multiple of 16): a launch of known memory traffic, used to scale

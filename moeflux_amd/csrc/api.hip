@@ -331,64 +331,62 @@ static int ensure_workspace(Ctx *c, int n_tok, int64_t kv_len, int layers = 1) {
                                   sdpa_workspace_ml_elems(Hq, Hkv, splits, n_tok));
 }
 
-// The plan of a prompt chunk on 32x32 tiles (not with a forced split count, which is the decode kernel's).  The first
-// plan that splits the cache allocates the workspace, whose size never changes; while the stream is being captured,
-// or without memory for it, the plan is one that needs none.
-static ChunkPlan chunk_plan(Ctx *c, int n_tok, int64_t kv_len) {
+// The plan of a prompt chunk (a forced split count is the split-K kernel's), and the memory it takes.  The first plan that
+// splits the cache on 32x32 tiles allocates their workspace, whose size never changes; without memory for it, or while
+// the stream is being captured, the plan is one that needs none.
+// Everything that sdpa_dev could still refuse is refused here, while the cache is as the caller left it.
+static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, ChunkPlan *out) {
     const mfa_config &g = c->cfg;
-    if (c->forced_splits || c->partial_only) return ChunkPlan{};
-    const auto plan = [&](size_t ws_elems) {
-        return sdpa_chunk_plan(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, kv_len, c->num_cus, ws_elems);
+    ChunkPlan &p = *out;
+    p = ChunkPlan{};
+    const auto plan = [&](size_t ws_elems, bool split_k) {
+        return sdpa_chunk_plan(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, kv_len, c->num_cus, kind,
+                               ChunkLimits{ws_elems, split_k});
     };
-    const ChunkPlan p = plan(kChunkPartElems);
-    if (p.splits <= 1 || c->chunk_part) return p;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return plan(0);
-    if (hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
-        (void)hipGetLastError();
-        c->chunk_part = nullptr;
-        return plan(0);
+    const auto capturing = [&] {
+        hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+        return hipStreamIsCapturing(c->stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+    };
+    if (!c->forced_splits && !c->partial_only) {
+        p = plan(kChunkPartElems, true);
+        if (c->chunk_route > 0 && g.kv_dtype == MFA_KV_BF16 && n_tok > 1) {
+            p = c->chunk_route == 1 ? ChunkPlan{ChunkRoute::Rows}
+                                    : sdpa_chunk_plan_of(g.num_attn_heads, g.num_kv_heads, n_tok, kv_len, c->chunk_route / 1000, c->chunk_route % 1000);
+            if (sdpa_chunk_part_elems(p, g.num_kv_heads, g.head_dim) > kChunkPartElems)
+                return fail(MFA_ERR_INVALID, "sdpa: %d splits of the chunk do not fit its workspace", p.splits);
+        }
+        if (p.route == ChunkRoute::Tiles32 && p.splits > 1 && !c->chunk_part) {
+            if (!capturing() && hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
+                (void)hipGetLastError();
+                c->chunk_part = nullptr;
+            }
+            if (c->chunk_part) c->chunk_part_elems = kChunkPartElems;
+            else p = plan(0, true);
+        }
     }
-    c->chunk_part_elems = kChunkPartElems;
-    return p;
-}
-
-// What sdpa_dev could still refuse for n_tok tokens over a cache of kv_len positions, checked
-// (and the split-K workspace grown) while the cache is as the caller left it.
-static int sdpa_prepare(Ctx *c, int n_tok, int64_t kv_len) {
-    const mfa_config &g = c->cfg;
-    if (chunk_plan(c, n_tok, kv_len).applies) return MFA_OK;
-    if (!c->forced_splits && !c->partial_only &&
-        sdpa_prefill_applies(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, n_tok, kv_len, c->num_cus))
-        return MFA_OK;   // one launch, no workspace
+    if (p.route != ChunkRoute::SplitK) return MFA_OK;
     const int64_t nhg = ((int64_t)n_tok * (g.num_attn_heads / g.num_kv_heads) + 15) / 16;
     if (nhg > 65535) return fail(MFA_ERR_SHAPE, "sdpa: too many query rows in one call");
-    if (n_tok > 1) MFA_TRY(ensure_workspace(c, n_tok, kv_len));
-    return MFA_OK;
+    if (n_tok == 1) return MFA_OK;
+    return ensure_workspace(c, n_tok, kv_len);
 }
 
 // n_tok tokens whose K/V rows are already in the cache (the last n_tok positions).
-static int sdpa_dev(Ctx *c, FullLayer *f, int n_tok, const float *q, const float *gate, float *out) {
+static int sdpa_dev(Ctx *c, FullLayer *f, int n_tok, const float *q, const float *gate, float *out, const ChunkPlan &p) {
     if (f->len <= 0) return fail(MFA_ERR_INVALID, "kv_len must be > 0 (got %d)", f->len);
-    const ChunkPlan p = chunk_plan(c, n_tok, f->len);
-    if (p.applies)
-        return launch_sdpa_chunk(c->stream, p, c->cfg.num_attn_heads, c->cfg.num_kv_heads, c->cfg.head_dim, n_tok, f->len,
-                                 c->plane_elems, f->k, f->v, ChunkQuery{q, gate, c->cfg.head_dim}, out, c->chunk_part,
-                                 c->chunk_part_elems);
-    if (!c->forced_splits && !c->partial_only &&
-        sdpa_prefill_applies(c->cfg.kv_dtype, c->cfg.num_attn_heads, c->cfg.num_kv_heads, n_tok, f->len,
-                             c->num_cus))
-        return launch_sdpa_prefill(c->stream, c->cfg.kv_dtype, c->cfg.num_attn_heads, c->cfg.num_kv_heads,
-                                   c->cfg.head_dim, n_tok, f->len, c->plane_elems, f->k, f->v, q, gate, out,
-                                   c->num_cus);
-    if (n_tok > 1) MFA_TRY(ensure_workspace(c, n_tok, f->len));
-    return launch_sdpa(c->stream, c->cfg.kv_dtype, c->cfg.num_attn_heads, c->cfg.num_kv_heads,
-                       c->cfg.head_dim, n_tok, f->len, c->plane_elems, f->k, f->v, q, gate, out,
-                       workspace(c), c->num_cus, c->forced_splits, c->partial_only);
+    const mfa_config &g = c->cfg;
+    if (p.route == ChunkRoute::Tiles32)
+        return launch_sdpa_chunk(c->stream, p, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, f->len, c->plane_elems, f->k,
+                                 f->v, ChunkQuery{q, gate, g.head_dim}, out, c->chunk_part, c->chunk_part_elems);
+    if (p.route == ChunkRoute::Rows)
+        return launch_sdpa_prefill(c->stream, g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, f->len,
+                                   c->plane_elems, f->k, f->v, q, gate, out, c->num_cus);
+    return launch_sdpa(c->stream, g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, f->len, c->plane_elems, f->k,
+                       f->v, q, gate, out, workspace(c), c->num_cus, c->forced_splits, c->partial_only);
 }
 
 static int sdpa_decode_dev(Ctx *c, FullLayer *f, const float *q, const float *gate, float *out) {
-    return sdpa_dev(c, f, 1, q, gate, out);
+    return sdpa_dev(c, f, 1, q, gate, out, ChunkPlan{});
 }
 
 static int kv_append_dev(Ctx *c, FullLayer *f, const float *k, const float *v, int64_t rows) {
@@ -765,12 +763,13 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
     if ((int64_t)f->len + T > c->cfg.kv_capacity)
         return fail(MFA_ERR_OVERFLOW, "kv cache overflow: len %d + %d > capacity %d", f->len, T, c->cfg.kv_capacity);
     const size_t qd = (size_t)c->q_dim() * T;
-    MFA_TRY(sdpa_prepare(c, T, (int64_t)f->len + T));
-    // The chunk kernel takes the query and its gate from the projection itself (unless the caller's result would
+    // The 32x32-tile kernel takes the query and its gate from the projection itself (unless the caller's result would
     // overwrite rows it has yet to read): all the launch ahead of it leaves is the tokens' rotation table.
-    const ChunkPlan plan = chunk_plan(c, T, (int64_t)f->len + T);
-    const bool raw = plan.applies && sdpa_chunk_takes_raw(c->cfg.head_dim, c->rotary_dim) &&
-                     (out_dev + qd <= q_proj_out_dev || q_proj_out_dev + 2 * qd <= out_dev);
+    const bool apart = out_dev + qd <= q_proj_out_dev || q_proj_out_dev + 2 * qd <= out_dev;
+    const ChunkQueryKind kind = apart && sdpa_chunk_takes_raw(c->cfg.head_dim, c->rotary_dim) ? ChunkQueryKind::Raw : ChunkQueryKind::RawPrologue;
+    ChunkPlan plan;
+    MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, kind, &plan));
+    const bool raw = plan.route == ChunkRoute::Tiles32 && kind == ChunkQueryKind::Raw;
     // Sized for either route (the table is T * rotary_dim floats, less than a head's rows), so that no later chunk of as
     // many tokens moves it: not one under capture, and none from under a graph that was captured.
     const size_t need = 2 * qd;
@@ -803,7 +802,7 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
                               k_dev + (size_t)off * c->kv_dim(), v_dev + (size_t)off * c->kv_dim(),
                               c->qg_chunk + (size_t)off * c->q_dim(), c->qg_chunk + qd + (size_t)off * c->q_dim(), n);
         }
-        if (rc == MFA_OK) rc = sdpa_dev(c, f, T, c->qg_chunk, c->qg_chunk + qd, out_dev);
+        if (rc == MFA_OK) rc = sdpa_dev(c, f, T, c->qg_chunk, c->qg_chunk + qd, out_dev, plan);
     }
     if (rc != MFA_OK) rollback_append(c, f, len0);   // a launch refused after all: the cache is as before the call
     return rc;
@@ -837,11 +836,12 @@ int mfa_prefill_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t T, const float *q_
     if ((int64_t)f->len + T > c->cfg.kv_capacity)
         return fail(MFA_ERR_OVERFLOW, "kv cache overflow: len %d + %d > capacity %d", f->len, T,
                     c->cfg.kv_capacity);
-    MFA_TRY(sdpa_prepare(c, T, (int64_t)f->len + T));
+    ChunkPlan plan;
+    MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, ChunkQueryKind::Normed, &plan));
     // append the whole chunk, then one causal pass: row t sees positions [0, len0 + t]
     const int32_t len0 = f->len;
     int rc = kv_append_dev(c, f, k_dev, v_dev, T);
-    if (rc == MFA_OK) rc = sdpa_dev(c, f, T, q_dev, q_gate_dev, out_dev);
+    if (rc == MFA_OK) rc = sdpa_dev(c, f, T, q_dev, q_gate_dev, out_dev, plan);
     if (rc != MFA_OK) rollback_append(c, f, len0);
     return rc;
 }
@@ -1262,6 +1262,25 @@ int32_t mfa_debug_max_splits(int32_t kv_dtype, int32_t Hq, int32_t Hkv, int32_t 
         num_cus <= 0)
         return -1;
     return sdpa_max_splits(kv_dtype, Hq, Hkv, D, max_len, num_cus, forced_splits);
+}
+
+int32_t mfa_debug_chunk_route(int32_t kv_dtype, int32_t Hq, int32_t Hkv, int32_t D, int32_t n_tok, int64_t kv_len,
+                              int32_t num_cus, int32_t raw) {
+    if (!sdpa_shape_supported(kv_dtype, D) || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || n_tok <= 0 || kv_len < n_tok || num_cus <= 0)
+        return -1;
+    const ChunkQueryKind kind = !raw ? ChunkQueryKind::Normed : sdpa_chunk_takes_raw(D, D / 4) ? ChunkQueryKind::Raw : ChunkQueryKind::RawPrologue;
+    const ChunkPlan p = sdpa_chunk_plan(kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, kind, ChunkLimits{kChunkPartElems, true});
+    return p.route == ChunkRoute::SplitK ? 0 : p.route == ChunkRoute::Rows ? 1 : 1000 * p.rw + p.splits;
+}
+
+int mfa_debug_set_chunk_route(mfa_ctx *ctx, int32_t route) {
+    Ctx *c = as_ctx(ctx);
+    if (!c) return fail(MFA_ERR_INVALID, "NULL context");
+    const int rw = route / 1000, splits = route % 1000;
+    if (route != -1 && route != 1 && !((rw == 2 || rw == 4) && splits >= 1 && splits <= kMaxChunkSplits))
+        return fail(MFA_ERR_INVALID, "chunk route %d", route);
+    c->chunk_route = route;
+    return MFA_OK;
 }
 
 int mfa_debug_copy_dev(mfa_ctx *ctx, void *dst_dev, const void *src_dev, size_t nbytes) {

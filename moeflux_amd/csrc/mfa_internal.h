@@ -164,6 +164,7 @@ struct Ctx {
     size_t part_o_elems = 0, part_ml_elems = 0;
     int32_t forced_splits = 0;
     int32_t partial_only = 0;
+    int32_t chunk_route = -1;    // of prompt chunks over a bf16 cache (mfa_debug_set_chunk_route)
     // partials of a split prompt chunk (sdpa_chunk.hip), allocated by the first one, of a size that never changes
     float *chunk_part = nullptr;
     size_t chunk_part_elems = 0;
@@ -284,17 +285,18 @@ int launch_attn_prologue_kv(hipStream_t s, int kv_dtype, int Hkv, int D, int rot
                             const float *k_in, const float *v_in, float2 *table, void *k_tiled, void *v_tiled);
 // sdpa_prefill.hip: the same contract for a chunk whose rows fill the machine without
 // splitting the cache (no workspace, one launch).
-bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_len, int num_cus);
 int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                         size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                         const float *gate, float *out, int num_cus);
 // sdpa_chunk.hip: the same for a bf16 cache on 32x32 matrix tiles; `splits` > 1 leaves partials in a
-// workspace and merges them in a second launch.
+// workspace and merges them in a second launch.  Which of the three a chunk takes is part of its plan.
+enum class ChunkRoute { SplitK, Rows, Tiles32 };   // launch_sdpa, launch_sdpa_prefill, launch_sdpa_chunk
 struct ChunkPlan {
-    bool applies;     // false: the split-K decode kernel serves the chunk
-    int rw, ks;       // row waves (32 rows each) and wave sets of a workgroup
-    int nrt;          // row tiles of 32 * rw rows per kv head
-    int splits, bps;  // splits of the cache, blocks of 32 positions per split
+    ChunkRoute route = ChunkRoute::SplitK;
+    // Tiles32
+    int rw = 0, ks = 0;       // row waves (32 rows each) and wave sets of a workgroup
+    int nrt = 0;              // row tiles of 32 * rw rows per kv head
+    int splits = 0, bps = 0;  // splits of the cache, blocks of 32 positions per split
 };
 // Workspace of a context: the partial rows of a split chunk are at most kChunkPartElems floats (33.5 MB, two
 // workgroups per CU of 128 rows x 128 channels), their maxima and sums a 32nd of that.
@@ -309,7 +311,20 @@ struct ChunkQuery {
     float eps = 0.f;
 };
 bool sdpa_chunk_takes_raw(int D, int rotary_dim);
-ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, size_t ws_elems);
+// What precedes a chunk's attention: nothing (the query is handed over), or the prologue of raw projections, of which the
+// Tiles32 route leaves the query to the attention launch where it can (sdpa_chunk_takes_raw).
+enum class ChunkQueryKind { Normed, Raw, RawPrologue };
+// What a plan may use: a workspace of ws_elems floats for split Tiles32 partials, and the split-K kernel.
+struct ChunkLimits {
+    size_t ws_elems;
+    bool split_k;
+};
+static constexpr int kMaxChunkSplits = 16;
+// The plan of the given shape of a workgroup, with at most `splits` splits.
+ChunkPlan sdpa_chunk_plan_of(int Hq, int Hkv, int n_tok, int64_t kv_len, int rw, int splits);
+size_t sdpa_chunk_part_elems(const ChunkPlan &p, int Hkv, int D);   // floats of its partials
+ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, ChunkQueryKind kind,
+                          const ChunkLimits &limits);
 int launch_sdpa_chunk(hipStream_t stream, const ChunkPlan &plan, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                       size_t plane_elems, const void *k_tiled, const void *v_tiled, const ChunkQuery &in, float *out,
                       float *ws, size_t ws_elems);

@@ -43,8 +43,6 @@ template <int N> __device__ inline void wait_pieces_and_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-static constexpr int kMaxChunkSplits = 16;
-
 struct ChunkArgs {
     const uint16_t *k, *v;
     size_t plane_elems;
@@ -558,30 +556,86 @@ __global__ __launch_bounds__(256) void sdpa_chunk_merge_kernel(const ChunkArgs a
 // Whether the kernel can norm and rotate the query rows itself (RowNorm).
 bool sdpa_chunk_takes_raw(int D, int rotary_dim) { return D >= 128 && rotary_dim * 4 == D; }
 
-// How a chunk is cut up: the shape of a workgroup and the splits of the cache of the smallest estimated cost, or no
-// plan at all where the split-K decode kernel (16-row groups, each streaming the cache by itself) is estimated
-// cheaper, which is where a chunk's rows are few and its cache is long.  The cost is the call's own time and one and a half
-// times the time of the whole device that it takes: a chunk's layers follow each other, but other sequences run beside them.
-// (34 chunks of 6 .. 1500 tokens behind 0 .. 12000 positions, every plan measured: this cost is on average 4 % behind the best
-// with three sequences side by side and 8 % in a call's own time; own time alone 7 and 5 %, three times the device's 2 and 15 %.)
-// Times in microseconds, fitted to launches measured over those chunks:
+// Which kernel takes a chunk, and how it is cut up.  Estimates in microseconds, with the kernels' constants by width
+// (64, 128, 256); `load` is workgroups per CU.
+//
+// On 32x32 tiles: the shape of a workgroup and the splits of the cache of the smallest cost, which is the call's own time and
+// one and a half times the time of the whole device that it takes: a chunk's layers follow each other, but other sequences may
+// run beside them.
 //   workgroup  kFixed (launch, query, first block, epilogue) + blocks per wave set * kBlock; a CU that holds two
 //              workgroups (head_dim <= 128) runs them 5 % faster than one after the other
 //   partials   written at 4.5 TB/s, merged at 7.5 TB/s with the gate and the result; 12 for the second launch
-//   decode     3 + the positions a CU streams * kStream, and its merge (6.9e-6 per output)
-// A split chunk's partials fit `ws_elems` floats.
-ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, size_t ws_elems) {
-    ChunkPlan best{};
-    if (kv_dtype != MFA_KV_BF16 || n_tok < 2 || !sdpa_shape_supported(kv_dtype, D)) return best;
-    static constexpr double kFixed[2][3] = {{6.0, 9.0, 12.0}, {7.0, 9.0, 14.0}}, kBlock[2][3] = {{0.5, 0.8, 1.58}, {0.55, 0.85, 1.85}};
+// A split chunk's partials fit limits.ws_elems floats.
+//
+// That kernel's workgroups begin slowly (32 query rows a wave in 512 registers), so that a short cache, or few rows before a
+// long one, are better served by 16-row groups: by sdpa_prefill (Rows) up to 2048 positions, by the split-K kernel beyond.  They
+// are taken where one sequence after itself is estimated faster with them (sequences side by side are bound by the
+// launches there, and so no slower).  The estimates are fitted to 800 chunks of 2 .. 1024 tokens behind 0 .. 16384 positions
+// (32 and 16 heads over 2 of 256, 32 over 4 and over 32 of 128, 16 over 2 of 64), normed and raw, every route of
+// every chunk measured: 8 % r.m.s. on a time, and of the routes they choose 29 of 1600 are more than 3 % slower than the
+// 16-row groups for one sequence, one 14 %; without them 418 were, up to 62 %, most of them small (2 .. 64 tokens of 32 heads over 2
+// of 256 from an empty cache 21 us a layer, 14 to 18 with 16-row groups).
+static constexpr double kFixed[2][3] = {{6.0, 9.0, 12.0}, {7.0, 9.0, 14.0}}, kBlock[2][3] = {{0.5, 0.8, 1.58}, {0.55, 0.85, 1.85}};
+
+struct ChunkShape {
+    int w, Hq, Hkv, D, n_tok;
+    int64_t rows, kv_len, nblk;
+    double num_cus;
+    bool causal() const { return kv_len - n_tok < n_tok; }   // most of the work is the triangle: tiles differ, the longest go first
+    double seen() const { return causal() ? ((double)(kv_len - n_tok) + 0.5 * n_tok) / (double)kv_len : 1.0; }
+    // the prologue of raw projections: all heads of a token, 16 bytes a q channel and fewer of k and v
+    double prologue() const { return 0.5 + 3.6e-6 * n_tok * (double)(Hq + 2 * Hkv) * D; }
+};
+
+// One sequence's time of a layer, prologue included, behind another of its own.
+static double tiles32_time(const ChunkShape &c, const ChunkPlan &p, ChunkQueryKind kind) {
+    static constexpr double kStart[2][3] = {{9.0, 10.5, 16.0}, {10.0, 12.0, 18.0}}, kStep[2][3] = {{0.6, 1.0, 1.8}, {0.6, 1.05, 1.9}};
+    static constexpr double kRawQuery[3] = {0.5, 1.4, 2.5};   // norm and rotation in the launch; k, v and table ahead of it
+    const int shape = p.ks - 1, slots = c.D <= 128 ? 2 : 1;
+    const double its = (p.bps + p.ks - 1) / p.ks, load = (double)p.nrt * c.Hkv * p.splits / c.num_cus, rounds = ceil(load / slots);
+    const double step = kStep[shape][c.w] * (load > 1 && slots == 2 ? 0.95 : 1.0), start = kStart[shape][c.w];
+    double t = c.causal() ? fmax(start + its * step, start * rounds + load * its * c.seen() * step) : start * rounds + ceil(load) * its * step;
+    if (p.splits > 1) t += 4.0 + 4.0 * p.nrt * c.Hkv * p.splits * 32.0 * p.rw * c.D / 9e6;
+    if (kind == ChunkQueryKind::Raw) t += kRawQuery[c.w] + 8e-6 * c.n_tok * (double)c.Hkv * c.D;
+    if (kind == ChunkQueryKind::RawPrologue) t += c.prologue();
+    return t;
+}
+static double rows_time(const ChunkShape &c, int64_t wgs, ChunkQueryKind kind) {
+    static constexpr double kStart[3] = {8.2, 9.8, 11.5}, kStep[3] = {0.69, 1.0, 1.45};
+    const double its = (double)(c.D <= 128 ? (c.nblk + 1) / 2 : c.nblk);   // two wave sets where there is room for them
+    return kStart[c.w] + its * kStep[c.w] + 3.5 * (double)wgs / c.num_cus + 0.8e-6 * (double)c.kv_len * c.Hkv * c.D +
+           (kind == ChunkQueryKind::Normed ? 0.0 : c.prologue());
+}
+// (a row group streams its kv head's cache by itself, from its XCD's L2 or from memory)
+static double split_k_time(const ChunkShape &c, ChunkQueryKind kind) {
+    static constexpr double kStream[3] = {0.005, 0.010, 0.0173};
+    const int64_t nhg = (c.rows + 15) / 16, groups = nhg * c.Hkv;
+    int64_t splits = (int64_t)c.num_cus / groups;
+    if (splits > c.nblk / 4) splits = c.nblk / 4;
+    if (splits < 1) splits = 1;
+    const double load = (double)(groups * splits) / c.num_cus, kv = (double)c.kv_len;
+    const double xcds = nhg < 8 ? (double)nhg : 8.0;
+    return 12.0 + fmax(ceil(load) * kv / (double)splits * kStream[c.w], 4.0 * kv * c.Hkv * c.D * xcds / 6.5e6) +
+           7e-6 * (double)c.rows * c.Hkv * c.D + (kind == ChunkQueryKind::Normed ? 0.0 : c.prologue());
+}
+
+ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len, int num_cus, ChunkQueryKind kind,
+                          const ChunkLimits &limits) {
+    ChunkPlan best;
+    if (n_tok < 2 || !sdpa_shape_supported(kv_dtype, D)) return best;
+    const int64_t rows = (int64_t)n_tok * (Hq / Hkv), row_wgs = ((rows + 15) / 16 + 3) / 4 * Hkv;
+    if (kv_dtype != MFA_KV_BF16) {
+        // a short cache (nothing to gain from splitting it), or rows that alone give half the CUs a workgroup
+        if ((kv_len + 15) / 16 <= 64 || row_wgs >= num_cus / 2) best.route = ChunkRoute::Rows;
+        return best;
+    }
+    const ChunkShape c{D == 64 ? 0 : D == 128 ? 1 : 2, Hq, Hkv, D, n_tok, rows, kv_len, (kv_len + 31) / 32, (double)num_cus};
+    const int w = c.w, slots = D <= 128 ? 2 : 1;
+    const int64_t nblk = c.nblk;
+    if ((rows + 127) * Hkv > INT32_MAX / 2 || nblk > INT32_MAX / 2) return best;   // 32-bit row and block numbers
     static constexpr double kStream[3] = {0.007, 0.0108, 0.0175};
     static constexpr double kLaunch = 12.0, kEmpty = 2.5;   // of a workgroup's fixed time, what its CU is free in
-    const int w = D == 64 ? 0 : D == 128 ? 1 : 2, slots = D <= 128 ? 2 : 1;
-    const int64_t rows = (int64_t)n_tok * (Hq / Hkv), nblk = (kv_len + 31) / 32;
-    if ((rows + 127) * Hkv > INT32_MAX / 2 || nblk > INT32_MAX / 2) return best;   // 32-bit row and block numbers
-    const double out_bytes = 8.0 * (double)rows * Hkv * D;
-    const bool causal = kv_len - n_tok < n_tok;   // most of the work is the triangle: tiles differ, the longest go first
-    const double seen = causal ? ((double)(kv_len - n_tok) + 0.5 * n_tok) / (double)kv_len : 1.0;
+    const double out_bytes = 8.0 * (double)rows * Hkv * D, seen = c.seen();
     double best_cost = 0;
     for (int shape = 0; shape < 2; shape++) {
         const int rw = shape ? 2 : 4, ks = shape ? 2 : 1;
@@ -590,39 +644,52 @@ ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64
             const int64_t bps = (nblk + want - 1) / want;
             if ((nblk + bps - 1) / bps != want) continue;
             const size_t elems = want > 1 ? (size_t)(nrt * Hkv * want) * 32 * rw * D : 0;
-            if (elems > ws_elems) break;
+            if (elems > limits.ws_elems) break;
             const double its = (double)((bps + ks - 1) / ks), load = (double)(nrt * Hkv * want) / num_cus, fixed = kFixed[shape][w];
             const double block = kBlock[shape][w] * (load > 1 && slots == 2 ? 0.95 : 1.0), rounds = ceil(load / slots);
-            double t = causal ? fmax(fixed + its * block, fixed * rounds + load * its * seen * block) : fixed * rounds + ceil(load) * its * block;
+            double t = c.causal() ? fmax(fixed + its * block, fixed * rounds + load * its * seen * block) : fixed * rounds + ceil(load) * its * block;
             double busy = load * (fixed - kEmpty + its * seen * block);
             if (want > 1) {
                 const double moved = 4.0 * elems / 4.5e6 + (4.0 * elems + out_bytes) / 7.5e6;
                 t += moved + kLaunch;
                 busy += moved;
             }
-            if (!best.applies || t + 1.5 * busy < best_cost) {
+            if (best.route != ChunkRoute::Tiles32 || t + 1.5 * busy < best_cost) {
                 best_cost = t + 1.5 * busy;
-                best = ChunkPlan{true, rw, ks, (int)nrt, (int)want, (int)bps};
+                best = ChunkPlan{ChunkRoute::Tiles32, rw, ks, (int)nrt, (int)want, (int)bps};
             }
         }
     }
-    // (a cache of at most 64 blocks is not worth the second launch of the decode kernel)
-    if (nblk > 64) {
+    const double own = tiles32_time(c, best, kind);
+    if (nblk <= 64) {
+        // (past a workgroup per CU the 32x32 tiles are faster at every length)
+        if (row_wgs <= num_cus && rows_time(c, row_wgs, kind) <= own) best = ChunkPlan{ChunkRoute::Rows};
+    } else if (limits.split_k && row_wgs < num_cus / 2) {
         const int64_t groups = (rows + 15) / 16 * Hkv;
         int64_t splits = num_cus / groups;
         if (splits > nblk / 4) splits = nblk / 4;
         if (splits < 1) splits = 1;
         const double load = (double)(groups * splits) / num_cus, stream = (double)kv_len / (double)splits * kStream[w], merge = out_bytes / 8 * 6.9e-6;
-        if (3.0 + ceil(load) * stream + kLaunch + merge + 1.5 * (load * (stream + 1.0) + merge) < best_cost) return ChunkPlan{};
+        if (3.0 + ceil(load) * stream + kLaunch + merge + 1.5 * (load * (stream + 1.0) + merge) < best_cost || split_k_time(c, kind) <= own)
+            best = ChunkPlan{};
     }
     return best;
+}
+
+ChunkPlan sdpa_chunk_plan_of(int Hq, int Hkv, int n_tok, int64_t kv_len, int rw, int splits) {
+    const int64_t rows = (int64_t)n_tok * (Hq / Hkv), nblk = (kv_len + 31) / 32, bps = (nblk + splits - 1) / splits;
+    return ChunkPlan{ChunkRoute::Tiles32, rw, rw == 4 ? 1 : 2, (int)((rows + 32 * rw - 1) / (32 * rw)), (int)((nblk + bps - 1) / bps), (int)bps};
+}
+
+size_t sdpa_chunk_part_elems(const ChunkPlan &p, int Hkv, int D) {
+    return p.splits > 1 ? (size_t)Hkv * p.nrt * p.splits * 32 * p.rw * D : 0;
 }
 
 int launch_sdpa_chunk(hipStream_t stream, const ChunkPlan &p, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                       size_t plane_elems, const void *k_tiled, const void *v_tiled, const ChunkQuery &in,
                       float *out, float *ws, size_t ws_elems) {
-    const size_t elems = p.splits > 1 ? (size_t)Hkv * p.nrt * p.splits * 32 * p.rw * D : 0;
-    if (!p.applies || elems > ws_elems) return fail(MFA_ERR_INVALID, "sdpa: chunk plan without its workspace");
+    const size_t elems = sdpa_chunk_part_elems(p, Hkv, D);
+    if (p.route != ChunkRoute::Tiles32 || elems > ws_elems) return fail(MFA_ERR_INVALID, "sdpa: chunk plan without its workspace");
     const int hpk = Hq / Hkv;
     ChunkArgs a{(const uint16_t *)k_tiled, (const uint16_t *)v_tiled, plane_elems, in, hpk, Hq, n_tok, kv_len - n_tok,
                 (1.0f / sqrtf((float)D)) * kLog2e, out, ws, ws + elems, p.nrt, p.splits, p.bps, Hkv * p.splits,

@@ -1,5 +1,6 @@
-// Causal attention of a prompt chunk over a tiled f32 KV cache, for chunks large enough
-// that the query rows alone fill the machine (a bf16 cache: sdpa_chunk.hip).
+// Causal attention of a prompt chunk over the tiled KV cache, for chunks large enough
+// that the query rows alone fill the machine, and for small chunks over short caches (of a bf16
+// cache these only: sdpa_chunk_plan).
 //
 // The reference has no batched prefill: eval_prompt is a token loop
 // (crates/moeflux/src/riir/mod.rs:1196-1214) whose every token runs the decode chain of
@@ -9,7 +10,7 @@
 // A workgroup is 4 waves; every wave owns RG groups of 16 query rows (rows of one kv
 // head: token-major, then the hpk query heads that share it) from start to end: its
 // query operands and its output tiles stay in registers and its soft-max needs no other
-// wave.  The workgroup walks the cache blocks (of V: 16 positions) that its rows may see; each
+// wave.  The workgroup walks the cache blocks (of V: 32 or 16 positions) that its rows may see; each
 // block's K and V (already in MFMA operand order in memory) is copied into LDS once by all 256 threads,
 // double buffered, and every wave takes its operands from there.  With RG = 2 an operand
 // read from LDS feeds two row groups.  Nothing is split along the cache, so the gated,
@@ -95,14 +96,18 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         fetch(std::integral_constant<int, 2>{}, 2);
         fetch(std::integral_constant<int, 3>{}, 3);
     }
+    // A bf16 cache's scores are products of the raw query, split into a bf16 high and low part, and are
+    // scaled as they leave the matrix core: a query that is exact in bf16 (what a bf16 model hands
+    // over) then has no low parts, and a wave all of whose rows are such leaves their products out.
     uint4 qr[RG][W::QREGS];
+    bool q_exact = true;
     int64_t limit[RG], limit_min[RG], limit_max[RG];
     bool full[RG];
 #pragma unroll
     for (int r = 0; r < RG; r++) {
         const RowGroup rows{kvh, hg0 + r, hpk, Hq, n_tok, kv_len0};
         if (KS == 1 || ks == 0) {   // uniform over the wave
-            W::load_q_regs(qr[r], q, lane, rows, qscale);
+            W::load_q_regs(qr[r], q, lane, rows, W::kScaleAfter ? 1.0f : qscale);
             if constexpr (KS > 1) {
 #pragma unroll
                 for (int i = 0; i < W::QREGS; i++) s_q[(rw * RG + r) * W::QREGS + i][lane] = qr[r][i];
@@ -123,6 +128,9 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
                 for (int i = 0; i < W::QREGS; i++) qr[r][i] = s_q[(rw * RG + r) * W::QREGS + i][lane];
         }
     }
+#pragma unroll
+    for (int r = 0; r < RG; r++) q_exact = q_exact && W::q_low_parts_zero(qr[r]);
+    q_exact = __all(q_exact);
     int64_t wave_max = limit_max[0];
 #pragma unroll
     for (int r = 1; r < RG; r++) wave_max = limit_max[r] > wave_max ? limit_max[r] : wave_max;
@@ -145,8 +153,13 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         uint4 kreg[NLOAD];
 #pragma unroll
         for (int i = 0; i < NLOAD; i++) kreg[i] = cur[i * 64 + lane];
+        if (q_exact) {
 #pragma unroll
-        for (int r = 0; r < RG; r++) W::scores_reg(kreg, qr[r], sc[r]);
+            for (int r = 0; r < RG; r++) W::template scores_reg<true>(kreg, qr[r], sc[r]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < RG; r++) W::template scores_reg<false>(kreg, qr[r], sc[r]);
+        }
     };
     auto finish = [&](int64_t b, const uint4 *cur, const typename W::Scores (&sc)[RG]) __attribute__((always_inline)) {
         uint4 p[RG][W::P_U4];
@@ -154,6 +167,9 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
         for (int r = 0; r < RG; r++) {
             float x[NX];
             W::unpack(sc[r], x);
+            // kScaleAfter: x is unscaled; the scale (positive) enters the row maximum once and the
+            // exponentials' arguments as a fused multiply-add
+            const float xs = W::kScaleAfter ? qscale : 1.0f;
             if (!full[r] || (b + 1) * W::BLK > limit_min[r]) {  // a block some row must not see in full
 #pragma unroll
                 for (int e = 0; e < NX; e++)
@@ -163,6 +179,7 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
 #pragma unroll
             for (int e = 1; e < NX; e++) m_loc = fmaxf(m_loc, x[e]);
             m_loc = rows_max(m_loc);
+            if constexpr (W::kScaleAfter) m_loc *= xs;
             // m_loc > -inf + 8 is false while the row has seen nothing, so m_ref stays
             // -inf; the exponent's reference is then 0 and every probability is 0.
             const bool move = m_loc > m_ref[r] + kLazyRescale;
@@ -175,7 +192,7 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
             float e[NX], psum = 0.f;
 #pragma unroll
             for (int i = 0; i < NX; i++) {
-                e[i] = fast_exp2(x[i] - ref);  // 0 for masked positions
+                e[i] = fast_exp2(W::kScaleAfter ? fmaf(x[i], xs, -ref) : x[i] - ref);  // 0 for masked positions
                 psum += e[i];
             }
             l_run[r] = l_run[r] * alpha + psum;
@@ -331,21 +348,10 @@ __global__ __launch_bounds__(64 * RW * KS) void sdpa_prefill_kernel(
     }
 }
 
-// Whether a chunk of n_tok tokens is better served by this kernel than by the split-K
-// row-group path: either the cache is short (nothing to gain from splitting it) or the
-// rows alone give at least half the CUs a workgroup.
-bool sdpa_prefill_applies(int kv_dtype, int Hq, int Hkv, int n_tok, int64_t kv_len, int num_cus) {
-    if (kv_dtype != MFA_KV_F32 || n_tok < 2) return false;
-    const int64_t nblk = (kv_len + 15) / 16;
-    const int64_t nhg = ((int64_t)n_tok * (Hq / Hkv) + 15) / 16;
-    const int64_t nwg = (nhg + 3) / 4 * Hkv;
-    return nblk <= 64 || nwg >= num_cus / 2;
-}
-
 int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                         size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                         const float *gate, float *out, int num_cus) {
-    if (kv_dtype != MFA_KV_F32 || !sdpa_shape_supported(kv_dtype, D))
+    if (!sdpa_shape_supported(kv_dtype, D))
         return fail(MFA_ERR_SHAPE, "sdpa: head_dim %d / kv dtype %d not supported", D, kv_dtype);
     if (n_tok <= 0 || kv_len < n_tok)
         return fail(MFA_ERR_INVALID, "sdpa: kv_len must be > 0 (got %lld for %d tokens)", (long long)kv_len, n_tok);
@@ -358,27 +364,33 @@ int launch_sdpa_prefill(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D
     //   split over two wave sets.  (2 x 2 x 2, four waves with two row groups each, was
     //   measured 35 % slower at 512 tokens: the two groups' instructions do not interleave;
     //   2 x 1 x 2, two small workgroups per CU, 15 % slower.)
-    const bool big = (nhg + 7) / 8 * Hkv >= 2 * (int64_t)num_cus && D <= 128;
-    const bool small = !big && D <= 128 && (nhg + 3) / 4 * Hkv < 2 * (int64_t)num_cus;
+    // A bf16 cache comes here with few rows only (sdpa_chunk_plan): always the small shape.
+    const bool f32 = kv_dtype == MFA_KV_F32;
+    const bool big = f32 && (nhg + 7) / 8 * Hkv >= 2 * (int64_t)num_cus && D <= 128;
+    const bool small = !big && D <= 128 && (!f32 || (nhg + 3) / 4 * Hkv < 2 * (int64_t)num_cus);
     const int rw = 4, rg = big ? 2 : 1;
     const int64_t nwg = (nhg + rw * rg - 1) / (rw * rg);
     if (nwg > 0x7fffffff || Hkv > 65535) return fail(MFA_ERR_SHAPE, "sdpa: too many query rows in one call");
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     const int64_t kv_len0 = kv_len - n_tok;
     const dim3 grid((unsigned)nwg, Hkv);
-#define MFA_LAUNCH(DD, RGG, DEP, KSS, RWW)                                                                          \
-    hipLaunchKernelGGL((sdpa_prefill_kernel<float, DD, RGG, DEP, KSS, RWW>), grid, dim3(64 * RWW * KSS), 0, stream, \
-                       (const float *)k_tiled, (const float *)v_tiled, plane_elems, q, gate, hpk, Hq, n_tok, kv_len0, \
+#define MFA_LAUNCH(KV, DD, RGG, DEP, KSS)                                                                       \
+    hipLaunchKernelGGL((sdpa_prefill_kernel<KV, DD, RGG, DEP, KSS, 4>), grid, dim3(256 * KSS), 0, stream,        \
+                       (const KV *)k_tiled, (const KV *)v_tiled, plane_elems, q, gate, hpk, Hq, n_tok, kv_len0,   \
                        qscale, out)
-    if (D == 256) MFA_LAUNCH(256, 1, 2, 1, 4);
+    if (!f32) {
+        if (D == 256) MFA_LAUNCH(uint16_t, 256, 1, 2, 1);
+        else if (D == 128) MFA_LAUNCH(uint16_t, 128, 1, 4, 2);
+        else MFA_LAUNCH(uint16_t, 64, 1, 4, 2);
+    } else if (D == 256) MFA_LAUNCH(float, 256, 1, 2, 1);
     else if (D == 128) {
-        if (big) MFA_LAUNCH(128, 2, 2, 1, 4);
-        else if (small) MFA_LAUNCH(128, 1, 4, 2, 4);
-        else MFA_LAUNCH(128, 1, 4, 1, 4);
+        if (big) MFA_LAUNCH(float, 128, 2, 2, 1);
+        else if (small) MFA_LAUNCH(float, 128, 1, 4, 2);
+        else MFA_LAUNCH(float, 128, 1, 4, 1);
     } else {
-        if (big) MFA_LAUNCH(64, 2, 2, 1, 4);
-        else if (small) MFA_LAUNCH(64, 1, 4, 2, 4);
-        else MFA_LAUNCH(64, 1, 4, 1, 4);
+        if (big) MFA_LAUNCH(float, 64, 2, 2, 1);
+        else if (small) MFA_LAUNCH(float, 64, 1, 4, 2);
+        else MFA_LAUNCH(float, 64, 1, 4, 1);
     }
 #undef MFA_LAUNCH
     MFA_HIP(hipGetLastError());

@@ -130,6 +130,7 @@ template <int D> struct Wave<uint16_t, D> {
     static constexpr int BLK = 32;
     static constexpr int KSTEPS = D / 32;   // MFMA k-steps per 16-position sub-tile
     static constexpr int NACC = D / 16;     // 16-wide output tiles of O^T
+    static constexpr int NLOAD = D / 16;    // 1 KiB loads of K per block
     static constexpr int QSLOTS = KSTEPS * 64;   // (k-step, lane) operand slots of the query
     static constexpr int QLDS_U4 = QSLOTS * 2;   // hi and lo
     static constexpr int QRAW_F4 = 2;            // float4 loads per slot
@@ -158,8 +159,55 @@ template <int D> struct Wave<uint16_t, D> {
         qlds[(s * 2 + 1) * 64 + lane] = lo;
     }
 
-    // The same operands in registers: per k-step a high and a low bf16 part.
+    // The same operands kept in registers by a wave that owns its row group: per k-step a
+    // high and a low bf16 part.
     static constexpr int QREGS = KSTEPS * 2;
+    __device__ static void load_q_regs(uint4 (&qr)[QREGS], const float *q, int lane, const RowGroup &rows,
+                                       float qscale) {
+        const int n = lane & 15, g = lane >> 4;
+        const bool ok = rows.valid(n);
+        const float *p = q + (ok ? rows.q_row(n) : 0) * D + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) {
+            float4 a = *(const float4 *)(p + 32 * s), b = *(const float4 *)(p + 32 * s + 4);
+            if (!ok) a = b = float4{0.f, 0.f, 0.f, 0.f};
+            split_pair(a.x * qscale, a.y * qscale, qr[2 * s].x, qr[2 * s + 1].x);
+            split_pair(a.z * qscale, a.w * qscale, qr[2 * s].y, qr[2 * s + 1].y);
+            split_pair(b.x * qscale, b.y * qscale, qr[2 * s].z, qr[2 * s + 1].z);
+            split_pair(b.z * qscale, b.w * qscale, qr[2 * s].w, qr[2 * s + 1].w);
+        }
+    }
+
+    struct Scores {
+        f32x4 s[2];
+    };
+
+    // K load li = 2*s + sub: both 16-position sub-tiles of a k-step share one read of the query operands.
+    // HI_ONLY: the query's low parts are all zero (a query that is exact in bf16), so their
+    // products are left out; the result is the same number.
+    template <bool HI_ONLY = false>
+    __device__ static void scores_reg(const uint4 (&kreg)[NLOAD], const uint4 (&qr)[QREGS], Scores &sc) {
+        sc.s[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+        sc.s[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) {
+#pragma unroll
+            for (int sub = 0; sub < 2; sub++) {
+                const bf16x8 a = as_bf16x8(kreg[2 * s + sub]);
+                sc.s[sub] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_bf16x8(qr[2 * s]), sc.s[sub], 0, 0, 0);
+                if constexpr (!HI_ONLY)
+                    sc.s[sub] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_bf16x8(qr[2 * s + 1]), sc.s[sub], 0, 0, 0);
+            }
+        }
+    }
+    // whether every low part of this lane's query operands is zero
+    __device__ static bool q_low_parts_zero(const uint4 (&qr)[QREGS]) {
+        unsigned any = 0;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) any |= (qr[2 * s + 1].x | qr[2 * s + 1].y | qr[2 * s + 1].z | qr[2 * s + 1].w) & 0x7fff7fffu;
+        return any == 0;
+    }
+    static constexpr bool kScaleAfter = true;   // scores leave the matrix core unscaled (prompt-chunk kernel)
 
     // One 1 KiB piece of K (16 positions x the 32 channels of k-step s) against the query
     // operands in registers: the piece's share of S^T[16 positions, 16 rows].
@@ -180,6 +228,24 @@ template <int D> struct Wave<uint16_t, D> {
         reinterpret_cast<uint2 *>(&pblk[1][lane])[h] = lo;
     }
 
+    static constexpr int NX = 8;  // scores per lane: row 4g+i of sub-tile `sub` is position 16*sub + 4g + i
+    __device__ static void unpack(const Scores &sc, float (&x)[NX]) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x[i] = sc.s[0][i];
+            x[4 + i] = sc.s[1][i];
+        }
+    }
+    __device__ static int64_t pos_of(int64_t blk, int g, int e) {
+        return blk * BLK + 16 * (e >> 2) + 4 * g + (e & 3);
+    }
+    // probabilities -> operand registers (slot e of lane group g is position pos_of(.., g, e))
+    __device__ static void pack_probs(const float (&e)[NX], uint4 (&p)[P_U4]) {
+        split_pair(e[0], e[1], p[0].x, p[1].x);
+        split_pair(e[2], e[3], p[0].y, p[1].y);
+        split_pair(e[4], e[5], p[0].z, p[1].z);
+        split_pair(e[6], e[7], p[0].w, p[1].w);
+    }
     __device__ static f32x4 pv(uint4 vreg, const uint4 (&p)[P_U4], f32x4 acc) {
         const bf16x8 a = as_bf16x8(vreg);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, as_bf16x8(p[0]), acc, 0, 0, 0);
@@ -233,6 +299,7 @@ template <int D> struct Wave<float, D> {
         f32x4 s;
     };
 
+    template <bool HI_ONLY = false>   // an f32 query has no parts
     __device__ static void scores_reg(const uint4 (&kreg)[NLOAD], const uint4 (&qr)[QREGS], Scores &sc) {
         sc.s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -245,6 +312,9 @@ template <int D> struct Wave<float, D> {
             sc.s = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, sc.s, 0, 0, 0);
         }
     }
+
+    __device__ static bool q_low_parts_zero(const uint4 (&)[QREGS]) { return false; }
+    static constexpr bool kScaleAfter = false;   // the query carries the scale
 
     // One 1 KiB piece of K (16 positions x the 16 channels of k-step s).
     __device__ static f32x4 score_step(uint4 kpiece, const uint4 (&qr)[QREGS], int s, f32x4 acc) {

@@ -158,6 +158,38 @@ def test_chunk_and_short_decode_in_a_captured_graph(mfa, oracle):
             assert rt().hipGraphExecDestroy(run) == 0 and rt().hipGraphDestroy(graph) == 0
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("route", [1, 2001, 4001, 2003, 4003])
+def test_every_form_against_the_oracle(mfa, oracle, route, d):
+    """16-row groups, and both shapes of the 32x32-tile kernel on the whole cache and on three splits of it, a row either
+    side of their tiles and of a block; from a normed query and from raw projections (rows of the oracle's prologue over
+    the cache as exported)."""
+    theta = 1.0e7
+    for Hq, Hkv, T, L0 in [(8, 2, 8, 0), (4, 1, 31, 1), (4, 1, 33, 31), (16, 1, 3, 61), (6, 2, 65, 64), (3, 3, 129, 290), (24, 1, 11, 95)]:
+        q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, T + L0)
+        qp = np.stack([q.reshape(T, Hq, d), g.reshape(T, Hq, d)], 2).reshape(T, Hq * 2 * d)
+        rng = np.random.default_rng(T)
+        norm = [oracle.f32_to_bf16(1.0 + 0.3 * rng.standard_normal(d)) for _ in range(2)]
+        with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+            c.set_full_weights(0, *norm)
+            c.set_rope(theta, d // 4)
+            assert c.lib.mfa_debug_set_chunk_route(c.h, route) == 0
+            for raw in (False, True):
+                c.memory_clear()
+                if L0:
+                    c.kv_import(0, k[:L0], v[:L0])
+                c.lib.mfa_debug_fill_workspace(c.h, 0x7FC00000)
+                out = c.prefill_full_attn(0, L0, qp, k[L0:], v[L0:]) if raw else c.prefill_attn(0, q, g, k[L0:], v[L0:])
+                kc, vc = c.kv_export(0)
+                qr = q
+                if raw:
+                    qr = np.stack([oracle.attn_prologue(L0 + t, Hq, Hkv, d, d // 4, theta, 1e-6, *norm, qp[t], k[L0 + t], v[L0 + t])[0]
+                                   for t in range(T)])
+                ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, qr, g, kc, vc).reshape(T, Hq * d)
+                assert rel_err(out, ref) <= TOL, (Hq, Hkv, T, L0, raw)
+                assert rel_err_rows(out, ref, d) <= 5 * TOL, (Hq, Hkv, T, L0, raw)
+
+
 class _Graph:
     """What `call` puts on a context's stream, captured (relaxed: other streams are not held up)."""
 

@@ -142,3 +142,22 @@ def test_inline_assembly_declares_m0():
                 writes += 1
                 assert '"m0"' in stmt, (f, stmt)
     assert writes > 0
+
+
+def test_prompt_chunks_take_the_kernel_that_is_faster_for_one_sequence():
+    """Few rows: 16-row groups, over the whole cache where it is short and over splits of it where it is long.  The
+    32x32 tiles from a few hundred tokens on at every length, and over lengths between, where they split the cache."""
+    lib = ffi.load()
+
+    def route(Hq, Hkv, d, T, L0, raw, dtype=ffi.KV_BF16):
+        return lib.mfa_debug_chunk_route(dtype, Hq, Hkv, d, T, L0 + T, 256, raw)
+
+    for Hq, Hkv, d in [(32, 2, 256), (16, 2, 256), (32, 4, 128), (16, 2, 64), (32, 32, 128)]:
+        for raw in (0, 1):
+            assert all(route(Hq, Hkv, d, T, L0, raw) == 1 for T in (2, 8, 32, 64) for L0 in (0, 40))
+            assert all(route(Hq, Hkv, d, T, L0, raw) == 0 for T in (2, 5) for L0 in (3001, 16384))
+            assert all(route(Hq, Hkv, d, 700, L0, raw) >= 2000 for L0 in (0, 100, 1000, 16384))
+            assert all(route(Hq, Hkv, d, 203, L0, raw) >= 2000 for L0 in (3001, 16384))
+            assert all(route(Hq, Hkv, d, T, 100, raw, ffi.KV_F32) == 1 for T in (2, 100, 700))
+    assert route(16, 2, 256, 1, 100, 0) == 0
+    assert route(16, 2, 256, 8, -1, 0) == -1
