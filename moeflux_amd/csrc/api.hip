@@ -318,6 +318,13 @@ static int ensure_workspace_elems(Ctx *c, size_t need_o, size_t need_ml) {
     return MFA_OK;
 }
 
+// Whether the split-K workspace holds a prompt chunk's partials (of one split: the launcher fits its plan to it).
+static bool split_k_workspace_holds(const Ctx *c, int n_tok) {
+    const mfa_config &g = c->cfg;
+    return sdpa_workspace_o_elems(g.num_attn_heads, g.num_kv_heads, g.head_dim, 1, n_tok) <= c->part_o_elems &&
+           sdpa_workspace_ml_elems(g.num_attn_heads, g.num_kv_heads, 1, n_tok) <= c->part_ml_elems;
+}
+
 // The split-K workspace is sized for decode at create time; a prompt chunk has n_tok times
 // the rows and grows it on first use.
 // `layers` > 1 sizes it for one launch over that many layers (layers * Hkv kv heads).
@@ -333,7 +340,7 @@ static int ensure_workspace(Ctx *c, int n_tok, int64_t kv_len, int layers = 1) {
 
 // The plan of a prompt chunk (a forced split count is the split-K kernel's), and the memory it takes.  The first plan that
 // splits the cache on 32x32 tiles allocates their workspace, whose size never changes; without memory for it, or while
-// the stream is being captured, the plan is one that needs none.
+// the stream is being captured, the plan is one that needs none.  Nor does a capture grow the split-K workspace.
 // Everything that sdpa_dev could still refuse is refused here, while the cache is as the caller left it.
 static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, ChunkPlan *out) {
     const mfa_config &g = c->cfg;
@@ -368,6 +375,10 @@ static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, Ch
     const int64_t nhg = ((int64_t)n_tok * (g.num_attn_heads / g.num_kv_heads) + 15) / 16;
     if (nhg > 65535) return fail(MFA_ERR_SHAPE, "sdpa: too many query rows in one call");
     if (n_tok == 1) return MFA_OK;
+    if (!c->forced_splits && !c->partial_only && !split_k_workspace_holds(c, n_tok) && capturing()) {
+        p = plan(c->chunk_part_elems, false);
+        if (p.route != ChunkRoute::SplitK) return MFA_OK;
+    }
     return ensure_workspace(c, n_tok, kv_len);
 }
 

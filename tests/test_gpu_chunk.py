@@ -254,3 +254,39 @@ def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first):
             c.sync()
             check(first)
         graph.close()
+
+
+@pytest.mark.parametrize("long", [8000, 0])
+def test_a_capture_takes_a_route_whose_memory_is_there(mfa, oracle, long):
+    """A chunk of few rows behind 2137 positions is the split-K kernel's, whose workspace grows with the tokens: captured
+    on a context that has not made room for it (the chunk before, behind another length, took another kernel, or none was
+    before), it takes a route that needs none."""
+    from moeflux_amd.hip import DeviceArray
+    Hq, Hkv, d, T, L0 = 16, 1, 64, 145, 2137
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, max(L0, long), 7)
+    ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, q, g, k[:L0 + T], v[:L0 + T]).reshape(T, Hq * d)
+    dq, dg, dk, dv = (DeviceArray.from_host(x) for x in (q, g, k[L0:L0 + T], v[L0:L0 + T]))
+    out = DeviceArray((T, Hq * d), zero=True)
+    with _ctx(mfa, Hq, Hkv, d, max(L0, long) + T) as c:
+        assert c.lib.mfa_debug_chunk_route(1, Hq, Hkv, d, T, L0 + T, 256, 0) == 0
+        assert c.lib.mfa_debug_chunk_route(1, Hq, Hkv, d, T, 8000 + T, 256, 0) > 1
+
+        def call():
+            return c.lib.mfa_prefill_attn_dev(c.h, 0, T, dq.ptr, dg.ptr, dk.ptr, dv.ptr, out.ptr)
+
+        if long:
+            c.kv_import(0, k[:long], v[:long])
+            assert call() == 0
+            c.sync()
+            c.memory_clear()
+        c.kv_import(0, k[:L0], v[:L0])
+        graph = _Graph(c, call)
+        for _ in range(3):
+            graph()
+            assert rel_err(out.to_host(), ref) <= TOL
+            c.memory_seq_rm(L0)
+            assert call() == 0      # eagerly: the split-K kernel, which makes its room
+            c.sync()
+            assert rel_err(out.to_host(), ref) <= TOL
+            c.memory_seq_rm(L0)
+        graph.close()
