@@ -363,9 +363,15 @@ static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, Ch
                 return fail(MFA_ERR_INVALID, "sdpa: %d splits of the chunk do not fit its workspace", p.splits);
         }
         if (p.route == ChunkRoute::Tiles32 && p.splits > 1 && !c->chunk_part) {
-            if (!capturing() && hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
-                (void)hipGetLastError();
-                c->chunk_part = nullptr;
+            if (!capturing()) {
+                // in the mode that leaves captures of other streams alone: an allocation in the usual one ends them
+                hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+                MFA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+                if (hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
+                    (void)hipGetLastError();
+                    c->chunk_part = nullptr;
+                }
+                MFA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
             }
             if (c->chunk_part) c->chunk_part_elems = kChunkPartElems;
             else p = plan(0, true);

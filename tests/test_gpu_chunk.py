@@ -290,3 +290,30 @@ def test_a_capture_takes_a_route_whose_memory_is_there(mfa, oracle, long):
             assert rel_err(out.to_host(), ref) <= TOL
             c.memory_seq_rm(L0)
         graph.close()
+
+
+def test_first_split_chunk_beside_another_streams_capture(mfa, oracle):
+    """A context's first split chunk allocates its workspace: while another stream is being captured in the mode that
+    holds up the whole process (hipStreamCaptureModeGlobal), neither the chunk nor that capture fails."""
+    import ctypes as C
+
+    from moeflux_amd.hip import rt
+    Hq, Hkv, d, T, L0 = 16, 2, 256, 50, 1990
+    q, g, k, v = _inputs(oracle, Hq, Hkv, d, T, L0, 9)
+    ref = oracle.prefill_attn(T, L0, Hq, Hkv, d, q, g, k, v).reshape(T, Hq * d)
+    from moeflux_amd.hip import DeviceArray
+    dq, dg, dk, dv = (DeviceArray.from_host(x) for x in (q, g, k[L0:], v[L0:]))
+    out = DeviceArray((T, Hq * d), zero=True)
+    other, graph = C.c_void_p(), C.c_void_p()
+    assert rt().hipStreamCreateWithFlags(C.byref(other), C.c_uint(1)) == 0
+    with _ctx(mfa, Hq, Hkv, d, L0 + T) as c:
+        c.kv_import(0, k[:L0], v[:L0])
+        assert c.lib.mfa_debug_chunk_route(1, Hq, Hkv, d, T, L0 + T, 256, 0) % 1000 > 1
+        assert rt().hipStreamBeginCapture(other, C.c_int(0)) == 0
+        rc = c.lib.mfa_prefill_attn_dev(c.h, 0, T, dq.ptr, dg.ptr, dk.ptr, dv.ptr, out.ptr)
+        end = rt().hipStreamEndCapture(other, C.byref(graph))
+        assert rc == 0, c.lib.mfa_last_error_string()
+        assert end == 0
+        c.sync()
+        assert rel_err(out.to_host(), ref) <= TOL
+    assert rt().hipGraphDestroy(graph) == 0 and rt().hipStreamDestroy(other) == 0
