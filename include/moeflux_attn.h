@@ -237,6 +237,7 @@ int mfa_attn_prologue_dev(mfa_ctx *ctx, int32_t layer, int32_t pos, const float 
  * (full_attn_forward.rs:234-389).  out: [Hq*head_dim]. */
 int mfa_full_attn_step(mfa_ctx *ctx, int32_t layer, int32_t pos, const float *q_proj_out,
                        const float *k, const float *v, float *out);
+/* (out_dev may lie over k_dev, not over q_proj_out_dev or v_dev.) */
 int mfa_full_attn_step_dev(mfa_ctx *ctx, int32_t layer, int32_t pos, const float *q_proj_out_dev,
                            const float *k_dev, const float *v_dev, float *out_dev);
 /* How many launches mfa_full_attn_step makes; no counterpart in the reference and no result
@@ -262,7 +263,8 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
 /* A chunk of T prompt tokens on one full-attention layer.  The reference has
  * no batched prefill: eval_prompt is a token loop (riir/mod.rs:1196-1214); the
  * result equals T successive mfa_kv_append + mfa_sdpa_decode calls.
- *   q, q_gate, out: [T, Hq*head_dim]; k, v: [T, num_kv_heads*head_dim]. */
+ *   q, q_gate, out: [T, Hq*head_dim]; k, v: [T, num_kv_heads*head_dim].
+ * out may be q or q_gate itself, and may lie over k or v. */
 int mfa_prefill_attn(mfa_ctx *ctx, int32_t layer, int32_t T, const float *q,
                      const float *q_gate, const float *k, const float *v, float *out);
 int mfa_prefill_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t T, const float *q_dev,

@@ -342,13 +342,13 @@ static int ensure_workspace(Ctx *c, int n_tok, int64_t kv_len, int layers = 1) {
 // splits the cache on 32x32 tiles allocates their workspace, whose size never changes; without memory for it, or while
 // the stream is being captured, the plan is one that needs none.  Nor does a capture grow the split-K workspace.
 // Everything that sdpa_dev could still refuse is refused here, while the cache is as the caller left it.
-static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, ChunkPlan *out) {
+static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, ChunkPlan *out, bool shifted = false) {
     const mfa_config &g = c->cfg;
     ChunkPlan &p = *out;
     p = ChunkPlan{};
     const auto plan = [&](size_t ws_elems, bool split_k) {
         return sdpa_chunk_plan(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, kv_len, c->num_cus, kind,
-                               ChunkLimits{ws_elems, split_k});
+                               ChunkLimits{ws_elems, split_k, shifted});
     };
     const auto capturing = [&] {
         hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
@@ -782,7 +782,7 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
     const size_t qd = (size_t)c->q_dim() * T;
     // The 32x32-tile kernel takes the query and its gate from the projection itself (unless the caller's result would
     // overwrite rows it has yet to read): all the launch ahead of it leaves is the tokens' rotation table.
-    const bool apart = out_dev + qd <= q_proj_out_dev || q_proj_out_dev + 2 * qd <= out_dev;
+    const bool apart = !overlap(out_dev, qd, q_proj_out_dev, 2 * qd);
     const ChunkQueryKind kind = apart && sdpa_chunk_takes_raw(c->cfg.head_dim, c->rotary_dim) ? ChunkQueryKind::Raw : ChunkQueryKind::RawPrologue;
     ChunkPlan plan;
     MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, kind, &plan));
@@ -853,8 +853,9 @@ int mfa_prefill_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t T, const float *q_
     if ((int64_t)f->len + T > c->cfg.kv_capacity)
         return fail(MFA_ERR_OVERFLOW, "kv cache overflow: len %d + %d > capacity %d", f->len, T,
                     c->cfg.kv_capacity);
+    const size_t qd = (size_t)c->q_dim() * T;
     ChunkPlan plan;
-    MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, ChunkQueryKind::Normed, &plan));
+    MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, ChunkQueryKind::Normed, &plan, out_dev != q_dev && overlap(out_dev, qd, q_dev, qd)));
     // append the whole chunk, then one causal pass: row t sees positions [0, len0 + t]
     const int32_t len0 = f->len;
     int rc = kv_append_dev(c, f, k_dev, v_dev, T);

@@ -212,6 +212,12 @@ int linear_import_from(Ctx *c, LinearLayer *l, const float *conv_dev);
 // ---- kernel launchers (device pointers, asynchronous on `stream`) ------------
 
 // sdpa_decode.hip
+// Whether [a, a + na) and [b, b + nb) share a float.
+inline bool overlap(const float *a, size_t na, const float *b, size_t nb) {
+    const uintptr_t a0 = (uintptr_t)a, b0 = (uintptr_t)b;
+    return a0 < b0 + nb * sizeof(float) && b0 < a0 + na * sizeof(float);
+}
+
 struct SdpaWorkspace {
     float *part_o;
     float *part_ml;
@@ -318,6 +324,9 @@ enum class ChunkQueryKind { Normed, Raw, RawPrologue };
 struct ChunkLimits {
     size_t ws_elems;
     bool split_k;
+    // The result lies over the query, but not row over row: before a long cache, where the split-K kernel reads all of the
+    // query before it writes any of the result, so must what takes its place.
+    bool shifted = false;
 };
 static constexpr int kMaxChunkSplits = 16;
 // The plan of the given shape of a workgroup, with at most `splits` splits.

@@ -636,11 +636,12 @@ ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64
     static constexpr double kStream[3] = {0.007, 0.0108, 0.0175};
     static constexpr double kLaunch = 12.0, kEmpty = 2.5;   // of a workgroup's fixed time, what its CU is free in
     const double out_bytes = 8.0 * (double)rows * Hkv * D, seen = c.seen();
+    const bool two_launches = limits.shifted && nblk > 64 && row_wgs < num_cus / 2;
     double best_cost = 0;
     for (int shape = 0; shape < 2; shape++) {
         const int rw = shape ? 2 : 4, ks = shape ? 2 : 1;
         const int64_t nrt = (rows + 32 * rw - 1) / (32 * rw);
-        for (int64_t want = 1; want <= kMaxChunkSplits && want <= nblk; want++) {
+        for (int64_t want = two_launches ? 2 : 1; want <= kMaxChunkSplits && want <= nblk; want++) {
             const int64_t bps = (nblk + want - 1) / want;
             if ((nblk + bps - 1) / bps != want) continue;
             const size_t elems = want > 1 ? (size_t)(nrt * Hkv * want) * 32 * rw * D : 0;
@@ -660,6 +661,7 @@ ChunkPlan sdpa_chunk_plan(int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64
             }
         }
     }
+    if (best.route != ChunkRoute::Tiles32) return best;
     const double own = tiles32_time(c, best, kind);
     if (nblk <= 64) {
         // (past a workgroup per CU the 32x32 tiles are faster at every length)

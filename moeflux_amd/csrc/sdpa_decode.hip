@@ -847,7 +847,10 @@ int launch_sdpa_step(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, i
     if (len0 < 0 || pos < 0) return fail(MFA_ERR_INVALID, "attention step: negative position");
     const int hpk = Hq / Hkv;
     SplitPlan plan;
-    const bool one = one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, ws);
+    // (one launch: a row group's result may be out before another's inputs are in, so they lie apart)
+    const size_t qd = (size_t)Hq * D, kd = (size_t)Hkv * D;
+    const bool one = !overlap(out, qd, q_proj, 2 * qd) && !overlap(out, qd, k_in, kd) && !overlap(out, qd, v_in, kd) &&
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, ws);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, 1, len0 > 0 ? len0 : 1, num_cus, forced_splits, ws));
     const OneLaunch ol{q_proj + D, out, 2 * D, ws.tickets};
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
@@ -878,7 +881,11 @@ int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_
         return fail(MFA_ERR_INVALID, "sdpa: kv_len must be > 0 (got %lld for %d tokens)", (long long)kv_len, n_tok);
     const int hpk = Hq / Hkv;
     SplitPlan plan;
-    const bool one = n_tok == 1 && gate && !partial_only && !defer_merge && one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, ws);
+    // (one launch: a row group's result may be out before another's query is in; in place it lies over its own)
+    const size_t qd = (size_t)Hq * D;
+    const bool apart = (out == q || !overlap(out, qd, q, qd)) && (out == gate || !overlap(out, qd, gate, qd));
+    const bool one = n_tok == 1 && gate && apart && !partial_only && !defer_merge &&
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, ws);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, forced_splits, ws));
     const OneLaunch ol{gate, out, D, ws.tickets};
     // scores are produced in log2 units: q is pre-multiplied by (1/sqrt(D)) * log2(e)

@@ -241,3 +241,62 @@ def test_short_caches_merge_in_the_attention_launch(mfa, oracle, Hq, Hkv, d, bf1
             c.set_num_splits(2)
             assert rel_err(outs[0], c.sdpa_decode(0, q, g)) <= tol, n
             c.set_num_splits(0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,d", [(32, 2, 256), (40, 2, 128)])
+@pytest.mark.parametrize("L", [1, 300, 768])
+def test_result_over_the_inputs(mfa, oracle, Hq, Hkv, d, L):
+    """A short decode whose result is its query, its gate, or lies over the query at an offset (a row group then writes
+    what another has yet to read, unless all is read first); a step whose result lies over its key projection."""
+    from moeflux_amd.hip import DeviceArray
+    q, g, k, v = sdpa_random_inputs(L, Hq, Hkv, d, L, bf16=True)
+    n = Hq * d
+    rng = np.random.default_rng(L)
+    qp, kn, vn = (rng.standard_normal(m).astype(np.float32) for m in (2 * n, Hkv * d, Hkv * d))
+    norm = [oracle.f32_to_bf16(1.0 + 0.1 * rng.standard_normal(d)) for _ in range(2)]
+    with _ctx(mfa, num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d, kv_capacity=L + 1, kv_dtype=1) as c:
+        c.set_full_weights(0, *norm)
+        c.kv_import(0, k, v)
+        want = c.sdpa_decode(0, q, g)
+        for where in ("q", "gate", -17 * d, -d, 4, d, 17 * d):
+            room = np.zeros(3 * n, np.float32)
+            room[n:2 * n] = q
+            buf, gate = DeviceArray.from_host(room), DeviceArray.from_host(g)
+            out = gate.ptr if where == "gate" else buf.offset(n + (0 if where == "q" else where))
+            assert c.lib.mfa_sdpa_decode_dev(c.h, 0, buf.offset(n), gate.ptr, out) == 0
+            c.sync()
+            got = gate.to_host() if where == "gate" else buf.to_host()[n + (0 if where == "q" else where):][:n]
+            assert rel_err(got, want) <= 1e-5, where     # (another route's order of sums)
+        want = c.full_attn_step(0, L, qp, kn, vn)
+        dq, dv = DeviceArray.from_host(qp), DeviceArray.from_host(vn)
+        for off in (0, d, n - 1 - (n - 1) % 4):     # where in the result the key projection lies
+            c.memory_seq_rm(L)
+            room = np.zeros(3 * n, np.float32)
+            room[n:n + Hkv * d] = kn
+            buf = DeviceArray.from_host(room)
+            assert c.lib.mfa_full_attn_step_dev(c.h, 0, L, dq.ptr, buf.offset(n), dv.ptr, buf.offset(n - off)) == 0
+            c.sync()
+            assert rel_err(buf.to_host()[n - off:][:n], want) <= 1e-5, off
+
+
+def test_chunk_result_shifted_over_the_query(mfa, oracle):
+    """Few rows before a long cache: whatever kernel takes them, all of the query is read before any of the result is written."""
+    from moeflux_amd.hip import DeviceArray
+    Hq, Hkv, d, T, L = 32, 4, 128, 145, 2100
+    rng = np.random.default_rng(1)
+    k, v = (oracle.bf16_to_f32(oracle.f32_to_bf16(rng.standard_normal((L + T, Hkv * d)).astype(np.float32))) for _ in range(2))
+    q, g = (rng.standard_normal((T, Hq * d)).astype(np.float32) for _ in range(2))
+    n = T * Hq * d
+    dg, dk, dv = (DeviceArray.from_host(x) for x in (g, k[L:], v[L:]))
+    with _ctx(mfa, num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d, kv_capacity=L + T, kv_dtype=1) as c:
+        assert c.lib.mfa_debug_chunk_route(1, Hq, Hkv, d, T, L + T, 256, 0) % 1000 == 1     # unsplit, where they lie apart
+        c.kv_import(0, k[:L], v[:L])
+        want = c.prefill_attn(0, q, g, k[L:], v[L:]).reshape(-1)
+        for off in (-64 * Hq * d, -4, 0, d, 100 * Hq * d):
+            c.memory_seq_rm(L)
+            room = np.zeros(3 * n, np.float32)
+            room[n:2 * n] = q.reshape(-1)
+            buf = DeviceArray.from_host(room)
+            assert c.lib.mfa_prefill_attn_dev(c.h, 0, T, buf.offset(n), dg.ptr, dk.ptr, dv.ptr, buf.offset(n + off)) == 0
+            c.sync()
+            assert rel_err(buf.to_host()[n + off:][:n], want) <= 1e-4, off
