@@ -119,7 +119,8 @@ int32_t mfa_kv_len(mfa_ctx *ctx, int32_t layer);
 /* Replaces both branches of full_attn_forward.rs:331-389: the four-kernel GPU
  * chain attn_scores_batched / attn_softmax_batched / attn_values_batched /
  * sigmoid_gate (linear_attn_forward.rs:850-902) and the sdpa_cpu fallback
- * (sdpa.rs:63-172), at every kv_len >= 1.  q, q_gate, out: [Hq*head_dim] f32. */
+ * (sdpa.rs:63-172), at every kv_len >= 1.  q, q_gate, out: [Hq*head_dim] f32.
+ * out_dev may be q_dev or q_gate_dev itself, and may lie over q_dev at an offset. */
 int mfa_sdpa_decode(mfa_ctx *ctx, int32_t layer, const float *q, const float *q_gate,
                     float *out);
 int mfa_sdpa_decode_dev(mfa_ctx *ctx, int32_t layer, const float *q_dev,
@@ -244,8 +245,11 @@ int mfa_full_attn_step_dev(mfa_ctx *ctx, int32_t layer, int32_t pos, const float
  * depends on it beyond rounding.  2 (default, where rotary_dim / 2 is a multiple of 8 channels
  * for a bf16 cache, 4 for f32): the attention launch norms and rotates its own query heads from
  * q_proj_out, attends to the positions the cache already holds, and scores and appends the new
- * token; the merge launch takes the token as one more split (a short cache, up to 1024 positions,
- * is merged by the attention launch itself: one launch).  3: prologue, attention, merge. */
+ * token; the merge launch takes the token as one more split.  A short cache takes one launch,
+ * whose workgroups hold a row from start to end: up to 10, 3 and 3 chunks of 64 positions at
+ * head_dim 64, 128 and 256 of a bf16 cache, 3, 2 and 1 of an f32 one.  3: prologue, attention, merge
+ * (attention and merge in one up to 12, 5 and 5 chunks, f32 4, 3 and 1, as mfa_sdpa_decode).
+ * A forced split count (mfa_set_num_splits) always takes the merge launch. */
 int mfa_set_step_launches(mfa_ctx *ctx, int32_t launches);
 /* The same for a chunk of T prompt tokens at positions pos0 .. pos0+T-1 (the token
  * loop of eval_prompt, riir/mod.rs:1196-1214, over full_attn_layer_forward): every

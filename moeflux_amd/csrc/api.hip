@@ -71,7 +71,7 @@ int release_stage_beyond_cap(Ctx *c) {
 }
 
 static SdpaWorkspace workspace(Ctx *c) {
-    return SdpaWorkspace{c->part_o, c->part_ml, c->part_o_elems, c->part_ml_elems, c->tickets};
+    return SdpaWorkspace{c->part_o, c->part_ml, c->part_o_elems, c->part_ml_elems};
 }
 
 static int h2d(Ctx *c, void *dst, const void *src, size_t bytes) {
@@ -215,12 +215,11 @@ static int create(const mfa_config *cfg, Ctx **out) {
         char *qg;
         MFA_TRY(slab_alloc(c, 2 * (size_t)cfg->num_attn_heads * cfg->head_dim * sizeof(float), &qg));
         c->qg_stage = (float *)qg;
-        // per (kv head, 16-row group): the new token's 16 scores; behind them all, the groups' tickets
+        // per (kv head, 16-row group): the new token's 16 scores
         const size_t groups = (size_t)cfg->num_kv_heads * ((cfg->num_attn_heads / cfg->num_kv_heads + 15) / 16);
         char *sc;
-        MFA_TRY(slab_alloc(c, groups * (16 * sizeof(float) + sizeof(unsigned)), &sc));
+        MFA_TRY(slab_alloc(c, groups * 16 * sizeof(float), &sc));
         c->step_score = (float *)sc;
-        c->tickets = (unsigned *)(sc + groups * 16 * sizeof(float));
         // variants.rs:245-250, 369: a quarter of the head is rotated, theta = 1e7
         MFA_TRY(set_rope(c, 1.0e7f, cfg->head_dim / 4));
         // room for the most splits any cache length up to the capacity gets
@@ -982,12 +981,10 @@ int mfa_token_sweep_dev(mfa_ctx *ctx, const float *full_q, const float *full_gat
     if (full_batch) {
         const int n = (int)c->full.size();
         MFA_TRY(ensure_workspace(c, 1, c->full[0].len, n));
-        SdpaWorkspace ws = workspace(c);
-        ws.tickets = nullptr;   // (they are one layer's)
         MFA_TRY(launch_sdpa(c->stream, c->cfg.kv_dtype, c->cfg.num_attn_heads * n, c->cfg.num_kv_heads * n,
                             c->cfg.head_dim, 1, c->full[0].len, c->plane_elems, c->full[0].k, c->full[0].v,
-                            full_q, full_gate, full_out, ws, c->num_cus, c->forced_splits,
-                            c->partial_only, lin_batch ? &merge : nullptr));
+                            full_q, full_gate, full_out, workspace(c), c->num_cus, c->forced_splits,
+                            c->partial_only, lin_batch ? &merge : nullptr, false));
     }
     if (lin_batch) {
         LinearLayer &l0 = c->lin[0];

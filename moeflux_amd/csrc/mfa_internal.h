@@ -151,7 +151,6 @@ struct Ctx {
     float *inv_freq = nullptr;
     int32_t rotary_dim = 0;
     float *qg_stage = nullptr;   // q and gate of mfa_full_attn_step, 2 * q_dim floats
-    unsigned *tickets = nullptr; // of the one-launch decode (SdpaWorkspace)
     float *step_score = nullptr; // the new token's score per query row of the two-launch attention step
     int32_t step_launches = 2;   // launches of mfa_full_attn_step: 2 (prologue inside the attention launch) or 3
     float *qg_chunk = nullptr;   // the same for a chunk of tokens (mfa_prefill_full_attn), grown on demand
@@ -222,8 +221,6 @@ struct SdpaWorkspace {
     float *part_o;
     float *part_ml;
     size_t part_o_elems, part_ml_elems;
-    // counters of a decode launch that merges its own partials, [Hkv][16-row groups], all 0; null: the merge is a launch
-    unsigned *tickets = nullptr;
 };
 bool sdpa_shape_supported(int kv_dtype, int head_dim);
 // Number of splits the launcher will use (for workspace sizing pass kv_len = capacity).
@@ -243,7 +240,7 @@ struct SdpaMergeTask {
 int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                 size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                 const float *gate, float *out, const SdpaWorkspace &ws, int num_cus,
-                int forced_splits, int partial_only = 0, SdpaMergeTask *defer_merge = nullptr);
+                int forced_splits, int partial_only = 0, SdpaMergeTask *defer_merge = nullptr, bool one_layer = true);
 // One decode token of a full-attention layer from its raw projections in two launches (the
 // attention launch norms and rotates the query itself and appends the token; the merge takes
 // the token as one more split).  len0: cache length before the call.

@@ -114,9 +114,10 @@ template <typename KV, int D, int NT> struct StepQuery {
         }
     }
 
-    // `tab`: the workgroup's (cos, sin) table (HeadRotor::table), complete before this call
+    // `tab`: the workgroup's (cos, sin) table (HeadRotor::table), complete before this call.  score_lds: where the token's
+    // scores go instead of sp.new_score (null: they go there).
     __device__ inline void finish(const StepPrologue &sp, const RowGroup &rows, float qscale, size_t plane_elems,
-                                  bool with_new, uint4 *qlds, int nhg, const float2 *tab) {
+                                  bool with_new, uint4 *qlds, int nhg, const float2 *tab, float *score_lds) {
         const int j = threadIdx.x % LPH, c0 = EPS * j;
         HeadRotor<EPS, D> hr;
         hr.init(j, sp.rotary_dim, tab);
@@ -139,9 +140,10 @@ template <typename KV, int D, int NT> struct StepQuery {
 #pragma unroll
                 for (int e = 0; e < EPS; e++) d = fmaf(qraw[i][e], knew[e], d);
                 d = lanes_sum<LPH>(d);
-                if (ok && j == 0)   // (at device scope, as the partials: a workgroup of another XCD may merge)
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, d * qscale), buffer_of(sp.new_score),
-                                                          (((rows.kvh * nhg + rows.hg) * 16 + n) * 4), 0, kThrough);
+                if (ok && j == 0) {
+                    if (score_lds) score_lds[n] = d * qscale;
+                    else sp.new_score[((size_t)rows.kvh * nhg + rows.hg) * 16 + n] = d * qscale;
+                }
             }
             if (in) {
                 float4 raw[W::QRAW_F4];
@@ -217,107 +219,13 @@ template <int N, int END, int STEP, typename F> __device__ __attribute__((always
     }
 }
 
-// A decode launch that merges its partials itself: every workgroup of a row group draws a ticket when its partial is
-// out, and the one that draws the last combines them all and writes the group's rows (nobody waits for anybody).  The
-// counter goes back to 0 with the last ticket.  For short caches: the merge as a launch of its own costs 3 us of host time,
-// which is what bounds layers this small, and 4 us of the device's; the hop through memory and the last workgroup's reading
-// cost about as long on the device (one_launch_plan).
+// A decode launch that is the whole of the attention, for a short cache: one workgroup per row group, whose rows go out normalised
+// and gated from the registers that hold them, a decode step's new token among their positions (one_launch_plan).
 struct OneLaunch {
     const float *gate;
     float *out;
     int gate_stride;
-    unsigned *tickets;   // [kv head][row group], 0 between launches
 };
-static constexpr int kOneSplits = 16;
-
-// Partials are stored and loaded at device scope (sc1), past the L2s of the XCDs, so that waiting for the stores ahead of the
-// ticket is all the ordering there is to do: with the fences of the memory model instead (the whole L2 written back and
-// invalidated by every workgroup) a call of 100 positions took 4 us longer and one of 3000 up to 6.
-template <typename KV, int D, bool STEP>
-__device__ inline void one_launch_merge(const OneLaunch &one, const float *part_o, const float *part_ml, int nsplit, int nhg, int hpk,
-                                        int Hq, int kvh, int hg, const std::conditional_t<STEP, StepPrologue, NoPrologue> &sp, int *s_last,
-                                        float (*s_stat)[32]) {
-    constexpr int NT = kWaves * 64, Q = D / 4;   // 16-byte pieces of a row
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's share of the partial is out
-    __syncthreads();
-    if (nsplit > 1) {
-        if (threadIdx.x == 0) {
-            unsigned *ticket = one.tickets + kvh * nhg + hg;
-            const bool last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)nsplit - 1;
-            if (last) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *s_last = last;
-        }
-        __syncthreads();
-        if (!*s_last) return;
-    }
-    const size_t pid0 = ((size_t)kvh * nhg + hg) * nsplit;
-    const __amdgpu_buffer_rsrc_t ob = buffer_of(part_o + pid0 * 16 * D), mlb = buffer_of(part_ml + pid0 * 32);
-    const int rows = hpk - 16 * hg < 16 ? hpk - 16 * hg : 16, items = rows * Q;
-    unsigned stat[kOneSplits * 32 / NT];
-#pragma unroll
-    for (int i = 0; i < kOneSplits * 32 / NT; i++) {
-        const int at = i * NT + threadIdx.x;
-        stat[i] = __builtin_amdgcn_raw_buffer_load_b32(mlb, (at < nsplit * 32 ? at : 0) * 4, 0, kThrough);
-    }
-    // NS: splits at most; PER: pieces a thread has in flight (all of their rows, gates and values requested at once)
-    auto combine = [&](auto ns_tag, auto per_tag) __attribute__((always_inline)) {
-        constexpr int NS = decltype(ns_tag)::value, PER = decltype(per_tag)::value;
-        for (int base = 0; base < items; base += PER * NT) {
-            u32x4 row[PER][NS];
-            float4 gate[PER], tok[PER];
-            float tok_score[PER];
-            auto piece = [&](int p) { const int i = base + p * NT + (int)threadIdx.x; return i < items ? i : items - 1; };
-#pragma unroll
-            for (int p = 0; p < PER; p++) {
-                const int item = piece(p), n = item / Q, c = 4 * (item % Q);
-#pragma unroll
-                for (int s = 0; s < NS; s++)
-                    row[p][s] = __builtin_amdgcn_raw_buffer_load_b128(ob, (((s < nsplit ? s : nsplit - 1) * 16 + n) * D + c) * 4, 0, kThrough);
-                gate[p] = load_f4(one.gate + ((size_t)kvh * hpk + 16 * hg + n) * one.gate_stride + c);
-                tok_score[p] = neg_inf();
-                tok[p] = float4{0.f, 0.f, 0.f, 0.f};
-                if constexpr (STEP) {
-                    tok_score[p] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(sp.new_score), ((kvh * nhg + hg) * 16 + n) * 4, 0, kThrough));
-                    const float4 v = load_f4(sp.v_in + (size_t)kvh * D + c);   // as the cache holds it
-                    tok[p] = float4{from_kv(to_kv<KV>(v.x)), from_kv(to_kv<KV>(v.y)), from_kv(to_kv<KV>(v.z)), from_kv(to_kv<KV>(v.w))};
-                }
-            }
-            if (base == 0) {
-#pragma unroll
-                for (int i = 0; i < kOneSplits * 32 / NT; i++) s_stat[(i * NT + threadIdx.x) / 32][threadIdx.x % 32] = __builtin_bit_cast(float, stat[i]);
-                __syncthreads();
-            }
-#pragma unroll
-            for (int p = 0; p < PER; p++) {
-                const int item = piece(p), n = item / Q, c = 4 * (item % Q);
-                float M = tok_score[p];
-#pragma unroll
-                for (int s = 0; s < NS; s++) M = fmaxf(M, s < nsplit ? s_stat[s][n] : neg_inf());
-                const float wt = tok_score[p] == neg_inf() ? 0.f : fast_exp2(tok_score[p] - M);
-                float den = wt;
-                float4 acc = {wt * tok[p].x, wt * tok[p].y, wt * tok[p].z, wt * tok[p].w};
-#pragma unroll
-                for (int s = 0; s < NS; s++) {
-                    const float m = s < nsplit ? s_stat[s][n] : neg_inf(), w = m == neg_inf() ? 0.f : fast_exp2(m - M);
-                    if (w != 0.f) {   // (a split without positions left its rows unwritten)
-                        const float4 x = __builtin_bit_cast(float4, row[p][s]);
-                        den += w * s_stat[s][16 + n];
-                        acc.x += w * x.x; acc.y += w * x.y; acc.z += w * x.z; acc.w += w * x.w;
-                    }
-                }
-                if (base + p * NT + (int)threadIdx.x < items)
-                    *(float4 *)(one.out + ((size_t)kvh * hpk + 16 * hg + n) * D + c) =
-                        float4{(acc.x / den) * merge_gate(one.gate, gate[p].x), (acc.y / den) * merge_gate(one.gate, gate[p].y),
-                               (acc.z / den) * merge_gate(one.gate, gate[p].z), (acc.w / den) * merge_gate(one.gate, gate[p].w)};
-            }
-        }
-    };
-    using std::integral_constant;
-    if (nsplit == 1) combine(integral_constant<int, 1>{}, integral_constant<int, 4>{});
-    else if (nsplit <= 4) combine(integral_constant<int, 4>{}, integral_constant<int, 4>{});
-    else if (nsplit <= 8) combine(integral_constant<int, 8>{}, integral_constant<int, 2>{});
-    else combine(integral_constant<int, kOneSplits>{}, integral_constant<int, 2>{});
-}
 
 template <typename KV, int D, bool STEP, bool ONE>
 __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
@@ -335,8 +243,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     __shared__ float sm[kWaves][16];
     __shared__ float sl[kWaves][16];
     __shared__ float2 s_tab[STEP ? 128 : 1];
-    __shared__ int s_last;
-    __shared__ float s_stat[ONE ? kOneSplits : 1][32];
+    __shared__ float s_score[16];   // ONE: the new token's score of each row
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
@@ -359,20 +266,79 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     int64_t c1 = (u0 + units_base + (split < units_rem ? 1 : 0)) * S::GRAN;
     if (c1 > nchunk) c1 = nchunk;
     const size_t pid = ((size_t)kvh * nhg + hg) * nsplit + split;
+    // ONE: what the rows' ends take, requested with the query.  Lane group g of tile t = 4 t + wave holds channels
+    // 16 (4 t + wave) + 4 g .. + 3 of row n.
+    float4 gate_in[ONE ? TPW : 1], tok_v[ONE && STEP ? TPW : 1];
+    const size_t out_row = (size_t)kvh * hpk + (rows.valid(n) ? 16 * hg + n : 0);
+    auto channel = [&](int t) { return 16 * (kWaves * t + wave) + 4 * g; };
+    auto request_outer = [&]() __attribute__((always_inline)) {
+        if constexpr (ONE) {
+#pragma unroll
+            for (int t = 0; t < TPW; t++) gate_in[t] = load_f4(one.gate + out_row * one.gate_stride + channel(t));
+            if constexpr (STEP) {
+#pragma unroll
+                for (int t = 0; t < TPW; t++) tok_v[t] = load_f4(sp.v_in + (size_t)kvh * D + channel(t));
+            }
+        }
+    };
+    // the gates' sigmoids and the token's value as the cache holds it, while the cache's first blocks are on their way
+    auto prepare_outer = [&]() __attribute__((always_inline)) {
+        if constexpr (ONE) {
+#pragma unroll
+            for (int t = 0; t < TPW; t++) {
+                float4 &x = gate_in[t];
+                x = float4{merge_gate(one.gate, x.x), merge_gate(one.gate, x.y), merge_gate(one.gate, x.z), merge_gate(one.gate, x.w)};
+                if constexpr (STEP) {
+                    float4 &v = tok_v[t];
+                    v = float4{from_kv(to_kv<KV>(v.x)), from_kv(to_kv<KV>(v.y)), from_kv(to_kv<KV>(v.z)), from_kv(to_kv<KV>(v.w))};
+                }
+            }
+        }
+    };
+    // the rows o (against maximum m, with sum l) and the token (its score in s_score), normalised and gated
+    auto finish_one = [&](const f32x4 (&o)[TPW], float m, float l) __attribute__((always_inline)) {
+        if constexpr (ONE) {
+            float M = m, ts = neg_inf();
+            if constexpr (STEP) {
+                ts = s_score[n];
+                M = fmaxf(M, ts);
+            }
+            const float w = m == neg_inf() ? 0.f : fast_exp2(m - M), wt = ts == neg_inf() ? 0.f : fast_exp2(ts - M);
+            const float den = w * l + wt;
+#pragma unroll
+            for (int t = 0; t < TPW; t++) {
+                float4 y = {w * o[t][0], w * o[t][1], w * o[t][2], w * o[t][3]};
+                if constexpr (STEP) {
+                    y.x += wt * tok_v[t].x; y.y += wt * tok_v[t].y; y.z += wt * tok_v[t].z; y.w += wt * tok_v[t].w;
+                }
+                if (rows.valid(n))
+                    *(float4 *)(one.out + out_row * D + channel(t)) =
+                        float4{(y.x / den) * gate_in[t].x, (y.y / den) * gate_in[t].y, (y.z / den) * gate_in[t].z, (y.w / den) * gate_in[t].w};
+            }
+        }
+    };
     if constexpr (STEP) {
         if (with_new && c0 >= c1) {
             // no positions for this split (an empty cache): its partial weighs nothing, the token is all there is
-            if (wave == 0 && g == 0) {
+            if (!ONE && wave == 0 && g == 0) {
                 const __amdgpu_buffer_rsrc_t mlb = buffer_of(part_ml + pid * 32);
                 __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, neg_inf()), mlb, n * 4, 0, kThrough);
                 __builtin_amdgcn_raw_buffer_store_b32(0u, mlb, (16 + n) * 4, 0, kThrough);
             }
             StepQuery<KV, D, NT> sq;
             sq.request(sp, rows);
+            request_outer();
             HeadRotor<sq.EPS, D>::table(sq.freq, sp.pos, sp.rotary_dim, s_tab);
             __syncthreads();
-            sq.finish(sp, rows, qscale, plane_elems, true, qlds, nhg, s_tab);
-            if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
+            sq.finish(sp, rows, qscale, plane_elems, true, qlds, nhg, s_tab, ONE ? s_score : nullptr);
+            if constexpr (ONE) {
+                f32x4 none[TPW];
+#pragma unroll
+                for (int t = 0; t < TPW; t++) none[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                prepare_outer();
+                lds_barrier();
+                finish_one(none, neg_inf(), 0.f);
+            }
             return;
         }
     }
@@ -384,7 +350,6 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, neg_inf()), mlb, n * 4, 0, kThrough);
             __builtin_amdgcn_raw_buffer_store_b32(0u, mlb, (16 + n) * 4, 0, kThrough);
         }
-        if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
         return;
     }
 
@@ -404,6 +369,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
             W::load_q_slot(qraw[i], q, slot, rows);
         }
     }
+    request_outer();
     // A CU returns load data in request order across its waves: hold the cache requests
     // back until every wave's query request is queued, or a late wave's query would
     // sit behind its siblings' cache data.
@@ -458,7 +424,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
         HeadRotor<sq.EPS, D>::table(sq.freq, sp.pos, sp.rotary_dim, s_tab);
         lds_barrier();
         rest_of_ring();
-        sq.finish(sp, rows, qscale, plane_elems, with_new, qlds, nhg, s_tab);
+        sq.finish(sp, rows, qscale, plane_elems, with_new, qlds, nhg, s_tab, ONE ? s_score : nullptr);
     } else {
 #pragma unroll
         for (int i = 0; i < NQ; i++) {
@@ -467,6 +433,7 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
         }
         rest_of_ring();
     }
+    prepare_outer();
     lds_barrier();
     uint4 qr[W::QREGS];
 #pragma unroll
@@ -573,6 +540,14 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     // ---- one partial per workgroup -----------------------------------------------
     l_run = rows_sum(l_run);
     if (g == 0) sl[wave][n] = l_run;
+    if constexpr (ONE) {
+        lds_barrier();
+        float lsum = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) lsum += sl[w][n];
+        finish_one(o, m_run, lsum);
+        return;
+    }
     const __amdgpu_buffer_rsrc_t ob = buffer_of(part_o + pid * 16 * D);
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
@@ -589,7 +564,6 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, m_run), mlb, n * 4, 0, kThrough);
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, lsum), mlb, (16 + n) * 4, 0, kThrough);
     }
-    if constexpr (ONE) one_launch_merge<KV, D, STEP>(one, part_o, part_ml, nsplit, nhg, hpk, Hq, kvh, hg, sp, &s_last, s_stat);
 }
 
 // The token a decode step has just appended, as one more split of the merge (MergeOut), and
@@ -811,26 +785,30 @@ static int fit_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int n
     return MFA_OK;
 }
 
-// Whether one launch serves a decode call (OneLaunch), and its plan: up to 1024 positions and 768 KiB of K and V per kv head,
-// in at most kOneSplits splits of a pass each.  Measured per layer, three sequences side by side: 7.4 -> 3.6 us at 20 .. 1000
-// positions (16 or 32 heads over 2 of 256, 32 over 4 of 128); one sequence after itself 7.6 -> 6.1 at 20, 8.8 -> 9.8 at 515, 8.5 -> 8.8
-// at 1000.  Past the limits the last workgroup's share of the merge, and the shares of the fewer splits, cost a single sequence
-// more than the launch they save (3000 positions: 9.8 -> 12 to 16.5 us).
-static constexpr int64_t kOnePositions = 1024, kOneBytes = 768 << 10;
-static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int64_t kv_len, int forced_splits, const SdpaWorkspace &ws) {
-    if (!ws.tickets || forced_splits > 0 || kv_len > kOnePositions) return false;
-    if (kv_len * D * (kv_dtype == MFA_KV_BF16 ? 4 : 8) > kOneBytes) return false;
+// Whether one launch serves a decode call (OneLaunch), and its plan: a cache of so few chunks of 64 positions that a workgroup
+// streams them in no more time than the second launch takes, for one sequence alone.  (A chunk takes it 0.12, 0.25 and 0.5 us
+// by width over a bf16 cache, over f32 0.3, 1.2 and 2.5; partials that another workgroup merges when a ticket says it is the last, in
+// one launch as well, cost a sequence 1.3 us and more over the two launches at 256 channels: the hop through memory is three trips.)
+// Calls one after the other, and one call and its wait, in us with one launch and with two:
+//   decode  16 heads over 2 of 256, bf16    64: 6.5, 9.1 and 19.2, 21.1   320: 7.5, 9.2 and 21.5, 22.6   515: 12.2, 9.3 and 24.4, 22.5
+//           32 over 4 of 128, bf16          64: 6.7, 9.3 and 18.2, 20.5   320: 6.7, 9.3 and 19.9, 21.2   768: 10.3, 9.4 and 22.8, 21.0
+//           32 over 4 of 128, f32           64: 6.7, 9.2 and 19.1, 21.2   192: 7.5, 9.4 and 21.7, 21.6   320: 10.4, 9.2 and 24.6, 21.6
+//   step    16 over 2 of 256, bf16         128: 10.5, 11.9 and 25.5, 26.8   256: 11.9, 11.3 and 26.8, 26.5
+// Three sequences side by side 6.6 and 9.3 (decode), 8.0 and 10.6 (step) at all these lengths: bound by the host's launches.
+static int one_launch_chunks(int kv_dtype, int D, bool step) {
+    static constexpr int kDecode[2][3] = {{12, 5, 5}, {4, 3, 1}}, kStep[2][3] = {{10, 3, 3}, {3, 2, 1}};
+    const int f32 = kv_dtype == MFA_KV_F32, w = D == 64 ? 0 : D == 128 ? 1 : 2;
+    return step ? kStep[f32][w] : kDecode[f32][w];
+}
+static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int64_t kv_len, int forced_splits, bool step) {
+    const int64_t nchunk = (kv_len + kKvChunk - 1) / kKvChunk;
+    if (forced_splits > 0 || nchunk > one_launch_chunks(kv_dtype, D, step)) return false;
     const int U = unit_chunks(kv_dtype, D);
-    const int64_t nchunk = (kv_len + kKvChunk - 1) / kKvChunk, nunits = nchunk > U ? (nchunk + U - 1) / U : 1;
-    const int64_t min_units = (min_pass_chunks(kv_dtype, D) + U - 1) / U;
-    int64_t splits = nunits / min_units;
-    if (splits > kOneSplits) splits = kOneSplits;
-    if (splits < 1) splits = 1;
     plan.nhg = (Hq / Hkv + 15) / 16;
-    plan.splits = (int)splits;
-    plan.base = (int)(nunits / splits);
-    plan.rem = (int)(nunits % splits);
-    return sdpa_workspace_o_elems(Hq, Hkv, D, plan.splits) <= ws.part_o_elems && sdpa_workspace_ml_elems(Hq, Hkv, plan.splits) <= ws.part_ml_elems;
+    plan.splits = 1;
+    plan.base = (int)((nchunk + U - 1) / U);
+    plan.rem = 0;
+    return true;
 }
 
 // One decode token of a full-attention layer from its raw projections in two launches: the
@@ -850,9 +828,9 @@ int launch_sdpa_step(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, i
     // (one launch: a row group's result may be out before another's inputs are in, so they lie apart)
     const size_t qd = (size_t)Hq * D, kd = (size_t)Hkv * D;
     const bool one = !overlap(out, qd, q_proj, 2 * qd) && !overlap(out, qd, k_in, kd) && !overlap(out, qd, v_in, kd) &&
-                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, ws);
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, true);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, 1, len0 > 0 ? len0 : 1, num_cus, forced_splits, ws));
-    const OneLaunch ol{q_proj + D, out, 2 * D, ws.tickets};
+    const OneLaunch ol{q_proj + D, out, 2 * D};
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     const StepPrologue sp{q_proj, k_in, v_in, q_norm, k_norm, inv_freq, rotary_dim, eps, pos, len0, new_score,
                           k_tiled, v_tiled, plan.splits - 1};
@@ -873,7 +851,7 @@ int launch_sdpa_step(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, i
 int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_tok, int64_t kv_len,
                 size_t plane_elems, const void *k_tiled, const void *v_tiled, const float *q,
                 const float *gate, float *out, const SdpaWorkspace &ws, int num_cus,
-                int forced_splits, int partial_only, SdpaMergeTask *defer_merge) {
+                int forced_splits, int partial_only, SdpaMergeTask *defer_merge, bool one_layer) {
     if (defer_merge) defer_merge->n_units = 0;
     if (!sdpa_shape_supported(kv_dtype, D))
         return fail(MFA_ERR_SHAPE, "sdpa: head_dim %d / kv dtype %d not supported", D, kv_dtype);
@@ -884,10 +862,10 @@ int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_
     // (one launch: a row group's result may be out before another's query is in; in place it lies over its own)
     const size_t qd = (size_t)Hq * D;
     const bool apart = (out == q || !overlap(out, qd, q, qd)) && (out == gate || !overlap(out, qd, gate, qd));
-    const bool one = n_tok == 1 && gate && apart && !partial_only && !defer_merge &&
-                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, ws);
+    const bool one = one_layer && n_tok == 1 && gate && apart && !partial_only && !defer_merge &&
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, false);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, forced_splits, ws));
-    const OneLaunch ol{gate, out, D, ws.tickets};
+    const OneLaunch ol{gate, out, D};
     // scores are produced in log2 units: q is pre-multiplied by (1/sqrt(D)) * log2(e)
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     launch_partial_any<false>(kv_dtype, D, stream, dim3(plan.splits, plan.nhg, Hkv), k_tiled, v_tiled, plane_elems, q,

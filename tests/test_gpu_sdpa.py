@@ -221,11 +221,13 @@ def test_shares_of_a_single_unit(mfa, oracle, Hq, Hkv, d, bf16):
     (16, 2, 256, True, (1, 127, 129, 515, 768, 769)), (32, 2, 256, True, (64, 640)), (40, 2, 128, True, (1023, 1024, 1025)),
     (32, 4, 128, False, (1, 63, 65, 767, 768, 769)), (4, 2, 64, True, (130, 1024)), (3, 1, 64, False, (500, 1024)),
     (18, 1, 256, False, (384, 385)),
+    (16, 2, 256, True, (319, 320, 321)), (32, 4, 128, True, (257, 320, 321)), (4, 2, 64, True, (767, 768, 769)),
+    (40, 2, 256, False, (1, 63, 64, 65)), (32, 4, 128, False, (191, 192, 193)), (3, 1, 64, False, (1, 255, 256, 257)),
 ])
 def test_short_caches_merge_in_the_attention_launch(mfa, oracle, Hq, Hkv, d, bf16, lens):
-    """Either side of the limits of the launch that merges its own partials (up to 1024 positions and 768 KiB per kv head;
-    more than 16 heads per kv head are two row groups): against the oracle, three calls in a row the same to the bit (the
-    counters are back at 0), over a workspace of NaN, and the merge launch (a forced split count) within rounding."""
+    """Either side of the limits of the launch that is the whole of a decode call (whole chunks of 64 positions; more than 16
+    heads per kv head are two row groups): against the oracle, three calls in a row the same to the bit, over a workspace of
+    NaN, and the merge launch (a forced split count) within rounding."""
     from moeflux_amd import Config
     top = max(lens)
     q, g, k, v = sdpa_random_inputs(top + d, Hq, Hkv, d, top, bf16=bf16)
@@ -300,3 +302,34 @@ def test_chunk_result_shifted_over_the_query(mfa, oracle):
             assert c.lib.mfa_prefill_attn_dev(c.h, 0, T, buf.offset(n), dg.ptr, dk.ptr, dv.ptr, buf.offset(n + off)) == 0
             c.sync()
             assert rel_err(buf.to_host()[n + off:][:n], want) <= 1e-4, off
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,bf16,lens", [
+    (16, 2, 256, True, (0, 1, 64, 65, 191, 192, 193)), (40, 2, 128, True, (0, 63, 192, 193)), (6, 2, 64, True, (0, 127, 640, 641)),
+    (32, 2, 256, False, (0, 1, 64, 65)), (3, 1, 128, False, (0, 127, 128, 129)), (16, 2, 64, False, (0, 192, 193)),
+])
+def test_short_steps_in_one_launch(mfa, oracle, Hq, Hkv, d, bf16, lens):
+    """A step either side of the limits of its one launch: against the oracle's prologue and attention over the cache as
+    exported, three times the same to the bit, and the forced split counts' two launches within rounding."""
+    rng = np.random.default_rng(d + Hq)
+    norm = [oracle.f32_to_bf16(1.0 + 0.1 * rng.standard_normal(d)) for _ in range(2)]
+    _, _, k, v = sdpa_random_inputs(d, Hq, Hkv, d, max(lens) + 1, bf16=bf16)
+    qp, kn, vn = (rng.standard_normal(m).astype(np.float32) for m in (2 * Hq * d, Hkv * d, Hkv * d))
+    tol = 1e-4 if bf16 else TOL_F32
+    with _ctx(mfa, num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d, kv_capacity=max(lens) + 1,
+              kv_dtype=1 if bf16 else 0) as c:
+        c.set_full_weights(0, *norm)
+        for n in lens:
+            outs = []
+            for splits in (0, 0, 0, 1, 2):
+                c.memory_clear()
+                if n:
+                    c.kv_import(0, k[:n], v[:n])
+                assert c.lib.mfa_debug_fill_workspace(c.h, 0x7FC00000) == 0
+                c.set_num_splits(splits)
+                outs.append(c.full_attn_step(0, n, qp, kn, vn))
+            kc, vc = c.kv_export(0)
+            rq, rg, _, _ = oracle.attn_prologue(n, Hq, Hkv, d, d // 4, 1.0e7, 1e-6, *norm, qp, kn, vn)
+            assert rel_err(outs[0], oracle.sdpa(n + 1, Hq, Hkv, d, rq, rg, kc, vc)) <= tol, n
+            assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2]), n
+            assert all(rel_err(outs[0], o) <= tol for o in outs[3:]), n
