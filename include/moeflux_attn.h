@@ -483,6 +483,9 @@ int32_t mfa_debug_chunk_route(int32_t kv_dtype, int32_t num_attn_heads, int32_t 
  * sizes.  A measurement and test switch; no result depends on it beyond rounding.  A chunk whose
  * partials would not fit the workspace is refused. */
 int mfa_debug_set_chunk_route(mfa_ctx *ctx, int32_t route);
+/* mfa_kv_export of the first `rows` positions (1 .. kv_capacity), whatever the layer's length: what
+ * a truncation leaves behind it.  No counterpart in the reference. */
+int mfa_debug_kv_export(mfa_ctx *ctx, int32_t layer, int32_t rows, float *k_out, float *v_out);
 
 /* A plain device-to-device copy kernel on the context's stream (nbytes read, nbytes
  * written, nbytes a multiple of 16): a launch of known memory traffic, used to scale

@@ -1153,22 +1153,33 @@ int32_t mfa_pos_max(mfa_ctx *ctx) {
     return m;
 }
 
+// The first `rows` positions of a layer's cache, row by row.
+static int kv_read(Ctx *c, const FullLayer *f, int32_t rows, float *k_out, float *v_out) {
+    const size_t n = (size_t)rows * c->kv_dim();
+    MFA_TRY(ensure_stage(c, 2 * n));
+    MFA_TRY(launch_kv_gather(c->stream, c->cfg.kv_dtype, c->cfg.num_kv_heads, c->cfg.head_dim,
+                             c->plane_elems, rows, f->k, f->v, c->stage, c->stage + n));
+    MFA_HIP(hipMemcpyAsync(k_out, c->stage, n * 4, hipMemcpyDeviceToHost, c->stream));
+    MFA_TRY(d2h_sync(c, v_out, c->stage + n, n * 4));
+    return release_stage_beyond_cap(c);
+}
+
 int mfa_kv_export(mfa_ctx *ctx, int32_t layer, int32_t max_rows, float *k_out, float *v_out) {
     Ctx *c = as_ctx(ctx);
     FullLayer *f;
     MFA_TRY(full_layer(c, layer, &f));
     if (!k_out || !v_out) return fail(MFA_ERR_INVALID, "NULL argument");
     if (max_rows < f->len) return fail(MFA_ERR_INVALID, "buffer holds %d rows, layer has %d", max_rows, f->len);
-    if (f->len == 0) return MFA_OK;
-    const size_t n = (size_t)f->len * c->kv_dim();
-    MFA_TRY(ensure_stage(c, 2 * n));
-    MFA_TRY(launch_kv_gather(c->stream, c->cfg.kv_dtype, c->cfg.num_kv_heads, c->cfg.head_dim,
-                             c->plane_elems, f->len, f->k, f->v, c->stage, c->stage + n));
-    MFA_HIP(hipMemcpyAsync(k_out, c->stage, n * 4, hipMemcpyDeviceToHost, c->stream));
-    MFA_TRY(d2h_sync(c, v_out, c->stage + n, n * 4));
-    return release_stage_beyond_cap(c);
+    return f->len == 0 ? MFA_OK : kv_read(c, f, f->len, k_out, v_out);
 }
 
+int mfa_debug_kv_export(mfa_ctx *ctx, int32_t layer, int32_t rows, float *k_out, float *v_out) {
+    Ctx *c = as_ctx(ctx);
+    FullLayer *f;
+    MFA_TRY(full_layer(c, layer, &f));
+    if (!k_out || !v_out || rows <= 0 || rows > c->cfg.kv_capacity) return fail(MFA_ERR_INVALID, "NULL argument or %d rows", rows);
+    return kv_read(c, f, rows, k_out, v_out);
+}
 
 void *mfa_host_alloc(int64_t bytes) {
     if (bytes <= 0) {

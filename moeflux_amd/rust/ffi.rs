@@ -156,6 +156,7 @@ extern "C" {
     pub fn mfa_debug_chunk_route(kv_dtype: i32, num_attn_heads: i32, num_kv_heads: i32, head_dim: i32,
         n_tok: i32, kv_len: i64, num_cus: i32, raw: i32) -> i32;
     pub fn mfa_debug_set_chunk_route(ctx: *mut mfa_ctx, route: i32) -> c_int;
+    pub fn mfa_debug_kv_export(ctx: *mut mfa_ctx, layer: i32, rows: i32, k: *mut f32, v: *mut f32) -> c_int;
     pub fn mfa_debug_copy_dev(ctx: *mut mfa_ctx, dst_dev: *mut c_void, src_dev: *const c_void,
         nbytes: usize) -> c_int;
     pub fn mfa_debug_read_dev(ctx: *mut mfa_ctx, src_dev: *const c_void, nbytes: usize, workgroups: i32) -> c_int;
