@@ -97,6 +97,9 @@ static void destroy(Ctx *c) {
     if (c->stage) (void)hipFree(c->stage);
     if (c->gdn_scratch) (void)hipFree(c->gdn_scratch);
     if (c->qg_chunk) (void)hipFree(c->qg_chunk);
+    if (c->rot_chunk) (void)hipFree(c->rot_chunk);
+    for (void *p : c->outgrown)
+        if (p) (void)hipFree(p);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -337,6 +340,42 @@ static int ensure_workspace(Ctx *c, int n_tok, int64_t kv_len, int layers = 1) {
                                   sdpa_workspace_ml_elems(Hq, Hkv, splits, n_tok));
 }
 
+static bool capturing(const Ctx *c) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(c->stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+
+// hipMalloc in the mode that leaves captures alone, this stream's and others': in the usual one it is refused, and ends them.
+static hipError_t malloc_beside_captures(void **p, size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return e;
+    e = hipMalloc(p, bytes);
+    const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+    return e != hipSuccess ? e : back;
+}
+
+// Grows a chunk's scratch buffer to `need` floats.  Each route of a chunk has a buffer of its own, so that no chunk of as many
+// tokens on the other moves it from under a captured graph; while the stream is captured nothing may be waited for or
+// freed, and what is outgrown then stays until the context ends.
+static int ensure_chunk_scratch(Ctx *c, float **buf, size_t *elems, size_t need) {
+    if (need <= *elems) return MFA_OK;
+    float *grown = nullptr;
+    if (capturing(c)) {
+        MFA_HIP(malloc_beside_captures((void **)&grown, need * sizeof(float)));
+        if (*buf) c->outgrown.push_back(*buf);
+    } else {
+        MFA_HIP(hipStreamSynchronize(c->stream));
+        if (*buf) MFA_HIP(hipFree(*buf));
+        *buf = nullptr;
+        *elems = 0;
+        MFA_HIP(hipMalloc((void **)&grown, need * sizeof(float)));
+    }
+    *buf = grown;
+    *elems = need;
+    return MFA_OK;
+}
+
 // The plan of a prompt chunk (a forced split count is the split-K kernel's), and the memory it takes.  The first plan that
 // splits the cache on 32x32 tiles allocates their workspace, whose size never changes; without memory for it, or while
 // the stream is being captured, the plan is one that needs none.  Nor does a capture grow the split-K workspace.
@@ -349,10 +388,6 @@ static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, Ch
         return sdpa_chunk_plan(g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, n_tok, kv_len, c->num_cus, kind,
                                ChunkLimits{ws_elems, split_k, shifted});
     };
-    const auto capturing = [&] {
-        hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-        return hipStreamIsCapturing(c->stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
-    };
     if (!c->forced_splits && !c->partial_only) {
         p = plan(kChunkPartElems, true);
         if (c->chunk_route > 0 && g.kv_dtype == MFA_KV_BF16 && n_tok > 1) {
@@ -362,15 +397,9 @@ static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, Ch
                 return fail(MFA_ERR_INVALID, "sdpa: %d splits of the chunk do not fit its workspace", p.splits);
         }
         if (p.route == ChunkRoute::Tiles32 && p.splits > 1 && !c->chunk_part) {
-            if (!capturing()) {
-                // in the mode that leaves captures of other streams alone: an allocation in the usual one ends them
-                hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-                MFA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-                if (hipMalloc((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
-                    (void)hipGetLastError();
-                    c->chunk_part = nullptr;
-                }
-                MFA_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+            if (!capturing(c) && malloc_beside_captures((void **)&c->chunk_part, (kChunkPartElems + kChunkPartElems / 32) * sizeof(float)) != hipSuccess) {
+                (void)hipGetLastError();
+                c->chunk_part = nullptr;
             }
             if (c->chunk_part) c->chunk_part_elems = kChunkPartElems;
             else p = plan(0, true);
@@ -380,7 +409,7 @@ static int chunk_plan(Ctx *c, int n_tok, int64_t kv_len, ChunkQueryKind kind, Ch
     const int64_t nhg = ((int64_t)n_tok * (g.num_attn_heads / g.num_kv_heads) + 15) / 16;
     if (nhg > 65535) return fail(MFA_ERR_SHAPE, "sdpa: too many query rows in one call");
     if (n_tok == 1) return MFA_OK;
-    if (!c->forced_splits && !c->partial_only && !split_k_workspace_holds(c, n_tok) && capturing()) {
+    if (!c->forced_splits && !c->partial_only && !split_k_workspace_holds(c, n_tok) && capturing(c)) {
         p = plan(c->chunk_part_elems, false);
         if (p.route != ChunkRoute::SplitK) return MFA_OK;
     }
@@ -786,27 +815,18 @@ int mfa_prefill_full_attn_dev(mfa_ctx *ctx, int32_t layer, int32_t pos0, int32_t
     ChunkPlan plan;
     MFA_TRY(chunk_plan(c, T, (int64_t)f->len + T, kind, &plan));
     const bool raw = plan.route == ChunkRoute::Tiles32 && kind == ChunkQueryKind::Raw;
-    // Sized for either route (the table is T * rotary_dim floats, less than a head's rows), so that no later chunk of as
-    // many tokens moves it: not one under capture, and none from under a graph that was captured.
-    const size_t need = 2 * qd;
-    if (need > c->qg_chunk_elems) {
-        MFA_HIP(hipStreamSynchronize(c->stream));
-        if (c->qg_chunk) MFA_HIP(hipFree(c->qg_chunk));
-        c->qg_chunk = nullptr;
-        c->qg_chunk_elems = 0;
-        MFA_HIP(hipMalloc((void **)&c->qg_chunk, need * sizeof(float)));
-        c->qg_chunk_elems = need;
-    }
+    MFA_TRY(raw ? ensure_chunk_scratch(c, &c->rot_chunk, &c->rot_chunk_elems, (size_t)T * c->rotary_dim)
+                : ensure_chunk_scratch(c, &c->qg_chunk, &c->qg_chunk_elems, 2 * qd));
     // the whole chunk is normed, rotated and appended, then one causal pass: row t sees positions [0, len0 + t]
     const int32_t len0 = f->len;
     int rc = MFA_OK;
     if (raw) {
         const int D = c->cfg.head_dim;
         rc = launch_attn_prologue_kv(c->stream, c->cfg.kv_dtype, c->cfg.num_kv_heads, D, c->rotary_dim, c->cfg.rms_norm_eps, T, pos0,
-                                     len0, c->plane_elems, f->k_norm, c->inv_freq, k_dev, v_dev, (float2 *)c->qg_chunk, f->k, f->v);
+                                     len0, c->plane_elems, f->k_norm, c->inv_freq, k_dev, v_dev, (float2 *)c->rot_chunk, f->k, f->v);
         if (rc == MFA_OK) {
             f->len += T;
-            const ChunkQuery in{q_proj_out_dev, q_proj_out_dev + D, 2 * D, f->q_norm, (const float2 *)c->qg_chunk, c->cfg.rms_norm_eps};
+            const ChunkQuery in{q_proj_out_dev, q_proj_out_dev + D, 2 * D, f->q_norm, (const float2 *)c->rot_chunk, c->cfg.rms_norm_eps};
             rc = launch_sdpa_chunk(c->stream, plan, c->cfg.num_attn_heads, c->cfg.num_kv_heads, D, T, f->len, c->plane_elems, f->k,
                                    f->v, in, out_dev, c->chunk_part, c->chunk_part_elems);
         }

@@ -155,6 +155,9 @@ struct Ctx {
     int32_t step_launches = 2;   // launches of mfa_full_attn_step: 2 (prologue inside the attention launch) or 3
     float *qg_chunk = nullptr;   // the same for a chunk of tokens (mfa_prefill_full_attn), grown on demand
     size_t qg_chunk_elems = 0;
+    float *rot_chunk = nullptr;  // the rotations of a chunk whose query the attention launch norms, grown on demand
+    size_t rot_chunk_elems = 0;
+    std::vector<void *> outgrown;   // buffers that a capture outgrew
     int64_t cap_pad = 0;        // kv capacity rounded up to whole K chunks
     size_t plane_elems = 0;     // elements of one (layer, K|V, kv head) plane
     // split-K workspace

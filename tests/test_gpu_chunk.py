@@ -213,11 +213,12 @@ class _Graph:
         assert self.rt.hipGraphExecDestroy(self.run) == 0 and self.rt.hipGraphDestroy(self.graph) == 0
 
 
+@pytest.mark.parametrize("few", [0, 40])
 @pytest.mark.parametrize("first", ["over the projection", "apart"])
-def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first):
+def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first, few):
     """A chunk whose result lies over its projection (a prologue of its own) captured behind one of as many tokens whose
-    result lies apart (query normed in the attention launch), and the other way round; then the first route again, eagerly,
-    and replays."""
+    result lies apart (query normed in the attention launch), and the other way round, on scratch that the capture makes or
+    (after a chunk of few tokens) grows; then the first route again, eagerly, and replays."""
     from moeflux_amd.hip import H2D, DeviceArray, rt
     Hq, Hkv, d, T = 16, 2, 256, 300
     rng = np.random.default_rng(4)
@@ -230,9 +231,9 @@ def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first):
         want = c.prefill_full_attn(0, 0, qp, k, v)
         bufs = {"apart": (DeviceArray.from_host(qp), DeviceArray((T, Hq * d), zero=True)), "over the projection": (DeviceArray.from_host(qp),) * 2}
 
-        def call(where):
+        def call(where, n=T):
             q, out = bufs[where]
-            return c.lib.mfa_prefill_full_attn_dev(c.h, 0, 0, T, q.ptr, dk.ptr, dv.ptr, out.ptr)
+            return c.lib.mfa_prefill_full_attn_dev(c.h, 0, 0, n, q.ptr, dk.ptr, dv.ptr, out.ptr)
 
         def check(where):
             assert rel_err(bufs[where][1].to_host().reshape(-1)[:T * Hq * d].reshape(T, Hq * d), want) <= TOL
@@ -241,6 +242,11 @@ def test_both_routes_of_a_raw_chunk_share_their_scratch(mfa, oracle, first):
         second = next(w for w in bufs if w != first)
     with _ctx(mfa, Hq, Hkv, d, T) as c:   # its scratch is of its own first chunk
         c.set_full_weights(0, *norm)
+        if few:
+            assert call(second, few) == 0
+            c.sync()
+            assert rt().hipMemcpy(bufs[second][0].ptr, qp.ctypes.data, qp.nbytes, H2D) == 0
+            c.memory_clear()
         assert call(first) == 0
         c.sync()
         check(first)
