@@ -245,11 +245,12 @@ int mfa_full_attn_step_dev(mfa_ctx *ctx, int32_t layer, int32_t pos, const float
  * depends on it beyond rounding.  2 (default, where rotary_dim / 2 is a multiple of 8 channels
  * for a bf16 cache, 4 for f32): the attention launch norms and rotates its own query heads from
  * q_proj_out, attends to the positions the cache already holds, and scores and appends the new
- * token; the merge launch takes the token as one more split.  A short cache takes one launch,
- * whose workgroups hold a row from start to end: up to 10, 3 and 3 chunks of 64 positions at
- * head_dim 64, 128 and 256 of a bf16 cache, 3, 2 and 1 of an f32 one.  3: prologue, attention, merge
- * (attention and merge in one up to 12, 5 and 5 chunks, f32 4, 3 and 1, as mfa_sdpa_decode).
- * A forced split count (mfa_set_num_splits) always takes the merge launch. */
+ * token; the merge launch takes the token as one more split.  A short cache takes one launch:
+ * up to 16, 13 and 3 chunks of 64 positions at head_dim 64, 128 and 256 of a bf16 cache, 16, 5 and
+ * 1 of an f32 one (with one or two query heads per kv head 5, 1, 1 and 1, 1, 1).  3: prologue,
+ * attention, merge, the last two in one launch as in mfa_sdpa_decode: up to 16, 9 and 5 chunks, f32
+ * 9, 3 and 1 (6, 2, 2 and 2, 1, 1).  A forced split count (mfa_set_num_splits) always takes the merge
+ * launch. */
 int mfa_set_step_launches(mfa_ctx *ctx, int32_t launches);
 /* The same for a chunk of T prompt tokens at positions pos0 .. pos0+T-1 (the token
  * loop of eval_prompt, riir/mod.rs:1196-1214, over full_attn_layer_forward): every

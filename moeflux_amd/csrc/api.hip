@@ -71,7 +71,7 @@ int release_stage_beyond_cap(Ctx *c) {
 }
 
 static SdpaWorkspace workspace(Ctx *c) {
-    return SdpaWorkspace{c->part_o, c->part_ml, c->part_o_elems, c->part_ml_elems};
+    return SdpaWorkspace{c->part_o, c->part_ml, c->part_o_elems, c->part_ml_elems, c->tickets};
 }
 
 static int h2d(Ctx *c, void *dst, const void *src, size_t bytes) {
@@ -218,11 +218,12 @@ static int create(const mfa_config *cfg, Ctx **out) {
         char *qg;
         MFA_TRY(slab_alloc(c, 2 * (size_t)cfg->num_attn_heads * cfg->head_dim * sizeof(float), &qg));
         c->qg_stage = (float *)qg;
-        // per (kv head, 16-row group): the new token's 16 scores
+        // per (kv head, 16-row group): the new token's 16 scores; behind them all, the groups' tickets
         const size_t groups = (size_t)cfg->num_kv_heads * ((cfg->num_attn_heads / cfg->num_kv_heads + 15) / 16);
         char *sc;
-        MFA_TRY(slab_alloc(c, groups * 16 * sizeof(float), &sc));
+        MFA_TRY(slab_alloc(c, groups * (16 * sizeof(float) + kOneTickets * sizeof(unsigned)), &sc));
         c->step_score = (float *)sc;
+        c->tickets = (unsigned *)(sc + groups * 16 * sizeof(float));
         // variants.rs:245-250, 369: a quarter of the head is rotated, theta = 1e7
         MFA_TRY(set_rope(c, 1.0e7f, cfg->head_dim / 4));
         // room for the most splits any cache length up to the capacity gets

@@ -151,6 +151,7 @@ struct Ctx {
     float *inv_freq = nullptr;
     int32_t rotary_dim = 0;
     float *qg_stage = nullptr;   // q and gate of mfa_full_attn_step, 2 * q_dim floats
+    unsigned *tickets = nullptr; // of the one-launch decode (SdpaWorkspace)
     float *step_score = nullptr; // the new token's score per query row of the two-launch attention step
     int32_t step_launches = 2;   // launches of mfa_full_attn_step: 2 (prologue inside the attention launch) or 3
     float *qg_chunk = nullptr;   // the same for a chunk of tokens (mfa_prefill_full_attn), grown on demand
@@ -224,7 +225,10 @@ struct SdpaWorkspace {
     float *part_o;
     float *part_ml;
     size_t part_o_elems, part_ml_elems;
+    // counters of a decode launch that merges its own partials, [Hkv][16-row groups][kOneTickets], all 0; null: no such launch
+    unsigned *tickets = nullptr;
 };
+static constexpr int kOneTickets = 4;   // one per wave of a workgroup
 bool sdpa_shape_supported(int kv_dtype, int head_dim);
 // Number of splits the launcher will use (for workspace sizing pass kv_len = capacity).
 int sdpa_max_splits(int kv_dtype, int Hq, int Hkv, int D, int64_t max_len, int num_cus, int forced);

@@ -219,13 +219,20 @@ template <int N, int END, int STEP, typename F> __device__ __attribute__((always
     }
 }
 
-// A decode launch that is the whole of the attention, for a short cache: one workgroup per row group, whose rows go out normalised
-// and gated from the registers that hold them, a decode step's new token among their positions (one_launch_plan).
+// A decode launch that is the whole of the attention, for a short cache.  With one workgroup per row group its rows go out
+// normalised and gated from the registers that hold them, a decode step's new token among their positions.  With several,
+// wave w of each holds the same output tiles: it puts its part of the partial out and draws a ticket, and the wave that draws
+// the last of tile set w adds the others' to its own (nobody waits for anybody; the counter goes back to 0 with the last
+// ticket).  A wave's stores are at device scope (sc1), past the L2s of the XCDs, and out before its ticket; that is all the
+// ordering there is to do (one_launch_plan).
 struct OneLaunch {
     const float *gate;
     float *out;
     int gate_stride;
+    unsigned *tickets;   // [kv head][row group][wave], 0 between launches
 };
+static constexpr int kOneSplits = 16;
+static_assert(kOneTickets == kWaves, "a ticket per wave");
 
 template <typename KV, int D, bool STEP, bool ONE>
 __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
@@ -295,14 +302,86 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
             }
         }
     };
-    // the rows o (against maximum m, with sum l) and the token (its score in s_score), normalised and gated
-    auto finish_one = [&](const f32x4 (&o)[TPW], float m, float l) __attribute__((always_inline)) {
+    auto finish_one = [&](f32x4 (&o)[TPW], float m, float l) __attribute__((always_inline)) {
         if constexpr (ONE) {
-            float M = m, ts = neg_inf();
-            if constexpr (STEP) {
-                ts = s_score[n];
-                M = fmaxf(M, ts);
+            float ts = neg_inf();
+            if constexpr (STEP) ts = with_new ? s_score[n] : neg_inf();
+            if (nsplit > 1) {
+                // this wave's tiles, and its own copy of the rows' (maximum, sum, token's score): a ticket orders a wave's own stores
+                const size_t pid0 = ((size_t)kvh * nhg + hg) * nsplit;
+                const __amdgpu_buffer_rsrc_t ob = buffer_of(part_o + pid0 * 16 * D), mlb = buffer_of(part_ml + (pid0 * kWaves) * 48);
+                const int stat = (split * kWaves + wave) * 48;
+                if (rows.valid(n)) {
+#pragma unroll
+                    for (int t = 0; t < TPW; t++)
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[t]), ob, ((split * 16 + n) * D + channel(t)) * 4, 0, kThrough);
+                }
+                if (g < 3) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, g == 0 ? m : g == 1 ? l : ts), mlb, (stat + 16 * g + n) * 4, 0, kThrough);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                unsigned *ticket = one.tickets + (kvh * nhg + hg) * kWaves + wave;
+                unsigned got = 0;
+                if (lane == 0) got = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                got = __builtin_amdgcn_readfirstlane(got);
+                if (got != (unsigned)nsplit - 1) return;
+                asm volatile("" ::: "memory");
+                if (lane == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                // in the order of the splits, whoever was the last: the same bits every time
+                float sm_[kOneSplits], sl_[kOneSplits];
+#pragma unroll
+                for (int s = 0; s < kOneSplits; s++) {
+                    if (s >= nsplit) continue;
+                    sm_[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mlb, ((s * kWaves + wave) * 48 + n) * 4, 0, kThrough));
+                    sl_[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mlb, ((s * kWaves + wave) * 48 + 16 + n) * 4, 0, kThrough));
+                }
+                if constexpr (STEP) ts = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(mlb, ((sp.token_split * kWaves + wave) * 48 + 32 + n) * 4, 0, kThrough));
+                f32x4 acc[TPW];
+#pragma unroll
+                for (int t = 0; t < TPW; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                float M = neg_inf(), den = 0.f;
+                auto batch = [&](auto ns_tag, int s0) __attribute__((always_inline)) {   // splits s0 .. s0 + NS - 1, in flight at a time
+                    constexpr int NS = decltype(ns_tag)::value;
+                    u32x4 x[NS][TPW];
+#pragma unroll
+                    for (int i = 0; i < NS; i++) {
+                        if (s0 + i >= nsplit || s0 + i == split) continue;
+                        if (rows.valid(n)) {
+#pragma unroll
+                            for (int t = 0; t < TPW; t++)
+                                x[i][t] = __builtin_amdgcn_raw_buffer_load_b128(ob, (((s0 + i) * 16 + n) * D + channel(t)) * 4, 0, kThrough);
+                        }
+                    }
+                    if (s0 == 0) {
+#pragma unroll
+                        for (int s = 0; s < kOneSplits; s++)
+                            if (s < nsplit) M = fmaxf(M, sm_[s]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < NS; i++) {
+                        const int s = s0 + i;
+                        if (s >= nsplit) continue;
+                        // a split without positions of the row has the maximum -inf and weighs nothing, whatever its rows hold
+                        const bool seen = sm_[s] != neg_inf();
+                        const float w = seen ? fast_exp2(sm_[s] - M) : 0.f;
+                        den = seen ? fmaf(w, sl_[s], den) : den;
+#pragma unroll
+                        for (int t = 0; t < TPW; t++) {
+                            const f32x4 y = s == split ? o[t] : __builtin_bit_cast(f32x4, x[i][t]);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[t][e] = seen ? fmaf(w, y[e], acc[t][e]) : acc[t][e];
+                        }
+                    }
+                };
+                if (nsplit <= 4) batch(std::integral_constant<int, 4>{}, 0);
+                else {
+                    batch(std::integral_constant<int, 8>{}, 0);
+                    if (nsplit > 8) batch(std::integral_constant<int, 8>{}, 8);
+                }
+#pragma unroll
+                for (int t = 0; t < TPW; t++) o[t] = acc[t];
+                m = M;
+                l = den;
             }
+            const float M = fmaxf(m, ts);
             const float w = m == neg_inf() ? 0.f : fast_exp2(m - M), wt = ts == neg_inf() ? 0.f : fast_exp2(ts - M);
             const float den = w * l + wt;
 #pragma unroll
@@ -345,6 +424,15 @@ __global__ __launch_bounds__(kWaves * 64) void sdpa_partial_kernel(
     if (c0 >= c1) {  // a split that lies wholly beyond what this group's rows may see
         // Its rows of part_o stay unwritten: the merge gives a split whose maximum is -inf the
         // weight 0 by selection, so whatever bytes the workspace holds there never enter a sum.
+        if constexpr (ONE) {
+            request_outer();
+            prepare_outer();
+            f32x4 none[TPW];
+#pragma unroll
+            for (int t = 0; t < TPW; t++) none[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            finish_one(none, neg_inf(), 0.f);
+            return;
+        }
         if (wave == 0 && g == 0) {
             const __amdgpu_buffer_rsrc_t mlb = buffer_of(part_ml + pid * 32);
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, neg_inf()), mlb, n * 4, 0, kThrough);
@@ -785,30 +873,44 @@ static int fit_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int n
     return MFA_OK;
 }
 
-// Whether one launch serves a decode call (OneLaunch), and its plan: a cache of so few chunks of 64 positions that a workgroup
-// streams them in no more time than the second launch takes, for one sequence alone.  (A chunk takes it 0.12, 0.25 and 0.5 us
-// by width over a bf16 cache, over f32 0.3, 1.2 and 2.5; partials that another workgroup merges when a ticket says it is the last, in
-// one launch as well, cost a sequence 1.3 us and more over the two launches at 256 channels: the hop through memory is three trips.)
-// Calls one after the other, and one call and its wait, in us with one launch and with two:
-//   decode  16 heads over 2 of 256, bf16    64: 6.5, 9.1 and 19.2, 21.1   320: 7.5, 9.2 and 21.5, 22.6   515: 12.2, 9.3 and 24.4, 22.5
-//           32 over 4 of 128, bf16          64: 6.7, 9.3 and 18.2, 20.5   320: 6.7, 9.3 and 19.9, 21.2   768: 10.3, 9.4 and 22.8, 21.0
-//           32 over 4 of 128, f32           64: 6.7, 9.2 and 19.1, 21.2   192: 7.5, 9.4 and 21.7, 21.6   320: 10.4, 9.2 and 24.6, 21.6
-//   step    16 over 2 of 256, bf16         128: 10.5, 11.9 and 25.5, 26.8   256: 11.9, 11.3 and 26.8, 26.5
-// Three sequences side by side 6.6 and 9.3 (decode), 8.0 and 10.6 (step) at all these lengths: bound by the host's launches.
-static int one_launch_chunks(int kv_dtype, int D, bool step) {
-    static constexpr int kDecode[2][3] = {{12, 5, 5}, {4, 3, 1}}, kStep[2][3] = {{10, 3, 3}, {3, 2, 1}};
-    const int f32 = kv_dtype == MFA_KV_F32, w = D == 64 ? 0 : D == 128 ? 1 : 2;
-    return step ? kStep[f32][w] : kDecode[f32][w];
-}
-static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int64_t kv_len, int forced_splits, bool step) {
+// Whether one launch serves a decode call (OneLaunch), and its plan, by the cache's chunks of 64 positions: where one sequence is
+// no slower with it than with two launches.  (Sequences side by side are bound by the host's launches: 7 us a layer against 10,
+// a step 8.2 against 11.)
+//   one workgroup per row group    streams a chunk in 0.12, 0.25 and 0.5 us by width over a bf16 cache, in 0.3, 1.2 and 2.5 over
+//                                  f32, and saves the second launch and two trips through memory
+//   several                        the partials, the ticket and the last wave's loads are three trips through memory, one more
+//                                  than the second launch; at 256 channels that and the bytes cost more than it saves
+// One sequence's calls one after the other, and one call and its wait, in us, with one launch and with two:
+//   decode  16 heads over 2 of 256, bf16   64: 7.1, 9.0 and 18.5, 20.3   310: 8.9, 9.0 and 21.3, 21.6   several 515: 9.6, 10.2 and 22.9, 22.1
+//           32 over 4 of 128, bf16         64: 7.1, 8.9 and 17.4, 19.6   320: 7.2, 9.0 and 19.6, 20.8   several 576: 7.3, 9.1 and 21.1, 21.1
+//           16 over 2 of 64, bf16          64: 7.1, 8.9 and 17.1, 19.4   768: 7.4, 9.0 and 20.4, 20.7   several 1024: 7.0, 10.0 and 20.4, 20.8
+//   step    16 over 2 of 256, bf16        116: 9.7, 11.3 and 24.0, 25.7  180: 10.4, 12.0 and 24.6, 26.3  several 500: 12.7, 11.8 and 27.1, 26.0
+//           32 over 4 of 128, bf16        116: 8.1, 10.2 and 21.6, 24.2  180: 8.3, 10.3 and 22.2, 24.7  several 820: 10.3, 11.7 and 24.5, 24.6
+// One or two query heads per kv head are 1.4 us slower in this form than three and more (all widths and row counts tried), with
+// two launches not: they get half the chunks, and one workgroup per row group.
+static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int D, int64_t kv_len, int forced_splits, bool step,
+                            const SdpaWorkspace &ws) {
+    static constexpr int kOne[2][2][3] = {{{12, 5, 5}, {4, 3, 1}}, {{10, 3, 3}, {3, 2, 1}}};      // [step][f32][width]
+    static constexpr int kSeveral[2][2][3] = {{{16, 9, 0}, {9, 0, 0}}, {{16, 13, 0}, {16, 5, 0}}};
+    const int f32 = kv_dtype == MFA_KV_F32, w = D == 64 ? 0 : D == 128 ? 1 : 2, hpk = Hq / Hkv;
     const int64_t nchunk = (kv_len + kKvChunk - 1) / kKvChunk;
-    if (forced_splits > 0 || nchunk > one_launch_chunks(kv_dtype, D, step)) return false;
     const int U = unit_chunks(kv_dtype, D);
-    plan.nhg = (Hq / Hkv + 15) / 16;
-    plan.splits = 1;
-    plan.base = (int)((nchunk + U - 1) / U);
-    plan.rem = 0;
-    return true;
+    const int64_t nunits = (nchunk + U - 1) / U;
+    if (forced_splits > 0) return false;
+    int64_t splits = 1;
+    const int one = kOne[step][f32][w];
+    if (nchunk > (hpk > 2 || one == 1 ? one : one / 2)) {
+        if (hpk <= 2 || nchunk > kSeveral[step][f32][w] || !ws.tickets) return false;
+        const int64_t per = (min_pass_chunks(kv_dtype, D) + U - 1) / U;   // a share is one pass
+        splits = (nunits + per - 1) / per;
+        if (splits > kOneSplits) splits = kOneSplits;
+    }
+    plan.nhg = (hpk + 15) / 16;
+    plan.splits = (int)splits;
+    plan.base = (int)(nunits / splits);
+    plan.rem = (int)(nunits % splits);
+    return splits == 1 || (sdpa_workspace_o_elems(Hq, Hkv, D, plan.splits) <= ws.part_o_elems &&
+                           (size_t)Hkv * plan.nhg * plan.splits * kWaves * 48 <= ws.part_ml_elems);
 }
 
 // One decode token of a full-attention layer from its raw projections in two launches: the
@@ -828,9 +930,9 @@ int launch_sdpa_step(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, i
     // (one launch: a row group's result may be out before another's inputs are in, so they lie apart)
     const size_t qd = (size_t)Hq * D, kd = (size_t)Hkv * D;
     const bool one = !overlap(out, qd, q_proj, 2 * qd) && !overlap(out, qd, k_in, kd) && !overlap(out, qd, v_in, kd) &&
-                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, true);
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, len0 > 0 ? len0 : 1, forced_splits, true, ws);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, 1, len0 > 0 ? len0 : 1, num_cus, forced_splits, ws));
-    const OneLaunch ol{q_proj + D, out, 2 * D};
+    const OneLaunch ol{q_proj + D, out, 2 * D, ws.tickets};
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     const StepPrologue sp{q_proj, k_in, v_in, q_norm, k_norm, inv_freq, rotary_dim, eps, pos, len0, new_score,
                           k_tiled, v_tiled, plan.splits - 1};
@@ -863,9 +965,9 @@ int launch_sdpa(hipStream_t stream, int kv_dtype, int Hq, int Hkv, int D, int n_
     const size_t qd = (size_t)Hq * D;
     const bool apart = (out == q || !overlap(out, qd, q, qd)) && (out == gate || !overlap(out, qd, gate, qd));
     const bool one = one_layer && n_tok == 1 && gate && apart && !partial_only && !defer_merge &&
-                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, false);
+                     one_launch_plan(plan, kv_dtype, Hq, Hkv, D, kv_len, forced_splits, false, ws);
     if (!one) MFA_TRY(fit_plan(plan, kv_dtype, Hq, Hkv, D, n_tok, kv_len, num_cus, forced_splits, ws));
-    const OneLaunch ol{gate, out, D};
+    const OneLaunch ol{gate, out, D, ws.tickets};
     // scores are produced in log2 units: q is pre-multiplied by (1/sqrt(D)) * log2(e)
     const float qscale = (1.0f / sqrtf((float)D)) * kLog2e;
     launch_partial_any<false>(kv_dtype, D, stream, dim3(plan.splits, plan.nhg, Hkv), k_tiled, v_tiled, plane_elems, q,

@@ -54,7 +54,7 @@ extern "C" int mfa_sdpa_decode_static_dev(mfa_ctx *ctx, int32_t layer, const flo
                     "mfa_sdpa_decode_static_dev: %d splits of %d kv heads need %zu bytes of partials, the static "
                     "scratch holds %zu (use mfa_sdpa_decode_dev, or fewer splits: mfa_set_num_splits)",
                     splits, g.num_kv_heads, (need_o + need_ml) * sizeof(float), static_scratch_bytes());
-    const SdpaWorkspace ws{base, base + kStaticOElems, kStaticOElems, kStaticMlElems};
+    const SdpaWorkspace ws{base, base + kStaticOElems, kStaticOElems, kStaticMlElems, c->tickets};
     return launch_sdpa(c->stream, g.kv_dtype, g.num_attn_heads, g.num_kv_heads, g.head_dim, 1, f->len, c->plane_elems,
                        f->k, f->v, q_dev, q_gate_dev, out_dev, ws, c->num_cus, c->forced_splits, 0);
 }

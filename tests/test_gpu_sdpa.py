@@ -221,13 +221,15 @@ def test_shares_of_a_single_unit(mfa, oracle, Hq, Hkv, d, bf16):
     (16, 2, 256, True, (1, 127, 129, 515, 768, 769)), (32, 2, 256, True, (64, 640)), (40, 2, 128, True, (1023, 1024, 1025)),
     (32, 4, 128, False, (1, 63, 65, 767, 768, 769)), (4, 2, 64, True, (130, 1024)), (3, 1, 64, False, (500, 1024)),
     (18, 1, 256, False, (384, 385)),
-    (16, 2, 256, True, (319, 320, 321)), (32, 4, 128, True, (257, 320, 321)), (4, 2, 64, True, (767, 768, 769)),
-    (40, 2, 256, False, (1, 63, 64, 65)), (32, 4, 128, False, (191, 192, 193)), (3, 1, 64, False, (1, 255, 256, 257)),
+    (16, 2, 256, True, (319, 320, 321)), (32, 4, 128, True, (257, 320, 321, 383, 575, 576, 577)), (40, 2, 128, True, (321, 513, 576)),
+    (6, 2, 64, True, (767, 768, 769, 833, 1024, 1025)), (4, 2, 64, True, (383, 384, 385)), (3, 3, 128, True, (127, 128, 129)),
+    (40, 2, 256, False, (1, 63, 64, 65)), (32, 4, 128, False, (191, 192, 193)), (3, 1, 64, False, (1, 255, 256, 257, 321, 576, 577)),
 ])
 def test_short_caches_merge_in_the_attention_launch(mfa, oracle, Hq, Hkv, d, bf16, lens):
-    """Either side of the limits of the launch that is the whole of a decode call (whole chunks of 64 positions; more than 16
-    heads per kv head are two row groups): against the oracle, three calls in a row the same to the bit, over a workspace of
-    NaN, and the merge launch (a forced split count) within rounding."""
+    """Either side of the limits of the launch that is the whole of a decode call (whole chunks of 64 positions, one workgroup per
+    row group and several; more than 16 heads per kv head are two row groups): against the oracle, three calls in a row the
+    same to the bit (the counters are back at 0), over a workspace of NaN, and the merge launch (a forced split count) within
+    rounding."""
     from moeflux_amd import Config
     top = max(lens)
     q, g, k, v = sdpa_random_inputs(top + d, Hq, Hkv, d, top, bf16=bf16)
@@ -305,8 +307,9 @@ def test_chunk_result_shifted_over_the_query(mfa, oracle):
 
 
 @pytest.mark.parametrize("Hq,Hkv,d,bf16,lens", [
-    (16, 2, 256, True, (0, 1, 64, 65, 191, 192, 193)), (40, 2, 128, True, (0, 63, 192, 193)), (6, 2, 64, True, (0, 127, 640, 641)),
-    (32, 2, 256, False, (0, 1, 64, 65)), (3, 1, 128, False, (0, 127, 128, 129)), (16, 2, 64, False, (0, 192, 193)),
+    (16, 2, 256, True, (0, 1, 64, 65, 191, 192, 193)), (40, 2, 128, True, (0, 63, 192, 193, 300, 832, 833)),
+    (6, 2, 64, True, (0, 127, 640, 641, 1024, 1025)), (2, 1, 128, True, (0, 64, 65, 200)),
+    (32, 2, 256, False, (0, 1, 64, 65)), (3, 1, 128, False, (0, 127, 128, 129, 257, 320, 321)), (16, 2, 64, False, (0, 192, 193, 600, 1024, 1025)),
 ])
 def test_short_steps_in_one_launch(mfa, oracle, Hq, Hkv, d, bf16, lens):
     """A step either side of the limits of its one launch: against the oracle's prologue and attention over the cache as
