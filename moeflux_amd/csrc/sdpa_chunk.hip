@@ -16,8 +16,8 @@
 // Rows that leave CUs idle split the cache (sdpa_chunk_plan).
 //
 // What bounds it: behind a long cache the matrix cores at the rate they sustain.  512 tokens of 32 heads
-// of 128 behind 32768 positions: 580 us with 16-row groups, 429 with this kernel, 384 with its soft-max
-// left out (both parts of query and probabilities are products, so 2.75e11 operations are 5.5e11 executed: 1.4 PFLOP/s).
+// of 128 behind 32768 positions, three sequences side by side: 580 us with 16-row groups, 429 with this kernel, 384 with its
+// soft-max left out (one call after the other, at a lower clock: 664 and 502) (both parts of query and probabilities are products, so 2.75e11 operations are 5.5e11 executed: 1.4 PFLOP/s).
 // Over short caches launch, query, first block and epilogue: 512 tokens from an empty cache 17 us,
 // of which the longest workgroup's eight blocks are 7.
 #include <cmath>
