@@ -229,6 +229,11 @@ struct SdpaWorkspace {
     unsigned *tickets = nullptr;
 };
 static constexpr int kOneTickets = 4;   // one per wave of a workgroup
+// Sizes of the file-scope scratch of mfa_sdpa_decode_static_dev: partial outputs [kv head][row group][split][16][D], then the
+// (max, sum) pairs.  A decode launch that merges its own partials keeps to them on any scratch, so that the route, and with
+// it the bits of the result, does not depend on which.
+static constexpr size_t kStaticOElems = (size_t)2 << 20;    // 8 MiB
+static constexpr size_t kStaticMlElems = (size_t)64 << 10;  // 256 KiB
 bool sdpa_shape_supported(int kv_dtype, int head_dim);
 // Number of splits the launcher will use (for workspace sizing pass kv_len = capacity).
 int sdpa_max_splits(int kv_dtype, int Hq, int Hkv, int D, int64_t max_len, int num_cus, int forced);

@@ -909,8 +909,8 @@ static bool one_launch_plan(SplitPlan &plan, int kv_dtype, int Hq, int Hkv, int 
     plan.splits = (int)splits;
     plan.base = (int)(nunits / splits);
     plan.rem = (int)(nunits % splits);
-    return splits == 1 || (sdpa_workspace_o_elems(Hq, Hkv, D, plan.splits) <= ws.part_o_elems &&
-                           (size_t)Hkv * plan.nhg * plan.splits * kWaves * 48 <= ws.part_ml_elems);
+    const size_t o = sdpa_workspace_o_elems(Hq, Hkv, D, plan.splits), stats = (size_t)Hkv * plan.nhg * plan.splits * kWaves * 48;
+    return splits == 1 || (o <= kStaticOElems && stats <= kStaticMlElems && o <= ws.part_o_elems && stats <= ws.part_ml_elems);
 }
 
 // One decode token of a full-attention layer from its raw projections in two launches: the

@@ -9,9 +9,6 @@
 
 namespace mfa {
 
-// partial outputs [kv head][row group][split][16][D] f32, then the (max, sum) pairs
-static constexpr size_t kStaticOElems = (size_t)2 << 20;    // 8 MiB
-static constexpr size_t kStaticMlElems = (size_t)64 << 10;  // 256 KiB
 static __device__ __align__(256) float scratch[kStaticOElems + kStaticMlElems];
 
 static constexpr int kMaxDevices = 64;

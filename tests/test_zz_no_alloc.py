@@ -48,6 +48,24 @@ def test_static_scratch_decode_equals_the_workspace_decode(mfa, oracle, bf16):
         assert np.array_equal(ws, st)
 
 
+@pytest.mark.parametrize("Hq,Hkv,d,n", [(32, 4, 128, 500), (16, 2, 64, 1000), (216, 72, 128, 576), (270, 90, 64, 1000)])
+def test_static_scratch_decode_takes_the_route_of_the_workspace(mfa, Hq, Hkv, d, n):
+    """Short caches whose partials one launch merges: the same bits on either scratch, also where the row groups are so
+    many that their statistics would not fit the static array."""
+    from moeflux_amd import Config
+    from moeflux_amd.hip import DeviceArray
+    rng = np.random.default_rng(n)
+    k, v = (rng.standard_normal((n, Hkv * d), dtype=np.float32) for _ in range(2))
+    with mfa.Ctx(Config(num_layers=1, full_attn_interval=1, num_attn_heads=Hq, num_kv_heads=Hkv, head_dim=d, kv_capacity=n, kv_dtype=1)) as c:
+        c.kv_import(0, k, v)
+        dq, dg = (DeviceArray.from_host(rng.standard_normal(Hq * d, dtype=np.float32)) for _ in range(2))
+        out = [DeviceArray((Hq * d,), zero=True) for _ in range(2)]
+        assert c.lib.mfa_sdpa_decode_dev(c.h, 0, dq.ptr, dg.ptr, out[0].ptr) == 0
+        assert c.lib.mfa_sdpa_decode_static_dev(c.h, 0, dq.ptr, dg.ptr, out[1].ptr) == 0
+        c.sync()
+        assert np.array_equal(out[0].to_host(), out[1].to_host())
+
+
 def test_static_scratch_decode_leaves_the_free_device_memory_as_it_was(mfa):
     """What the entry point is for: no allocation.  Free device memory (hipMemGetInfo) is read before
     and after calls over cache lengths that change the split plan from 1 workgroup per row group to
