@@ -15,10 +15,11 @@
 // Everything before D depends on the inputs only and is computed for all blocks of the
 // chunk at once (gdn_wy_kernel, one workgroup per (block, value head)); the four
 // products that involve the state run block after block with the state in registers
-// (gdn_wy_recur_kernel, one workgroup per 16 rows of a head's state, rows being
-// independent).  All products are v_mfma_f32_16x16x4_f32.
+// (gdn_wy_recur_kernel, one workgroup per 32 rows of a head's state, rows being
+// independent).  The products before D are v_mfma_f32_16x16x4_f32; those that involve the state are
+// v_mfma_f32_16x16x32_f16 over operands split into two f16 numbers (see wy_split4).
 //
-// Operand conventions of that instruction (lane l, m = n = l % 16, g = l / 16):
+// Operand conventions of the f32 instruction (lane l, m = n = l % 16, g = l / 16):
 // A[m][g], B[g][n] in; D[4g+i][n], i = 0..3, out.  A contraction over 16 values is done as
 // 4 instructions i = 0..3 in which lane group g contributes value number 4g+i: then one
 // float4 (values 4g..4g+3) feeds the four instructions, and a D tile can be used as the
@@ -26,6 +27,7 @@
 #include <type_traits>
 
 #include "gdn_device.h"
+#include "sdpa_wave.h"
 
 namespace mfa {
 
@@ -58,9 +60,44 @@ __device__ inline float4 as_f4(wy_f32x4 v) { return float4{v[0], v[1], v[2], v[3
 // a 16-byte load kept as a vector register value (members of a struct of operands)
 __device__ inline wy_f32x4 load_v4(const float *p) { return *reinterpret_cast<const wy_f32x4 *>(p); }
 
+// f32 x scaled by a power of two as the sum of two f16 numbers, hi = f16(x), lo = f16(x - hi): 22 bits, what is left out is below
+// 2^-24 of x (2^-39 of the scale for x below 2^-16 of it, where lo is subnormal), the size of x's own rounding.
+// Of a product hi hi + hi lo + lo hi is formed (lo lo too where it costs nothing) and summed in f32, as the f32 instruction does,
+// in 16 clocks for 32 contracted values and term instead of 256.  W, q^, the decayed k^ and M are at most 1 by construction
+// (unit keys, beta <= 1, decays <= 1, and every row of W is beta e^L k^ under a chain of contractions), so they carry a fixed
+// scale; the state's and D's scales are those of the largest value of a tile's row, taken as the tile is formed.
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+static constexpr float kWyScale = 16384.f;   // 2^14: the largest f16 is 65504
+__device__ inline uint32_t wy_pack(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2)); }
+__device__ inline void wy_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = wy_pack(a - (float)h[0], b - (float)h[1]);
+}
+// four values as 16 bytes: hi of all, lo of all
+__device__ inline u32x4 wy_split4(float a, float b, float c, float d) {
+    uint32_t h0, h1, l0, l1;
+    wy_split2(a, b, h0, l0);
+    wy_split2(c, d, h1, l1);
+    return u32x4{h0, h1, l0, l1};
+}
+__device__ inline u32x4 wy_split4_unit(float a, float b, float c, float d) {   // of values of at most 1
+    return wy_split4(a * kWyScale, b * kWyScale, c * kWyScale, d * kWyScale);
+}
+// The scale of values of at most mx (2^14 <= mx scale < 2^15, less for mx below 2^-87) and what undoes it together with kWyScale.
+__device__ inline void wy_scale(float mx, float &scale, float &undo) {
+    const int e = max((int)(__builtin_bit_cast(uint32_t, mx) >> 23), 40);   // mx >= 0
+    scale = __builtin_bit_cast(float, (uint32_t)(268 - e) << 23);
+    undo = __builtin_bit_cast(float, (uint32_t)(e - 28) << 23);
+}
+__device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+}
+
 // Per (block, value head) outputs, block-major then head, each cut into 16x16 tiles that
-// are stored the way the recurrence kernel's lanes read them, 16 bytes per lane and
-// 1 KiB per tile (a row-major matrix read as an A operand has neighbouring lanes 512
+// are stored the way the recurrence kernel's lanes read them, 16 bytes per lane (four f32 values of Ut, the two f16 parts of
+// four values of the others) and 1 KiB per tile (a row-major matrix read as an A operand has neighbouring lanes 512
 // bytes apart, which the memory pipeline serves at a fraction of its rate):
 //   Wt [token tile w][col tile c], Qt likewise, Mt [w][token tile tau], Kt [col tile c][tau]
 //   (= diag(e^{L_C-L}) K transposed): lane (m, g) holds X[16 row-tile + m][16 col-tile + 4g + i];
@@ -79,8 +116,8 @@ template <int DK, bool FUSED>
 __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     int Hk, int Hv, int T, const float *__restrict__ qn, const float *__restrict__ kn,
     const float *__restrict__ vv, const float *__restrict__ lg, const float *__restrict__ bg,
-    float *__restrict__ Wt, float *__restrict__ Qt, float *__restrict__ Ut, float *__restrict__ Mt,
-    float *__restrict__ Kt, float *__restrict__ eLc, WyInputs in) {
+    u32x4 *__restrict__ Wt, u32x4 *__restrict__ Qt, float *__restrict__ Ut, u32x4 *__restrict__ Mt,
+    u32x4 *__restrict__ Kt, float *__restrict__ eLc, WyInputs in) {
     constexpr int DV = DK;
     constexpr int NK = DK / 16;
     constexpr int LDK = DK + 4;  // row strides chosen so that 16-byte row reads by 8 lanes hit all banks
@@ -338,12 +375,13 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 const float d = sR[row] > col ? 0.f : __builtin_amdgcn_exp2f((dl < 0.f ? dl : 0.f) * 1.4426950408889634f);
                 mv[i] = (col <= row) ? d * acc[i] : 0.f;
             }
-            *reinterpret_cast<wy_f32x4 *>(Mt + ((slot * 4 + I) * 4 + J) * 256 + lane * 4) = mv;
+            Mt[((slot * 4 + I) * 4 + J) * 64 + lane] = wy_split4_unit(mv[0], mv[1], mv[2], mv[3]);
         }
     }
     for (int i = tid; i < 4 * NK * 64; i += NTHR) {  // q^ tiles, before v takes its place
         const int tile = i >> 6, l = i & 63, w = tile / NK, c = tile % NK;
-        *(float4 *)(Qt + (slot * 4 * NK + tile) * 256 + l * 4) = lds_f4(&sQ[16 * w + (l & 15)][16 * c + 4 * (l >> 4)]);
+        const float4 q = lds_f4(&sQ[16 * w + (l & 15)][16 * c + 4 * (l >> 4)]);
+        Qt[(slot * 4 * NK + tile) * 64 + l] = wy_split4_unit(q.x, q.y, q.z, q.w);
     }
     __syncthreads();
 
@@ -357,8 +395,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             const int i = tid + u * NTHR, tile = i >> 6, l = i & 63, c = tile >> 2, tau = tile & 3;
             const int kk = 16 * c + (l & 15), j4 = 16 * tau + 4 * (l >> 4);
             const float4 e = lds_f4(&sKd[j4]);
-            const float4 o = {e.x * sK[j4 + 0][kk], e.y * sK[j4 + 1][kk], e.z * sK[j4 + 2][kk], e.w * sK[j4 + 3][kk]};
-            *(float4 *)(Kt + (slot * NK * 4 + tile) * 256 + l * 4) = o;
+            Kt[(slot * NK * 4 + tile) * 64 + l] = wy_split4_unit(e.x * sK[j4 + 0][kk], e.y * sK[j4 + 1][kk], e.z * sK[j4 + 2][kk], e.w * sK[j4 + 3][kk]);
         }
         if constexpr (!FUSED) {
 #pragma unroll
@@ -449,146 +486,202 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             const size_t tile = (slot * 4 + tau) * NK + NCT * wave + ct;
             // U as computed (a D tile), W in A-operand order
             *reinterpret_cast<wy_f32x4 *>(Ut + tile * 256 + lane * 4) = au;
-            *reinterpret_cast<wy_f32x4 *>(Wt + tile * 256 + lane * 4) = aw;
+            Wt[tile * 64 + lane] = wy_split4_unit(aw[0], aw[1], aw[2], aw[3]);
         }
     }
 }
 
-// grid (Hv, DV/16), 256 threads.  The 16 rows of the state are kept by every wave, in the
-// layout of a D tile per 16 columns (lane (n, g): S[row0+n][16c+4g+i]), which is also the B
-// operand of a contraction over the columns.  Wave w serves tokens 16w .. 16w+15 of each
-// block and the column tiles (DK/64)*w .. of the state update.
-// 256 registers a wave (it took 260): a CU then holds two workgroups, of 64 heads' 512 or of two sequences' launches, and
-// one computes while the other waits at a block's barriers (512 tokens, six layers of 32 heads 275 -> 261 us a pass with
-// three sequences side by side).
+// grid (Hv, DV/32), 512 threads: 32 rows of one head's state, as two groups of 16.  Waves w and w + 4 serve tokens 16w .. 16w+15
+// of each block, the first with W (and then D), the second with q^ (and then O); in the update of the state wave 4 rg + s owns
+// columns 32s .. 32s+31 of row group rg, in f32, and hands them to all waves as f16 parts with the scale of each row's largest
+// value there.  (Lane (n, g) of a tile that the update leaves holds row n, columns 16c+4g+i: with c = 2s, 2s+1 its own eight
+// values are the B operand of a 32-wide contraction over them, k-slot e < 4 being column 32s+4g+e, e >= 4 column 32s+16+4g+e-4;
+// a tile of D likewise tokens 16w+4g+i of row n.  The A side has hi and lo of the same four values in its k-slots 0-3 and 4-7, so
+// against a D operand that repeats its values one instruction adds two of the products.)
+// Bound by the two exchanges a block and by the CU's 64 bytes a clock of operands.  512 tokens of 32 heads take 25 us on half the
+// CUs (f32 instructions, 16 rows a workgroup: 25 us on all of them): six layers 241 -> 205 us a pass with three sequences side by
+// side, 2000 tokens of one layer 162 -> 128, of 64 heads 337 -> 261.
 template <int DK>
-__global__ __launch_bounds__(256, 2) void gdn_wy_recur_kernel(
-    int Hk, int Hv, int T, const float *__restrict__ Wt, const float *__restrict__ Qt,
-    const float *__restrict__ Ut, const float *__restrict__ Mt, const float *__restrict__ Kt,
+__global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
+    int Hk, int Hv, int T, const u32x4 *__restrict__ Wt, const u32x4 *__restrict__ Qt,
+    const float *__restrict__ Ut, const u32x4 *__restrict__ Mt, const u32x4 *__restrict__ Kt,
     const float *__restrict__ eLc, float *__restrict__ ssm, float *__restrict__ o_raw) {
     constexpr int DV = DK;
     constexpr int NK = DK / 16;   // column tiles of the state
-    constexpr int NKW = NK / 4;   // of which a wave updates
-    __shared__ wy_f32x4 s_d[4][64];    // D tiles of the block, by token tile
-    __shared__ wy_f32x4 s_st[NK][64];  // the updated state
+    constexpr int NS = DK / 32;   // 32-column steps of a contraction over them
+    __shared__ u32x4 s_s[2][NS][2][64];    // state [row group][step][hi|lo]
+    __shared__ u32x4 s_d[2][2][4][2][64];  // D [block % 2][row group][token tile][hi twice|lo twice]
+    __shared__ float s_su[2][NS][16], s_du[2][2][4][16];   // what undoes their scales, per row
 
-    const int vh = wy_head_of(blockIdx.x, Hk, Hv), row0 = blockIdx.y * 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int vh = wy_head_of(blockIdx.x, Hk, Hv), row0 = blockIdx.y * 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, g = lane >> 4;
-    float *srow = ssm + ((size_t)vh * DV + row0 + m) * DK + 4 * g;
-    wy_f32x4 st[NK];
-#pragma unroll
-    for (int c = 0; c < NK; c++) {
-        const float4 v = load_f4(srow + 16 * c);
-        st[c] = wy_f32x4{v.x, v.y, v.z, v.w};
-    }
-
-    // A block's operands live in registers and are requested one block ahead, all of them
-    // before the block's first barrier: the W and q^ rows of this wave's tokens and its U
-    // entries into the registers the block has just consumed, its M rows, e^L and the K
-    // columns of its share of the update into a second set (two blocks per loop pass,
-    // the sets swapping roles).  Requests past the last block re-read it.
+    const int w = wave & 3, rgu = wave >> 2;   // token tile; of the update: row group, and step w
+    const bool owner = w < NS;
     const int nblk = (T + kC - 1) / kC;
-    struct Late {
-        wy_f32x4 mt[4], kd[NKW][4], el;
+    auto slot_of = [&](int blk) { return (size_t)(blk < nblk ? blk : nblk - 1) * Hv + vh; };   // past the end: the last block again
+
+    float *srow = ssm + ((size_t)vh * DV + row0 + 16 * rgu + m) * DK + 32 * (owner ? w : 0) + 4 * g;
+    wy_f32x4 st[2] = {load_v4(srow), load_v4(srow + 16)};
+    auto publish_state = [&]() __attribute__((always_inline)) {
+        float mx = 0.f, sc, un;
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(st[ct][i]));
+        wy_scale(rows_max(mx), sc, un);
+        const u32x4 a = wy_split4(st[0][0] * sc, st[0][1] * sc, st[0][2] * sc, st[0][3] * sc);
+        const u32x4 b = wy_split4(st[1][0] * sc, st[1][1] * sc, st[1][2] * sc, st[1][3] * sc);
+        s_s[rgu][w][0][lane] = u32x4{a[0], a[1], b[0], b[1]};
+        s_s[rgu][w][1][lane] = u32x4{a[2], a[3], b[2], b[3]};
+        if (g == 0) s_su[rgu][w][m] = un;
+    };
+
+    // ROLE 0: W, D; ROLE 1: q^, O.  D and the state are the chain that the next block waits for; O of a block is formed a block
+    // later, beside the chain (its waves give way to the others: s_setprio).  An operand's register takes the next block's
+    // request as soon as it has been used.  Requests go through a descriptor of the block's operand, so that they cost a
+    // scalar addition each and no vector one.
+    const int lane16 = lane * 16;
+    auto run = [&](auto role_tag) __attribute__((always_inline)) {
+        constexpr int ROLE = decltype(role_tag)::value;
+        u32x4 pw[NK], mt[4], kd[2][4];
+        wy_f32x4 pu[2], el, o[2];
         float elc;
-    };
-    float4 pw[NK], pq[NK], pu;
-    auto slot_of = [&](int blk) { return (size_t)(blk < nblk ? blk : nblk - 1) * Hv + vh; };
-    // The requests for the next block are issued between the matrix instructions of the
-    // first product (an instruction occupies the matrix core for 32 clocks, the wave's issue
-    // slot for a few), column tile by column tile as its W and q^ registers come free;
-    // the second set's 6 + 4*NKW requests are spread over the same loop.
-    auto fetch_wq = [&](int blk, int c) __attribute__((always_inline)) {
-        const size_t off = (slot_of(blk) * 4 + wave) * NK * 256 + lane * 4;
-        pw[c] = load_f4(Wt + off + c * 256);
-        pq[c] = load_f4(Qt + off + c * 256);
-    };
-    auto fetch_u = [&](int blk) __attribute__((always_inline)) {
-        pu = load_f4(Ut + ((slot_of(blk) * 4 + wave) * NK + blockIdx.y) * 256 + lane * 4);
-    };
-    constexpr int NLATE = 6 + 4 * NKW;                 // requests of a Late set
-    constexpr int LATE_PER_C = (NLATE + NK - 1) / NK;  // of which per column tile
-    auto fetch_late = [&](Late &p, int blk, int j) __attribute__((always_inline)) {
-        const size_t slot = slot_of(blk);
-        if (j < 4) p.mt[j] = load_v4(Mt + ((slot * 4 + wave) * 4 + (j <= wave ? j : wave)) * 256 + lane * 4);
-        else if (j == 4) p.el = load_v4(eLc + slot * kC + 16 * wave + 4 * g);
-        else if (j == 5) p.elc = eLc[slot * kC + kC - 1];
-        else if (j < NLATE) {
-            const int kt = (j - 6) / 4, tau = (j - 6) % 4;
-            p.kd[kt][tau] = load_v4(Kt + ((slot * NK + NKW * wave + kt) * 4 + tau) * 256 + lane * 4);
-        }
-    };
-    auto block = [&](int blk, const Late &cur, Late &nxt) __attribute__((always_inline)) {
-        const int t0 = blk * kC;
-        // ---- W S0^T and Q S0^T for this wave's 16 tokens ------------------------------
-        wy_f32x4 p1 = {0.f, 0.f, 0.f, 0.f}, p2 = p1;
-#pragma unroll
-        for (int c = 0; c < NK; c++) {
-            p1 = mfma4(pw[c], as_f4(st[c]), p1);
-            p2 = mfma4(pq[c], as_f4(st[c]), p2);
-            fetch_wq(blk + 1, c);
-#pragma unroll
-            for (int u = 0; u < LATE_PER_C; u++) fetch_late(nxt, blk + 1, c * LATE_PER_C + u);
-            // keep this column tile's requests between its matrix instructions (left to itself the
-            // scheduler gathers all requests at the end of the product, where nothing hides their issue)
-            __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 2 + LATE_PER_C, 0);
-        }
-        // ---- D = U - W S0^T: lane (n, g) holds tokens 16w+4g+i of state row row0+n ----
-        wy_f32x4 d;
-        d[0] = pu.x - p1[0]; d[1] = pu.y - p1[1]; d[2] = pu.z - p1[2]; d[3] = pu.w - p1[3];
-        fetch_u(blk + 1);
-        s_d[wave][lane] = d;
-        __syncthreads();
-        // ---- O = diag(e^L) Q S0^T + M D ------------------------------------------------
-        wy_f32x4 o = cur.el * p2;
-#pragma unroll
-        for (int tau = 0; tau < 4; tau++)
-            if (tau <= wave) o = mfma4(as_f4(cur.mt[tau]), as_f4(s_d[tau][lane]), o);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int t = t0 + 16 * wave + 4 * g + i;
-            if (t < T) o_raw[((size_t)t * Hv + vh) * DV + row0 + m] = o[i];
-        }
-        // ---- S' = e^{L_C} S0 + D^T diag(e^{L_C-L}) K, column tiles NKW*w .. ------------
-        // (written out per wave so that the state tile is a compile-time register choice)
-        auto update = [&](auto wtag) __attribute__((always_inline)) {
-            constexpr int w = decltype(wtag)::value;
-#pragma unroll
-            for (int kt = 0; kt < NKW; kt++) {
-                constexpr int c0 = NKW * w;
-                wy_f32x4 acc = st[c0 + kt] * cur.elc;
-#pragma unroll
-                for (int tau = 0; tau < 4; tau++)
-                    acc = mfma4(as_f4(cur.kd[kt][tau]), as_f4(s_d[tau][lane]), acc);
-                s_st[c0 + kt][lane] = acc;
-            }
+        auto load = [&](__amdgpu_buffer_rsrc_t r, int tile) __attribute__((always_inline)) {
+            return __builtin_amdgcn_raw_buffer_load_b128(r, lane16, tile * 1024, 0);
         };
-        if (wave == 0) update(std::integral_constant<int, 0>{});
-        else if (wave == 1) update(std::integral_constant<int, 1>{});
-        else if (wave == 2) update(std::integral_constant<int, 2>{});
-        else update(std::integral_constant<int, 3>{});
-        __syncthreads();
+        auto w_of = [&](int blk) { return buffer_of((ROLE == 0 ? Wt : Qt) + (slot_of(blk) * 4 + w) * NK * 64); };
+        auto fetch_u = [&](int blk) __attribute__((always_inline)) {
+            const auto r = buffer_of(Ut + ((slot_of(blk) * 4 + w) * NK + 2 * blockIdx.y) * 256);
 #pragma unroll
-        for (int c = 0; c < NK; c++) st[c] = s_st[c][lane];
-    };
-    Late la, lb;
+            for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(r, rg));
+        };
+        auto fetch_el = [&](int blk) __attribute__((always_inline)) {
+            el = __builtin_bit_cast(wy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(eLc + slot_of(blk) * kC + 16 * w), g * 16, 0, 0));
+        };
+        auto fetch_m = [&](int blk) __attribute__((always_inline)) {
+            const auto r = buffer_of(Mt + (slot_of(blk) * 4 + w) * 4 * 64);
 #pragma unroll
-    for (int c = 0; c < NK; c++) fetch_wq(0, c);
-    fetch_u(0);
+            for (int tau = 0; tau < 4; tau++) mt[tau] = load(r, tau <= w ? tau : w);
+        };
+        auto fetch_k = [&](int blk) __attribute__((always_inline)) {
+            const size_t slot = slot_of(blk);
+            const auto r = buffer_of(Kt + (slot * NK + 2 * (owner ? w : 0)) * 4 * 64);
+            elc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(eLc + slot * kC + kC - 1), 0, 0, 0));
 #pragma unroll
-    for (int j = 0; j < NLATE; j++) fetch_late(la, 0, j);
-    for (int blk = 0; blk < nblk; blk += 2) {
-        block(blk, la, lb);
-        if (blk + 1 < nblk) block(blk + 1, lb, la);  // uniform over the workgroup
-    }
-    if (wave == 0) {
+            for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-        for (int c = 0; c < NK; c++) {
-            gdn_f32x4 v = {st[c][0], st[c][1], st[c][2], st[c][3]};
-            *reinterpret_cast<gdn_f32x4 *>(srow + 16 * c) = v;
+                for (int tau = 0; tau < 4; tau++) kd[ct][tau] = load(r, 4 * ct + tau);
+        };
+        // O of block blk = (what diag(e^L) q^ S0^T left in o) + M D
+        auto finish_o = [&](int blk) __attribute__((always_inline)) {
+            const u32x4(*sd)[4][2][64] = s_d[blk & 1];
+            const float(*du)[4][16] = s_du[blk & 1];
+#pragma unroll
+            for (int tau = 0; tau < 4; tau++)
+                if (tau <= w) {
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) {
+                        wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                        acc = wy_mfma(mt[tau], sd[rg][tau][1][lane], acc);
+                        acc = wy_mfma(mt[tau], sd[rg][tau][0][lane], acc);
+                        o[rg] += acc * du[rg][tau][m];
+                    }
+                }
+            const int rows = T - (blk * kC + 16 * w) - 4 * g;   // tokens from this lane's first on
+            float *dst = o_raw + ((size_t)(blk * kC + 16 * w) * Hv + vh) * DV + row0;
+            const int stride = Hv * DV, off = 4 * g * stride + m;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i < rows) {
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) dst[off + i * stride + 16 * rg] = o[rg][i];
+                }
+        };
+        {
+            const auto r = w_of(0);
+#pragma unroll
+            for (int c = 0; c < NK; c++) pw[c] = load(r, c);
         }
+        if (ROLE == 0) fetch_u(0);
+        else fetch_el(0);
+        fetch_k(0);
+        if (owner) publish_state();
+        __syncthreads();
+        for (int blk = 0; blk < nblk; blk++) {
+            // ---- W S0^T, or q^ S0^T, for this wave's 16 tokens ------------------------------
+            if constexpr (ROLE == 0) __builtin_amdgcn_s_setprio(1);
+            if constexpr (ROLE == 1) {
+                if (blk > 0) {
+                    finish_o(blk - 1);
+                }
+                fetch_m(blk);
+            }
+            wy_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            const auto r = w_of(blk + 1);
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                const u32x4 a = pw[2 * s], b = pw[2 * s + 1];
+                const u32x4 hi = {a[0], a[1], b[0], b[1]}, lo = {a[2], a[3], b[2], b[3]};
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++) {
+                    const u32x4 sh = s_s[rg][s][0][lane], sl = s_s[rg][s][1][lane];
+                    wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                    acc = wy_mfma(lo, sh, acc);
+                    acc = wy_mfma(hi, sl, acc);
+                    acc = wy_mfma(hi, sh, acc);
+                    p[rg] += acc * s_su[rg][s][m];
+                }
+                pw[2 * s] = load(r, 2 * s);
+                pw[2 * s + 1] = load(r, 2 * s + 1);
+            }
+            if constexpr (ROLE == 0) {
+                // ---- D = U - W S0^T: lane (n, g) holds tokens 16w+4g+i of state row n of the group ----
+                const wy_f32x4 d[2] = {pu[0] - p[0], pu[1] - p[1]};
+                fetch_u(blk + 1);
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++) {
+                    float sc, un;
+                    wy_scale(rows_max(fmaxf(fmaxf(fabsf(d[rg][0]), fabsf(d[rg][1])), fmaxf(fabsf(d[rg][2]), fabsf(d[rg][3])))), sc, un);
+                    const u32x4 x = wy_split4(d[rg][0] * sc, d[rg][1] * sc, d[rg][2] * sc, d[rg][3] * sc);
+                    s_d[blk & 1][rg][w][0][lane] = u32x4{x[0], x[1], x[0], x[1]};
+                    s_d[blk & 1][rg][w][1][lane] = u32x4{x[2], x[3], x[2], x[3]};
+                    if (g == 0) s_du[blk & 1][rg][w][m] = un;
+                }
+            } else {
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++) o[rg] = el * p[rg];
+                fetch_el(blk + 1);
+            }
+            __syncthreads();
+            // ---- S' = e^{L_C} S0 + D^T diag(e^{L_C-L}) K, this wave's columns and rows ------
+            if (owner) {
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) st[ct] *= elc;
+#pragma unroll
+                for (int tau = 0; tau < 4; tau++) {
+                    const u32x4 dh = s_d[blk & 1][rgu][tau][0][lane], dl = s_d[blk & 1][rgu][tau][1][lane];
+                    const float un = s_du[blk & 1][rgu][tau][m];
+#pragma unroll
+                    for (int ct = 0; ct < 2; ct++) {
+                        wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                        acc = wy_mfma(kd[ct][tau], dl, acc);
+                        acc = wy_mfma(kd[ct][tau], dh, acc);
+                        st[ct] += acc * un;
+                    }
+                }
+                publish_state();
+                fetch_k(blk + 1);
+            }
+            __syncthreads();
+        }
+        if constexpr (ROLE == 1) finish_o(nblk - 1);
+    };
+    if (rgu == 0) run(std::integral_constant<int, 0>{});
+    else run(std::integral_constant<int, 1>{});
+    if (owner) {
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) *reinterpret_cast<wy_f32x4 *>(srow + 16 * ct) = st[ct];
     }
 }
 
@@ -608,23 +701,24 @@ int launch_gdn_wy(hipStream_t s, int Hk, int Hv, int dk, int dv, int T, const fl
     const size_t nblk = ((size_t)T + kC - 1) / kC;
     if (nblk > 65535) return fail(MFA_ERR_SHAPE, "gdn blocked form: too many tokens in one call");
     const size_t slots = nblk * Hv;
-    float *Wt = scratch;
-    float *Qt = Wt + slots * kC * dk;
-    float *Kt = Qt + slots * kC * dk;
-    float *Ut = Kt + slots * kC * dk;
-    float *Mt = Ut + slots * kC * dv;
-    float *eLc = Mt + slots * kC * kC;
+    // (an operand's two f16 parts take the four bytes of the f32 value they stand for)
+    u32x4 *Wt = reinterpret_cast<u32x4 *>(scratch);
+    u32x4 *Qt = Wt + slots * kC * dk / 4;
+    u32x4 *Kt = Qt + slots * kC * dk / 4;
+    float *Ut = reinterpret_cast<float *>(Kt + slots * kC * dk / 4);
+    u32x4 *Mt = reinterpret_cast<u32x4 *>(Ut + slots * kC * dv);
+    float *eLc = reinterpret_cast<float *>(Mt + slots * kC * kC / 4);
     const WyInputs none{};
 #define MFA_WY(DKK, FU)                                                                                             \
     hipLaunchKernelGGL((gdn_wy_kernel<DKK, FU>), dim3(Hv, (unsigned)nblk), dim3(DKK * 4), 0, s, Hk, Hv, T, qn, kn, vv, \
                        lg, bg, Wt, Qt, Ut, Mt, Kt, eLc, in ? *in : none)
     if (dk == 128) {
         if (in) MFA_WY(128, true); else MFA_WY(128, false);
-        hipLaunchKernelGGL((gdn_wy_recur_kernel<128>), dim3(Hv, dv / 16), dim3(256), 0, s, Hk, Hv, T, Wt, Qt, Ut,
+        hipLaunchKernelGGL((gdn_wy_recur_kernel<128>), dim3(Hv, dv / 32), dim3(512), 0, s, Hk, Hv, T, Wt, Qt, Ut,
                            Mt, Kt, eLc, ssm, o_raw);
     } else {
         if (in) MFA_WY(64, true); else MFA_WY(64, false);
-        hipLaunchKernelGGL((gdn_wy_recur_kernel<64>), dim3(Hv, dv / 16), dim3(256), 0, s, Hk, Hv, T, Wt, Qt, Ut,
+        hipLaunchKernelGGL((gdn_wy_recur_kernel<64>), dim3(Hv, dv / 32), dim3(512), 0, s, Hk, Hv, T, Wt, Qt, Ut,
                            Mt, Kt, eLc, ssm, o_raw);
     }
 #undef MFA_WY
