@@ -16,8 +16,8 @@
 // chunk at once (gdn_wy_kernel, one workgroup per (block, value head)); the four
 // products that involve the state run block after block with the state in registers
 // (gdn_wy_recur_kernel, one workgroup per 32 rows of a head's state, rows being
-// independent).  The products before D are v_mfma_f32_16x16x4_f32; those that involve the state are
-// v_mfma_f32_16x16x32_f16 over operands split into two f16 numbers (see wy_split4).
+// independent).  The products are v_mfma_f32_16x16x32_f16 over operands split into two f16 numbers (see wy_split4), the
+// inversion's small ones v_mfma_f32_16x16x4_f32.
 //
 // Operand conventions of the f32 instruction (lane l, m = n = l % 16, g = l / 16):
 // A[m][g], B[g][n] in; D[4g+i][n], i = 0..3, out.  A contraction over 16 values is done as
@@ -68,22 +68,30 @@ __device__ inline wy_f32x4 load_v4(const float *p) { return *reinterpret_cast<co
 // scale; the state's and D's scales are those of the largest value of a tile's row, taken as the tile is formed.
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;   // (LDS holding f32 and f16 parts in turn is read and written as vectors, which alias anything)
 static constexpr float kWyScale = 16384.f;   // 2^14: the largest f16 is 65504
-__device__ inline uint32_t wy_pack(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2)); }
-__device__ inline void wy_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-    const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
-    hi = __builtin_bit_cast(uint32_t, h);
-    lo = wy_pack(a - (float)h[0], b - (float)h[1]);
-}
-// four values as 16 bytes: hi of all, lo of all
-__device__ inline u32x4 wy_split4(float a, float b, float c, float d) {
+// Four values times scale as 16 bytes: hi of all, lo of all.  v_fma_mix*_f16 multiplies, subtracts hi where there is one, and
+// rounds, in one instruction per value and part (multiply, convert, convert back, subtract, convert are four).
+// The compiler does not see into the assembly: a result that went to the upper half of its register may be read one wait state
+// later at the earliest, which the order of the eight and the last no-op keep; and no result of a matrix instruction may come in
+// directly (its wait states are the compiler's to place), which callers see to with an instruction in between.
+__device__ inline u32x4 wy_split4(float a, float b, float c, float d, float scale) {
     uint32_t h0, h1, l0, l1;
-    wy_split2(a, b, h0, l0);
-    wy_split2(c, d, h1, l1);
+    asm("v_fma_mixlo_f16 %0, %4, %8, 0\n\t"
+        "v_fma_mixlo_f16 %1, %6, %8, 0\n\t"
+        "v_fma_mixhi_f16 %0, %5, %8, 0\n\t"
+        "v_fma_mixhi_f16 %1, %7, %8, 0\n\t"
+        "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %6, %8, -%1 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, %5, %8, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, %7, %8, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 0"
+        : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1) : "v"(a), "v"(b), "v"(c), "v"(d), "v"(scale));
     return u32x4{h0, h1, l0, l1};
 }
-__device__ inline u32x4 wy_split4_unit(float a, float b, float c, float d) {   // of values of at most 1
-    return wy_split4(a * kWyScale, b * kWyScale, c * kWyScale, d * kWyScale);
+__device__ inline u32x4 wy_split4_unit(float a, float b, float c, float d) { return wy_split4(a, b, c, d, kWyScale); }   // of values of at most 1
+__device__ inline wy_f32x4 wy_fma(wy_f32x4 a, float s, wy_f32x4 c) {
+    return wy_f32x4{fmaf(a[0], s, c[0]), fmaf(a[1], s, c[1]), fmaf(a[2], s, c[2]), fmaf(a[3], s, c[3])};
 }
 // The scale of values of at most mx (2^14 <= mx scale < 2^15, less for mx below 2^-87) and what undoes it together with kWyScale.
 __device__ inline void wy_scale(float mx, float &scale, float &undo) {
@@ -107,6 +115,10 @@ __device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
 //
 // grid (Hv, blocks), one wave per 16 columns of K (DK/16 waves: two per SIMD at DK = 128, so that one
 // has matrix work while the other waits for LDS or stores a tile).
+// A workgroup's 28 k clocks (39 k on f32 instructions) are 9 k until its inputs are there, 3 k of norms, 3.5 k for the two
+// triangles, 2.3 k for the diagonal blocks beside K', 4.7 k for the levels beside phase 3's operands, 4 k for W and U: 512 tokens of 32
+// heads 21.8 -> 16.9 us.  At 128 registers, so that a CU holds two (it takes 144 and holds one), it spills: no faster at 2000
+// tokens with three sequences side by side (120.5 us a pass either way), 2 us slower at 512.
 // FUSED: the block's inputs come straight from the layer's inputs (WyInputs): what
 // gdn_chunk_pre_kernel computes for the token-by-token form is done here per (block, value head) -
 // conv + SiLU of the head's q, k and v channels, the per-token q/k norm, the decay's logarithm and
@@ -119,32 +131,32 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     u32x4 *__restrict__ Wt, u32x4 *__restrict__ Qt, float *__restrict__ Ut, u32x4 *__restrict__ Mt,
     u32x4 *__restrict__ Kt, float *__restrict__ eLc, WyInputs in) {
     constexpr int DV = DK;
-    constexpr int NK = DK / 16;
-    constexpr int LDK = DK + 4;  // row strides chosen so that 16-byte row reads by 8 lanes hit all banks
+    constexpr int NK = DK / 16, NS = DK / 32;
+    constexpr int LDK = DK + 4;  // row strides (4-byte units) chosen so that 16-byte row reads by 8 lanes hit all banks
     constexpr int LDC = kC + 4;
-    constexpr int NW = NK;        // waves
+    constexpr int NW = NK;        // waves; wave c owns columns 16c .. 16c+15 of W and of U
     constexpr int NTHR = 64 * NW;
-    constexpr int NCT = 1;        // 16-wide column tiles of W (and of U) per wave
-    static_assert(!FUSED || NCT == 1, "a wave's v is one column tile");
+    // A row of k^ or q^ is f32 until it is normed and then the f16 parts in its place (hi of all channels, then lo of all), v stays
+    // in the registers of the wave that multiplies it, T and its f16 parts lie where q^ and A were.
     __shared__ __align__(16) float sK[kC][LDK];
-    // FUSED keeps to half a CU's LDS (81664 bytes of 163840; it was 137472), so that a CU holds two workgroups, of one launch or
-    // of two sequences': v stays in the registers of the wave that multiplies it, A is its ten lower tiles, and T lies
-    // where q^ was.  The kernel waits on memory, LDS and its substitution chain far more than on its products (512 tokens,
-    // six layers 261 -> 237 us a pass with three sequences side by side; 2000 tokens of one layer 176 -> 154).
-    __shared__ __align__(16) float sQ[kC][LDK];  // q^, later v (FUSED: later T)
-    __shared__ __align__(16) float sA[10][16][20];   // tile (I, J <= I) at I (I + 1) / 2 + J
-    __shared__ __align__(16) float sTown[FUSED ? 1 : kC][LDC];
-    static_assert(LDC <= LDK, "T fits where q^ was");
-    float(*sT)[LDC] = FUSED ? reinterpret_cast<float(*)[LDC]>(&sQ[0][0]) : sTown;
+    constexpr int TPARTS = 6 * 2 * 64 * 4;           // f16 parts of T times a factor per token: [(token tile, 32-token step)][hi|lo][64] x 16 bytes
+    constexpr int QROOM = kC * LDK > kC * LDC + TPARTS ? kC * LDK : kC * LDC + TPARTS;
+    __shared__ __align__(16) float sQroom[QROOM];    // q^, later T and T diag(beta)
+    __shared__ __align__(16) float sA[10][16][20];   // tile (I, J <= I) at I (I + 1) / 2 + J; later T diag(beta e^L)
+    float(*sQ)[LDK] = reinterpret_cast<float(*)[LDK]>(&sQroom[0]);
+    float(*sT)[LDC] = reinterpret_cast<float(*)[LDC]>(&sQroom[0]);
+    u32x4(*sTu)[2][64] = reinterpret_cast<u32x4(*)[2][64]>(&sQroom[kC * LDC]);
+    u32x4(*sTw)[2][64] = reinterpret_cast<u32x4(*)[2][64]>(&sA[0][0][0]);
+    static_assert(TPARTS * sizeof(float) <= sizeof(sA), "T's parts fit where A was");
     __shared__ __align__(16) float sL[kC], sB[kC], sCw[kC], sKd[kC];
-    __shared__ int sR[kC];
+    __shared__ __align__(16) int sR[kC];
 
     // heads along x: a head's blocks are produced on the XCD whose L2 the recurrence kernel
     // (heads along x as well) will read them through
     const int vh = wy_head_of(blockIdx.x, Hk, Hv), blk = blockIdx.y, kh = vh / (Hv / Hk);
     const int t0 = blk * kC;
     const int nt = (T - t0 < kC) ? T - t0 : kC;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = lane & 15, g = lane >> 4;
     const size_t slot = (size_t)blk * Hv + vh;
 
@@ -152,9 +164,42 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     // Everything the block reads is requested here, in the order of use (loads return in the
     // order of their requests): the gates, k^ and q^, and v, which waits in registers for phase 2.
     float lg_in = 0.f, bg_in = 0.f;
-    constexpr int NLV = kC * (DV / 4) / NTHR;
-    float4 va[FUSED ? 1 : NLV];
-    float vreg[4][4];   // FUSED: v of tokens 16 s + 4 g + i, channel 16 wave + m, phase 3's operand
+    float vreg[4][4];   // v of tokens 16 s + 4 g + i, channel 16 wave + m, phase 3's operand
+    // Cumulative log decay (wave 0), restarted after every token whose decay is zero: where the
+    // reference's exp() underflows (log g below log FLT_MIN; -inf when its softplus overflows,
+    // linear_attn.rs:357-370) the token forgets everything before it, and no factor e^{L_i-L_j}
+    // may be formed across it (-inf - -inf).  sR[t] is the last such token up to and
+    // including t (-1: none); a pair (row, col) decays to exactly 0 when sR[row] > col.
+    auto scan_gates = [&]() __attribute__((always_inline)) {
+        const bool dead = lg_in < -87.3f;
+        float l = dead ? 0.f : lg_in;
+        bool seg = dead;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const float u = __shfl_up(l, d, 64);
+            const int su = __shfl_up((int)seg, d, 64);
+            if (lane >= d) {
+                if (!seg) l += u;
+                seg = seg || su;
+            }
+        }
+        const unsigned long long kills = __ballot(dead) & ((2ull << lane) - 1ull);
+        const int r = kills ? 63 - __builtin_clzll(kills) : -1;
+        const float el = r >= 0 ? 0.f : expf(l);      // decay since the block's first token
+        sL[lane] = l;
+        sR[lane] = r;
+        sB[lane] = bg_in;
+        sCw[lane] = bg_in * el;
+        eLc[slot * kC + lane] = el;
+        sKd[lane] = __shfl(r, 63, 64) > lane ? 0.f : expf(__shfl(l, 63, 64) - l);  // e^{L_C - L_t}
+    };
+    // a row of k^ or q^ as its f16 parts: channels c .. c + 3, y scale (at most 1)
+    auto put4 = [&](float *row, int c, float4 y, float scale) __attribute__((always_inline)) {
+        const u32x4 x = wy_split4(y.x, y.y, y.z, y.w, scale * kWyScale);
+        uint32_t *r = reinterpret_cast<uint32_t *>(row);
+        *reinterpret_cast<u32x2 *>(r + c / 2) = u32x2{x[0], x[1]};
+        *reinterpret_cast<u32x2 *>(r + DK / 2 + c / 2) = u32x2{x[2], x[3]};
+    };
     if constexpr (FUSED) {
         constexpr int NCONV = 2 * DK, TT = 16;               // q and k channels of the head; tokens per run
         constexpr int NU = NCONV * (kC / TT) / NTHR;          // (channel, run) units per thread
@@ -249,6 +294,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             lg_in = -a_cap * sp;
             bg_in = 1.0f / (1.0f + expf(-b_in));
         }
+        if (wave == 0) scan_gates();   // ahead of the barrier, which waves 4 .. 7 reach last
         __syncthreads();
         // per-token norm of q and k (infer.m:2655-2667: x * inv_rms, then q *= (1/sqrt(dk))^2,
         // k *= 1/sqrt(dk)): NTHR / (2 kC) lanes per (token, q|k) row, in place
@@ -269,20 +315,18 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             if (LPP == 4) ss = dpp_add<0x4E>(ss);
             const float inv_scale = 1.0f / sqrtf((float)DK);
             const float inv_rms = 1.0f / sqrtf(ss / (float)DK + 1e-6f);
-            const float sc = is_q ? inv_scale * inv_scale : inv_scale;
+            const float sc = inv_rms * (is_q ? inv_scale * inv_scale : inv_scale);
 #pragma unroll
-            for (int i = 0; i < EPL / 4; i++) {
-                float4 y = {x[i].x * inv_rms, x[i].y * inv_rms, x[i].z * inv_rms, x[i].w * inv_rms};
-                y.x *= sc; y.y *= sc; y.z *= sc; y.w *= sc;
-                *(float4 *)(row + 4 * i) = y;
-            }
+            for (int i = 0; i < EPL / 4; i++) put4(is_q ? sQ[tt] : sK[tt], EPL * sub + 4 * i, x[i], sc);   // (a row's lanes are one wave's: all have read it)
         }
     } else {
-    if (wave == 0 && lane < nt) {
-        lg_in = lg[(size_t)(t0 + lane) * Hv + vh];
-        bg_in = bg[(size_t)(t0 + lane) * Hv + vh];
-    }
-    {
+        if (wave == 0) {
+            if (lane < nt) {
+                lg_in = lg[(size_t)(t0 + lane) * Hv + vh];
+                bg_in = bg[(size_t)(t0 + lane) * Hv + vh];
+            }
+            scan_gates();
+        }
         constexpr int NL = kC * (DK / 4) / NTHR;
         float4 a[NL], b[NL];
 #pragma unroll
@@ -293,120 +337,121 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             b[u] = load_f4(qn + src);
         }
 #pragma unroll
-        for (int u = 0; u < NLV; u++) {
-            const int i = tid + u * NTHR, tt = i / (DV / 4), x = (i % (DV / 4)) * 4;
-            va[u] = load_f4(vv + ((size_t)(t0 + (tt < nt ? tt : nt - 1)) * Hv + vh) * DV + x);
-        }
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tt = 16 * s + 4 * g + i;
+                vreg[s][i] = vv[((size_t)(t0 + (tt < nt ? tt : nt - 1)) * Hv + vh) * DV + 16 * wave + m];
+                if (tt >= nt) vreg[s][i] = 0.f;
+            }
 #pragma unroll
         for (int u = 0; u < NL; u++) {
             const int i = tid + u * NTHR, tt = i / (DK / 4), x = (i % (DK / 4)) * 4;
             const float keep = tt < nt ? 1.f : 0.f;  // padded tokens are zero rows
-            *(float4 *)&sK[tt][x] = float4{a[u].x * keep, a[u].y * keep, a[u].z * keep, a[u].w * keep};
-            *(float4 *)&sQ[tt][x] = float4{b[u].x * keep, b[u].y * keep, b[u].z * keep, b[u].w * keep};
+            put4(sK[tt], x, float4{a[u].x * keep, a[u].y * keep, a[u].z * keep, a[u].w * keep}, 1.f);
+            put4(sQ[tt], x, float4{b[u].x * keep, b[u].y * keep, b[u].z * keep, b[u].w * keep}, 1.f);
         }
-    }
-    }
-    if (wave == 0) {
-        // Cumulative log decay, restarted after every token whose decay is zero: where the
-        // reference's exp() underflows (log g below log FLT_MIN; -inf when its softplus overflows,
-        // linear_attn.rs:357-370) the token forgets everything before it, and no factor e^{L_i-L_j}
-        // may be formed across it (-inf - -inf).  sR[t] is the last such token up to and
-        // including t (-1: none); a pair (row, col) decays to exactly 0 when sR[row] > col.
-        const bool dead = lg_in < -87.3f;
-        float l = dead ? 0.f : lg_in;
-        bool seg = dead;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const float u = __shfl_up(l, d, 64);
-            const int su = __shfl_up((int)seg, d, 64);
-            if (lane >= d) {
-                if (!seg) l += u;
-                seg = seg || su;
-            }
-        }
-        const unsigned long long kills = __ballot(dead) & ((2ull << lane) - 1ull);
-        const int r = kills ? 63 - __builtin_clzll(kills) : -1;
-        const float b = bg_in;
-        const float el = r >= 0 ? 0.f : expf(l);      // decay since the block's first token
-        sL[lane] = l;
-        sR[lane] = r;
-        sB[lane] = b;
-        sCw[lane] = b * el;
-        eLc[slot * kC + lane] = el;
-        sKd[lane] = __shfl(r, 63, 64) > lane ? 0.f : expf(__shfl(l, 63, 64) - l);  // e^{L_C - L_t}
     }
     __syncthreads();
+
+    // Operands from the rows: eight channels of a row; four tokens (t .. t + 3, t = 16 tau + 4 g) of channel 16 c + m.
+    auto row_part = [&](const float *row, int s, int part) __attribute__((always_inline)) {
+        return *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint32_t *>(row) + part * (DK / 2) + 16 * s + 4 * g);
+    };
+    auto col_part = [&](int tau, int c, int part) __attribute__((always_inline)) {
+        typedef short i16x4 __attribute__((ext_vector_type(4)));
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(sK[16 * tau + 4 * g + (m >> 2)]) + part * (DK / 2) + 8 * c + 2 * (m & 3);
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (i16x4 __attribute__((address_space(3))) *)(__attribute__((address_space(3))) uint32_t *)p));
+    };
+    const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    constexpr float kUnscale2 = 1.f / (kWyScale * kWyScale);
 
     // ---- phase 1: the lower tiles of K K^T (-> A) and of Q K^T (-> M) -----------------
-    // 10 tiles (I, J <= I) each; 20 jobs of DK/4 instructions dealt round the waves.
+    // A job is a row tile I of one of the two and its tiles J <= I; the jobs of a SIMD's two waves add up to five tiles.  Written
+    // out per job, so that the reads of a tile's operands overlap the tile before it.
+    auto gram = [&](auto kind_tag, auto I_tag) __attribute__((always_inline)) {
+        constexpr int kind = decltype(kind_tag)::value, I = decltype(I_tag)::value;
+        u32x4 ih[NS], il[NS];
 #pragma unroll
-    for (int r = 0; r < (20 + NW - 1) / NW; r++) {
-        const int job = wave + NW * r;
-        if (job >= 20) break;   // uniform over the wave
-        const int kind = job / 10, idx = job % 10;
-        const int I = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-        const int J = idx - I * (I + 1) / 2;
-        wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        if (kind == 0) {
+        for (int s = 0; s < NS; s++) {
+            const float *row = kind ? sQ[16 * I + m] : sK[16 * I + m];
+            ih[s] = row_part(row, s, 0);
+            il[s] = row_part(row, s, 1);
+        }
 #pragma unroll
-            for (int s = 0; s < DK / 16; s++)
-                acc = mfma4(lds_f4(&sK[16 * I + m][16 * s + 4 * g]), lds_f4(&sK[16 * J + m][16 * s + 4 * g]), acc);
-            // lane (n = m, g) holds rows 16I + 4g + i of column 16J + n
-            const int col = 16 * J + m;
+        for (int J = 0; J <= I; J++) {
+            u32x4 jh[NS], jl[NS];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int row = 16 * I + 4 * g + i;
-                const float dl = sL[row] - sL[col];
-                const float d = sR[row] > col ? 0.f : __builtin_amdgcn_exp2f((dl < 0.f ? dl : 0.f) * 1.4426950408889634f);  // v_exp_f32: 1 ulp
-                sA[idx][4 * g + i][m] = (col < row) ? sB[row] * d * acc[i] : 0.f;
+            for (int s = 0; s < NS; s++) jh[s] = row_part(sK[16 * J + m], s, 0), jl[s] = row_part(sK[16 * J + m], s, 1);
+            wy_f32x4 lh = zero, hl = zero, hh = zero;
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                // K K^T: lane (n = m, g) gets rows 16I + 4g + i of column 16J + n.  Q K^T as the tile transposed (k^ as the A side):
+                // columns 16J + 4g + i of row 16I + n, which is this lane's 16 bytes of tile (I, J) in A-operand order
+                lh = kind ? wy_mfma(jl[s], ih[s], lh) : wy_mfma(il[s], jh[s], lh);
+                hl = kind ? wy_mfma(jh[s], il[s], hl) : wy_mfma(ih[s], jl[s], hl);
+                hh = kind ? wy_mfma(jh[s], ih[s], hh) : wy_mfma(ih[s], jh[s], hh);
             }
-        } else {
-            // the tile transposed (k^ as the A side): lane (n = m, g) then holds columns 16J + 4g + i of
-            // row 16I + n, which is this lane's 16 bytes of tile (I, J) in A-operand order
+            const wy_f32x4 acc = ((lh + hl) + hh) * kUnscale2;
+            const int one = kind ? 16 * I + m : 16 * J + m, four = (kind ? 16 * J : 16 * I) + 4 * g;   // this lane's row (column), columns (rows)
+            const float4 l4 = lds_f4(&sL[four]);
+            const float lf[4] = {l4.x, l4.y, l4.z, l4.w}, l1 = sL[one];
+            wy_f32x4 y;
+            if constexpr (kind) {
+                const int r1 = sR[one];
 #pragma unroll
-            for (int s = 0; s < DK / 16; s++)
-                acc = mfma4(lds_f4(&sK[16 * J + m][16 * s + 4 * g]), lds_f4(&sQ[16 * I + m][16 * s + 4 * g]), acc);
-            const int row = 16 * I + m;
-            wy_f32x4 mv;
+                for (int i = 0; i < 4; i++) {
+                    const float d = r1 > four + i ? 0.f : __builtin_amdgcn_exp2f(fminf(l1 - lf[i], 0.f) * 1.4426950408889634f);  // v_exp_f32: 1 ulp
+                    y[i] = (I > J || four + i <= one) ? d * acc[i] : 0.f;
+                }
+                Mt[((slot * 4 + I) * 4 + J) * 64 + lane] = wy_split4_unit(y[0], y[1], y[2], y[3]);
+            } else {
+                const float4 b4 = lds_f4(&sB[four]);
+                const int4 r4 = *reinterpret_cast<const int4 *>(&sR[four]);
+                const float bf[4] = {b4.x, b4.y, b4.z, b4.w};
+                const int rf[4] = {r4.x, r4.y, r4.z, r4.w};
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int col = 16 * J + 4 * g + i;
-                const float dl = sL[row] - sL[col];
-                const float d = sR[row] > col ? 0.f : __builtin_amdgcn_exp2f((dl < 0.f ? dl : 0.f) * 1.4426950408889634f);
-                mv[i] = (col <= row) ? d * acc[i] : 0.f;
+                for (int i = 0; i < 4; i++) {
+                    const float d = rf[i] > one ? 0.f : __builtin_amdgcn_exp2f(fminf(lf[i] - l1, 0.f) * 1.4426950408889634f);
+                    sA[I * (I + 1) / 2 + J][4 * g + i][m] = (I > J || one < four + i) ? bf[i] * d * acc[i] : 0.f;
+                }
             }
-            Mt[((slot * 4 + I) * 4 + J) * 64 + lane] = wy_split4_unit(mv[0], mv[1], mv[2], mv[3]);
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < 8 / NW; r++) {
+        using std::integral_constant;
+        switch (wave + NW * r) {   // uniform over the wave
+            case 0: gram(integral_constant<int, 0>{}, integral_constant<int, 0>{}); break;
+            case 1: gram(integral_constant<int, 0>{}, integral_constant<int, 1>{}); break;
+            case 2: gram(integral_constant<int, 0>{}, integral_constant<int, 2>{}); break;
+            case 3: gram(integral_constant<int, 0>{}, integral_constant<int, 3>{}); break;
+            case 4: gram(integral_constant<int, 1>{}, integral_constant<int, 3>{}); break;
+            case 5: gram(integral_constant<int, 1>{}, integral_constant<int, 2>{}); break;
+            case 6: gram(integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
+            default: gram(integral_constant<int, 1>{}, integral_constant<int, 0>{}); break;
         }
     }
-    for (int i = tid; i < 4 * NK * 64; i += NTHR) {  // q^ tiles, before v takes its place
-        const int tile = i >> 6, l = i & 63, w = tile / NK, c = tile % NK;
-        const float4 q = lds_f4(&sQ[16 * w + (l & 15)][16 * c + 4 * (l >> 4)]);
-        Qt[(slot * 4 * NK + tile) * 64 + l] = wy_split4_unit(q.x, q.y, q.z, q.w);
+#pragma unroll
+    for (int u = 0; u < 4 * NK / NW; u++) {  // q^ tiles, before T takes their place
+        const int tile = wave + NW * u, w = tile / NK, c = tile % NK;
+        const uint32_t *row = reinterpret_cast<const uint32_t *>(sQ[16 * w + m]) + 8 * c + 2 * g;
+        const u32x2 hi = *reinterpret_cast<const u32x2 *>(row), lo = *reinterpret_cast<const u32x2 *>(row + DK / 2);
+        Qt[(slot * 4 * NK + tile) * 64 + lane] = u32x4{hi[0], hi[1], lo[0], lo[1]};
     }
     __syncthreads();
 
-    // ---- phase 2: diag(e^{L_C - L}) K transposed goes out, v comes in, and
+    // ---- phase 2: diag(e^{L_C - L}) K transposed goes out, and
     //      T = (I + A)^-1 by blocks of 16: the diagonal blocks by forward substitution (one
     //      per wave, a column per lane), the blocks below them level by level from
     //      T_IJ = -T_II sum_{J <= K < I} A_IK T_KJ on the matrix cores -----------------------
-    {
-#pragma unroll
-        for (int u = 0; u < NK * 4 * 64 / NTHR; u++) {
-            const int i = tid + u * NTHR, tile = i >> 6, l = i & 63, c = tile >> 2, tau = tile & 3;
-            const int kk = 16 * c + (l & 15), j4 = 16 * tau + 4 * (l >> 4);
-            const float4 e = lds_f4(&sKd[j4]);
-            Kt[(slot * NK * 4 + tile) * 64 + l] = wy_split4_unit(e.x * sK[j4 + 0][kk], e.y * sK[j4 + 1][kk], e.z * sK[j4 + 2][kk], e.w * sK[j4 + 3][kk]);
-        }
-        if constexpr (!FUSED) {
-#pragma unroll
-            for (int u = 0; u < NLV; u++) {
-                const int i = tid + u * NTHR, tt = i / (DV / 4), x = (i % (DV / 4)) * 4;
-                const float keep = tt < nt ? 1.f : 0.f;
-                *(float4 *)&sQ[tt][x] = float4{va[u].x * keep, va[u].y * keep, va[u].z * keep, va[u].w * keep};
-            }
-        }
-    }
-    if (wave < 4) {
+    // k^ of four tokens from its parts (exact), times kWyScale
+    auto whole = [&](u32x2 hi, u32x2 lo) __attribute__((always_inline)) {
+        const f16x2 h0 = __builtin_bit_cast(f16x2, (uint32_t)hi[0]), h1 = __builtin_bit_cast(f16x2, (uint32_t)hi[1]), l0 = __builtin_bit_cast(f16x2, (uint32_t)lo[0]), l1 = __builtin_bit_cast(f16x2, (uint32_t)lo[1]);
+        return float4{(float)h0[0] + (float)l0[0], (float)h0[1] + (float)l0[1], (float)h1[0] + (float)l1[0], (float)h1[1] + (float)l1[1]};
+    };
+    if (NW == 4 || wave < 4) {
         // block `wave`; the four lane groups compute the same 16 columns, group 0 stores
         const int r0 = 16 * wave;
         float t[16];
@@ -425,12 +470,43 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             if (g == 0) sT[r0 + i][r0 + m] = acc;
         }
     }
+    // the waves without a diagonal block take the tiles of K' (all waves where each has one)
+    if (NW == 4 || wave >= 4) {
+#pragma unroll
+        for (int u = 0; u < NK; u++) {
+            const int tile = (wave & 3) + 4 * u, c = tile >> 2, tau = tile & 3;
+            const float4 e = lds_f4(&sKd[16 * tau + 4 * g]);
+            const float4 k = whole(col_part(tau, c, 0), col_part(tau, c, 1));
+            Kt[(slot * NK * 4 + tile) * 64 + lane] = wy_split4(k.x * e.x, k.y * e.y, k.z * e.z, k.w * e.w, 1.f);
+        }
+    }
     __syncthreads();
+    // phase 3's K and V operands of the wave's columns, for all four token tiles: here, where most waves would wait for the levels
+    u32x4 kwh[2], kwl[2], vuh[2], vul[2];
+    float v_undo;
+    {
+        float mx = 0.f, sc;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(vreg[s][i]));
+        wy_scale(rows_max(mx), sc, v_undo);
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            const u32x2 h0 = col_part(2 * p, wave, 0), h1 = col_part(2 * p + 1, wave, 0), l0 = col_part(2 * p, wave, 1), l1 = col_part(2 * p + 1, wave, 1);
+            kwh[p] = u32x4{h0[0], h0[1], h1[0], h1[1]};
+            kwl[p] = u32x4{l0[0], l0[1], l1[0], l1[1]};
+            const u32x4 y0 = wy_split4(vreg[2 * p][0], vreg[2 * p][1], vreg[2 * p][2], vreg[2 * p][3], sc);
+            const u32x4 y1 = wy_split4(vreg[2 * p + 1][0], vreg[2 * p + 1][1], vreg[2 * p + 1][2], vreg[2 * p + 1][3], sc);
+            vuh[p] = u32x4{y0[0], y0[1], y1[0], y1[1]};
+            vul[p] = u32x4{y0[2], y0[3], y1[2], y1[3]};
+        }
+    }
 #pragma unroll
     for (int lvl = 1; lvl < 4; lvl++) {
         if (wave < 4 - lvl) {  // block (I, J) = (wave + lvl, wave)
             const int I = wave + lvl, J = wave;
-            wy_f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            wy_f32x4 x = zero;
             for (int K = J; K < I; K++) {
                 float4 bt;
                 bt.x = sT[16 * K + 4 * g + 0][16 * J + m];
@@ -440,67 +516,75 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                 x = mfma4(lds_f4(&sA[I * (I + 1) / 2 + K][m][4 * g]), bt, x);
             }
             // x is held as rows 4g+i of column m: already the B operand of T_II x
-            wy_f32x4 r = {0.f, 0.f, 0.f, 0.f};
+            wy_f32x4 r = zero;
             r = mfma4(lds_f4(&sT[16 * I + m][16 * I + 4 * g]), as_f4(x), r);
 #pragma unroll
             for (int i = 0; i < 4; i++) sT[16 * I + 4 * g + i][16 * J + m] = -r[i];
         }
         __syncthreads();
     }
+    // The f16 parts of T diag(beta e^L) and T diag(beta) (T is at most 1: its column j is what an impulse at token j leaves of itself in
+    // later ones); step p of token tile tau holds tokens 32p .. 32p+31, zeros above the diagonal
+#pragma unroll
+    for (int u = 0; u < 12 / NW + (12 % NW != 0); u++) {
+        const int half = wave + NW * u;   // (tau, token tile): (0,0) (0,1) (1,0) (1,1) (2,0) .. (3,3)
+        if (half < 12) {
+            const int tau = half < 4 ? half >> 1 : 2 + ((half - 4) >> 2), s = half < 4 ? half & 1 : (half - 4) & 3;
+            const float4 t = s <= tau ? lds_f4(&sT[16 * tau + m][16 * s + 4 * g]) : float4{0.f, 0.f, 0.f, 0.f};
+            const float4 cw = lds_f4(&sCw[16 * s + 4 * g]), cb = lds_f4(&sB[16 * s + 4 * g]);
+            const u32x4 x = wy_split4_unit(t.x * cw.x, t.y * cw.y, t.z * cw.z, t.w * cw.w);
+            const u32x4 y = wy_split4_unit(t.x * cb.x, t.y * cb.y, t.z * cb.z, t.w * cb.w);
+#pragma unroll
+            for (int part = 0; part < 2; part++) {
+                reinterpret_cast<u32x2 *>(&sTw[half >> 1][part][lane])[half & 1] = u32x2{x[2 * part], x[2 * part + 1]};
+                reinterpret_cast<u32x2 *>(&sTu[half >> 1][part][lane])[half & 1] = u32x2{y[2 * part], y[2 * part + 1]};
+            }
+        }
+    }
+    __syncthreads();
 
     // ---- phase 3: W = T diag(beta e^L) K and U = T diag(beta) V -------------------------
-    // Wave w owns column tiles NCT*w .. of both; the K and V operands of those columns are
-    // read once and serve all four token tiles.
-    float bK[4][NCT][4], bV[4][NCT][4];
+    u32x4 tw[6][2], tu[6][2];
 #pragma unroll
-    for (int s = 0; s < 4; s++)
+    for (int at = 0; at < 6; at++)
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                bK[s][ct][i] = sK[16 * s + 4 * g + i][16 * (NCT * wave + ct) + m];
-                bV[s][ct][i] = FUSED ? vreg[s][i] : sQ[16 * s + 4 * g + i][16 * (NCT * wave + ct) + m];
-            }
+        for (int part = 0; part < 2; part++) tw[at][part] = sTw[at][part][lane], tu[at][part] = sTu[at][part][lane];
+    __builtin_amdgcn_sched_barrier(0);   // all reads ahead of the first product
 #pragma unroll
     for (int tau = 0; tau < 4; tau++) {
-        wy_f32x4 aw4[NCT], au4[NCT];
+        wy_f32x4 aw = zero, au = zero;
 #pragma unroll
-        for (int ct = 0; ct < NCT; ct++) aw4[ct] = au4[ct] = wy_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s <= tau; s++) {
-            const float4 t4 = lds_f4(&sT[16 * tau + m][16 * s + 4 * g]);
-            const float4 cw = lds_f4(&sCw[16 * s + 4 * g]), cb = lds_f4(&sB[16 * s + 4 * g]);
-            const float4 tw = {t4.x * cw.x, t4.y * cw.y, t4.z * cw.z, t4.w * cw.w};
-            const float4 tu = {t4.x * cb.x, t4.y * cb.y, t4.z * cb.z, t4.w * cb.w};
-#pragma unroll
-            for (int ct = 0; ct < NCT; ct++) {
-                // W transposed (K as the A side): lane (n = m, g) then holds columns 16c + 4g + i of
-                // token 16 tau + n, its 16 bytes of the tile in A-operand order
-                aw4[ct] = mfma4(float4{bK[s][ct][0], bK[s][ct][1], bK[s][ct][2], bK[s][ct][3]}, tw, aw4[ct]);
-                au4[ct] = mfma4(tu, float4{bV[s][ct][0], bV[s][ct][1], bV[s][ct][2], bV[s][ct][3]}, au4[ct]);
-            }
+        for (int p = 0; p <= tau / 2; p++) {
+            const int at = tau < 2 ? tau : 2 + 2 * (tau - 2) + p;
+            // W transposed (K as the A side): lane (n = m, g) then holds columns 16c + 4g + i of
+            // token 16 tau + n, its 16 bytes of the tile in A-operand order
+            aw = wy_mfma(kwl[p], tw[at][0], aw);
+            au = wy_mfma(tu[at][1], vuh[p], au);
+            aw = wy_mfma(kwh[p], tw[at][1], aw);
+            au = wy_mfma(tu[at][0], vul[p], au);
+            aw = wy_mfma(kwh[p], tw[at][0], aw);
+            au = wy_mfma(tu[at][0], vuh[p], au);
         }
-#pragma unroll
-        for (int ct = 0; ct < NCT; ct++) {
-            const wy_f32x4 aw = aw4[ct], au = au4[ct];
-            const size_t tile = (slot * 4 + tau) * NK + NCT * wave + ct;
-            // U as computed (a D tile), W in A-operand order
-            *reinterpret_cast<wy_f32x4 *>(Ut + tile * 256 + lane * 4) = au;
-            Wt[tile * 64 + lane] = wy_split4_unit(aw[0], aw[1], aw[2], aw[3]);
-        }
+        const size_t tile = (slot * 4 + tau) * NK + wave;
+        // U as computed (a D tile), W in A-operand order
+        *reinterpret_cast<wy_f32x4 *>(Ut + tile * 256 + lane * 4) = au * v_undo;
+        const wy_f32x4 w4 = aw * (1.f / kWyScale);   // (the instruction between the product and wy_split4)
+        Wt[tile * 64 + lane] = wy_split4(w4[0], w4[1], w4[2], w4[3], 1.f);
     }
 }
 
-// grid (Hv, DV/32), 512 threads: 32 rows of one head's state, as two groups of 16.  Waves w and w + 4 serve tokens 16w .. 16w+15
-// of each block, the first with W (and then D), the second with q^ (and then O); in the update of the state wave 4 rg + s owns
-// columns 32s .. 32s+31 of row group rg, in f32, and hands them to all waves as f16 parts with the scale of each row's largest
-// value there.  (Lane (n, g) of a tile that the update leaves holds row n, columns 16c+4g+i: with c = 2s, 2s+1 its own eight
-// values are the B operand of a 32-wide contraction over them, k-slot e < 4 being column 32s+4g+e, e >= 4 column 32s+16+4g+e-4;
-// a tile of D likewise tokens 16w+4g+i of row n.  The A side has hi and lo of the same four values in its k-slots 0-3 and 4-7, so
-// against a D operand that repeats its values one instruction adds two of the products.)
-// Bound by the two exchanges a block and by the CU's 64 bytes a clock of operands.  512 tokens of 32 heads take 25 us on half the
-// CUs (f32 instructions, 16 rows a workgroup: 25 us on all of them): six layers 241 -> 205 us a pass with three sequences side by
-// side, 2000 tokens of one layer 162 -> 128, of 64 heads 337 -> 261.
+// grid (Hv, DV/32), 512 threads: 32 rows of one head's state, as two groups of 16.  Waves 0-3 are the chain that each block waits
+// for: wave w forms D of tokens 16w .. 16w+15 from W, and owns columns 32w .. 32w+31 of the state, in f32, which it updates
+// and hands to all waves as f16 parts with the scale of each row's largest value there.  Waves 4-7 form O of the same
+// tokens from q^, a block later, beside the chain.  (Lane (n, g) of a tile that the update leaves holds row n, columns 16c+4g+i: with
+// c = 2w, 2w+1 its own eight values are the B operand of a 32-wide contraction over them, k-slot e < 4 being column 32w+4g+e,
+// e >= 4 column 32w+16+4g+e-4; a tile of D likewise tokens 16w+4g+i of row n.  The A side has hi and lo of the same four values in its
+// k-slots 0-3 and 4-7, so against a D operand that repeats its values one instruction adds two of the products.)
+// Bound by the chain: 4.4 k clocks a block (two exchanges through LDS, 56 matrix and 300 vector instructions in a row), on half the
+// CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.7 us; six layers'
+// chunks with this and the block precompute below 238 -> 186 us a pass with three sequences side by side, one sequence 54.8 -> 47.7 a layer;
+// 2000 tokens 162 -> 121 and 163 -> 144, of 64 heads 337 -> 248 and 331 -> 247.  Tried and not kept: the operands touched two blocks
+// ahead to have them in the L2 (24.5 us), O beside D of the same block (24.6).
 template <int DK>
 __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
     int Hk, int Hv, int T, const u32x4 *__restrict__ Wt, const u32x4 *__restrict__ Qt,
@@ -509,179 +593,264 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
     constexpr int DV = DK;
     constexpr int NK = DK / 16;   // column tiles of the state
     constexpr int NS = DK / 32;   // 32-column steps of a contraction over them
-    __shared__ u32x4 s_s[2][NS][2][64];    // state [row group][step][hi|lo]
-    __shared__ u32x4 s_d[2][2][4][2][64];  // D [block % 2][row group][token tile][hi twice|lo twice]
-    __shared__ float s_su[2][NS][16], s_du[2][2][4][16];   // what undoes their scales, per row
+    __shared__ u32x4 s_s[2][2][NS][2][64];   // state [block % 2][row group][step][hi|lo]
+    __shared__ u32x4 s_d[2][2][4][2][64];    // D [block % 2][row group][token tile][hi twice|lo twice]
+    __shared__ float s_su[2][2][NS][16], s_du[2][2][4][16];   // what undoes their scales, per row
 
     const int vh = wy_head_of(blockIdx.x, Hk, Hv), row0 = blockIdx.y * 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m = lane & 15, g = lane >> 4;
-    const int w = wave & 3, rgu = wave >> 2;   // token tile; of the update: row group, and step w
-    const bool owner = w < NS;
+    const int m = lane & 15, g = lane >> 4, w = wave & 3, lane16 = lane * 16;
     const int nblk = (T + kC - 1) / kC;
-    auto slot_of = [&](int blk) { return (size_t)(blk < nblk ? blk : nblk - 1) * Hv + vh; };   // past the end: the last block again
-
-    float *srow = ssm + ((size_t)vh * DV + row0 + 16 * rgu + m) * DK + 32 * (owner ? w : 0) + 4 * g;
-    wy_f32x4 st[2] = {load_v4(srow), load_v4(srow + 16)};
-    auto publish_state = [&]() __attribute__((always_inline)) {
-        float mx = 0.f, sc, un;
+    // Requests go through a descriptor of the block's operand, so that they cost no vector addition.  Past the last block: that one again.
+    auto slot_of = [&](int blk) { return (size_t)(blk < nblk ? blk : nblk - 1) * Hv + vh; };
+    auto load = [&](__amdgpu_buffer_rsrc_t r, int tile) __attribute__((always_inline)) {
+        return __builtin_amdgcn_raw_buffer_load_b128(r, lane16, tile * 1024, 0);
+    };
+    u32x4 pw[NK];   // W, or q^, of tokens 16w .. 16w+15: a register takes the next block's request as soon as it has been used
+    auto w_of = [&](const u32x4 *X, int blk) { return buffer_of(X + (slot_of(blk) * 4 + w) * NK * 64); };
+    auto fetch_all_w = [&](const u32x4 *X) __attribute__((always_inline)) {
+        const auto r = w_of(X, 0);
 #pragma unroll
-        for (int ct = 0; ct < 2; ct++)
+        for (int c = 0; c < NK; c++) pw[c] = load(r, c);
+    };
+    // X S0^T of this wave's 16 tokens, X = W or q^, both row groups
+    auto times_state = [&](const u32x4 *X, int blk, wy_f32x4 (&p)[2]) __attribute__((always_inline)) {
+        // All LDS reads first, and the three terms of every (step, row group) in turn, so that no instruction waits for the one
+        // before it (left alone the compiler reads each operand just ahead of its product: 5.2 k clocks a block instead of 4.4 k).
+        u32x4 sh[NS][2], sl[NS][2];
+        float un[NS][2];
 #pragma unroll
-            for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(st[ct][i]));
-        wy_scale(rows_max(mx), sc, un);
-        const u32x4 a = wy_split4(st[0][0] * sc, st[0][1] * sc, st[0][2] * sc, st[0][3] * sc);
-        const u32x4 b = wy_split4(st[1][0] * sc, st[1][1] * sc, st[1][2] * sc, st[1][3] * sc);
-        s_s[rgu][w][0][lane] = u32x4{a[0], a[1], b[0], b[1]};
-        s_s[rgu][w][1][lane] = u32x4{a[2], a[3], b[2], b[3]};
-        if (g == 0) s_su[rgu][w][m] = un;
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) sh[s][rg] = s_s[blk & 1][rg][s][0][lane], sl[s][rg] = s_s[blk & 1][rg][s][1][lane];
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) un[s][rg] = s_su[blk & 1][rg][s][m];
+        __builtin_amdgcn_sched_barrier(0);
+        wy_f32x4 acc[NS][2];
+        u32x4 hi[NS], lo[NS];
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const u32x4 a = pw[2 * s], b = pw[2 * s + 1];
+            hi[s] = u32x4{a[0], a[1], b[0], b[1]};
+            lo[s] = u32x4{a[2], a[3], b[2], b[3]};
+        }
+        const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(lo[s], sh[s][rg], zero);
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(hi[s], sl[s][rg], acc[s][rg]);
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(hi[s], sh[s][rg], acc[s][rg]);
+        const auto r = w_of(X, blk + 1);
+#pragma unroll
+        for (int c = 0; c < NK; c++) pw[c] = load(r, c);
+#pragma unroll
+        for (int rg = 0; rg < 2; rg++) {
+            p[rg] = acc[0][rg] * un[0][rg];
+#pragma unroll
+            for (int s = 1; s < NS; s++) p[rg] = wy_fma(acc[s][rg], un[s][rg], p[rg]);
+        }
     };
 
-    // ROLE 0: W, D; ROLE 1: q^, O.  D and the state are the chain that the next block waits for; O of a block is formed a block
-    // later, beside the chain (its waves give way to the others: s_setprio).  An operand's register takes the next block's
-    // request as soon as it has been used.  Requests go through a descriptor of the block's operand, so that they cost a
-    // scalar addition each and no vector one.
-    const int lane16 = lane * 16;
-    auto run = [&](auto role_tag) __attribute__((always_inline)) {
-        constexpr int ROLE = decltype(role_tag)::value;
-        u32x4 pw[NK], mt[4], kd[2][4];
-        wy_f32x4 pu[2], el, o[2];
-        float elc;
-        auto load = [&](__amdgpu_buffer_rsrc_t r, int tile) __attribute__((always_inline)) {
-            return __builtin_amdgcn_raw_buffer_load_b128(r, lane16, tile * 1024, 0);
-        };
-        auto w_of = [&](int blk) { return buffer_of((ROLE == 0 ? Wt : Qt) + (slot_of(blk) * 4 + w) * NK * 64); };
-        auto fetch_u = [&](int blk) __attribute__((always_inline)) {
-            const auto r = buffer_of(Ut + ((slot_of(blk) * 4 + w) * NK + 2 * blockIdx.y) * 256);
+    if (wave < 4) {
+        // ================= the chain: D, and the state =================
+        __builtin_amdgcn_s_setprio(1);   // the other waves' work is wanted a block later
+        const bool owner = w < NS;       // of columns 32w .. 32w+31 of the state
+        float *srow = ssm + ((size_t)vh * DV + row0 + m) * DK + 32 * (owner ? w : 0) + 4 * g;
+        wy_f32x4 st[2][2];               // [row group][column tile]
 #pragma unroll
-            for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(r, rg));
+        for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) st[rg][ct] = load_v4(srow + 16 * rg * DK + 16 * ct);
+        auto publish_state = [&](int buf) __attribute__((always_inline)) {
+            float mx[2];
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) {
+                mx[rg] = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) mx[rg] = fmaxf(fmaxf(mx[rg], fabsf(st[rg][0][i])), fabsf(st[rg][1][i]));
+            }
+            rows_max2(mx[0], mx[1]);
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) {
+                float sc, un;
+                wy_scale(mx[rg], sc, un);
+                const u32x4 a = wy_split4(st[rg][0][0], st[rg][0][1], st[rg][0][2], st[rg][0][3], sc);
+                const u32x4 b = wy_split4(st[rg][1][0], st[rg][1][1], st[rg][1][2], st[rg][1][3], sc);
+                s_s[buf][rg][w][0][lane] = u32x4{a[0], a[1], b[0], b[1]};
+                s_s[buf][rg][w][1][lane] = u32x4{a[2], a[3], b[2], b[3]};
+                if (g == 0) s_su[buf][rg][w][m] = un;
+            }
         };
-        auto fetch_el = [&](int blk) __attribute__((always_inline)) {
-            el = __builtin_bit_cast(wy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(eLc + slot_of(blk) * kC + 16 * w), g * 16, 0, 0));
+        u32x4 kd[2][4];
+        wy_f32x4 pu[2];
+        float elc;
+        auto u_of = [&](int blk) { return buffer_of(Ut + ((slot_of(blk) * 4 + w) * NK + 2 * blockIdx.y) * 256); };
+        auto k_of = [&](int blk) { return buffer_of(Kt + (slot_of(blk) * NK + 2 * (owner ? w : 0)) * 4 * 64); };
+        auto fetch_elc = [&](int blk) __attribute__((always_inline)) {
+            elc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(eLc + slot_of(blk) * kC + kC - 1), 0, 0, 0));
         };
+        fetch_all_w(Wt);
+        {
+            const auto ru = u_of(0), rk = k_of(0);
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(ru, rg));
+            fetch_elc(0);
+#pragma unroll
+            for (int tau = 0; tau < 4; tau++)
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) kd[ct][tau] = load(rk, 4 * ct + tau);
+        }
+        if (owner) publish_state(0);
+        __syncthreads();
+        for (int blk = 0; blk < nblk; blk++) {
+            // ---- D = U - W S0^T: lane (n, g) holds tokens 16w+4g+i of state row n of the group ----
+            wy_f32x4 p[2];
+            times_state(Wt, blk, p);
+            const wy_f32x4 d[2] = {pu[0] - p[0], pu[1] - p[1]};
+            const auto ru = u_of(blk + 1);
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(ru, rg));
+            float mx[2];
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++)
+                mx[rg] = fmaxf(fmaxf(fabsf(d[rg][0]), fabsf(d[rg][1])), fmaxf(fabsf(d[rg][2]), fabsf(d[rg][3])));
+            rows_max2(mx[0], mx[1]);
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++) {
+                float sc, un;
+                wy_scale(mx[rg], sc, un);
+                const u32x4 x = wy_split4(d[rg][0], d[rg][1], d[rg][2], d[rg][3], sc);
+                s_d[blk & 1][rg][w][0][lane] = u32x4{x[0], x[1], x[0], x[1]};
+                s_d[blk & 1][rg][w][1][lane] = u32x4{x[2], x[3], x[2], x[3]};
+                if (g == 0) s_du[blk & 1][rg][w][m] = un;
+            }
+            __syncthreads();
+            // ---- S' = e^{L_C} S0 + D^T diag(e^{L_C-L}) K, this wave's columns ------
+            if (owner) {
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                    for (int ct = 0; ct < 2; ct++) st[rg][ct] *= elc;
+                const auto rk = k_of(blk + 1);
+                fetch_elc(blk + 1);
+                u32x4 dh[4][2], dl[4][2];
+                float un[4][2];
+#pragma unroll
+                for (int tau = 0; tau < 4; tau++)
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) dl[tau][rg] = s_d[blk & 1][rg][tau][1][lane], dh[tau][rg] = s_d[blk & 1][rg][tau][0][lane];
+#pragma unroll
+                for (int tau = 0; tau < 4; tau++)
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) un[tau][rg] = s_du[blk & 1][rg][tau][m];
+                __builtin_amdgcn_sched_barrier(0);
+                const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int th = 0; th < 4; th += 2) {
+                    wy_f32x4 acc[2][2][2];
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                            for (int ct = 0; ct < 2; ct++) acc[t][rg][ct] = wy_mfma(kd[ct][th + t], dl[th + t][rg], zero);
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                            for (int ct = 0; ct < 2; ct++) acc[t][rg][ct] = wy_mfma(kd[ct][th + t], dh[th + t][rg], acc[t][rg][ct]);
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+#pragma unroll
+                        for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                            for (int ct = 0; ct < 2; ct++) st[rg][ct] = wy_fma(acc[t][rg][ct], un[th + t][rg], st[rg][ct]);
+#pragma unroll
+                        for (int ct = 0; ct < 2; ct++) kd[ct][th + t] = load(rk, 4 * ct + th + t);
+                    }
+                }
+                publish_state((blk + 1) & 1);
+            }
+            __syncthreads();
+        }
+        __syncthreads();   // the other waves' last block
+        if (owner) {
+#pragma unroll
+            for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) *reinterpret_cast<wy_f32x4 *>(srow + 16 * rg * DK + 16 * ct) = st[rg][ct];
+        }
+    } else {
+        // ================= O = diag(e^L) q^ S0^T + M D, a block behind =================
+        u32x4 mt[4];
+        wy_f32x4 el;
         auto fetch_m = [&](int blk) __attribute__((always_inline)) {
             const auto r = buffer_of(Mt + (slot_of(blk) * 4 + w) * 4 * 64);
 #pragma unroll
             for (int tau = 0; tau < 4; tau++) mt[tau] = load(r, tau <= w ? tau : w);
         };
-        auto fetch_k = [&](int blk) __attribute__((always_inline)) {
-            const size_t slot = slot_of(blk);
-            const auto r = buffer_of(Kt + (slot * NK + 2 * (owner ? w : 0)) * 4 * 64);
-            elc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(eLc + slot * kC + kC - 1), 0, 0, 0));
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                for (int tau = 0; tau < 4; tau++) kd[ct][tau] = load(r, 4 * ct + tau);
+        auto fetch_el = [&](int blk) __attribute__((always_inline)) {
+            el = __builtin_bit_cast(wy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(eLc + slot_of(blk) * kC + 16 * w), g * 16, 0, 0));
         };
-        // O of block blk = (what diag(e^L) q^ S0^T left in o) + M D
-        auto finish_o = [&](int blk) __attribute__((always_inline)) {
-            const u32x4(*sd)[4][2][64] = s_d[blk & 1];
-            const float(*du)[4][16] = s_du[blk & 1];
+        const int stride = Hv * DV;
+        fetch_all_w(Qt);
+        fetch_el(0);
+        fetch_m(0);
+        __syncthreads();
+        __syncthreads();
+        __syncthreads();   // block 0: its D and the state behind it are there
+        for (int blk = 0; blk < nblk; blk++) {
+            wy_f32x4 o[2];
+            times_state(Qt, blk, o);
+            o[0] *= el;
+            o[1] *= el;
+            fetch_el(blk + 1);
+            __syncthreads();   // the state of this block may be written over
+            // (tiles past the diagonal repeat the last one; their products are left out of the sum)
+            u32x4 dh[4][2], dl[4][2];
+            float un[4][2];
+#pragma unroll
+            for (int tau = 0; tau < 4; tau++)
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++) dl[tau][rg] = s_d[blk & 1][rg][tau][1][lane], dh[tau][rg] = s_d[blk & 1][rg][tau][0][lane];
+#pragma unroll
+            for (int tau = 0; tau < 4; tau++)
+#pragma unroll
+                for (int rg = 0; rg < 2; rg++) un[tau][rg] = s_du[blk & 1][rg][tau][m];
+            __builtin_amdgcn_sched_barrier(0);
+            const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+            wy_f32x4 acc[4][2];
 #pragma unroll
             for (int tau = 0; tau < 4; tau++)
                 if (tau <= w) {
 #pragma unroll
-                    for (int rg = 0; rg < 2; rg++) {
-                        wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                        acc = wy_mfma(mt[tau], sd[rg][tau][1][lane], acc);
-                        acc = wy_mfma(mt[tau], sd[rg][tau][0][lane], acc);
-                        o[rg] += acc * du[rg][tau][m];
-                    }
+                    for (int rg = 0; rg < 2; rg++) acc[tau][rg] = wy_mfma(mt[tau], dl[tau][rg], zero);
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) acc[tau][rg] = wy_mfma(mt[tau], dh[tau][rg], acc[tau][rg]);
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) o[rg] = wy_fma(acc[tau][rg], un[tau][rg], o[rg]);
                 }
-            const int rows = T - (blk * kC + 16 * w) - 4 * g;   // tokens from this lane's first on
+            fetch_m(blk + 1);
+            const int left = T - (blk * kC + 16 * w) - 4 * g;   // tokens from this lane's first on
             float *dst = o_raw + ((size_t)(blk * kC + 16 * w) * Hv + vh) * DV + row0;
-            const int stride = Hv * DV, off = 4 * g * stride + m;
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                if (i < rows) {
+                if (i < left) {
 #pragma unroll
-                    for (int rg = 0; rg < 2; rg++) dst[off + i * stride + 16 * rg] = o[rg][i];
+                    for (int rg = 0; rg < 2; rg++) dst[(4 * g + i) * stride + m + 16 * rg] = o[rg][i];
                 }
-        };
-        {
-            const auto r = w_of(0);
-#pragma unroll
-            for (int c = 0; c < NK; c++) pw[c] = load(r, c);
+            if (blk + 1 < nblk) __syncthreads();   // this block's D may be written over
         }
-        if (ROLE == 0) fetch_u(0);
-        else fetch_el(0);
-        fetch_k(0);
-        if (owner) publish_state();
-        __syncthreads();
-        for (int blk = 0; blk < nblk; blk++) {
-            // ---- W S0^T, or q^ S0^T, for this wave's 16 tokens ------------------------------
-            if constexpr (ROLE == 0) __builtin_amdgcn_s_setprio(1);
-            if constexpr (ROLE == 1) {
-                if (blk > 0) {
-                    finish_o(blk - 1);
-                }
-                fetch_m(blk);
-            }
-            wy_f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-            const auto r = w_of(blk + 1);
-#pragma unroll
-            for (int s = 0; s < NS; s++) {
-                const u32x4 a = pw[2 * s], b = pw[2 * s + 1];
-                const u32x4 hi = {a[0], a[1], b[0], b[1]}, lo = {a[2], a[3], b[2], b[3]};
-#pragma unroll
-                for (int rg = 0; rg < 2; rg++) {
-                    const u32x4 sh = s_s[rg][s][0][lane], sl = s_s[rg][s][1][lane];
-                    wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                    acc = wy_mfma(lo, sh, acc);
-                    acc = wy_mfma(hi, sl, acc);
-                    acc = wy_mfma(hi, sh, acc);
-                    p[rg] += acc * s_su[rg][s][m];
-                }
-                pw[2 * s] = load(r, 2 * s);
-                pw[2 * s + 1] = load(r, 2 * s + 1);
-            }
-            if constexpr (ROLE == 0) {
-                // ---- D = U - W S0^T: lane (n, g) holds tokens 16w+4g+i of state row n of the group ----
-                const wy_f32x4 d[2] = {pu[0] - p[0], pu[1] - p[1]};
-                fetch_u(blk + 1);
-#pragma unroll
-                for (int rg = 0; rg < 2; rg++) {
-                    float sc, un;
-                    wy_scale(rows_max(fmaxf(fmaxf(fabsf(d[rg][0]), fabsf(d[rg][1])), fmaxf(fabsf(d[rg][2]), fabsf(d[rg][3])))), sc, un);
-                    const u32x4 x = wy_split4(d[rg][0] * sc, d[rg][1] * sc, d[rg][2] * sc, d[rg][3] * sc);
-                    s_d[blk & 1][rg][w][0][lane] = u32x4{x[0], x[1], x[0], x[1]};
-                    s_d[blk & 1][rg][w][1][lane] = u32x4{x[2], x[3], x[2], x[3]};
-                    if (g == 0) s_du[blk & 1][rg][w][m] = un;
-                }
-            } else {
-#pragma unroll
-                for (int rg = 0; rg < 2; rg++) o[rg] = el * p[rg];
-                fetch_el(blk + 1);
-            }
-            __syncthreads();
-            // ---- S' = e^{L_C} S0 + D^T diag(e^{L_C-L}) K, this wave's columns and rows ------
-            if (owner) {
-#pragma unroll
-                for (int ct = 0; ct < 2; ct++) st[ct] *= elc;
-#pragma unroll
-                for (int tau = 0; tau < 4; tau++) {
-                    const u32x4 dh = s_d[blk & 1][rgu][tau][0][lane], dl = s_d[blk & 1][rgu][tau][1][lane];
-                    const float un = s_du[blk & 1][rgu][tau][m];
-#pragma unroll
-                    for (int ct = 0; ct < 2; ct++) {
-                        wy_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                        acc = wy_mfma(kd[ct][tau], dl, acc);
-                        acc = wy_mfma(kd[ct][tau], dh, acc);
-                        st[ct] += acc * un;
-                    }
-                }
-                publish_state();
-                fetch_k(blk + 1);
-            }
-            __syncthreads();
-        }
-        if constexpr (ROLE == 1) finish_o(nblk - 1);
-    };
-    if (rgu == 0) run(std::integral_constant<int, 0>{});
-    else run(std::integral_constant<int, 1>{});
-    if (owner) {
-#pragma unroll
-        for (int ct = 0; ct < 2; ct++) *reinterpret_cast<wy_f32x4 *>(srow + 16 * ct) = st[ct];
     }
 }
 
