@@ -268,10 +268,11 @@ int launch_sdpa_merge(hipStream_t stream, const SdpaWorkspace &ws, int splits, i
                       int n_tok, const float *gate, float *out);
 // mla_sdpa.hip: one query token of H heads against a latent cache [L, R] + rotary keys [L, P].
 struct MlaPlan {
-    int splits;     // workgroups along the cache
-    int bps;        // 16-position blocks per split
-    int nhg;        // 16-head groups
-    int nwg_heads;  // workgroups along the heads (4 groups each)
+    int splits;      // workgroups along the cache
+    int per_split;   // positions of a split
+    int nhg;         // 16-head groups
+    int head_tiles;  // of which a workgroup serves this many (4: the streaming kernel)
+    int groups;      // workgroups along the heads
 };
 bool mla_shape_supported(int kv_lora_rank, int qk_rope_head_dim);
 MlaPlan mla_plan(int H, int L, int num_cus, int forced_splits = 0);

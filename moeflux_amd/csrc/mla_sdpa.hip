@@ -4,14 +4,30 @@
 // Per head h:  s[t] = (q'[h] . latent[t] + q_pe[h] . rope_k[t]) * scale,  w = softmax(s),
 //              out[h] = sum_t w[t] latent[t].
 // Every head reads the same keys ([latent | rope_k], R + P wide) and the same values
-// (latent): the heads are the free dimension of both products, so they form the N side
-// of MFMA tiles and the cache is read once per 64 heads instead of once per head.
+// (latent): the heads are the free dimension of both products, so they form one side of
+// the MFMA tiles and a workgroup reads its positions once for all of its heads.
 //
 // Both products run on the bf16 matrix pipeline at f32-like accuracy: every f32 operand x
 // is split into bf16 parts hi = bf16(x), lo = bf16(x - hi)  (x = hi + lo to 2^-18 x), and a
 // product a b is evaluated as a_hi b_hi + a_hi b_lo + a_lo b_hi with f32 accumulation.
 //
-//   mla_partial_kernel<R, P>   grid (splits, ceil(H / 64)); 8 waves in two roles.  Wave hg
+// Two kernels (mla_plan chooses); partials (unnormalised O, running max and sum per head) go to the workspace in the
+// layout of the decode kernel's partials, and sdpa_merge_kernel combines them.
+//
+//   mla_rounds_kernel<NHT>   a workgroup (8 waves) serves 16 NHT heads and walks its share of the cache in rounds of 128
+//     positions, each in two phases:
+//       scores   a wave owns 16 positions of the round and forms their scores against every head of the workgroup: keys
+//                come from memory in whole lines and change lanes through 4 KiB of the wave's own LDS (mla_operands); the queries,
+//                split once per workgroup, are B operands in LDS;
+//       values   a wave owns 64 channels: lane (n, g) reads channels 4 n .. 4 n + 3 of positions 4 g + e and 16 + 4 g + e
+//                (256 contiguous bytes per row), so that the four channels are B operands of four tiles and no value is ever
+//                transposed; the probabilities are A operands in LDS, in exactly the registers the scores left them in.
+//     Nothing passes between waves but the rows' maxima and the probabilities: two barriers a round.  For caches of few rounds:
+//     its workgroups start 3 us sooner than the other kernel's, and with 16 or 32 heads each they leave a half or a quarter of the
+//     partials.  It converts each row twice per workgroup, so that with more than
+//     three rounds the vector ALU (10 k of a round's 19 k clocks at 32 heads) costs more than that saves.
+//
+//   mla_stream_kernel<R, P>   grid (splits, ceil(H / 64)); 8 waves in two roles.  Wave hg
 //     (0..3) computes the scores and the softmax of head group hg, wave 4 + hg accumulates
 //     that group's values; the two share a SIMD and run one block apart, so that one of
 //     them always has matrix work while the other converts, exponentiates or stores:
@@ -34,13 +50,267 @@
 //     The value waves fetch and split 6 of a block's 16 latent rows (two channels per
 //     thread), the score waves the other 10 and the rotary keys: the split at which the call is
 //     fastest (12 / 4, which evens out the clocks the two roles spend per block, is 4 % slower).
-//     Partials (unnormalised O, running max and sum per head) go to the workspace in the
-//     layout of the decode kernel's partials, and sdpa_merge_kernel combines them.
+#include <algorithm>
+
 #include "sdpa_wave.h"
 
 namespace mfa {
 
 __device__ inline f32x4 mla_load4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+
+static constexpr int kMlaWaves = 8;
+
+// hi and lo operand halves of eight values
+__device__ inline void mla_split8(const f32x4 &a, const f32x4 &b, bf16x8 &hi, bf16x8 &lo) {
+    uint4 h, l;
+    split_pair(a[0], a[1], h.x, l.x);
+    split_pair(a[2], a[3], h.y, l.y);
+    split_pair(b[0], b[1], h.z, l.z);
+    split_pair(b[2], b[3], h.w, l.w);
+    hi = as_bf16x8(h);
+    lo = as_bf16x8(l);
+}
+
+// 16 rows x 64 channels, read as four requests of four rows (256 contiguous bytes each: lane l has channels 4 (l % 16) .. + 3 of row
+// 4 r + l / 16), as the operands of two 32-channel steps: step k takes channels 32 k + 8 g .. + 7 of row n into lane (n, g).  They
+// change lanes through 4 KiB of LDS of the wave's own (LDS executes a wave's instructions in order: no barrier).  Requested in
+// operand order instead, neighbouring lanes in different rows, a request takes 49 clocks of the CU's 16; exchanged by DPP selects
+// (32 for the 16 values a lane holds) these cost 20 clocks each as soon as a SIMD has two waves.
+static constexpr int kMlaRow = 68;   // floats from row to row: 16 neighbouring lanes then read 16 different groups of four banks
+__device__ inline void mla_operands(const f32x4 (&x)[4], float *buf, int lane, bf16x8 (&hi)[2], bf16x8 (&lo)[2]) {
+    const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int r = 0; r < 4; r++) *reinterpret_cast<f32x4 *>(buf + (4 * r + g) * kMlaRow + 4 * n) = x[r];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const float *at = buf + n * kMlaRow + 32 * k + 8 * g;
+        mla_split8(mla_load4(at), mla_load4(at + 4), hi[k], lo[k]);
+    }
+}
+
+// Workgroup id -> (split, head group).  Workgroups go to the 8 XCDs in turn; those of one split read the same rows and sit on
+// one XCD, one after the other, so that the rows come through its L2 once.
+template <int NHT>
+__global__ __launch_bounds__(kMlaWaves * 64, 2) void mla_rounds_kernel(
+    const float *__restrict__ q_prime, const float *__restrict__ q_pe, const float *__restrict__ latent,
+    const float *__restrict__ rope_k, int H, int L, int nsplit, int ngroups, int per_split, float qscale,
+    float *__restrict__ part_o, float *__restrict__ part_ml) {
+    constexpr int R = 512, P = 64;
+    constexpr int NS = (R + P) / 64, NSL = R / 64;   // 64-channel steps of the scores; of which latent
+    constexpr int HW = 16 * NHT;                     // heads of a workgroup
+    constexpr int WPOS = 16, ROUND = kMlaWaves * WPOS;   // positions of a wave, of a round
+    constexpr int D = 2;                             // steps of keys in flight
+    __shared__ uint4 sq[2 * NS][NHT][2][64];         // queries [32 channels][head tile][hi|lo], operand order
+    __shared__ uint4 sp[ROUND / 32][NHT][2][64];     // probabilities [32 positions][head tile][hi|lo], operand order
+    __shared__ __attribute__((aligned(16))) float smax[HW][kMlaWaves];
+    __shared__ float ssum[kMlaWaves][HW];
+    __shared__ __attribute__((aligned(16))) float kbuf[kMlaWaves][16 * kMlaRow];   // see mla_operands
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    float *buf = kbuf[wave];
+    const int id = blockIdx.x, xi = id >> 3;
+    const int split = (xi / ngroups) * 8 + (id & 7), group = xi % ngroups;
+    if (split >= nsplit) return;   // uniform over the workgroup, ahead of every barrier
+    const int h0 = group * HW;
+    const int p0 = split * per_split, p1 = min(p0 + per_split, L);   // p0 < p1: the plan has no empty split
+
+    // queries: 16 heads x 64 channels per unit, split into LDS
+    {
+        constexpr int NU = (NS * NHT + kMlaWaves - 1) / kMlaWaves;
+        f32x4 x[NU][4];
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            const int u = min(wave + kMlaWaves * i, NS * NHT - 1), s = u / NHT, ht = u % NHT;
+            const float *base = s < NSL ? q_prime + 64 * s : q_pe;
+            const int width = s < NSL ? R : P;
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[i][r] = mla_load4(base + ((unsigned)min(h0 + 16 * ht + 4 * r + g, H - 1) * width + 4 * n));
+        }
+#pragma unroll
+        for (int i = 0; i < NU; i++) {
+            const int u = min(wave + kMlaWaves * i, NS * NHT - 1), s = u / NHT, ht = u % NHT;
+            bf16x8 hi[2], lo[2];
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[i][r] *= qscale;
+            mla_operands(x[i], buf, lane, hi, lo);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                sq[2 * s + k][ht][0][lane] = __builtin_bit_cast(uint4, hi[k]);
+                sq[2 * s + k][ht][1][lane] = __builtin_bit_cast(uint4, lo[k]);
+            }
+        }
+    }
+
+    f32x4 o[4][NHT];   // lane (channel slot n, g): heads 16 ht + 4 g + i, channel 64 wave + 4 n + j
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int ht = 0; ht < NHT; ht++) o[j][ht] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run[NHT], l_run[NHT];   // of head 16 ht + n: maximum over everything seen, this lane's part of the sum
+#pragma unroll
+    for (int ht = 0; ht < NHT; ht++) m_run[ht] = neg_inf(), l_run[ht] = 0.f;
+
+    f32x4 kr[D][4];
+    // step s of the keys of the round that starts at r0 (rows past the cache's end: its last one, masked below)
+    auto fetch_k = [&](int r0, int s) __attribute__((always_inline)) {
+        const float *base = s < NSL ? latent + (size_t)r0 * R + 64 * s : rope_k + (size_t)r0 * P;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const unsigned row = min(WPOS * wave + 4 * r + g, L - 1 - r0);
+            kr[s % D][r] = mla_load4(base + (row * (s < NSL ? R : P) + 4 * n));
+        }
+    };
+    f32x4 vr[2][8];
+    auto fetch_v = [&](int r0, int ks, int slot) __attribute__((always_inline)) {
+        const float *base = latent + (size_t)r0 * R;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const unsigned row = min(32 * ks + (e < 4 ? 4 * g + e : 12 + 4 * g + e), L - 1 - r0);
+            vr[slot][e] = mla_load4(base + (row * R + 64 * wave + 4 * n));
+        }
+    };
+    bool mine = p0 + WPOS * wave < p1;   // whether the wave has positions in the round
+    if (mine) {
+#pragma unroll
+        for (int s = 0; s < D; s++) fetch_k(p0, s);
+    }
+    __syncthreads();
+
+    for (int r0 = p0; r0 < p1; r0 += ROUND) {
+        const int npos = min(p1 - r0, ROUND);
+        const int pairs = (npos + 63) / 64;   // of 32-position steps of the values
+        // ---- scores ---------------------------------------------------------------------------------------------
+        f32x4 sc[NHT];   // rows = positions 4 g + i, column = head n (log2 units)
+        if (mine) {
+#pragma unroll
+            for (int ht = 0; ht < NHT; ht++) sc[ht] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                bf16x8 kh[2], kl[2];
+                mla_operands(kr[s % D], buf, lane, kh, kl);
+                if (s + D < NS) fetch_k(r0, s + D);
+                if (s == NS - D) fetch_v(r0, 0, 0);
+                if (s == NS - D + 1) fetch_v(r0, 1, 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+#pragma unroll
+                    for (int ht = 0; ht < NHT; ht++) {
+                        const bf16x8 qh = as_bf16x8(sq[2 * s + k][ht][0][lane]), ql = as_bf16x8(sq[2 * s + k][ht][1][lane]);
+                        sc[ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl[k], qh, sc[ht], 0, 0, 0);
+                        sc[ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[k], ql, sc[ht], 0, 0, 0);
+                        sc[ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh[k], qh, sc[ht], 0, 0, 0);
+                    }
+            }
+#pragma unroll
+            for (int ht = 0; ht < NHT; ht++) {
+                float mb = neg_inf();
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (r0 + WPOS * wave + 4 * g + i >= p1) sc[ht][i] = neg_inf();
+                    mb = fmaxf(mb, sc[ht][i]);
+                }
+                mb = rows_max(mb);
+                if (g == 0) smax[16 * ht + n][wave] = mb;
+            }
+        } else {
+            fetch_v(r0, 0, 0);
+            fetch_v(r0, 1, 1);
+#pragma unroll
+            for (int ht = 0; ht < NHT; ht++) {
+                sc[ht] = f32x4{neg_inf(), neg_inf(), neg_inf(), neg_inf()};
+                if (g == 0) smax[16 * ht + n][wave] = neg_inf();
+            }
+        }
+        __syncthreads();
+        // ---- probabilities ----------------------------------------------------------------------------------------
+        float alpha[NHT];
+#pragma unroll
+        for (int ht = 0; ht < NHT; ht++) {
+            const f32x4 a = mla_load4(&smax[16 * ht + n][0]), b = mla_load4(&smax[16 * ht + n][4]);
+            const float m = fmaxf(m_run[ht], fmaxf(fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3])), fmaxf(fmaxf(b[0], b[1]), fmaxf(b[2], b[3]))));
+            alpha[ht] = fast_exp2(m_run[ht] - m);   // 0 in the first round
+            m_run[ht] = m;
+            float p[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[i] = fast_exp2(sc[ht][i] - m);
+            l_run[ht] = l_run[ht] * alpha[ht] + ((p[0] + p[1]) + (p[2] + p[3]));
+            uint2 ph, pl;
+            split_pair(p[0], p[1], ph.x, pl.x);
+            split_pair(p[2], p[3], ph.y, pl.y);
+            reinterpret_cast<uint2 *>(&sp[wave >> 1][ht][0][lane])[wave & 1] = ph;
+            reinterpret_cast<uint2 *>(&sp[wave >> 1][ht][1][lane])[wave & 1] = pl;
+        }
+        if (r0 != p0) {
+#pragma unroll
+            for (int ht = 0; ht < NHT; ht++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float a = __shfl(alpha[ht], 4 * g + i, 64);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) o[j][ht][i] *= a;
+                }
+        }
+        __syncthreads();
+        // ---- values -------------------------------------------------------------------------------------------------
+        auto accumulate = [&](int ks, int slot) __attribute__((always_inline)) {
+            bf16x8 vh[4], vl[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                mla_split8(f32x4{vr[slot][0][j], vr[slot][1][j], vr[slot][2][j], vr[slot][3][j]},
+                           f32x4{vr[slot][4][j], vr[slot][5][j], vr[slot][6][j], vr[slot][7][j]}, vh[j], vl[j]);
+            if (ks + 2 < 2 * pairs) fetch_v(r0, ks + 2, slot);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ht = 0; ht < NHT; ht++) {
+                const bf16x8 ph = as_bf16x8(sp[ks][ht][0][lane]), pl = as_bf16x8(sp[ks][ht][1][lane]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    o[j][ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vl[j], o[j][ht], 0, 0, 0);   // (without it the result is 5 % further off)
+                    o[j][ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vl[j], o[j][ht], 0, 0, 0);
+                    o[j][ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vh[j], o[j][ht], 0, 0, 0);
+                    o[j][ht] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vh[j], o[j][ht], 0, 0, 0);
+                }
+            }
+        };
+        const int next = r0 + ROUND;
+        for (int pr = 0; pr + 1 < pairs; pr++) {
+            accumulate(2 * pr, 0);
+            accumulate(2 * pr + 1, 1);
+        }
+        mine = next + WPOS * wave < p1;
+        if (mine) {
+#pragma unroll
+            for (int s = 0; s < D; s++) fetch_k(next, s);
+        }
+        accumulate(2 * pairs - 2, 0);
+        accumulate(2 * pairs - 1, 1);
+    }
+
+    // ---- partials ------------------------------------------------------------------------------------------------------
+#pragma unroll
+    for (int ht = 0; ht < NHT; ht++) {
+        const float l = rows_sum(l_run[ht]);
+        if (g == 0) ssum[wave][16 * ht + n] = l;
+        if (h0 + 16 * ht < H) {
+            const size_t pid = (size_t)(group * NHT + ht) * nsplit + split;
+            float *po = part_o + (pid * 16 + 4 * g) * R + 64 * wave + 4 * n;
+#pragma unroll
+            for (int i = 0; i < 4; i++) *reinterpret_cast<f32x4 *>(po + i * R) = f32x4{o[0][ht][i], o[1][ht][i], o[2][ht][i], o[3][ht][i]};
+            if (wave == 0 && g == 0) part_ml[pid * 32 + n] = m_run[ht];
+        }
+    }
+    __syncthreads();
+    if (tid < HW && h0 + (tid & ~15) < H) {
+        float l = 0.f;
+#pragma unroll
+        for (int w = 0; w < kMlaWaves; w++) l += ssum[w][tid];
+        part_ml[((size_t)(group * NHT + tid / 16) * nsplit + split) * 32 + 16 + (tid & 15)] = l;
+    }
+}
+
 __device__ inline f32x2 mla_load2(const float *p) { return *reinterpret_cast<const f32x2 *>(p); }
 __device__ inline bf16x8 mla_lds8(const void *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
@@ -57,7 +327,7 @@ static constexpr int kMlaHG = 4;      // 16-head groups per workgroup
 static constexpr float kMlaLazy = 8.f;
 
 template <int R, int P>
-__global__ __launch_bounds__(kMlaHG * 128) void mla_partial_kernel(
+__global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
     const float *__restrict__ q_prime, const float *__restrict__ q_pe, const float *__restrict__ latent,
     const float *__restrict__ rope_k, int H, int L, int blocks_per_split, float qscale,
     float *__restrict__ part_o, float *__restrict__ part_ml) {
@@ -130,22 +400,29 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_partial_kernel(
             }
         };
         fetch(b0);
-        // the 16 queries as B operands: lane (n, g) holds head n, channels 32 s + 8 g .. + 7 of [q' | q_pe]
+        // the 16 queries as B operands: lane (n, g) holds head n, channels 32 s + 8 g .. + 7 of [q' | q_pe].  Read row by row in whole
+        // lines and exchanged through LDS, three 64-channel steps at a time (requested in operand order they took 3 us of the launch).
         bf16x8 qh[NS], ql[NS];
         {
-            const int head = min(hg * 16 + n, H - 1);
+            static_assert(kMlaHG * 16 * kMlaRow * 4 <= KBUF, "the exchange buffers fit one block buffer");
+            float *buf = reinterpret_cast<float *>(smem + 2 * KBUF) + hgl * 16 * kMlaRow;   // block b0 + 2 is written after the barriers below
+            f32x4 x[3][4];
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                const int c0 = 32 * s + 8 * g;
-                const float *src = (c0 < R) ? q_prime + (size_t)head * R + c0 : q_pe + (size_t)head * P + (c0 - R);
-                const f32x4 a = mla_load4(src) * qscale, b = mla_load4(src + 4) * qscale;
-                uint4 hi, lo;
-                split_pair(a[0], a[1], hi.x, lo.x);
-                split_pair(a[2], a[3], hi.y, lo.y);
-                split_pair(b[0], b[1], hi.z, lo.z);
-                split_pair(b[2], b[3], hi.w, lo.w);
-                qh[s] = as_bf16x8(hi);
-                ql[s] = as_bf16x8(lo);
+            for (int t = 0; t < DK / 64; t += 3) {
+#pragma unroll
+                for (int u = 0; u < 3; u++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const unsigned head = min(hg * 16 + 4 * r + g, H - 1);
+                        x[u][r] = (64 * (t + u) < R ? mla_load4(q_prime + 64 * (t + u) + (head * R + 4 * n)) : mla_load4(q_pe + (head * P + 4 * n))) * qscale;
+                    }
+#pragma unroll
+                for (int u = 0; u < 3; u++) {
+                    bf16x8 hi[2], lo[2];
+                    mla_operands(x[u], buf, lane, hi, lo);
+#pragma unroll
+                    for (int k = 0; k < 2; k++) qh[2 * (t + u) + k] = hi[k], ql[2 * (t + u) + k] = lo[k];
+                }
             }
         }
         float m_ref = neg_inf(), l_sum = 0.f;
@@ -277,19 +554,35 @@ bool mla_shape_supported(int kv_lora_rank, int qk_rope_head_dim) {
     return kv_lora_rank == 512 && qk_rope_head_dim == 64;
 }
 
-// Partition of the cache's blocks over workgroups: enough splits that every CU has a
-// workgroup, never more than there are blocks.
+// Partition of the heads and of the cache over workgroups, a workgroup per CU.  Which kernel (us a layer, one call after the
+// other / three sequences side by side, in brackets the streaming kernel with its queries read in operand order):
+//   rounds, 16 heads  where one round of 128 positions is enough: 128 heads over 200 positions 11.5 / 7.6 (17.0 / 8.4), 1500
+//                     14.8 / 11.1 (26.1 / 15.1), 4096 18.1 / 13.9 (27.7 / 20.9); 64 over 2000 14.5 / 10.8 (24.0 / 11.4), 8192 18.7 / 13.7
+//                     (28.8 / 22.6).  17 to 32 heads, whose two groups share an L2: up to three rounds, 32 over 32768 26.0 / 25.7
+//                     (33.8 / 28.9), 49000 33.9 / 36.0 (40.0 / 36.4).  Up to 16 heads, where nobody shares the second read of
+//                     the rows: up to 80 positions, 16 over 16384 19.9 / 15.2 (23.6 / 15.9), but 32768 32.0 / 24.8 (30.5 / 25.3)
+//   rounds, 32 heads  up to two rounds: 128 over 8192 24.3 / 18.5 (28.6 / 24.4), 16384 31.7 / 28.3 (34.0 / 32.6), but 24000
+//                     40.8 / 39.8 (41.5 / 39.4); 64 over 32768 33.8 / 31.3 (38.0 / 36.5)
+//   streaming, 64     beyond: 128 over 32768 45.5 / 47.4 (47.5 / 47.8)
 MlaPlan mla_plan(int H, int L, int num_cus, int forced_splits) {
     MlaPlan p;
     p.nhg = (H + 15) / 16;
-    p.nwg_heads = (p.nhg + kMlaHG - 1) / kMlaHG;
-    const int nblk = (L + kMlaBlk - 1) / kMlaBlk;
-    int splits = forced_splits > 0 ? forced_splits : (num_cus + p.nwg_heads - 1) / p.nwg_heads;
-    if (splits > nblk) splits = nblk;
-    if (splits > 1024) splits = 1024;
-    if (splits < 1) splits = 1;
-    p.bps = (nblk + splits - 1) / splits;
-    p.splits = (nblk + p.bps - 1) / p.bps;
+    auto rounds = [&](int tiles) {   // of a workgroup that serves `tiles` head groups
+        const int64_t groups = (p.nhg + tiles - 1) / tiles;
+        return (L * groups + 128 * (int64_t)num_cus - 1) / (128 * (int64_t)num_cus);
+    };
+    const bool few = p.nhg == 1 ? L <= 80 * (int64_t)num_cus : rounds(1) <= (p.nhg == 2 ? 3 : 1);
+    p.head_tiles = few ? 1 : p.nhg > 2 && rounds(2) <= 2 ? 2 : kMlaHG;
+    p.groups = (p.nhg + p.head_tiles - 1) / p.head_tiles;
+    // (rounded down for the rounds kernel: with 48 heads' three groups one workgroup too many would run alone)
+    int splits = forced_splits > 0 ? forced_splits : p.head_tiles == kMlaHG ? (num_cus + p.groups - 1) / p.groups : num_cus / p.groups;
+    splits = std::max(1, std::min(splits, 1024));
+    // whole blocks of 16 positions; a share of less than two leaves more partials than it saves time
+    const int blocks = (L + 15) / 16;
+    int per = (blocks + splits - 1) / splits;
+    if (forced_splits <= 0 && p.head_tiles < kMlaHG) per = std::max(per, 2);
+    p.per_split = 16 * per;
+    p.splits = (blocks + per - 1) / per;
     return p;
 }
 
@@ -305,8 +598,18 @@ int launch_mla_sdpa_folded(hipStream_t stream, int H, int R, int P, int L, float
     if (ws.part_o_elems < mla_workspace_o_elems(plan, R) || ws.part_ml_elems < mla_workspace_ml_elems(plan))
         return fail(MFA_ERR_INVALID, "latent attention: workspace too small for %d splits", plan.splits);
     const float qscale = softmax_scale * 1.4426950408889634f;  // scores in log2 units
-    hipLaunchKernelGGL((mla_partial_kernel<512, 64>), dim3(plan.splits, plan.nwg_heads), dim3(kMlaHG * 128), 0,
-                       stream, q_prime, q_pe, latent, rope_k, H, L, plan.bps, qscale, ws.part_o, ws.part_ml);
+    if (plan.head_tiles == kMlaHG) {
+        hipLaunchKernelGGL((mla_stream_kernel<512, 64>), dim3(plan.splits, plan.groups), dim3(kMlaHG * 128), 0,
+                           stream, q_prime, q_pe, latent, rope_k, H, L, plan.per_split / kMlaBlk, qscale, ws.part_o, ws.part_ml);
+    } else {
+        const dim3 grid((unsigned)((plan.splits + 7) / 8 * 8 * plan.groups));   // see mla_rounds_kernel: a split's workgroups on one XCD
+#define MFA_MLA(HT)                                                                                                \
+    hipLaunchKernelGGL((mla_rounds_kernel<HT>), grid, dim3(kMlaWaves * 64), 0, stream, q_prime, q_pe, latent, rope_k, \
+                       H, L, plan.splits, plan.groups, plan.per_split, qscale, ws.part_o, ws.part_ml)
+        if (plan.head_tiles == 1) MFA_MLA(1);
+        else MFA_MLA(2);
+#undef MFA_MLA
+    }
     MFA_HIP(hipGetLastError());
     return launch_sdpa_merge(stream, ws, plan.splits, /*hpk=*/H, /*Hq=*/H, plan.nhg, R, /*n_tok=*/1,
                              /*gate=*/nullptr, out);

@@ -129,6 +129,38 @@ def test_mla_size_independent_properties(mfa):
     assert rel_err(twice, half) <= TOL_F32
 
 
+@pytest.mark.parametrize("H,L", [(16, 33), (17, 127), (33, 129), (16, 20480), (16, 20481), (48, 9999), (128, 4096),
+                                 (128, 4097), (40, 16500), (128, 16384), (128, 16385), (30, 49152), (30, 49153)])
+def test_mla_kernels_at_their_borders(mfa, H, L):
+    """Both sides of every border between the kernels (16 heads a workgroup, 32, the streaming one: on 256 CUs 128 heads
+    change at 4096 and 16384 positions, 16 at 20480, 30 at 49152), ragged ends of a split, of a round and of a 32-position step, head counts that
+    leave a workgroup's last group empty; a maximum that rises from round to round (the last positions score highest).
+    Against float64: products of two-part operands leave 2^-17 of an operand's size, 4e-6 as measured over these
+    inputs, and the bar is the oracle's."""
+    qp, qe, lat, rk = _random(H + L, H, L)
+    lat *= np.linspace(0.2, 1.5, L, dtype=np.float32)[:, None]
+    scale = 1.0 / np.sqrt(192.0)
+    q, k = np.concatenate([qp, qe], 1).astype(np.float64), np.concatenate([lat, rk], 1).astype(np.float64)
+    s = (q @ k.T) * scale
+    w = np.exp(s - s.max(1, keepdims=True))
+    ref = (w / w.sum(1, keepdims=True)) @ lat.astype(np.float64)
+    out = mfa.mla_sdpa_folded(H, R, P, L, scale, qp, qe, lat, rk)
+    assert rel_err(out, ref.reshape(-1)) <= TOL_F32
+
+
+def test_mla_not_a_number_and_infinity_stay_in_their_heads(mfa):
+    """A query row that is not finite spoils its own head and no other of its tile; a row of the cache past the end is
+    never read into a result."""
+    H, L = 20, 200
+    qp, qe, lat, rk = _random(77, H, L)
+    clean = mfa.mla_sdpa_folded(H, R, P, L, 0.07, qp, qe, lat, rk).reshape(H, R)
+    qp[3, 5], qp[17, 0] = np.nan, np.inf
+    out = mfa.mla_sdpa_folded(H, R, P, L, 0.07, qp, qe, lat, rk).reshape(H, R)
+    others = [h for h in range(H) if h not in (3, 17)]
+    assert np.isnan(out[3]).all() and np.isnan(out[17]).all()
+    assert np.array_equal(out[others], clean[others])
+
+
 def test_mla_errors(mfa):
     from moeflux_amd import ffi
     lib = ffi.load()
