@@ -51,6 +51,7 @@
 //     thread), the score waves the other 10 and the rotary keys: the split at which the call is
 //     fastest (12 / 4, which evens out the clocks the two roles spend per block, is 4 % slower).
 #include <algorithm>
+#include <type_traits>
 
 #include "sdpa_wave.h"
 
@@ -325,6 +326,7 @@ __device__ inline mla_i16x4 mla_lds_tr(const unsigned char *p) {
 static constexpr int kMlaBlk = 16;    // positions per block
 static constexpr int kMlaHG = 4;      // 16-head groups per workgroup
 static constexpr float kMlaLazy = 8.f;
+static constexpr int kMlaMayMove = 0x2 | 0x4 | 0x10 | 0x200;   // sched_barrier: vector and scalar ALU, memory and LDS writes may cross
 
 template <int R, int P>
 __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
@@ -367,39 +369,42 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
     auto clampb =[&](int b) { return min(b, b1 - 1); };  // requests past the range repeat its last block; nobody reads them
     // block b lives in buffer (b - b0) % 3
     auto bufof =[&](int b) { return smem + ((b - b0) % 3) * KBUF; };
+    // A block's rows are requested two blocks before they are written to LDS, in two sets of registers, and 16 bytes a lane: with
+    // that and the operands read ahead of the products (below) 128 heads over 32768 positions take 43.7 us instead of 46.5.
+    // (Neither by itself gains: a block's 3.9 k clocks are 1.9 k of matrix time at a clock that the matrix load pulls down, 1 k of
+    // conversion and 1.4 k of LDS reads at least.  Tried and not kept: 32 heads a wave over half of the channels, half the LDS
+    // reads but a barrier more a block (50.2 us), either role's waves ahead of the other's by priority, 4 or 8 rows staged by the value waves.)
+    const int srow = rtid >> 7, scol = rtid & 127;   // 128 threads x 4 channels a latent row
+    const std::integral_constant<int, 0> zero{};
+    const std::integral_constant<int, 1> one{};
+    auto put4 = [&](unsigned char *at, const f32x4 &x) __attribute__((always_inline)) {
+        uint2 hi, lo;
+        split_pair(x[0], x[1], hi.x, lo.x);
+        split_pair(x[2], x[3], hi.y, lo.y);
+        *reinterpret_cast<uint2 *>(at) = hi;
+        *reinterpret_cast<uint2 *>(at + KPLANE) = lo;
+    };
 
     if (score_role) {
         // ================= scores and softmax of head group hgl =================
-        // staging: the rotary keys, two channels at positions rp and rp + 8, and the latent rows the value waves leave
-        const int rp = rtid >> 5, rc2 = rtid & 31;
-        f32x2 rraw[2], lraw[kMlaBlk - VPOS];
-        auto fetch =[&](int b) {
+        // staging: four channels of one rotary key, and of every second of the latent rows that the value waves leave
+        constexpr int NR = (kMlaBlk - VPOS) / 2;
+        f32x4 rraw[2], lraw[2][NR];   // [block % 2 from b0 + 1 on]
+        auto fetch =[&](int b, auto slot) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
+            rraw[S] = mla_load4(rope_k + (size_t)min(clampb(b) * kMlaBlk + (rtid >> 4), L - 1) * P + 4 * (rtid & 15));
 #pragma unroll
-            for (int k = 0; k < 2; k++)
-                rraw[k] = mla_load2(rope_k + (size_t)min(clampb(b) * kMlaBlk + rp + 8 * k, L - 1) * P + 2 * rc2);
-#pragma unroll
-            for (int j = VPOS; j < kMlaBlk; j++)
-                lraw[j - VPOS] = mla_load2(latent + (size_t)min(clampb(b) * kMlaBlk + j, L - 1) * R + 2 * rtid);
+            for (int j = 0; j < NR; j++)
+                lraw[S][j] = mla_load4(latent + (size_t)min(clampb(b) * kMlaBlk + VPOS + 2 * j + srow, L - 1) * R + 4 * scol);
         };
-        const int kr_off = (rp * KROW + R + 2 * rc2) * 2;
-        auto commit =[&](int b) {
+        auto commit =[&](int b, auto slot) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
             unsigned char *base = bufof(b);
+            put4(base + ((rtid >> 4) * KROW + R + 4 * (rtid & 15)) * 2, rraw[S]);
 #pragma unroll
-            for (int k = 0; k < 2; k++) {
-                uint32_t rh, rl;
-                split_pair(rraw[k][0], rraw[k][1], rh, rl);
-                *reinterpret_cast<uint32_t *>(base + kr_off + 8 * k * KROW * 2) = rh;
-                *reinterpret_cast<uint32_t *>(base + kr_off + 8 * k * KROW * 2 + KPLANE) = rl;
-            }
-#pragma unroll
-            for (int j = VPOS; j < kMlaBlk; j++) {   // the last latent rows of the block, channels 2 rtid, 2 rtid + 1
-                uint32_t hi, lo;
-                split_pair(lraw[j - VPOS][0], lraw[j - VPOS][1], hi, lo);
-                *reinterpret_cast<uint32_t *>(base + 4 * rtid + j * KROW * 2) = hi;
-                *reinterpret_cast<uint32_t *>(base + 4 * rtid + j * KROW * 2 + KPLANE) = lo;
-            }
+            for (int j = 0; j < NR; j++) put4(base + ((VPOS + 2 * j + srow) * KROW + 4 * scol) * 2, lraw[S][j]);
         };
-        fetch(b0);
+        fetch(b0, zero);
         // the 16 queries as B operands: lane (n, g) holds head n, channels 32 s + 8 g .. + 7 of [q' | q_pe].  Read row by row in whole
         // lines and exchanged through LDS, three 64-channel steps at a time (requested in operand order they took 3 us of the launch).
         bf16x8 qh[NS], ql[NS];
@@ -427,26 +432,43 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
         }
         float m_ref = neg_inf(), l_sum = 0.f;
         const int kr_rd = (n * KROW + 8 * g) * 2;   // [hi][position n][8 g]; lo at + KPLANE; step s at + 64 s
-        commit(b0);
-        fetch(b0 + 1);
+        commit(b0, zero);
+        fetch(b0 + 1, zero);
+        fetch(b0 + 2, one);
         __syncthreads();
         // iteration b0 - 1: block b0 is scored, nothing is accumulated yet; then one iteration per block
-        for (int it = b0 - 1; it < b1 - 1; it++) {
+        auto iteration = [&](int it, auto slot) __attribute__((always_inline)) {
             const int b = it + 1;   // the block scored in this iteration
             const unsigned char *base = bufof(b);
             f32x4 sc = {0.f, 0.f, 0.f, 0.f};  // rows = positions 4g + i, column = head n (log2 units)
+            // operands two to four steps ahead of the products (left alone the compiler reads them one step ahead, and every step
+            // waits for LDS); only matrix instructions and LDS reads keep their places
+            constexpr int GS = 2;
+            bf16x8 ah[2][GS], al[2][GS];
+            auto read_keys = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                const bf16x8 ah = mla_lds8(base + kr_rd + 64 * s);
-                const bf16x8 al = mla_lds8(base + kr_rd + 64 * s + KPLANE);
-                sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, qh[s], sc, 0, 0, 0);
-                sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, ql[s], sc, 0, 0, 0);
-                sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, qh[s], sc, 0, 0, 0);
+                for (int i = 0; i < GS; i++) {
+                    ah[q & 1][i] = mla_lds8(base + kr_rd + 64 * (GS * q + i));
+                    al[q & 1][i] = mla_lds8(base + kr_rd + 64 * (GS * q + i) + KPLANE);
+                }
+            };
+            static_assert(NS % GS == 0, "whole groups");
+            read_keys(0);
+#pragma unroll
+            for (int q = 0; q < NS / GS; q++) {
+                if (q + 1 < NS / GS) read_keys(q + 1);
+                __builtin_amdgcn_sched_barrier(kMlaMayMove);
+#pragma unroll
+                for (int i = 0; i < GS; i++) {
+                    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[q & 1][i], qh[GS * q + i], sc, 0, 0, 0);
+                    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q & 1][i], ql[GS * q + i], sc, 0, 0, 0);
+                    sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q & 1][i], qh[GS * q + i], sc, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(kMlaMayMove);
             }
-            // the rotary keys of block it + 2 (its buffer was accumulated from in the previous
-            // iteration); block it + 3 is requested
-            commit(it + 2);
-            fetch(it + 3);
+            // block it + 2 (its buffer was accumulated from in the previous iteration); block it + 4 is requested
+            commit(it + 2, slot);
+            fetch(it + 4, slot);
             {
                 const int pos0 = b * kMlaBlk + 4 * g;
 #pragma unroll
@@ -475,6 +497,10 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
                 if (g == 0) abuf[b & 1][hgl][n] = alpha;
             }
             __syncthreads();
+        };
+        for (int it = b0 - 1; it < b1 - 1; it += 2) {
+            iteration(it, zero);
+            if (it + 1 < b1 - 1) iteration(it + 1, one);
         }
         l_sum = rows_sum(l_sum);
         if (active && g == 0) {
@@ -484,23 +510,19 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
         __syncthreads();  // iteration b1 - 1: the value waves accumulate the last block
     } else {
         // ================= values of head group hgl =================
-        // staging: the latent rows, channels 2 c2, 2 c2 + 1 at the block's first VPOS positions
-        const int c2 = rtid;
-        f32x2 raw[VPOS];
-        auto fetch =[&](int b) {
+        // staging: four channels of every second of the block's first VPOS latent rows
+        f32x4 raw[2][VPOS / 2];
+        auto fetch =[&](int b, auto slot) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
 #pragma unroll
-            for (int j = 0; j < VPOS; j++)
-                raw[j] = mla_load2(latent + (size_t)min(clampb(b) * kMlaBlk + j, L - 1) * R + 2 * c2);
+            for (int j = 0; j < VPOS / 2; j++)
+                raw[S][j] = mla_load4(latent + (size_t)min(clampb(b) * kMlaBlk + 2 * j + srow, L - 1) * R + 4 * scol);
         };
-        auto commit =[&](int b) {
-            unsigned char *base = bufof(b) + 4 * c2;
+        auto commit =[&](int b, auto slot) __attribute__((always_inline)) {
+            constexpr int S = decltype(slot)::value;
+            unsigned char *base = bufof(b);
 #pragma unroll
-            for (int j = 0; j < VPOS; j++) {
-                uint32_t hi, lo;
-                split_pair(raw[j][0], raw[j][1], hi, lo);
-                *reinterpret_cast<uint32_t *>(base + j * KROW * 2) = hi;
-                *reinterpret_cast<uint32_t *>(base + j * KROW * 2 + KPLANE) = lo;
-            }
+            for (int j = 0; j < VPOS / 2; j++) put4(base + ((2 * j + srow) * KROW + 4 * scol) * 2, raw[S][j]);
         };
         f32x4 o[NT];
 #pragma unroll
@@ -510,17 +532,18 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
         // at positions 8 (g & 1) .. + 3 [+ 4]
         const bool hi_slots = g < 2;
         const int tr_rd = (hi_slots ? 0 : KPLANE) + ((8 * (g & 1) + (n >> 2)) * KROW + 4 * (n & 3)) * 2;
-        fetch(b0);
-        commit(b0);
-        fetch(b0 + 1);
+        fetch(b0, zero);
+        commit(b0, zero);
+        fetch(b0 + 1, zero);
+        fetch(b0 + 2, one);
         __syncthreads();
         // iteration b0 - 1: no weights yet
-        commit(b0 + 1);
-        fetch(b0 + 2);
+        commit(b0 + 1, zero);
+        fetch(b0 + 3, zero);
         __syncthreads();
-        for (int it = b0; it < b1; it++) {
-            commit(it + 2);    // its buffer held block it - 1
-            fetch(it + 3);
+        auto iteration = [&](int it, auto slot) __attribute__((always_inline)) {
+            commit(it + 2, slot);    // its buffer held block it - 1
+            fetch(it + 4, slot);
             const unsigned char *base = bufof(it) + tr_rd;
             // lane (n, g): weights of head n at positions 8 (g & 1) .. + 7
             const bf16x8 pb_h = mla_lds8(&pbuf[it & 1][hgl][0][n][8 * (g & 1)]);
@@ -530,16 +553,34 @@ __global__ __launch_bounds__(kMlaHG * 128) void mla_stream_kernel(
 #pragma unroll
                 for (int t = 0; t < NT; t++) o[t] *= alpha;
             }
+            // operands four tiles ahead of the products, as above
+            constexpr int GT = 4;
+            bf16x8 a[2][GT];
+            auto read_values = [&](int q) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const mla_i16x4 a0 = mla_lds_tr(base + 32 * t);
-                const mla_i16x4 a1 = mla_lds_tr(base + 32 * t + 4 * KROW * 2);
-                const mla_i16x8 a8 = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-                const bf16x8 a = __builtin_bit_cast(bf16x8, a8);
-                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb_l, o[t], 0, 0, 0);
-                o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb_h, o[t], 0, 0, 0);
+                for (int i = 0; i < GT; i++) {
+                    const mla_i16x4 a0 = mla_lds_tr(base + 32 * (GT * q + i));
+                    const mla_i16x4 a1 = mla_lds_tr(base + 32 * (GT * q + i) + 4 * KROW * 2);
+                    const mla_i16x8 a8 = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    a[q & 1][i] = __builtin_bit_cast(bf16x8, a8);
+                }
+            };
+            read_values(0);
+#pragma unroll
+            for (int q = 0; q < NT / GT; q++) {
+                if (q + 1 < NT / GT) read_values(q + 1);
+                __builtin_amdgcn_sched_barrier(kMlaMayMove);
+#pragma unroll
+                for (int i = 0; i < GT; i++) o[GT * q + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q & 1][i], pb_l, o[GT * q + i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < GT; i++) o[GT * q + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q & 1][i], pb_h, o[GT * q + i], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(kMlaMayMove);
             }
             __syncthreads();
+        };
+        for (int it = b0; it < b1; it += 2) {
+            iteration(it, one);
+            if (it + 1 < b1) iteration(it + 1, zero);
         }
         // o[t][i] is channel 16 t + 4g + i of head n
         if (active) {
@@ -563,7 +604,7 @@ bool mla_shape_supported(int kv_lora_rank, int qk_rope_head_dim) {
 //                     the rows: up to 80 positions, 16 over 16384 19.9 / 15.2 (23.6 / 15.9), but 32768 32.0 / 24.8 (30.5 / 25.3)
 //   rounds, 32 heads  up to two rounds: 128 over 8192 24.3 / 18.5 (28.6 / 24.4), 16384 31.7 / 28.3 (34.0 / 32.6), but 24000
 //                     40.8 / 39.8 (41.5 / 39.4); 64 over 32768 33.8 / 31.3 (38.0 / 36.5)
-//   streaming, 64     beyond: 128 over 32768 45.5 / 47.4 (47.5 / 47.8)
+//   streaming, 64     beyond: 128 over 32768 43.7 / 44.5 (47.9 / 48.7), 65536 76.5 / 74.7 (79.5 / 79.8)
 MlaPlan mla_plan(int H, int L, int num_cus, int forced_splits) {
     MlaPlan p;
     p.nhg = (H + 15) / 16;
