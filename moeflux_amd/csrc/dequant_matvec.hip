@@ -369,10 +369,10 @@ int launch_dequant_matvec_4bit(hipStream_t stream, int n, const uint32_t *const 
     (void)num_cus;
 #define MV_LAUNCH(W)                                                                                              \
     do {                                                                                                          \
-        if (sb16 && tiled) hipLaunchKernelGGL((dequant_matvec_mfma_kernel<W, true, true>), grid, dim3(W * 64), 0, stream, sp, tl);   \
-        else if (sb16) hipLaunchKernelGGL((dequant_matvec_mfma_kernel<W, true, false>), grid, dim3(W * 64), 0, stream, sp, tl);      \
-        else if (tiled) hipLaunchKernelGGL((dequant_matvec_mfma_kernel<W, false, true>), grid, dim3(W * 64), 0, stream, sp, tl);     \
-        else hipLaunchKernelGGL((dequant_matvec_mfma_kernel<W, false, false>), grid, dim3(W * 64), 0, stream, sp, tl);               \
+        if (sb16 && tiled) launch_kernel(dequant_matvec_mfma_kernel<W, true, true>, grid, dim3(W * 64), stream, sp, tl);   \
+        else if (sb16) launch_kernel(dequant_matvec_mfma_kernel<W, true, false>, grid, dim3(W * 64), stream, sp, tl);      \
+        else if (tiled) launch_kernel(dequant_matvec_mfma_kernel<W, false, true>, grid, dim3(W * 64), stream, sp, tl);     \
+        else launch_kernel(dequant_matvec_mfma_kernel<W, false, false>, grid, dim3(W * 64), stream, sp, tl);               \
     } while (0)
     if (max_in <= 1024) MV_LAUNCH(1);
     else if (max_in <= 2048) MV_LAUNCH(2);

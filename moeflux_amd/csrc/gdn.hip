@@ -376,7 +376,7 @@ int launch_gdn_step(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float 
                     Hv, dk, dv, K);
     const int slot_new = (int)(step % K);
 #define MFA_GDN(DKK, KCC)                                                                       \
-    hipLaunchKernelGGL((gdn_step_kernel<DKK, DKK, KCC>), dim3(Hv, n_layers), dim3(DKK * 8), 0, s, Hk, Hv, K, eps, \
+    launch_kernel(gdn_step_kernel<DKK, DKK, KCC>, dim3(Hv, n_layers), dim3(DKK * 8), s, Hk, Hv, K, eps, \
                        w.conv_w, w.a_log, w.dt_bias, w.norm_w, conv_ring, slot_new, ssm, qkv_in, z,  \
                        alpha, beta, out)
     if (merge && merge->n_units > 0) {
@@ -385,7 +385,7 @@ int launch_gdn_step(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float 
         const int merge_rows = (merge->n_units + per_row - 1) / per_row;
         if (n_layers + merge_rows > 65535) return fail(MFA_ERR_INVALID, "gdn_step: bad layer count %d", n_layers);
 #define MFA_GDN_M(DKK, KCC)                                                                                       \
-    hipLaunchKernelGGL((gdn_step_merge_kernel<DKK, DKK, KCC>), dim3(Hv, merge_rows + n_layers), dim3(DKK * 8), 0, s, Hk, \
+    launch_kernel(gdn_step_merge_kernel<DKK, DKK, KCC>, dim3(Hv, merge_rows + n_layers), dim3(DKK * 8), s, Hk, \
                        Hv, K, eps, w.conv_w, w.a_log, w.dt_bias, w.norm_w, conv_ring, slot_new, ssm, qkv_in, z,   \
                        alpha, beta, out, *merge, merge_rows)
         if (dk == 128 && K == 4) MFA_GDN_M(128, 4);

@@ -640,13 +640,12 @@ int launch_mla_sdpa_folded(hipStream_t stream, int H, int R, int P, int L, float
         return fail(MFA_ERR_INVALID, "latent attention: workspace too small for %d splits", plan.splits);
     const float qscale = softmax_scale * 1.4426950408889634f;  // scores in log2 units
     if (plan.head_tiles == kMlaHG) {
-        hipLaunchKernelGGL((mla_stream_kernel<512, 64>), dim3(plan.splits, plan.groups), dim3(kMlaHG * 128), 0,
-                           stream, q_prime, q_pe, latent, rope_k, H, L, plan.per_split / kMlaBlk, qscale, ws.part_o, ws.part_ml);
+        launch_kernel(mla_stream_kernel<512, 64>, dim3(plan.splits, plan.groups), dim3(kMlaHG * 128), stream, q_prime, q_pe, latent, rope_k, H, L, plan.per_split / kMlaBlk, qscale, ws.part_o, ws.part_ml);
     } else {
         const dim3 grid((unsigned)((plan.splits + 7) / 8 * 8 * plan.groups));   // see mla_rounds_kernel: a split's workgroups on one XCD
 #define MFA_MLA(HT)                                                                                                \
-    hipLaunchKernelGGL((mla_rounds_kernel<HT>), grid, dim3(kMlaWaves * 64), 0, stream, q_prime, q_pe, latent, rope_k, \
-                       H, L, plan.splits, plan.groups, plan.per_split, qscale, ws.part_o, ws.part_ml)
+    launch_kernel(mla_rounds_kernel<HT>, grid, dim3(kMlaWaves * 64), stream, q_prime, q_pe, latent, rope_k, \
+                  H, L, plan.splits, plan.groups, plan.per_split, qscale, ws.part_o, ws.part_ml)
         if (plan.head_tiles == 1) MFA_MLA(1);
         else MFA_MLA(2);
 #undef MFA_MLA

@@ -714,13 +714,13 @@ static void launch_merge_kernels(hipStream_t stream, const float *part_o, const 
 #define MFA_MERGE(TOKK)                                                                                                 \
     do {                                                                                                                \
         if (splits <= 8)                                                                                                \
-            hipLaunchKernelGGL((sdpa_merge_few_kernel<8, TOKK>), few, dim3(256), 0, stream, part_o, part_ml, splits, hpk, \
+            launch_kernel(sdpa_merge_few_kernel<8, TOKK>, few, dim3(256), stream, part_o, part_ml, splits, hpk, \
                                Hq, nhg, D, n_units, gate, out, ex);                                                     \
         else if (splits <= 16)                                                                                          \
-            hipLaunchKernelGGL((sdpa_merge_few_kernel<16, TOKK>), few, dim3(256), 0, stream, part_o, part_ml, splits,   \
+            launch_kernel(sdpa_merge_few_kernel<16, TOKK>, few, dim3(256), stream, part_o, part_ml, splits,   \
                                hpk, Hq, nhg, D, n_units, gate, out, ex);                                                \
         else                                                                                                            \
-            hipLaunchKernelGGL(sdpa_merge_kernel<TOKK>, dim3(n_tok * Hq, D / 64), dim3(256), 0, stream, part_o, part_ml, \
+            launch_kernel(sdpa_merge_kernel<TOKK>, dim3(n_tok * Hq, D / 64), dim3(256), stream, part_o, part_ml, \
                                splits, hpk, Hq, nhg, D, gate, out, ex);                                                 \
     } while (0)
     if (extra) MFA_MERGE(true); else MFA_MERGE(false);
@@ -826,10 +826,10 @@ static void launch_partial(hipStream_t stream, dim3 grid, const void *k, const v
                            const float *q, int hpk, int Hq, int n_tok, int64_t kv_len0, const SplitPlan &plan,
                            float qscale, float *po, float *pml, const SP &sp, const OneLaunch *one) {
     if (one)
-        hipLaunchKernelGGL((sdpa_partial_kernel<KV, D, STEP, true>), grid, dim3(kWaves * 64), 0, stream, (const KV *)k, (const KV *)v,
+        launch_kernel(sdpa_partial_kernel<KV, D, STEP, true>, grid, dim3(kWaves * 64), stream, (const KV *)k, (const KV *)v,
                            plane_elems, q, hpk, Hq, n_tok, kv_len0, plan.base, plan.rem, qscale, po, pml, sp, *one);
     else
-        hipLaunchKernelGGL((sdpa_partial_kernel<KV, D, STEP, false>), grid, dim3(kWaves * 64), 0, stream, (const KV *)k, (const KV *)v,
+        launch_kernel(sdpa_partial_kernel<KV, D, STEP, false>, grid, dim3(kWaves * 64), stream, (const KV *)k, (const KV *)v,
                            plane_elems, q, hpk, Hq, n_tok, kv_len0, plan.base, plan.rem, qscale, po, pml, sp, OneLaunch{});
 }
 
