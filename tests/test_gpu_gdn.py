@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from tests.util import TOL_F32, GdnCase, idx, rel_err
+from tests.util import TOL_F32, GdnCase, idx, rel_err, rel_err_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -196,6 +196,49 @@ def test_blocked_form_on_hard_inputs(mfa, mutate):
     assert np.isfinite(out).all()
     assert rel_err(out, ref_out) <= TOL_F32 and rel_err(ssm, ref_ssm) <= TOL_F32
     assert np.array_equal(conv.reshape(-1), ref_conv)
+
+
+@pytest.mark.parametrize("dk,Hk,Hv,K,T", [(128, 2, 4, 4, 48), (128, 1, 3, 3, 65), (64, 2, 2, 4, 128), (64, 1, 4, 2, 200)])
+def test_blocked_form_keeps_each_row_of_the_state_to_its_own_scale(mfa, dk, Hk, Hv, K, T):
+    """The blocked form splits its operands into scaled f16 parts; a row of the state and of the values is independent
+    of the others, so each is held to TOL_F32 of its own largest value: rows from 2^-60 to 2^60 side by side, one of
+    2^-100 (below the split's smallest scale), one of 2^80 and a row of zeros with no input.  22 bits an operand and three of the four terms
+    leave 2^-22 of a product, 64 of them and up to four blocks stay below 2^-17 < TOL_F32.  A row that holds NaN or
+    infinity changes no bit of any other row of the state and leaves the other heads' outputs as they were."""
+    case = GdnCase(900 + T, Hk, Hv, dk, dk, K=K, T=T)
+    rng = np.random.default_rng(T)
+    scale = np.exp2(rng.integers(-60, 61, Hv * dk)).astype(np.float32)
+    scale[1], scale[dk + 17], scale[2 * dk - 1] = 0.0, 2.0 ** -100, 2.0 ** 80
+    v0 = 2 * Hk * dk                      # SiLU is linear for the small rows and the identity for the large ones
+    case.qkv[:, v0:] = np.abs(case.qkv[:, v0:]) * scale
+    case.conv_w = case.conv_w.copy()
+    case.conv_w.reshape(case.C, K)[v0:] &= 0x7fff
+    case.conv_state = np.abs(case.conv_state)
+    case.conv_state.reshape(K - 1, case.C)[:, v0:] *= scale
+    case.ssm_state = (case.ssm_state.reshape(Hv * dk, dk) * scale[:, None]).reshape(-1)
+    _, ref_conv, ref_ssm = case.oracle()
+
+    def run(state):
+        with _ctx(mfa, case) as c:
+            c.linear_state_import(0, case.conv_state, state)
+            out = c.prefill_gdn(0, case.qkv, case.z, case.alpha, case.beta)
+            conv, ssm = c.linear_state_export(0)
+        return out, conv, ssm.reshape(Hv * dk, dk)
+
+    out, conv, ssm = run(case.ssm_state)
+    assert np.array_equal(conv.reshape(-1), ref_conv)
+    assert np.isfinite(ssm).all() and not ssm[1].any()
+    assert rel_err_rows(ssm, ref_ssm, dk) <= TOL_F32
+    for bad in (np.nan, np.inf):
+        state = case.ssm_state.copy()
+        row = dk + 5                      # a row of head 1
+        state[row * dk + 7] = bad
+        out2, _, ssm2 = run(state)
+        rows = np.arange(Hv * dk) != row
+        assert not np.isfinite(ssm2[row]).all()
+        assert np.array_equal(ssm2[rows], ssm[rows])
+        heads = np.arange(Hv) != 1
+        assert np.array_equal(out2.reshape(T, Hv, dk)[:, heads], out.reshape(T, Hv, dk)[:, heads])
 
 
 def test_chunk_at_the_a17b_head_counts(mfa):
