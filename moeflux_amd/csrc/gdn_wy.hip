@@ -107,7 +107,7 @@ __device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
 // are stored the way the recurrence kernel's lanes read them, 16 bytes per lane (four f32 values of Ut, the two f16 parts of
 // four values of the others) and 1 KiB per tile (a row-major matrix read as an A operand has neighbouring lanes 512
 // bytes apart, which the memory pipeline serves at a fraction of its rate):
-//   Wt [token tile w][col tile c], Qt likewise, Mt [w][token tile tau], Kt [col tile c][tau]
+//   Wt [token tile w][col tile c], Qt likewise (in the slot of the first value head that shares q^), Mt [w][token tile tau], Kt [col tile c][tau]
 //   (= diag(e^{L_C-L}) K transposed): lane (m, g) holds X[16 row-tile + m][16 col-tile + 4g + i];
 //   Ut [w][col tile c]: lane (n, g) holds U[16w + 4g + i][16c + n]  (a D tile as computed);
 //   eL [64] (e^{L_t}; eL[63] = e^{L_C} because padded tokens do not decay).
@@ -123,7 +123,8 @@ __device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
 // gdn_chunk_pre_kernel computes for the token-by-token form is done here per (block, value head) -
 // conv + SiLU of the head's q, k and v channels, the per-token q/k norm, the decay's logarithm and
 // beta - so the chunk needs no launch and no arrays for them.  A k-head's q and k are formed by
-// each of the value heads that share it.
+// each of the value heads that share it; q^ goes out once, each of them writing a part (a layer's 512 tokens with three sequences side by
+// side: 2 value heads a k head 31.7 -> 31.3 us, 4 64.2 -> 59.9; 2000 tokens of 2 117.4 -> 114.4).
 template <int DK, bool FUSED>
 __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     int Hk, int Hv, int T, const float *__restrict__ qn, const float *__restrict__ kn,
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 
     // heads along x: a head's blocks are produced on the XCD whose L2 the recurrence kernel
     // (heads along x as well) will read them through
-    const int vh = wy_head_of(blockIdx.x, Hk, Hv), blk = blockIdx.y, kh = vh / (Hv / Hk);
+    const int vh = wy_head_of(blockIdx.x, Hk, Hv), blk = blockIdx.y, heads = Hv / Hk, kh = vh / heads;
     const int t0 = blk * kC;
     const int nt = (T - t0 < kC) ? T - t0 : kC;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -434,11 +435,12 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
         }
     }
 #pragma unroll
-    for (int u = 0; u < 4 * NK / NW; u++) {  // q^ tiles, before T takes their place
+    for (int u = 0; u < 4 * NK / NW; u++) {  // q^ tiles, before T takes their place: once per k head, by its value heads in turn
+        if (u % heads != vh % heads) continue;
         const int tile = wave + NW * u, w = tile / NK, c = tile % NK;
         const uint32_t *row = reinterpret_cast<const uint32_t *>(sQ[16 * w + m]) + 8 * c + 2 * g;
         const u32x2 hi = *reinterpret_cast<const u32x2 *>(row), lo = *reinterpret_cast<const u32x2 *>(row + DK / 2);
-        Qt[(slot * 4 * NK + tile) * 64 + lane] = u32x4{hi[0], hi[1], lo[0], lo[1]};
+        Qt[((slot - vh % heads) * 4 * NK + tile) * 64 + lane] = u32x4{hi[0], hi[1], lo[0], lo[1]};
     }
     __syncthreads();
 
@@ -582,7 +584,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 // k-slots 0-3 and 4-7, so against a D operand that repeats its values one instruction adds two of the products.)
 // Bound by the chain: 4.4 k clocks a block (two exchanges through LDS, 56 matrix and 300 vector instructions in a row), on half the
 // CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.7 us; six layers'
-// chunks with this and the block precompute below 238 -> 186 us a pass with three sequences side by side, one sequence 54.8 -> 47.7 a layer;
+// chunks with this and the block precompute above 238 -> 186 us a pass with three sequences side by side, one sequence 54.8 -> 47.7 a layer;
 // 2000 tokens 162 -> 121 and 163 -> 144, of 64 heads 337 -> 248 and 331 -> 247.  Tried and not kept: the operands touched two blocks
 // ahead to have them in the L2 (24.5 us), O beside D of the same block (24.6).
 template <int DK>
@@ -603,18 +605,19 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
     const int nblk = (T + kC - 1) / kC;
     // Requests go through a descriptor of the block's operand, so that they cost no vector addition.  Past the last block: that one again.
     auto slot_of = [&](int blk) { return (size_t)(blk < nblk ? blk : nblk - 1) * Hv + vh; };
+    const int shared = vh % (Hv / Hk);   // q^ is its k head's, in the slot of the first of the value heads
     auto load = [&](__amdgpu_buffer_rsrc_t r, int tile) __attribute__((always_inline)) {
         return __builtin_amdgcn_raw_buffer_load_b128(r, lane16, tile * 1024, 0);
     };
     u32x4 pw[NK];   // W, or q^, of tokens 16w .. 16w+15: a register takes the next block's request as soon as it has been used
-    auto w_of = [&](const u32x4 *X, int blk) { return buffer_of(X + (slot_of(blk) * 4 + w) * NK * 64); };
-    auto fetch_all_w = [&](const u32x4 *X) __attribute__((always_inline)) {
-        const auto r = w_of(X, 0);
+    auto w_of = [&](const u32x4 *X, int back, int blk) { return buffer_of(X + ((slot_of(blk) - back) * 4 + w) * NK * 64); };
+    auto fetch_all_w = [&](const u32x4 *X, int back) __attribute__((always_inline)) {
+        const auto r = w_of(X, back, 0);
 #pragma unroll
         for (int c = 0; c < NK; c++) pw[c] = load(r, c);
     };
-    // X S0^T of this wave's 16 tokens, X = W or q^, both row groups
-    auto times_state = [&](const u32x4 *X, int blk, wy_f32x4 (&p)[2]) __attribute__((always_inline)) {
+    // X S0^T of this wave's 16 tokens, X = W or q^ (which lies `back` slots ahead of the head's own), both row groups
+    auto times_state = [&](const u32x4 *X, int back, int blk, wy_f32x4 (&p)[2]) __attribute__((always_inline)) {
         // All LDS reads first, and the three terms of every (step, row group) in turn, so that no instruction waits for the one
         // before it (left alone the compiler reads each operand just ahead of its product: 5.2 k clocks a block instead of 4.4 k).
         u32x4 sh[NS][2], sl[NS][2];
@@ -649,7 +652,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         for (int s = 0; s < NS; s++)
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(hi[s], sh[s][rg], acc[s][rg]);
-        const auto r = w_of(X, blk + 1);
+        const auto r = w_of(X, back, blk + 1);
 #pragma unroll
         for (int c = 0; c < NK; c++) pw[c] = load(r, c);
 #pragma unroll
@@ -698,7 +701,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         auto fetch_elc = [&](int blk) __attribute__((always_inline)) {
             elc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(eLc + slot_of(blk) * kC + kC - 1), 0, 0, 0));
         };
-        fetch_all_w(Wt);
+        fetch_all_w(Wt, 0);
         {
             const auto ru = u_of(0), rk = k_of(0);
 #pragma unroll
@@ -714,7 +717,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         for (int blk = 0; blk < nblk; blk++) {
             // ---- D = U - W S0^T: lane (n, g) holds tokens 16w+4g+i of state row n of the group ----
             wy_f32x4 p[2];
-            times_state(Wt, blk, p);
+            times_state(Wt, 0, blk, p);
             const wy_f32x4 d[2] = {pu[0] - p[0], pu[1] - p[1]};
             const auto ru = u_of(blk + 1);
 #pragma unroll
@@ -803,7 +806,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
             el = __builtin_bit_cast(wy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(eLc + slot_of(blk) * kC + 16 * w), g * 16, 0, 0));
         };
         const int stride = Hv * DV;
-        fetch_all_w(Qt);
+        fetch_all_w(Qt, shared);
         fetch_el(0);
         fetch_m(0);
         __syncthreads();
@@ -811,7 +814,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         __syncthreads();   // block 0: its D and the state behind it are there
         for (int blk = 0; blk < nblk; blk++) {
             wy_f32x4 o[2];
-            times_state(Qt, blk, o);
+            times_state(Qt, shared, blk, o);
             o[0] *= el;
             o[1] *= el;
             fetch_el(blk + 1);
