@@ -25,7 +25,7 @@
 //     Nothing passes between waves but the rows' maxima and the probabilities: two barriers a round.  For caches of few rounds:
 //     its workgroups start 3 us sooner than the other kernel's, and with 16 or 32 heads each they leave a half or a quarter of the
 //     partials.  It converts each row twice per workgroup, so that with more than
-//     three rounds the vector ALU (10 k of a round's 19 k clocks at 32 heads) costs more than that saves.
+//     two rounds of 32 heads the vector ALU (10 k of a round's 19 k clocks at 32 heads) costs more than that saves.
 //
 //   mla_stream_kernel<R, P>   grid (splits, ceil(H / 64)); 8 waves in two roles.  Wave hg
 //     (0..3) computes the scores and the softmax of head group hg, wave 4 + hg accumulates
