@@ -117,7 +117,7 @@ __device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
 // has matrix work while the other waits for LDS or stores a tile).
 // A workgroup's 28 k clocks (39 k on f32 instructions) are 9 k until its inputs are there, 3 k of norms, 3.5 k for the two
 // triangles, 2.3 k for the diagonal blocks beside K', 4.7 k for the levels beside phase 3's operands, 4 k for W and U: 512 tokens of 32
-// heads 21.8 -> 16.9 us.  At 128 registers, so that a CU holds two (it takes 144 and holds one), it spills: no faster at 2000
+// heads 21.5 -> 15.8 us.  At 128 registers, so that a CU holds two (it takes 144 and holds one), it spills: no faster at 2000
 // tokens with three sequences side by side (120.5 us a pass either way), 2 us slower at 512.
 // FUSED: the block's inputs come straight from the layer's inputs (WyInputs): what
 // gdn_chunk_pre_kernel computes for the token-by-token form is done here per (block, value head) -
@@ -583,9 +583,9 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
 // e >= 4 column 32w+16+4g+e-4; a tile of D likewise tokens 16w+4g+i of row n.  The A side has hi and lo of the same four values in its
 // k-slots 0-3 and 4-7, so against a D operand that repeats its values one instruction adds two of the products.)
 // Bound by the chain: 4.4 k clocks a block (two exchanges through LDS, 56 matrix and 300 vector instructions in a row), on half the
-// CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.7 us; six layers'
-// chunks with this and the block precompute above 238 -> 186 us a pass with three sequences side by side, one sequence 54.8 -> 47.7 a layer;
-// 2000 tokens 162 -> 121 and 163 -> 144, of 64 heads 337 -> 248 and 331 -> 247.  Tried and not kept: the operands touched two blocks
+// CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.2 us; six layers'
+// chunks with this and the block precompute above 238 -> 180 us a pass with three sequences side by side, one sequence 54.8 -> 47.6 a layer;
+// 2000 tokens 162 -> 118 and 163 -> 144, of 64 heads 337 -> 231 and 331 -> 241.  Tried and not kept: the operands touched two blocks
 // ahead to have them in the L2 (24.5 us), O beside D of the same block (24.6).
 template <int DK>
 __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
