@@ -252,6 +252,21 @@ def test_chunk_at_the_a17b_head_counts(mfa):
     assert rel_err(out, ref_out) <= TOL_F32 and rel_err(ssm, ref_ssm) <= TOL_F32
 
 
+@pytest.mark.parametrize("K", [4, 3])
+@pytest.mark.parametrize("T", [256, 257, 385])
+def test_blocked_form_at_and_past_a_workgroup_per_cu(mfa, K, T):
+    """64 heads of 128 channels: four blocks are a workgroup per CU, from five on two share one and the block precompute
+    runs in fewer registers; with the conv inside it (width 4) and ahead of it."""
+    case = GdnCase(60 + T + K, 16, 64, 128, 128, K=K, T=T)
+    ref_out, ref_conv, ref_ssm = case.oracle()
+    with _ctx(mfa, case) as c:
+        c.linear_state_import(0, case.conv_state, case.ssm_state)
+        out = c.prefill_gdn(0, case.qkv, case.z, case.alpha, case.beta)
+        conv, ssm = c.linear_state_export(0)
+    assert rel_err(out, ref_out) <= TOL_F32 and rel_err(ssm, ref_ssm) <= TOL_F32
+    assert np.array_equal(conv.reshape(-1), ref_conv)
+
+
 def test_prompt_longer_than_one_segment(mfa):
     """A prompt of more than 4096 tokens goes through the chunk kernels in 4096-token segments; the
     ring and the state carry from one segment to the next as they do between calls."""
