@@ -945,7 +945,7 @@ int mfa_prefill_gdn_dev(mfa_ctx *ctx, int32_t layer, int32_t T, const float *qkv
         MFA_TRY(launch_gdn_chunk(c->stream, g.linear_num_k_heads, g.linear_num_v_heads, g.linear_key_dim,
                                  g.linear_value_dim, g.conv_kernel_size, g.rms_norm_eps, n, l->w,
                                  l->conv_ring, l->step, l->ssm, qkv_in_dev + off * C, z_dev + off * tv,
-                                 alpha_dev + off * Hv, beta_dev + off * Hv, c->gdn_scratch, out_dev + off * tv, c->num_cus));
+                                 alpha_dev + off * Hv, beta_dev + off * Hv, c->gdn_scratch, out_dev + off * tv));
         l->step += n;
     }
     return MFA_OK;

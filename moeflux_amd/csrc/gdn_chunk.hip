@@ -272,7 +272,7 @@ size_t gdn_chunk_scratch_elems(int Hk, int Hv, int dk, int dv, int T) {
 int launch_gdn_chunk(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float eps, int T,
                      const LinearWeights &w, float *conv_ring, int64_t step, float *ssm,
                      const float *qkv_in, const float *z, const float *alpha, const float *beta,
-                     float *scratch, float *out, int num_cus) {
+                     float *scratch, float *out) {
     if (!gdn_shape_supported(Hk, Hv, dk, dv, K))
         return fail(MFA_ERR_SHAPE, "gdn chunk: shape Hk=%d Hv=%d dk=%d dv=%d K=%d not supported", Hk, Hv,
                     dk, dv, K);
@@ -293,7 +293,7 @@ int launch_gdn_chunk(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float
     if (blocked && K == 4) {
         // the blocks of the blocked form compute conv, norms and gates themselves
         const WyInputs in{qkv_in, conv_ring, w.conv_w, w.a_log, w.dt_bias, alpha, beta, K, (int)(step % K)};
-        MFA_TRY(launch_gdn_wy(s, Hk, Hv, dk, dv, T, nullptr, nullptr, nullptr, nullptr, nullptr, wy, ssm, o_raw, num_cus, &in));
+        MFA_TRY(launch_gdn_wy(s, Hk, Hv, dk, dv, T, nullptr, nullptr, nullptr, nullptr, nullptr, wy, ssm, o_raw, &in));
     } else {
         if (dk == 128)
             hipLaunchKernelGGL((gdn_chunk_pre_kernel<128>), dim3((T + kPreTok - 1) / kPreTok, Hk + nvb + 1), dim3(256), 0, s,
@@ -305,7 +305,7 @@ int launch_gdn_chunk(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float
                                vv, gd, bg, kq, lg);
         MFA_HIP(hipGetLastError());
         if (blocked)
-            MFA_TRY(launch_gdn_wy(s, Hk, Hv, dk, dv, T, qn, kn, vv, lg, bg, wy, ssm, o_raw, num_cus));
+            MFA_TRY(launch_gdn_wy(s, Hk, Hv, dk, dv, T, qn, kn, vv, lg, bg, wy, ssm, o_raw));
         else if (dk == 128)
             hipLaunchKernelGGL((gdn_chunk_recur_kernel<128, 128>), dim3(Hv, 128 / 16), dim3(256), 0, s, Hk, Hv, T, qn,
                                kn, vv, gd, bg, kq, ssm, o_raw);

@@ -117,20 +117,16 @@ __device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
 // has matrix work while the other waits for LDS or stores a tile).
 // A workgroup's 28 k clocks (39 k on f32 instructions) are 9 k until its inputs are there, 3 k of norms, 3.5 k for the two
 // triangles, 2.3 k for the diagonal blocks beside K', 4.7 k for the levels beside phase 3's operands, 4 k for W and U: 512 tokens of 32
-// heads 21.5 -> 15.8 us.
-// TWO: in 128 registers, so that a CU holds two of them (144 leave room for one); phase 3 then reads T's parts as it needs them.  Where
-// there are more workgroups than CUs (a layer, one call after the other / three sequences side by side): 600 tokens of 32 heads 61.5 -> 58.6 /
-// 37.8 -> 38.2 us, 1000 78.7 -> 74.6 / 59.9 -> 59.6, 2000 143.0 -> 137.6 / 117.7 -> 115.0, 300 of 64 heads 53.6 -> 50.5 / 40.3 -> 40.7, 512 66.1 ->
-// 64.2 / 60.3 -> 60.0, 2000 239 -> 230 / 232 -> 228; up to one a CU the requests of the first phase go out later for want of registers: 512
-// tokens of 32 heads 47.1 -> 48.9 / 30.7 -> 31.0, so not there.
+// heads 21.5 -> 15.8 us.  At 128 registers, so that a CU holds two (it takes 144 and holds one), it spills: no faster at 2000
+// tokens with three sequences side by side (120.5 us a pass either way), 2 us slower at 512.
 // FUSED: the block's inputs come straight from the layer's inputs (WyInputs): what
 // gdn_chunk_pre_kernel computes for the token-by-token form is done here per (block, value head) -
 // conv + SiLU of the head's q, k and v channels, the per-token q/k norm, the decay's logarithm and
 // beta - so the chunk needs no launch and no arrays for them.  A k-head's q and k are formed by
 // each of the value heads that share it; q^ goes out once, each of them writing a part (a layer's 512 tokens with three sequences side by
 // side: 2 value heads a k head 31.7 -> 31.3 us, 4 64.2 -> 59.9; 2000 tokens of 2 117.4 -> 114.4).
-template <int DK, bool FUSED, bool TWO>
-__global__ __launch_bounds__(DK * 4, TWO ? 4 : 1) void gdn_wy_kernel(
+template <int DK, bool FUSED>
+__global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     int Hk, int Hv, int T, const float *__restrict__ qn, const float *__restrict__ kn,
     const float *__restrict__ vv, const float *__restrict__ lg, const float *__restrict__ bg,
     u32x4 *__restrict__ Wt, u32x4 *__restrict__ Qt, float *__restrict__ Ut, u32x4 *__restrict__ Mt,
@@ -551,18 +547,14 @@ __global__ __launch_bounds__(DK * 4, TWO ? 4 : 1) void gdn_wy_kernel(
 
     // ---- phase 3: W = T diag(beta e^L) K and U = T diag(beta) V -------------------------
     u32x4 tw[6][2], tu[6][2];
-    auto read_t = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-        for (int at = from; at < to; at++)
+    for (int at = 0; at < 6; at++)
 #pragma unroll
-            for (int part = 0; part < 2; part++) tw[at][part] = sTw[at][part][lane], tu[at][part] = sTu[at][part][lane];
-        __builtin_amdgcn_sched_barrier(0);   // these reads ahead of the first product
-    };
-    read_t(0, TWO ? 2 : 6);
+        for (int part = 0; part < 2; part++) tw[at][part] = sTw[at][part][lane], tu[at][part] = sTu[at][part][lane];
+    __builtin_amdgcn_sched_barrier(0);   // all reads ahead of the first product
 #pragma unroll
     for (int tau = 0; tau < 4; tau++) {
         wy_f32x4 aw = zero, au = zero;
-        if (TWO && tau >= 2) read_t(2 * tau - 2, 2 * tau);
 #pragma unroll
         for (int p = 0; p <= tau / 2; p++) {
             const int at = tau < 2 ? tau : 2 + 2 * (tau - 2) + p;
@@ -593,7 +585,7 @@ __global__ __launch_bounds__(DK * 4, TWO ? 4 : 1) void gdn_wy_kernel(
 // Bound by the chain: 4.4 k clocks a block (two exchanges through LDS, 56 matrix and 300 vector instructions in a row), on half the
 // CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.2 us; six layers'
 // chunks with this and the block precompute above 238 -> 180 us a pass with three sequences side by side, one sequence 54.8 -> 47.6 a layer;
-// 2000 tokens 162 -> 115 and 163 -> 138, of 64 heads 337 -> 228 and 331 -> 230.  Tried and not kept: the operands touched two blocks
+// 2000 tokens 162 -> 118 and 163 -> 144, of 64 heads 337 -> 231 and 331 -> 241.  Tried and not kept: the operands touched two blocks
 // ahead to have them in the L2 (24.5 us), O beside D of the same block (24.6).
 template <int DK>
 __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
@@ -875,7 +867,7 @@ size_t gdn_wy_scratch_elems(int Hv, int dk, int dv, int T) {
 // decay, beta gate) as gdn_chunk_pre_kernel leaves them.
 int launch_gdn_wy(hipStream_t s, int Hk, int Hv, int dk, int dv, int T, const float *qn, const float *kn,
                   const float *vv, const float *lg, const float *bg, float *scratch, float *ssm,
-                  float *o_raw, int num_cus, const WyInputs *in) {
+                  float *o_raw, const WyInputs *in) {
     if (dk != dv || (dk != 64 && dk != 128))
         return fail(MFA_ERR_SHAPE, "gdn blocked form: dk=%d dv=%d not supported", dk, dv);
     const size_t nblk = ((size_t)T + kC - 1) / kC;
@@ -889,19 +881,15 @@ int launch_gdn_wy(hipStream_t s, int Hk, int Hv, int dk, int dv, int T, const fl
     u32x4 *Mt = reinterpret_cast<u32x4 *>(Ut + slots * kC * dv);
     float *eLc = reinterpret_cast<float *>(Mt + slots * kC * kC / 4);
     const WyInputs none{};
-    const bool two = slots > (size_t)num_cus;   // (see TWO)
-#define MFA_WY(DKK, FU, TW)                                                                                         \
-    hipLaunchKernelGGL((gdn_wy_kernel<DKK, FU, TW>), dim3(Hv, (unsigned)nblk), dim3(DKK * 4), 0, s, Hk, Hv, T, qn, kn, vv, \
+#define MFA_WY(DKK, FU)                                                                                             \
+    hipLaunchKernelGGL((gdn_wy_kernel<DKK, FU>), dim3(Hv, (unsigned)nblk), dim3(DKK * 4), 0, s, Hk, Hv, T, qn, kn, vv, \
                        lg, bg, Wt, Qt, Ut, Mt, Kt, eLc, in ? *in : none)
     if (dk == 128) {
-        if (in && two) MFA_WY(128, true, true);
-        else if (in) MFA_WY(128, true, false);
-        else if (two) MFA_WY(128, false, true);
-        else MFA_WY(128, false, false);
+        if (in) MFA_WY(128, true); else MFA_WY(128, false);
         hipLaunchKernelGGL((gdn_wy_recur_kernel<128>), dim3(Hv, dv / 32), dim3(512), 0, s, Hk, Hv, T, Wt, Qt, Ut,
                            Mt, Kt, eLc, ssm, o_raw);
     } else {
-        if (in) MFA_WY(64, true, false); else MFA_WY(64, false, false);
+        if (in) MFA_WY(64, true); else MFA_WY(64, false);
         hipLaunchKernelGGL((gdn_wy_recur_kernel<64>), dim3(Hv, dv / 32), dim3(512), 0, s, Hk, Hv, T, Wt, Qt, Ut,
                            Mt, Kt, eLc, ssm, o_raw);
     }

@@ -417,11 +417,11 @@ struct WyInputs {
 };
 int launch_gdn_wy(hipStream_t s, int Hk, int Hv, int dk, int dv, int T, const float *qn, const float *kn,
                   const float *vv, const float *lg, const float *bg, float *scratch, float *ssm,
-                  float *o_raw, int num_cus, const WyInputs *in = nullptr);
+                  float *o_raw, const WyInputs *in = nullptr);
 int launch_gdn_chunk(hipStream_t s, int Hk, int Hv, int dk, int dv, int K, float eps, int T,
                      const LinearWeights &w, float *conv_ring, int64_t step, float *ssm,
                      const float *qkv_in, const float *z, const float *alpha, const float *beta,
-                     float *scratch, float *out, int num_cus);
+                     float *scratch, float *out);
 int launch_conv1d_step(hipStream_t s, int C, int K, float *conv_state, const float *in,
                        const uint16_t *w, float *out);
 int launch_rms_norm_qk(hipStream_t s, int Hk, int dk, float *q, float *k);

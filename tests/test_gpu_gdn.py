@@ -255,8 +255,8 @@ def test_chunk_at_the_a17b_head_counts(mfa):
 @pytest.mark.parametrize("K", [4, 3])
 @pytest.mark.parametrize("T", [256, 257, 385])
 def test_blocked_form_at_and_past_a_workgroup_per_cu(mfa, K, T):
-    """64 heads of 128 channels: four blocks are a workgroup per CU, from five on two share one and the block precompute
-    runs in fewer registers; with the conv inside it (width 4) and ahead of it."""
+    """64 heads of 128 channels: four blocks are a workgroup of the block precompute per CU, from five on a CU has more than
+    one; with the conv inside it (width 4) and ahead of it."""
     case = GdnCase(60 + T + K, 16, 64, 128, 128, K=K, T=T)
     ref_out, ref_conv, ref_ssm = case.oracle()
     with _ctx(mfa, case) as c:
