@@ -926,7 +926,7 @@ int mfa_prefill_gdn_dev(mfa_ctx *ctx, int32_t layer, int32_t T, const float *qkv
     if (T == 1) return gdn_step_dev(c, l, qkv_in_dev, z_dev, alpha_dev, beta_dev, out_dev);
     if (!l->w.set) return fail(MFA_ERR_INVALID, "linear layer weights not set (mfa_set_linear_weights)");
     const mfa_config &g = c->cfg;
-    // Long prompts go through in segments, which bounds the scratch (about 57 KB per token
+    // Long prompts go through in segments, which bounds the scratch (about 148 KB per token
     // at the 16/32-head, 128-wide shape); the ring and the state carry over as between calls.
     const int kSeg = 4096;
     const size_t need = gdn_chunk_scratch_elems(g.linear_num_k_heads, g.linear_num_v_heads,

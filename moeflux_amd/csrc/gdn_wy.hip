@@ -16,7 +16,7 @@
 // chunk at once (gdn_wy_kernel, one workgroup per (block, value head)); the four
 // products that involve the state run block after block with the state in registers
 // (gdn_wy_recur_kernel, one workgroup per 32 rows of a head's state, rows being
-// independent).  The products are v_mfma_f32_16x16x32_f16 over operands split into two f16 numbers (see wy_split4), the
+// independent).  The products are v_mfma_f32_16x16x32_bf16 over operands split into three bf16 numbers (see wy_split4), the
 // inversion's small ones v_mfma_f32_16x16x4_f32.
 //
 // Operand conventions of the f32 instruction (lane l, m = n = l % 16, g = l / 16):
@@ -60,95 +60,111 @@ __device__ inline float4 as_f4(wy_f32x4 v) { return float4{v[0], v[1], v[2], v[3
 // a 16-byte load kept as a vector register value (members of a struct of operands)
 __device__ inline wy_f32x4 load_v4(const float *p) { return *reinterpret_cast<const wy_f32x4 *>(p); }
 
-// f32 x scaled by a power of two as the sum of two f16 numbers, hi = f16(x), lo = f16(x - hi): 22 bits, what is left out is below
-// 2^-24 of x (2^-39 of the scale for x below 2^-16 of it, where lo is subnormal), the size of x's own rounding.
-// Of a product hi hi + hi lo + lo hi is formed (lo lo too where it costs nothing) and summed in f32, as the f32 instruction does,
-// in 16 clocks for 32 contracted values and term instead of 256.  W, q^, the decayed k^ and M are at most 1 by construction
-// (unit keys, beta <= 1, decays <= 1, and every row of W is beta e^L k^ under a chain of contractions), so they carry a fixed
-// scale; the state's and D's scales are those of the largest value of a tile's row, taken as the tile is formed.
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;   // (LDS holding f32 and f16 parts in turn is read and written as vectors, which alias anything)
-static constexpr float kWyScale = 16384.f;   // 2^14: the largest f16 is 65504
-// Four values times scale as 16 bytes: hi of all, lo of all.  v_fma_mix*_f16 multiplies, subtracts hi where there is one, and
-// rounds, in one instruction per value and part (multiply, convert, convert back, subtract, convert are four).
-// The compiler does not see into the assembly: a result that went to the upper half of its register may be read one wait state
-// later at the earliest, which the order of the eight and the last no-op keep; and no result of a matrix instruction may come in
-// directly (its wait states are the compiler's to place), which callers see to with an instruction in between.
-__device__ inline u32x4 wy_split4(float a, float b, float c, float d, float scale) {
-    uint32_t h0, h1, l0, l1;
-    asm("v_fma_mixlo_f16 %0, %4, %8, 0\n\t"
-        "v_fma_mixlo_f16 %1, %6, %8, 0\n\t"
-        "v_fma_mixhi_f16 %0, %5, %8, 0\n\t"
-        "v_fma_mixhi_f16 %1, %7, %8, 0\n\t"
-        "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %3, %6, %8, -%1 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %2, %5, %8, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixhi_f16 %3, %7, %8, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "s_nop 0"
-        : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1) : "v"(a), "v"(b), "v"(c), "v"(d), "v"(scale));
-    return u32x4{h0, h1, l0, l1};
+// An f32 x as the sum of three bf16 numbers, h = bf16(x), m = bf16(x - h), l = x - h - m: exact, 24 bits are 8 + 8 + 8, and bf16 has
+// f32's exponents, so that every value keeps its own scale, whatever lies beside it in a tile.  (Two f16 parts are half the terms
+// and two bytes less, but share a scale along a contraction: a token 1e8 times the others took the bits of the tokens ahead of it, and
+// small W, T or K' under a fixed scale lost theirs.)  Below 2^-102 l loses its last bits; within 2^-9 of the largest f32 h is infinite.
+// Of a product all but m l, l m and l l is formed and summed in f32: what is left out is below 2^-24 of it.  Six
+// instructions take 96 clocks for 32 contracted values, f32 instructions 256.
+// Contractions over a block's tokens go in steps of 32, and of 16 where the next 16 lie past the diagonal: zeros
+// there would carry a later token's infinity or NaN into earlier ones.
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;   // (LDS holding f32 and bf16 parts in turn is read and written as vectors, which alias anything)
+struct WyFour { u32x2 p[3]; };    // h, m, l of four values
+struct WyEight { u32x4 p[3]; };
+__device__ inline void wy_split2(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
+    auto low = [](uint32_t x) { return __builtin_bit_cast(float, x << 16); };
+    auto high = [](uint32_t x) { return __builtin_bit_cast(float, x & 0xffff0000u); };
+    h = pack_bf16(a, b);
+    a -= low(h), b -= high(h);
+    m = pack_bf16(a, b);
+    l = pack_bf16(a - low(m), b - high(m));
 }
-__device__ inline u32x4 wy_split4_unit(float a, float b, float c, float d) { return wy_split4(a, b, c, d, kWyScale); }   // of values of at most 1
+__device__ inline WyFour wy_split4(float a, float b, float c, float d) {
+    uint32_t h0, h1, m0, m1, l0, l1;
+    wy_split2(a, b, h0, m0, l0);
+    wy_split2(c, d, h1, m1, l1);
+    return {{u32x2{h0, h1}, u32x2{m0, m1}, u32x2{l0, l1}}};
+}
+__device__ inline WyFour wy_split4(const wy_f32x4 &x) { return wy_split4(x[0], x[1], x[2], x[3]); }
+__device__ inline WyEight wy_join(const WyFour &x, const WyFour &y) {
+    WyEight r;
+#pragma unroll
+    for (int i = 0; i < 3; i++) r.p[i] = u32x4{x.p[i][0], x.p[i][1], y.p[i][0], y.p[i][1]};
+    return r;
+}
+// the four values whose parts these are
+__device__ inline wy_f32x4 wy_whole(const WyFour &x) {
+    wy_f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        auto low = [&](int k) { return __builtin_bit_cast(float, (uint32_t)x.p[k][i] << 16); };
+        auto high = [&](int k) { return __builtin_bit_cast(float, (uint32_t)x.p[k][i] & 0xffff0000u); };
+        r[2 * i] = low(0) + (low(1) + low(2));
+        r[2 * i + 1] = high(0) + (high(1) + high(2));
+    }
+    return r;
+}
 __device__ inline wy_f32x4 wy_fma(wy_f32x4 a, float s, wy_f32x4 c) {
     return wy_f32x4{fmaf(a[0], s, c[0]), fmaf(a[1], s, c[1]), fmaf(a[2], s, c[2]), fmaf(a[3], s, c[3])};
 }
-// The scale of values of at most mx (2^14 <= mx scale < 2^15, less for mx below 2^-87) and what undoes it together with kWyScale.
-__device__ inline void wy_scale(float mx, float &scale, float &undo) {
-    const int e = max((int)(__builtin_bit_cast(uint32_t, mx) >> 23), 40);   // mx >= 0
-    scale = __builtin_bit_cast(float, (uint32_t)(268 - e) << 23);
-    undo = __builtin_bit_cast(float, (uint32_t)(e - 28) << 23);
+static constexpr int kWyA[6] = {2, 0, 1, 1, 0, 0}, kWyB[6] = {0, 2, 1, 0, 1, 0};   // parts of the terms, smallest first
+__device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {   // 32 contracted values: the lane group's four of one 16, then of the next
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
 }
-__device__ inline wy_f32x4 wy_mfma(u32x4 a, u32x4 b, wy_f32x4 acc) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+__device__ inline wy_f32x4 wy_mfma_first(u32x4 a, u32x4 b, wy_f32x4 acc) {   // the first 16 of them
+    typedef short i16x4 __attribute__((ext_vector_type(4)));
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, u32x2{a[0], a[1]}), __builtin_bit_cast(i16x4, u32x2{b[0], b[1]}), acc, 0, 0, 0);
 }
 
-// Per (block, value head) outputs, block-major then head, each cut into 16x16 tiles that
-// are stored the way the recurrence kernel's lanes read them, 16 bytes per lane (four f32 values of Ut, the two f16 parts of
-// four values of the others) and 1 KiB per tile (a row-major matrix read as an A operand has neighbouring lanes 512
-// bytes apart, which the memory pipeline serves at a fraction of its rate):
-//   Wt [token tile w][col tile c], Qt likewise (in the slot of the first value head that shares q^), Mt [w][token tile tau], Kt [col tile c][tau]
-//   (= diag(e^{L_C-L}) K transposed): lane (m, g) holds X[16 row-tile + m][16 col-tile + 4g + i];
+// Per (block, value head) outputs, block-major then head, each cut into tiles that are stored the way the recurrence kernel's lanes
+// read them, 1 KiB of 16 bytes per lane (a row-major matrix read as an A operand has neighbouring lanes 512 bytes apart, which the
+// memory pipeline serves at a fraction of its rate).  A tile of W, q^ or K' is 16 rows by 32 contracted values and consists of three
+// such pieces, the bf16 parts h, m and l; M and U stay f32, in tiles of 16 by 16:
+//   Wt [token tile w][32 channels s], Qt likewise (in the slot of the first value head that shares q^), Kt [col tile c][32 tokens p]
+//   (= diag(e^{L_C-L}) K transposed): lane (m, g) holds X[16 row-tile + m][32 col-tile + 4g + i] and [.. + 16 + 4g + i];
+//   Mt [w][token tile tau]: lane (m, g) holds M[16w + m][16 tau + 4g + i];
 //   Ut [w][col tile c]: lane (n, g) holds U[16w + 4g + i][16c + n]  (a D tile as computed);
 //   eL [64] (e^{L_t}; eL[63] = e^{L_C} because padded tokens do not decay).
 // Tokens past the end of the chunk are padded with beta = 0, log g = 0, k = q = v = 0.
 //
 // grid (Hv, blocks), one wave per 16 columns of K (DK/16 waves: two per SIMD at DK = 128, so that one
 // has matrix work while the other waits for LDS or stores a tile).
-// A workgroup's 28 k clocks (39 k on f32 instructions) are 9 k until its inputs are there, 3 k of norms, 3.5 k for the two
-// triangles, 2.3 k for the diagonal blocks beside K', 4.7 k for the levels beside phase 3's operands, 4 k for W and U: 512 tokens of 32
-// heads 21.5 -> 15.8 us.  At 128 registers, so that a CU holds two (it takes 144 and holds one), it spills: no faster at 2000
-// tokens with three sequences side by side (120.5 us a pass either way), 2 us slower at 512.
+// A workgroup's 31 k clocks (39 k on f32 instructions) are 9 k until its inputs are there, 3.6 k of norms and their splits, 5 k for the two
+// triangles, 3 k for the diagonal blocks beside K', 3.5 k for the levels beside phase 3's operands, 1.4 k for T's parts and 4 to 6 k for W and U;
+// 512 tokens of 32 heads 20.9 us on f32 instructions, 19.4.  It takes 245 registers and 120 KiB, a CU to a workgroup.
+// Measured beside: q^ split by the wave that multiplies it, and the triangles' jobs by whole row tiles (20.2, the longest job 6.5 k clocks);
+// q^ out as f32 and split by the recurrence (19.0, but 26.7 there).
 // FUSED: the block's inputs come straight from the layer's inputs (WyInputs): what
 // gdn_chunk_pre_kernel computes for the token-by-token form is done here per (block, value head) -
 // conv + SiLU of the head's q, k and v channels, the per-token q/k norm, the decay's logarithm and
 // beta - so the chunk needs no launch and no arrays for them.  A k-head's q and k are formed by
-// each of the value heads that share it; q^ goes out once, each of them writing a part (a layer's 512 tokens with three sequences side by
-// side: 2 value heads a k head 31.7 -> 31.3 us, 4 64.2 -> 59.9; 2000 tokens of 2 117.4 -> 114.4).
+// each of the value heads that share it; q^ goes out once, each of them writing a part.
 template <int DK, bool FUSED>
 __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     int Hk, int Hv, int T, const float *__restrict__ qn, const float *__restrict__ kn,
     const float *__restrict__ vv, const float *__restrict__ lg, const float *__restrict__ bg,
-    u32x4 *__restrict__ Wt, u32x4 *__restrict__ Qt, float *__restrict__ Ut, u32x4 *__restrict__ Mt,
+    u32x4 *__restrict__ Wt, u32x4 *__restrict__ Qt, float *__restrict__ Ut, float *__restrict__ Mt,
     u32x4 *__restrict__ Kt, float *__restrict__ eLc, WyInputs in) {
     constexpr int DV = DK;
     constexpr int NK = DK / 16, NS = DK / 32;
-    constexpr int LDK = DK + 4;  // row strides (4-byte units) chosen so that 16-byte row reads by 8 lanes hit all banks
-    constexpr int LDC = kC + 4;
-    constexpr int NW = NK;        // waves; wave c owns columns 16c .. 16c+15 of W and of U
+    // row strides (4-byte units) chosen so that 16-byte row reads by 8 lanes hit all banks
+    constexpr int LDK = 3 * DK / 2 + 20, LDC = kC + 4;
+    constexpr int NW = NK;        // waves; wave c owns columns 16c .. 16c+15 of U
     constexpr int NTHR = 64 * NW;
-    // A row of k^ or q^ is f32 until it is normed and then the f16 parts in its place (hi of all channels, then lo of all), v stays
-    // in the registers of the wave that multiplies it, T and its f16 parts lie where q^ and A were.
-    __shared__ __align__(16) float sK[kC][LDK];
-    constexpr int TPARTS = 6 * 2 * 64 * 4;           // f16 parts of T times a factor per token: [(token tile, 32-token step)][hi|lo][64] x 16 bytes
+    // A row of k^ or q^ is f32 until it is normed and then its bf16 parts in its place (h of all channels, m, l; of each 32 channels in the
+    // order of an operand's lanes), v stays in the registers of the wave that multiplies it.  T lies where q^ was, its parts behind it
+    // and where k^ was.
+    constexpr int TPARTS = 6 * 3 * 64 * 4;           // parts of T times a factor per token: [(token tile, 32-token step)][h|m|l][64] x 16 bytes
+    constexpr int KROOM = kC * LDK > TPARTS ? kC * LDK : TPARTS;
     constexpr int QROOM = kC * LDK > kC * LDC + TPARTS ? kC * LDK : kC * LDC + TPARTS;
+    __shared__ __align__(16) float sKroom[KROOM];    // k^, later T diag(beta e^L)
     __shared__ __align__(16) float sQroom[QROOM];    // q^, later T and T diag(beta)
-    __shared__ __align__(16) float sA[10][16][20];   // tile (I, J <= I) at I (I + 1) / 2 + J; later T diag(beta e^L)
+    __shared__ __align__(16) float sA[10][16][20];   // tile (I, J <= I) at I (I + 1) / 2 + J
+    float(*sK)[LDK] = reinterpret_cast<float(*)[LDK]>(&sKroom[0]);
     float(*sQ)[LDK] = reinterpret_cast<float(*)[LDK]>(&sQroom[0]);
     float(*sT)[LDC] = reinterpret_cast<float(*)[LDC]>(&sQroom[0]);
-    u32x4(*sTu)[2][64] = reinterpret_cast<u32x4(*)[2][64]>(&sQroom[kC * LDC]);
-    u32x4(*sTw)[2][64] = reinterpret_cast<u32x4(*)[2][64]>(&sA[0][0][0]);
-    static_assert(TPARTS * sizeof(float) <= sizeof(sA), "T's parts fit where A was");
+    u32x4(*sTu)[3][64] = reinterpret_cast<u32x4(*)[3][64]>(&sQroom[kC * LDC]);
+    u32x4(*sTw)[3][64] = reinterpret_cast<u32x4(*)[3][64]>(&sKroom[0]);
     __shared__ __align__(16) float sL[kC], sB[kC], sCw[kC], sKd[kC];
     __shared__ __align__(16) int sR[kC];
 
@@ -194,12 +210,12 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
         eLc[slot * kC + lane] = el;
         sKd[lane] = __shfl(r, 63, 64) > lane ? 0.f : expf(__shfl(l, 63, 64) - l);  // e^{L_C - L_t}
     };
-    // a row of k^ or q^ as its f16 parts: channels c .. c + 3, y scale (at most 1)
-    auto put4 = [&](float *row, int c, float4 y, float scale) __attribute__((always_inline)) {
-        const u32x4 x = wy_split4(y.x, y.y, y.z, y.w, scale * kWyScale);
-        uint32_t *r = reinterpret_cast<uint32_t *>(row);
-        *reinterpret_cast<u32x2 *>(r + c / 2) = u32x2{x[0], x[1]};
-        *reinterpret_cast<u32x2 *>(r + DK / 2 + c / 2) = u32x2{x[2], x[3]};
+    // four channels c .. c + 3 of a row of k^ or q^ as their parts
+    auto put4 = [&](float *row, int c, float4 y) __attribute__((always_inline)) {
+        const WyFour x = wy_split4(y.x, y.y, y.z, y.w);
+        uint32_t *r = reinterpret_cast<uint32_t *>(row) + 16 * (c >> 5) + 4 * ((c >> 2) & 3) + 2 * ((c >> 4) & 1);
+#pragma unroll
+        for (int part = 0; part < 3; part++) *reinterpret_cast<u32x2 *>(r + part * (DK / 2)) = x.p[part];
     };
     if constexpr (FUSED) {
         constexpr int NCONV = 2 * DK, TT = 16;               // q and k channels of the head; tokens per run
@@ -304,21 +320,25 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
         {
             const int p = tid / LPP, sub = tid % LPP, tt = p % kC;
             const bool is_q = p < kC;
-            float *row = (is_q ? sQ[tt] : sK[tt]) + EPL * sub;
+            float *row = is_q ? sQ[tt] : sK[tt];
             float4 x[EPL / 4];
             float ss = 0.f;
 #pragma unroll
             for (int i = 0; i < EPL / 4; i++) {
-                x[i] = lds_f4(row + 4 * i);
+                x[i] = lds_f4(row + 4 * (LPP * i + sub));
                 ss += x[i].x * x[i].x + x[i].y * x[i].y + x[i].z * x[i].z + x[i].w * x[i].w;
             }
             ss = dpp_add<0xB1>(ss);
             if (LPP == 4) ss = dpp_add<0x4E>(ss);
             const float inv_scale = 1.0f / sqrtf((float)DK);
             const float inv_rms = 1.0f / sqrtf(ss / (float)DK + 1e-6f);
-            const float sc = inv_rms * (is_q ? inv_scale * inv_scale : inv_scale);
+            const float sc = is_q ? inv_scale * inv_scale : inv_scale;
 #pragma unroll
-            for (int i = 0; i < EPL / 4; i++) put4(is_q ? sQ[tt] : sK[tt], EPL * sub + 4 * i, x[i], sc);   // (a row's lanes are one wave's: all have read it)
+            for (int i = 0; i < EPL / 4; i++) {
+                float4 y = {x[i].x * inv_rms, x[i].y * inv_rms, x[i].z * inv_rms, x[i].w * inv_rms};
+                y.x *= sc; y.y *= sc; y.z *= sc; y.w *= sc;
+                put4(row, 4 * (LPP * i + sub), y);   // (a row's lanes are one wave's: all have read it)
+            }
         }
     } else {
         if (wave == 0) {
@@ -349,52 +369,56 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
         for (int u = 0; u < NL; u++) {
             const int i = tid + u * NTHR, tt = i / (DK / 4), x = (i % (DK / 4)) * 4;
             const float keep = tt < nt ? 1.f : 0.f;  // padded tokens are zero rows
-            put4(sK[tt], x, float4{a[u].x * keep, a[u].y * keep, a[u].z * keep, a[u].w * keep}, 1.f);
-            put4(sQ[tt], x, float4{b[u].x * keep, b[u].y * keep, b[u].z * keep, b[u].w * keep}, 1.f);
+            put4(sK[tt], x, float4{a[u].x * keep, a[u].y * keep, a[u].z * keep, a[u].w * keep});
+            put4(sQ[tt], x, float4{b[u].x * keep, b[u].y * keep, b[u].z * keep, b[u].w * keep});
         }
     }
     __syncthreads();
 
     // Operands from the rows: eight channels of a row; four tokens (t .. t + 3, t = 16 tau + 4 g) of channel 16 c + m.
-    auto row_part = [&](const float *row, int s, int part) __attribute__((always_inline)) {
-        return *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint32_t *>(row) + part * (DK / 2) + 16 * s + 4 * g);
+    auto row_of = [&](const float *row, int s) __attribute__((always_inline)) {
+        WyEight r;
+#pragma unroll
+        for (int part = 0; part < 3; part++)
+            r.p[part] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint32_t *>(row) + part * (DK / 2) + 16 * s + 4 * g);
+        return r;
     };
-    auto col_part = [&](int tau, int c, int part) __attribute__((always_inline)) {
+    auto col_of = [&](int tau, int c) __attribute__((always_inline)) {
         typedef short i16x4 __attribute__((ext_vector_type(4)));
-        const uint32_t *p = reinterpret_cast<const uint32_t *>(sK[16 * tau + 4 * g + (m >> 2)]) + part * (DK / 2) + 8 * c + 2 * (m & 3);
-        return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (i16x4 __attribute__((address_space(3))) *)(__attribute__((address_space(3))) uint32_t *)p));
+        const uint32_t *p = reinterpret_cast<const uint32_t *>(sK[16 * tau + 4 * g + (m >> 2)]) + 16 * (c >> 1) + 4 * (m & 3) + 2 * (c & 1);
+        WyFour r;
+#pragma unroll
+        for (int part = 0; part < 3; part++)
+            r.p[part] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (i16x4 __attribute__((address_space(3))) *)(__attribute__((address_space(3))) uint32_t *)(p + part * (DK / 2))));
+        return r;
     };
     const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    constexpr float kUnscale2 = 1.f / (kWyScale * kWyScale);
 
     // ---- phase 1: the lower tiles of K K^T (-> A) and of Q K^T (-> M) -----------------
-    // A job is a row tile I of one of the two and its tiles J <= I; the jobs of a SIMD's two waves add up to five tiles.  Written
+    // A job is two tiles of M, or three, of which M's (that take longer) is at most one.  Written
     // out per job, so that the reads of a tile's operands overlap the tile before it.
-    auto gram = [&](auto kind_tag, auto I_tag) __attribute__((always_inline)) {
-        constexpr int kind = decltype(kind_tag)::value, I = decltype(I_tag)::value;
-        u32x4 ih[NS], il[NS];
+    auto gram = [&](auto kind_tag, auto I_tag, auto from_tag, auto to_tag) __attribute__((always_inline)) {
+        constexpr int kind = decltype(kind_tag)::value, I = decltype(I_tag)::value, J0 = decltype(from_tag)::value, J1 = decltype(to_tag)::value;
+        WyEight own[NS];
 #pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const float *row = kind ? sQ[16 * I + m] : sK[16 * I + m];
-            ih[s] = row_part(row, s, 0);
-            il[s] = row_part(row, s, 1);
-        }
+        for (int s = 0; s < NS; s++) own[s] = row_of(kind ? sQ[16 * I + m] : sK[16 * I + m], s);
 #pragma unroll
-        for (int J = 0; J <= I; J++) {
-            u32x4 jh[NS], jl[NS];
+        for (int J = J0; J <= J1; J++) {
+            WyEight other[NS];
 #pragma unroll
-            for (int s = 0; s < NS; s++) jh[s] = row_part(sK[16 * J + m], s, 0), jl[s] = row_part(sK[16 * J + m], s, 1);
-            wy_f32x4 lh = zero, hl = zero, hh = zero;
+            for (int s = 0; s < NS; s++) other[s] = row_of(sK[16 * J + m], s);
+            wy_f32x4 term[6];
 #pragma unroll
-            for (int s = 0; s < NS; s++) {
-                // K K^T: lane (n = m, g) gets rows 16I + 4g + i of column 16J + n.  Q K^T as the tile transposed (k^ as the A side):
-                // columns 16J + 4g + i of row 16I + n, which is this lane's 16 bytes of tile (I, J) in A-operand order
-                lh = kind ? wy_mfma(jl[s], ih[s], lh) : wy_mfma(il[s], jh[s], lh);
-                hl = kind ? wy_mfma(jh[s], il[s], hl) : wy_mfma(ih[s], jl[s], hl);
-                hh = kind ? wy_mfma(jh[s], ih[s], hh) : wy_mfma(ih[s], jh[s], hh);
-            }
-            const wy_f32x4 acc = ((lh + hl) + hh) * kUnscale2;
+            for (int t = 0; t < 6; t++) term[t] = zero;
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int t = 0; t < 6; t++)
+                    // K K^T: lane (n = m, g) gets rows 16I + 4g + i of column 16J + n.  Q K^T as the tile transposed (k^ as the A side):
+                    // columns 16J + 4g + i of row 16I + n, which is this lane's part of tile (I, J) in A-operand order
+                    term[t] = kind ? wy_mfma(other[s].p[kWyA[t]], own[s].p[kWyB[t]], term[t]) : wy_mfma(own[s].p[kWyA[t]], other[s].p[kWyB[t]], term[t]);
+            const wy_f32x4 acc = ((term[0] + term[1]) + term[2]) + (term[3] + term[4]) + term[5];
             const int one = kind ? 16 * I + m : 16 * J + m, four = (kind ? 16 * J : 16 * I) + 4 * g;   // this lane's row (column), columns (rows)
             const float4 l4 = lds_f4(&sL[four]);
             const float lf[4] = {l4.x, l4.y, l4.z, l4.w}, l1 = sL[one];
@@ -406,7 +430,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
                     const float d = r1 > four + i ? 0.f : __builtin_amdgcn_exp2f(fminf(l1 - lf[i], 0.f) * 1.4426950408889634f);  // v_exp_f32: 1 ulp
                     y[i] = (I > J || four + i <= one) ? d * acc[i] : 0.f;
                 }
-                Mt[((slot * 4 + I) * 4 + J) * 64 + lane] = wy_split4_unit(y[0], y[1], y[2], y[3]);
+                *reinterpret_cast<wy_f32x4 *>(Mt + (((slot * 4 + I) * 4 + J) * 64 + lane) * 4) = y;
             } else {
                 const float4 b4 = lds_f4(&sB[four]);
                 const int4 r4 = *reinterpret_cast<const int4 *>(&sR[four]);
@@ -422,25 +446,28 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     };
 #pragma unroll
     for (int r = 0; r < 8 / NW; r++) {
-        using std::integral_constant;
+        const std::integral_constant<int, 0> c0{};
+        const std::integral_constant<int, 1> c1{};
+        const std::integral_constant<int, 2> c2{};
+        const std::integral_constant<int, 3> c3{};
         switch (wave + NW * r) {   // uniform over the wave
-            case 0: gram(integral_constant<int, 0>{}, integral_constant<int, 0>{}); break;
-            case 1: gram(integral_constant<int, 0>{}, integral_constant<int, 1>{}); break;
-            case 2: gram(integral_constant<int, 0>{}, integral_constant<int, 2>{}); break;
-            case 3: gram(integral_constant<int, 0>{}, integral_constant<int, 3>{}); break;
-            case 4: gram(integral_constant<int, 1>{}, integral_constant<int, 3>{}); break;
-            case 5: gram(integral_constant<int, 1>{}, integral_constant<int, 2>{}); break;
-            case 6: gram(integral_constant<int, 1>{}, integral_constant<int, 1>{}); break;
-            default: gram(integral_constant<int, 1>{}, integral_constant<int, 0>{}); break;
+            case 0: gram(c0, c0, c0, c0); gram(c0, c1, c0, c1); break;
+            case 1: gram(c0, c2, c0, c2); break;
+            case 2: gram(c0, c3, c0, c1); gram(c1, c0, c0, c0); break;
+            case 3: gram(c0, c3, c2, c3); gram(c1, c2, c2, c2); break;
+            case 4: gram(c1, c3, c0, c1); break;
+            case 5: gram(c1, c3, c2, c3); break;
+            case 6: gram(c1, c1, c0, c1); break;
+            default: gram(c1, c2, c0, c1); break;
         }
     }
 #pragma unroll
-    for (int u = 0; u < 4 * NK / NW; u++) {  // q^ tiles, before T takes their place: once per k head, by its value heads in turn
+    for (int u = 0; u < 4 * NS / NW; u++) {  // q^ tiles, before T takes their place: once per k head, by its value heads in turn
         if (u % heads != vh % heads) continue;
-        const int tile = wave + NW * u, w = tile / NK, c = tile % NK;
-        const uint32_t *row = reinterpret_cast<const uint32_t *>(sQ[16 * w + m]) + 8 * c + 2 * g;
-        const u32x2 hi = *reinterpret_cast<const u32x2 *>(row), lo = *reinterpret_cast<const u32x2 *>(row + DK / 2);
-        Qt[((slot - vh % heads) * 4 * NK + tile) * 64 + lane] = u32x4{hi[0], hi[1], lo[0], lo[1]};
+        const int tile = wave + NW * u;
+        const WyEight x = row_of(sQ[16 * (tile / NS) + m], tile % NS);
+#pragma unroll
+        for (int part = 0; part < 3; part++) Qt[(((slot - vh % heads) * 4 * NS + tile) * 3 + part) * 64 + lane] = x.p[part];
     }
     __syncthreads();
 
@@ -448,11 +475,6 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     //      T = (I + A)^-1 by blocks of 16: the diagonal blocks by forward substitution (one
     //      per wave, a column per lane), the blocks below them level by level from
     //      T_IJ = -T_II sum_{J <= K < I} A_IK T_KJ on the matrix cores -----------------------
-    // k^ of four tokens from its parts (exact), times kWyScale
-    auto whole = [&](u32x2 hi, u32x2 lo) __attribute__((always_inline)) {
-        const f16x2 h0 = __builtin_bit_cast(f16x2, (uint32_t)hi[0]), h1 = __builtin_bit_cast(f16x2, (uint32_t)hi[1]), l0 = __builtin_bit_cast(f16x2, (uint32_t)lo[0]), l1 = __builtin_bit_cast(f16x2, (uint32_t)lo[1]);
-        return float4{(float)h0[0] + (float)l0[0], (float)h0[1] + (float)l0[1], (float)h1[0] + (float)l1[0], (float)h1[1] + (float)l1[1]};
-    };
     if (NW == 4 || wave < 4) {
         // block `wave`; the four lane groups compute the same 16 columns, group 0 stores
         const int r0 = 16 * wave;
@@ -475,34 +497,32 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     // the waves without a diagonal block take the tiles of K' (all waves where each has one)
     if (NW == 4 || wave >= 4) {
 #pragma unroll
-        for (int u = 0; u < NK; u++) {
-            const int tile = (wave & 3) + 4 * u, c = tile >> 2, tau = tile & 3;
-            const float4 e = lds_f4(&sKd[16 * tau + 4 * g]);
-            const float4 k = whole(col_part(tau, c, 0), col_part(tau, c, 1));
-            Kt[(slot * NK * 4 + tile) * 64 + lane] = wy_split4(k.x * e.x, k.y * e.y, k.z * e.z, k.w * e.w, 1.f);
+        for (int u = 0; u < NK / 2; u++) {
+            const int tile = (wave & 3) + 4 * u, c = tile >> 1, p = tile & 1;
+            WyFour x[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float4 e = lds_f4(&sKd[32 * p + 16 * h + 4 * g]);
+                const wy_f32x4 k = wy_whole(col_of(2 * p + h, c));
+                x[h] = wy_split4(k[0] * e.x, k[1] * e.y, k[2] * e.z, k[3] * e.w);
+            }
+            const WyEight y = wy_join(x[0], x[1]);
+#pragma unroll
+            for (int part = 0; part < 3; part++) Kt[((slot * NK * 2 + tile) * 3 + part) * 64 + lane] = y.p[part];
         }
     }
     __syncthreads();
-    // phase 3's K and V operands of the wave's columns, for all four token tiles: here, where most waves would wait for the levels
-    u32x4 kwh[2], kwl[2], vuh[2], vul[2];
-    float v_undo;
-    {
-        float mx = 0.f, sc;
+    // phase 3's operands, for all four token tiles: here, where most waves would wait for the levels.  V of the wave's 16 columns; K of
+    // 32 columns, of which the wave forms W for two of the four token tiles: the first and the last, or those between
+    static_assert(NW == 2 * NS, "two waves to 32 columns");
+    const int wcol = wave % NS;
+    WyEight vu[2], kw[2][2];
 #pragma unroll
-        for (int s = 0; s < 4; s++)
+    for (int p = 0; p < 2; p++) {
+        vu[p] = wy_join(wy_split4(vreg[2 * p][0], vreg[2 * p][1], vreg[2 * p][2], vreg[2 * p][3]),
+                        wy_split4(vreg[2 * p + 1][0], vreg[2 * p + 1][1], vreg[2 * p + 1][2], vreg[2 * p + 1][3]));
 #pragma unroll
-            for (int i = 0; i < 4; i++) mx = fmaxf(mx, fabsf(vreg[s][i]));
-        wy_scale(rows_max(mx), sc, v_undo);
-#pragma unroll
-        for (int p = 0; p < 2; p++) {
-            const u32x2 h0 = col_part(2 * p, wave, 0), h1 = col_part(2 * p + 1, wave, 0), l0 = col_part(2 * p, wave, 1), l1 = col_part(2 * p + 1, wave, 1);
-            kwh[p] = u32x4{h0[0], h0[1], h1[0], h1[1]};
-            kwl[p] = u32x4{l0[0], l0[1], l1[0], l1[1]};
-            const u32x4 y0 = wy_split4(vreg[2 * p][0], vreg[2 * p][1], vreg[2 * p][2], vreg[2 * p][3], sc);
-            const u32x4 y1 = wy_split4(vreg[2 * p + 1][0], vreg[2 * p + 1][1], vreg[2 * p + 1][2], vreg[2 * p + 1][3], sc);
-            vuh[p] = u32x4{y0[0], y0[1], y1[0], y1[1]};
-            vul[p] = u32x4{y0[2], y0[3], y1[2], y1[3]};
-        }
+        for (int ct = 0; ct < 2; ct++) kw[ct][p] = wy_join(col_of(2 * p, 2 * wcol + ct), col_of(2 * p + 1, 2 * wcol + ct));
     }
 #pragma unroll
     for (int lvl = 1; lvl < 4; lvl++) {
@@ -525,79 +545,102 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
         }
         __syncthreads();
     }
-    // The f16 parts of T diag(beta e^L) and T diag(beta) (T is at most 1: its column j is what an impulse at token j leaves of itself in
-    // later ones); step p of token tile tau holds tokens 32p .. 32p+31, zeros above the diagonal
+    // The parts of T diag(beta e^L) and T diag(beta), tile (tau, s <= tau) at tau (tau + 1) / 2 + s
 #pragma unroll
-    for (int u = 0; u < 12 / NW + (12 % NW != 0); u++) {
-        const int half = wave + NW * u;   // (tau, token tile): (0,0) (0,1) (1,0) (1,1) (2,0) .. (3,3)
-        if (half < 12) {
-            const int tau = half < 4 ? half >> 1 : 2 + ((half - 4) >> 2), s = half < 4 ? half & 1 : (half - 4) & 3;
-            const float4 t = s <= tau ? lds_f4(&sT[16 * tau + m][16 * s + 4 * g]) : float4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < (10 + NW - 1) / NW; u++) {
+        const int tile = wave + NW * u;
+        if (tile < 10) {
+            const int tau = tile >= 6 ? 3 : tile >= 3 ? 2 : tile >= 1 ? 1 : 0, s = tile - tau * (tau + 1) / 2;
+            const int at = (tau < 2 ? tau : 2 * tau - 2) + (s >> 1);
+            const float4 t = lds_f4(&sT[16 * tau + m][16 * s + 4 * g]);
             const float4 cw = lds_f4(&sCw[16 * s + 4 * g]), cb = lds_f4(&sB[16 * s + 4 * g]);
-            const u32x4 x = wy_split4_unit(t.x * cw.x, t.y * cw.y, t.z * cw.z, t.w * cw.w);
-            const u32x4 y = wy_split4_unit(t.x * cb.x, t.y * cb.y, t.z * cb.z, t.w * cb.w);
+            const WyFour x = wy_split4(t.x * cw.x, t.y * cw.y, t.z * cw.z, t.w * cw.w);
+            const WyFour y = wy_split4(t.x * cb.x, t.y * cb.y, t.z * cb.z, t.w * cb.w);
 #pragma unroll
-            for (int part = 0; part < 2; part++) {
-                reinterpret_cast<u32x2 *>(&sTw[half >> 1][part][lane])[half & 1] = u32x2{x[2 * part], x[2 * part + 1]};
-                reinterpret_cast<u32x2 *>(&sTu[half >> 1][part][lane])[half & 1] = u32x2{y[2 * part], y[2 * part + 1]};
+            for (int part = 0; part < 3; part++) {
+                reinterpret_cast<u32x2 *>(&sTw[at][part][lane])[s & 1] = x.p[part];
+                reinterpret_cast<u32x2 *>(&sTu[at][part][lane])[s & 1] = y.p[part];
             }
         }
     }
     __syncthreads();
 
     // ---- phase 3: W = T diag(beta e^L) K and U = T diag(beta) V -------------------------
-    u32x4 tw[6][2], tu[6][2];
+    auto times_t = [&](auto first) __attribute__((always_inline)) {
+        WyEight tu[2][2], tw[2][2];   // [token tile % 2][step]
+        auto is_mine = [](int tau) { return (tau == 0 || tau == 3) == decltype(first)::value; };   // whether the wave forms W of these tokens
+        auto read_t = [&](int tau) __attribute__((always_inline)) {
 #pragma unroll
-    for (int at = 0; at < 6; at++)
+            for (int p = 0; p <= tau / 2; p++)
 #pragma unroll
-        for (int part = 0; part < 2; part++) tw[at][part] = sTw[at][part][lane], tu[at][part] = sTu[at][part][lane];
-    __builtin_amdgcn_sched_barrier(0);   // all reads ahead of the first product
+                for (int part = 0; part < 3; part++) {
+                    const int at = tau < 2 ? tau : 2 * tau - 2 + p;
+                    tu[tau % 2][p].p[part] = sTu[at][part][lane];
+                    if (is_mine(tau)) tw[tau % 2][p].p[part] = sTw[at][part][lane];
+                }
+        };
+        read_t(0);
 #pragma unroll
-    for (int tau = 0; tau < 4; tau++) {
-        wy_f32x4 aw = zero, au = zero;
+        for (int tau = 0; tau < 4; tau++) {
+            if (tau < 3) read_t(tau + 1);
+            __builtin_amdgcn_sched_barrier(0);   // the next tile's reads ahead of this one's products
+            const bool mine = is_mine(tau);
+            wy_f32x4 au[2] = {zero, zero}, aw[2][2] = {{zero, zero}, {zero, zero}};
 #pragma unroll
-        for (int p = 0; p <= tau / 2; p++) {
-            const int at = tau < 2 ? tau : 2 + 2 * (tau - 2) + p;
-            // W transposed (K as the A side): lane (n = m, g) then holds columns 16c + 4g + i of
-            // token 16 tau + n, its 16 bytes of the tile in A-operand order
-            aw = wy_mfma(kwl[p], tw[at][0], aw);
-            au = wy_mfma(tu[at][1], vuh[p], au);
-            aw = wy_mfma(kwh[p], tw[at][1], aw);
-            au = wy_mfma(tu[at][0], vul[p], au);
-            aw = wy_mfma(kwh[p], tw[at][0], aw);
-            au = wy_mfma(tu[at][0], vuh[p], au);
+            for (int p = 0; p <= tau / 2; p++) {
+                const bool half = 2 * p == tau;
+                const WyEight &u8 = tu[tau % 2][p], &w8 = tw[tau % 2][p];
+#pragma unroll
+                for (int t = 0; t < 6; t++) {
+                    const int x = (t & 1) * 3 + t / 2, a = kWyA[x], b = kWyB[x];   // the two sums in turn
+                    wy_f32x4 &u = au[x >= 3];
+                    u = half ? wy_mfma_first(u8.p[a], vu[p].p[b], u) : wy_mfma(u8.p[a], vu[p].p[b], u);
+                    if (mine) {
+                        // W transposed (K as the A side): lane (n = m, g) then holds columns 16c + 4g + i of
+                        // token 16 tau + n, its part of the tile in A-operand order
+#pragma unroll
+                        for (int ct = 0; ct < 2; ct++) {
+                            wy_f32x4 &w = aw[ct][x >= 3];
+                            w = half ? wy_mfma_first(kw[ct][p].p[a], w8.p[b], w) : wy_mfma(kw[ct][p].p[a], w8.p[b], w);
+                        }
+                    }
+                }
+            }
+            // U as computed (a D tile), W in A-operand order
+            *reinterpret_cast<wy_f32x4 *>(Ut + ((slot * 4 + tau) * NK + wave) * 256 + lane * 4) = au[0] + au[1];
+            if (mine) {
+                const WyEight w = wy_join(wy_split4(aw[0][0] + aw[0][1]), wy_split4(aw[1][0] + aw[1][1]));
+#pragma unroll
+                for (int part = 0; part < 3; part++) Wt[(((slot * 4 + tau) * NS + wcol) * 3 + part) * 64 + lane] = w.p[part];
+            }
         }
-        const size_t tile = (slot * 4 + tau) * NK + wave;
-        // U as computed (a D tile), W in A-operand order
-        *reinterpret_cast<wy_f32x4 *>(Ut + tile * 256 + lane * 4) = au * v_undo;
-        const wy_f32x4 w4 = aw * (1.f / kWyScale);   // (the instruction between the product and wy_split4)
-        Wt[tile * 64 + lane] = wy_split4(w4[0], w4[1], w4[2], w4[3], 1.f);
-    }
+    };
+    if (wave < NS) times_t(std::true_type{});
+    else times_t(std::false_type{});
 }
 
 // grid (Hv, DV/32), 512 threads: 32 rows of one head's state, as two groups of 16.  Waves 0-3 are the chain that each block waits
 // for: wave w forms D of tokens 16w .. 16w+15 from W, and owns columns 32w .. 32w+31 of the state, in f32, which it updates
-// and hands to all waves as f16 parts with the scale of each row's largest value there.  Waves 4-7 form O of the same
-// tokens from q^, a block later, beside the chain.  (Lane (n, g) of a tile that the update leaves holds row n, columns 16c+4g+i: with
-// c = 2w, 2w+1 its own eight values are the B operand of a 32-wide contraction over them, k-slot e < 4 being column 32w+4g+e,
-// e >= 4 column 32w+16+4g+e-4; a tile of D likewise tokens 16w+4g+i of row n.  The A side has hi and lo of the same four values in its
-// k-slots 0-3 and 4-7, so against a D operand that repeats its values one instruction adds two of the products.)
-// Bound by the chain: 4.4 k clocks a block (two exchanges through LDS, 56 matrix and 300 vector instructions in a row), on half the
-// CUs at 32 heads.  512 tokens of 32 heads 25.4 us (f32 instructions, 16 rows a workgroup, all CUs) -> 21.2 us; six layers'
-// chunks with this and the block precompute above 238 -> 180 us a pass with three sequences side by side, one sequence 54.8 -> 47.6 a layer;
-// 2000 tokens 162 -> 118 and 163 -> 144, of 64 heads 337 -> 231 and 331 -> 241.  Tried and not kept: the operands touched two blocks
-// ahead to have them in the L2 (24.5 us), O beside D of the same block (24.6).
+// and hands to all waves as parts.  Waves 4-7 form O of the same tokens: q^ S0^T while the chain updates the state, M D while it
+// forms the next block's D, so that LDS and matrix core are shared evenly.  (Lane (n, g) of a tile that the update leaves holds row n,
+// columns 16c+4g+i: with c = 2w, 2w+1 its own eight values are the B operand of a 32-wide contraction over them, k-slot e < 4 being
+// column 32w+4g+e, e >= 4 column 32w+16+4g+e-4; two tiles of D likewise tokens 32p+4g+i and 32p+16+4g+i of row n.)
+// A block takes 6.0 k clocks, 5.0 k without its operand requests (timing only): a chain of two exchanges through LDS, 96 matrix and 250 vector
+// instructions, and 160 KB of operands a CU.  512 tokens of 32 heads on half the CUs 23.8 us (f32 instructions, 16 rows a
+// workgroup: 25.4 on all of them; q^ S0^T beside the next block's D, and requests after the last product: 25.2).
+// A layer with this and the block precompute above against both on f32 instructions, with three sequences side by side / one call after
+// the other: 512 tokens of 32 heads 40.0 / 54.5 -> 36.9 / 52.3 us, 1000 79.1 / 89.2 -> 73.4 / 89.6, 2000 156 / 159 -> 144 / 163,
+// 512 of 64 heads 84.4 / 89.3 -> 73.7 / 78.7.  (f16 pairs: 31.2 / 47.1, 57.9 / 77.9, 114 / 138, 60.3 / 64.3.)
 template <int DK>
 __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
     int Hk, int Hv, int T, const u32x4 *__restrict__ Wt, const u32x4 *__restrict__ Qt,
-    const float *__restrict__ Ut, const u32x4 *__restrict__ Mt, const u32x4 *__restrict__ Kt,
+    const float *__restrict__ Ut, const float *__restrict__ Mt, const u32x4 *__restrict__ Kt,
     const float *__restrict__ eLc, float *__restrict__ ssm, float *__restrict__ o_raw) {
     constexpr int DV = DK;
     constexpr int NK = DK / 16;   // column tiles of the state
     constexpr int NS = DK / 32;   // 32-column steps of a contraction over them
-    __shared__ u32x4 s_s[2][2][NS][2][64];   // state [block % 2][row group][step][hi|lo]
-    __shared__ u32x4 s_d[2][2][4][2][64];    // D [block % 2][row group][token tile][hi twice|lo twice]
-    __shared__ float s_su[2][2][NS][16], s_du[2][2][4][16];   // what undoes their scales, per row
+    __shared__ u32x4 s_s[2][2][NS][3][64];   // state [block % 2][row group][step][h|m|l]
+    __shared__ u32x4 s_d[2][2][2][3][64];    // D [block % 2][row group][32 tokens][h|m|l]
 
     const int vh = wy_head_of(blockIdx.x, Hk, Hv), row0 = blockIdx.y * 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -609,58 +652,46 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
     auto load = [&](__amdgpu_buffer_rsrc_t r, int tile) __attribute__((always_inline)) {
         return __builtin_amdgcn_raw_buffer_load_b128(r, lane16, tile * 1024, 0);
     };
-    u32x4 pw[NK];   // W, or q^, of tokens 16w .. 16w+15: a register takes the next block's request as soon as it has been used
-    auto w_of = [&](const u32x4 *X, int back, int blk) { return buffer_of(X + ((slot_of(blk) - back) * 4 + w) * NK * 64); };
+    WyEight pw[NS];   // W, or q^, of tokens 16w .. 16w+15: a register takes the next block's request as soon as it has been used
+    auto w_of = [&](const u32x4 *X, int back, int blk) { return buffer_of(X + ((slot_of(blk) - back) * 4 + w) * NS * 3 * 64); };
+    auto fetch_w = [&](__amdgpu_buffer_rsrc_t r, int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int part = 0; part < 3; part++) pw[s].p[part] = load(r, 3 * s + part);
+    };
     auto fetch_all_w = [&](const u32x4 *X, int back) __attribute__((always_inline)) {
         const auto r = w_of(X, back, 0);
 #pragma unroll
-        for (int c = 0; c < NK; c++) pw[c] = load(r, c);
+        for (int s = 0; s < NS; s++) fetch_w(r, s);
     };
     // X S0^T of this wave's 16 tokens, X = W or q^ (which lies `back` slots ahead of the head's own), both row groups
     auto times_state = [&](const u32x4 *X, int back, int blk, wy_f32x4 (&p)[2]) __attribute__((always_inline)) {
-        // All LDS reads first, and the three terms of every (step, row group) in turn, so that no instruction waits for the one
-        // before it (left alone the compiler reads each operand just ahead of its product: 5.2 k clocks a block instead of 4.4 k).
-        u32x4 sh[NS][2], sl[NS][2];
-        float un[NS][2];
+        // All LDS reads first, and four sums in turn, so that no instruction waits for the one
+        // before it (left alone the compiler reads each operand just ahead of its product).
+        WyEight st[NS][2];
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
-            for (int rg = 0; rg < 2; rg++) sh[s][rg] = s_s[blk & 1][rg][s][0][lane], sl[s][rg] = s_s[blk & 1][rg][s][1][lane];
+            for (int rg = 0; rg < 2; rg++)
 #pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++) un[s][rg] = s_su[blk & 1][rg][s][m];
+                for (int part = 0; part < 3; part++) st[s][rg].p[part] = s_s[blk & 1][rg][s][part][lane];
         __builtin_amdgcn_sched_barrier(0);
-        wy_f32x4 acc[NS][2];
-        u32x4 hi[NS], lo[NS];
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const u32x4 a = pw[2 * s], b = pw[2 * s + 1];
-            hi[s] = u32x4{a[0], a[1], b[0], b[1]};
-            lo[s] = u32x4{a[2], a[3], b[2], b[3]};
-        }
         const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(lo[s], sh[s][rg], zero);
-#pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(hi[s], sl[s][rg], acc[s][rg]);
-#pragma unroll
-        for (int s = 0; s < NS; s++)
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++) acc[s][rg] = wy_mfma(hi[s], sh[s][rg], acc[s][rg]);
+        wy_f32x4 acc[2][2] = {{zero, zero}, {zero, zero}};
         const auto r = w_of(X, back, blk + 1);
 #pragma unroll
-        for (int c = 0; c < NK; c++) pw[c] = load(r, c);
+        for (int s = 0; s < NS; s += 2) {
 #pragma unroll
-        for (int rg = 0; rg < 2; rg++) {
-            p[rg] = acc[0][rg] * un[0][rg];
+            for (int t = 0; t < 6; t++)
 #pragma unroll
-            for (int s = 1; s < NS; s++) p[rg] = wy_fma(acc[s][rg], un[s][rg], p[rg]);
+                for (int x = 0; x < 2; x++)
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++) acc[x][rg] = wy_mfma(pw[s + x].p[kWyA[t]], st[s + x][rg].p[kWyB[t]], acc[x][rg]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_w(r, s);
+            fetch_w(r, s + 1);
         }
+#pragma unroll
+        for (int rg = 0; rg < 2; rg++) p[rg] = acc[0][rg] + acc[1][rg];
     };
 
     if (wave < 4) {
@@ -674,32 +705,26 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
 #pragma unroll
             for (int ct = 0; ct < 2; ct++) st[rg][ct] = load_v4(srow + 16 * rg * DK + 16 * ct);
         auto publish_state = [&](int buf) __attribute__((always_inline)) {
-            float mx[2];
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) {
-                mx[rg] = 0.f;
+                const WyEight x = wy_join(wy_split4(st[rg][0]), wy_split4(st[rg][1]));
 #pragma unroll
-                for (int i = 0; i < 4; i++) mx[rg] = fmaxf(fmaxf(mx[rg], fabsf(st[rg][0][i])), fabsf(st[rg][1][i]));
-            }
-            rows_max2(mx[0], mx[1]);
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++) {
-                float sc, un;
-                wy_scale(mx[rg], sc, un);
-                const u32x4 a = wy_split4(st[rg][0][0], st[rg][0][1], st[rg][0][2], st[rg][0][3], sc);
-                const u32x4 b = wy_split4(st[rg][1][0], st[rg][1][1], st[rg][1][2], st[rg][1][3], sc);
-                s_s[buf][rg][w][0][lane] = u32x4{a[0], a[1], b[0], b[1]};
-                s_s[buf][rg][w][1][lane] = u32x4{a[2], a[3], b[2], b[3]};
-                if (g == 0) s_su[buf][rg][w][m] = un;
+                for (int part = 0; part < 3; part++) s_s[buf][rg][w][part][lane] = x.p[part];
             }
         };
-        u32x4 kd[2][4];
+        WyEight kd[2][2];   // [column tile][32 tokens]
         wy_f32x4 pu[2];
         float elc;
         auto u_of = [&](int blk) { return buffer_of(Ut + ((slot_of(blk) * 4 + w) * NK + 2 * blockIdx.y) * 256); };
-        auto k_of = [&](int blk) { return buffer_of(Kt + (slot_of(blk) * NK + 2 * (owner ? w : 0)) * 4 * 64); };
+        auto k_of = [&](int blk) { return buffer_of(Kt + (slot_of(blk) * NK + 2 * (owner ? w : 0)) * 2 * 3 * 64); };
         auto fetch_elc = [&](int blk) __attribute__((always_inline)) {
             elc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buffer_of(eLc + slot_of(blk) * kC + kC - 1), 0, 0, 0));
+        };
+        auto fetch_k = [&](__amdgpu_buffer_rsrc_t r, int p) __attribute__((always_inline)) {
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int part = 0; part < 3; part++) kd[ct][p].p[part] = load(r, (2 * ct + p) * 3 + part);
         };
         fetch_all_w(Wt, 0);
         {
@@ -707,10 +732,8 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(ru, rg));
             fetch_elc(0);
-#pragma unroll
-            for (int tau = 0; tau < 4; tau++)
-#pragma unroll
-                for (int ct = 0; ct < 2; ct++) kd[ct][tau] = load(rk, 4 * ct + tau);
+            fetch_k(rk, 0);
+            fetch_k(rk, 1);
         }
         if (owner) publish_state(0);
         __syncthreads();
@@ -722,71 +745,45 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
             const auto ru = u_of(blk + 1);
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) pu[rg] = __builtin_bit_cast(wy_f32x4, load(ru, rg));
-            float mx[2];
-#pragma unroll
-            for (int rg = 0; rg < 2; rg++)
-                mx[rg] = fmaxf(fmaxf(fabsf(d[rg][0]), fabsf(d[rg][1])), fmaxf(fabsf(d[rg][2]), fabsf(d[rg][3])));
-            rows_max2(mx[0], mx[1]);
 #pragma unroll
             for (int rg = 0; rg < 2; rg++) {
-                float sc, un;
-                wy_scale(mx[rg], sc, un);
-                const u32x4 x = wy_split4(d[rg][0], d[rg][1], d[rg][2], d[rg][3], sc);
-                s_d[blk & 1][rg][w][0][lane] = u32x4{x[0], x[1], x[0], x[1]};
-                s_d[blk & 1][rg][w][1][lane] = u32x4{x[2], x[3], x[2], x[3]};
-                if (g == 0) s_du[blk & 1][rg][w][m] = un;
+                const WyFour x = wy_split4(d[rg]);
+#pragma unroll
+                for (int part = 0; part < 3; part++) reinterpret_cast<u32x2 *>(&s_d[blk & 1][rg][w >> 1][part][lane])[w & 1] = x.p[part];
             }
             __syncthreads();
             // ---- S' = e^{L_C} S0 + D^T diag(e^{L_C-L}) K, this wave's columns ------
             if (owner) {
+const auto rk = k_of(blk + 1);
+                WyEight dd[2][2];
+#pragma unroll
+                for (int p = 0; p < 2; p++)
+#pragma unroll
+                    for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                        for (int part = 0; part < 3; part++) dd[p][rg].p[part] = s_d[blk & 1][rg][p][part][lane];
+                __builtin_amdgcn_sched_barrier(0);
+                const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+                wy_f32x4 acc[2][2] = {{zero, zero}, {zero, zero}};
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+#pragma unroll
+                    for (int t = 0; t < 6; t++)
+#pragma unroll
+                        for (int rg = 0; rg < 2; rg++)
+#pragma unroll
+                            for (int ct = 0; ct < 2; ct++) acc[rg][ct] = wy_mfma(kd[ct][p].p[kWyA[t]], dd[p][rg].p[kWyB[t]], acc[rg][ct]);
+                    fetch_k(rk, p);
+                }
 #pragma unroll
                 for (int rg = 0; rg < 2; rg++)
 #pragma unroll
-                    for (int ct = 0; ct < 2; ct++) st[rg][ct] *= elc;
-                const auto rk = k_of(blk + 1);
+                    for (int ct = 0; ct < 2; ct++) st[rg][ct] = wy_fma(st[rg][ct], elc, acc[rg][ct]);
                 fetch_elc(blk + 1);
-                u32x4 dh[4][2], dl[4][2];
-                float un[4][2];
-#pragma unroll
-                for (int tau = 0; tau < 4; tau++)
-#pragma unroll
-                    for (int rg = 0; rg < 2; rg++) dl[tau][rg] = s_d[blk & 1][rg][tau][1][lane], dh[tau][rg] = s_d[blk & 1][rg][tau][0][lane];
-#pragma unroll
-                for (int tau = 0; tau < 4; tau++)
-#pragma unroll
-                    for (int rg = 0; rg < 2; rg++) un[tau][rg] = s_du[blk & 1][rg][tau][m];
-                __builtin_amdgcn_sched_barrier(0);
-                const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int th = 0; th < 4; th += 2) {
-                    wy_f32x4 acc[2][2][2];
-#pragma unroll
-                    for (int t = 0; t < 2; t++)
-#pragma unroll
-                        for (int rg = 0; rg < 2; rg++)
-#pragma unroll
-                            for (int ct = 0; ct < 2; ct++) acc[t][rg][ct] = wy_mfma(kd[ct][th + t], dl[th + t][rg], zero);
-#pragma unroll
-                    for (int t = 0; t < 2; t++)
-#pragma unroll
-                        for (int rg = 0; rg < 2; rg++)
-#pragma unroll
-                            for (int ct = 0; ct < 2; ct++) acc[t][rg][ct] = wy_mfma(kd[ct][th + t], dh[th + t][rg], acc[t][rg][ct]);
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-#pragma unroll
-                        for (int rg = 0; rg < 2; rg++)
-#pragma unroll
-                            for (int ct = 0; ct < 2; ct++) st[rg][ct] = wy_fma(acc[t][rg][ct], un[th + t][rg], st[rg][ct]);
-#pragma unroll
-                        for (int ct = 0; ct < 2; ct++) kd[ct][th + t] = load(rk, 4 * ct + th + t);
-                    }
-                }
                 publish_state((blk + 1) & 1);
             }
             __syncthreads();
         }
-        __syncthreads();   // the other waves' last block
         if (owner) {
 #pragma unroll
             for (int rg = 0; rg < 2; rg++)
@@ -795,12 +792,12 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         }
     } else {
         // ================= O = diag(e^L) q^ S0^T + M D, a block behind =================
-        u32x4 mt[4];
-        wy_f32x4 el;
+        // M comes as f32 and is split here: these waves wait for the chain's D
+        wy_f32x4 rm[4], el;
         auto fetch_m = [&](int blk) __attribute__((always_inline)) {
-            const auto r = buffer_of(Mt + (slot_of(blk) * 4 + w) * 4 * 64);
+            const auto r = buffer_of(Mt + (slot_of(blk) * 4 + w) * 4 * 256);
 #pragma unroll
-            for (int tau = 0; tau < 4; tau++) mt[tau] = load(r, tau <= w ? tau : w);
+            for (int tau = 0; tau < 4; tau++) rm[tau] = __builtin_bit_cast(wy_f32x4, load(r, tau <= w ? tau : w));   // (past the diagonal there is nothing)
         };
         auto fetch_el = [&](int blk) __attribute__((always_inline)) {
             el = __builtin_bit_cast(wy_f32x4, __builtin_amdgcn_raw_buffer_load_b128(buffer_of(eLc + slot_of(blk) * kC + 16 * w), g * 16, 0, 0));
@@ -811,38 +808,43 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
         fetch_m(0);
         __syncthreads();
         __syncthreads();
-        __syncthreads();   // block 0: its D and the state behind it are there
         for (int blk = 0; blk < nblk; blk++) {
+            // beside the update of this block's state
             wy_f32x4 o[2];
             times_state(Qt, shared, blk, o);
             o[0] *= el;
             o[1] *= el;
             fetch_el(blk + 1);
-            __syncthreads();   // the state of this block may be written over
-            // (tiles past the diagonal repeat the last one; their products are left out of the sum)
-            u32x4 dh[4][2], dl[4][2];
-            float un[4][2];
+            __syncthreads();
+            // beside the next block's D
+WyEight dd[2][2];
 #pragma unroll
-            for (int tau = 0; tau < 4; tau++)
+            for (int p = 0; p < 2; p++)
 #pragma unroll
-                for (int rg = 0; rg < 2; rg++) dl[tau][rg] = s_d[blk & 1][rg][tau][1][lane], dh[tau][rg] = s_d[blk & 1][rg][tau][0][lane];
+                for (int rg = 0; rg < 2; rg++)
 #pragma unroll
-            for (int tau = 0; tau < 4; tau++)
-#pragma unroll
-                for (int rg = 0; rg < 2; rg++) un[tau][rg] = s_du[blk & 1][rg][tau][m];
+                    for (int part = 0; part < 3; part++) dd[p][rg].p[part] = s_d[blk & 1][rg][p][part][lane];
             __builtin_amdgcn_sched_barrier(0);
             const wy_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            wy_f32x4 acc[4][2];
+            wy_f32x4 acc[2][2] = {{zero, zero}, {zero, zero}};
+            auto add = [&](int p, auto half) __attribute__((always_inline)) {
+                const WyEight mt = wy_join(wy_split4(rm[2 * p]), decltype(half)::value ? WyFour{} : wy_split4(rm[2 * p + 1]));
 #pragma unroll
-            for (int tau = 0; tau < 4; tau++)
-                if (tau <= w) {
+                for (int t = 0; t < 6; t++)
 #pragma unroll
-                    for (int rg = 0; rg < 2; rg++) acc[tau][rg] = wy_mfma(mt[tau], dl[tau][rg], zero);
+                    for (int rg = 0; rg < 2; rg++) {
+                        const int x = (t & 1) * 3 + t / 2;   // the two sums in turn
+                        const u32x4 a = mt.p[kWyA[x]], b = dd[p][rg].p[kWyB[x]];
+                        acc[t & 1][rg] = decltype(half)::value ? wy_mfma_first(a, b, acc[t & 1][rg]) : wy_mfma(a, b, acc[t & 1][rg]);
+                    }
+            };
 #pragma unroll
-                    for (int rg = 0; rg < 2; rg++) acc[tau][rg] = wy_mfma(mt[tau], dh[tau][rg], acc[tau][rg]);
+            for (int p = 0; p < 2; p++) {
+                if (2 * p < w) add(p, std::false_type{});
+                else if (2 * p == w) add(p, std::true_type{});
+            }
 #pragma unroll
-                    for (int rg = 0; rg < 2; rg++) o[rg] = wy_fma(acc[tau][rg], un[tau][rg], o[rg]);
-                }
+            for (int rg = 0; rg < 2; rg++) o[rg] += acc[0][rg] + acc[1][rg];
             fetch_m(blk + 1);
             const int left = T - (blk * kC + 16 * w) - 4 * g;   // tokens from this lane's first on
             float *dst = o_raw + ((size_t)(blk * kC + 16 * w) * Hv + vh) * DV + row0;
@@ -859,7 +861,7 @@ __global__ __launch_bounds__(512, 2) void gdn_wy_recur_kernel(
 
 size_t gdn_wy_scratch_elems(int Hv, int dk, int dv, int T) {
     const size_t nblk = ((size_t)T + kC - 1) / kC;
-    return nblk * Hv * (3 * (size_t)kC * dk + (size_t)kC * dv + (size_t)kC * kC + kC);
+    return nblk * Hv * (9 * (size_t)kC * dk / 2 + (size_t)kC * dv + (size_t)kC * kC + kC);
 }
 
 // o_raw [T, Hv*dv].  The blocks' inputs come from the layer's inputs (`in`; qn .. bg are then unused
@@ -873,13 +875,13 @@ int launch_gdn_wy(hipStream_t s, int Hk, int Hv, int dk, int dv, int T, const fl
     const size_t nblk = ((size_t)T + kC - 1) / kC;
     if (nblk > 65535) return fail(MFA_ERR_SHAPE, "gdn blocked form: too many tokens in one call");
     const size_t slots = nblk * Hv;
-    // (an operand's two f16 parts take the four bytes of the f32 value they stand for)
+    // (the parts of W, q^ and K' take six bytes a value)
     u32x4 *Wt = reinterpret_cast<u32x4 *>(scratch);
-    u32x4 *Qt = Wt + slots * kC * dk / 4;
-    u32x4 *Kt = Qt + slots * kC * dk / 4;
-    float *Ut = reinterpret_cast<float *>(Kt + slots * kC * dk / 4);
-    u32x4 *Mt = reinterpret_cast<u32x4 *>(Ut + slots * kC * dv);
-    float *eLc = reinterpret_cast<float *>(Mt + slots * kC * kC / 4);
+    u32x4 *Qt = Wt + slots * kC * dk * 3 / 8;
+    u32x4 *Kt = Qt + slots * kC * dk * 3 / 8;
+    float *Ut = reinterpret_cast<float *>(Kt + slots * kC * dk * 3 / 8);
+    float *Mt = Ut + slots * kC * dv;
+    float *eLc = Mt + slots * kC * kC;
     const WyInputs none{};
 #define MFA_WY(DKK, FU)                                                                                             \
     hipLaunchKernelGGL((gdn_wy_kernel<DKK, FU>), dim3(Hv, (unsigned)nblk), dim3(DKK * 4), 0, s, Hk, Hv, T, qn, kn, vv, \

@@ -35,15 +35,6 @@ __device__ inline float rows_max(float v) {
     rows_swap32(a, b);
     return fmaxf(a, b);
 }
-__device__ inline void rows_max2(float &u, float &v) {   // of two values at once
-    float a = u, b = u, c = v, d = v;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-    a = b = fmaxf(a, b);
-    c = d = fmaxf(c, d);
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\tv_permlane32_swap_b32 %2, %3\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
-    u = fmaxf(a, b);
-    v = fmaxf(c, d);
-}
 __device__ inline float rows_sum(float v) {
     float a = v, b = v;
     rows_swap16(a, b);

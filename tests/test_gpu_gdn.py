@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from tests.util import TOL_F32, GdnCase, idx, rel_err, rel_err_rows
+from tests.util import TOL_F32, GdnCase, idx, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -198,12 +198,28 @@ def test_blocked_form_on_hard_inputs(mfa, mutate):
     assert np.array_equal(conv.reshape(-1), ref_conv)
 
 
+def _run(mfa, case, state=None):
+    """(out [T, Hv, dv], conv history, state [Hv dv, dk]) of the chunk call."""
+    with _ctx(mfa, case) as c:
+        c.linear_state_import(0, case.conv_state, case.ssm_state if state is None else state)
+        out = c.prefill_gdn(0, case.qkv, case.z, case.alpha, case.beta)
+        conv, ssm = c.linear_state_export(0)
+    return out.reshape(case.T, case.Hv, case.dv), conv.reshape(-1), ssm.reshape(case.Hv * case.dv, case.dk)
+
+
+def _own_scale_err(a, b, row_len):
+    """Worst max|a_row - b_row| / max|b_row| over the rows, however small a row is; rows of zeros have to be zeros."""
+    a, b = (np.asarray(x, np.float64).reshape(-1, row_len) for x in (a, b))
+    top = np.abs(b).max(axis=1)
+    assert not a[top == 0].any()
+    return float((np.abs(a - b).max(axis=1)[top > 0] / top[top > 0]).max())
+
+
 @pytest.mark.parametrize("dk,Hk,Hv,K,T", [(128, 2, 4, 4, 48), (128, 1, 3, 3, 65), (64, 2, 2, 4, 128), (64, 1, 4, 2, 200)])
 def test_blocked_form_keeps_each_row_of_the_state_to_its_own_scale(mfa, dk, Hk, Hv, K, T):
-    """The blocked form splits its operands into scaled f16 parts; a row of the state and of the values is independent
-    of the others, so each is held to TOL_F32 of its own largest value: rows from 2^-60 to 2^60 side by side, one of
-    2^-100 (below the split's smallest scale), one of 2^80 and a row of zeros with no input.  22 bits an operand and three of the four terms
-    leave 2^-22 of a product, 64 of them and up to four blocks stay below 2^-17 < TOL_F32.  A row that holds NaN or
+    """A row of the state and of the values is independent of the others, so each is held to TOL_F32 of its own largest
+    value: rows from 2^-60 to 2^60 side by side, one of 2^-100 (the smallest whose three bf16 parts are all exact is 2^-102),
+    one of 2^80 and a row of zeros with no input.  A row that holds NaN or
     infinity changes no bit of any other row of the state and leaves the other heads' outputs as they were."""
     case = GdnCase(900 + T, Hk, Hv, dk, dk, K=K, T=T)
     rng = np.random.default_rng(T)
@@ -218,27 +234,100 @@ def test_blocked_form_keeps_each_row_of_the_state_to_its_own_scale(mfa, dk, Hk, 
     case.ssm_state = (case.ssm_state.reshape(Hv * dk, dk) * scale[:, None]).reshape(-1)
     _, ref_conv, ref_ssm = case.oracle()
 
-    def run(state):
-        with _ctx(mfa, case) as c:
-            c.linear_state_import(0, case.conv_state, state)
-            out = c.prefill_gdn(0, case.qkv, case.z, case.alpha, case.beta)
-            conv, ssm = c.linear_state_export(0)
-        return out, conv, ssm.reshape(Hv * dk, dk)
-
-    out, conv, ssm = run(case.ssm_state)
-    assert np.array_equal(conv.reshape(-1), ref_conv)
+    out, conv, ssm = _run(mfa, case)
+    assert np.array_equal(conv, ref_conv)
     assert np.isfinite(ssm).all() and not ssm[1].any()
-    assert rel_err_rows(ssm, ref_ssm, dk) <= TOL_F32
+    assert _own_scale_err(ssm, ref_ssm, dk) <= TOL_F32
     for bad in (np.nan, np.inf):
         state = case.ssm_state.copy()
         row = dk + 5                      # a row of head 1
         state[row * dk + 7] = bad
-        out2, _, ssm2 = run(state)
+        out2, _, ssm2 = _run(mfa, case, state)
         rows = np.arange(Hv * dk) != row
         assert not np.isfinite(ssm2[row]).all()
         assert np.array_equal(ssm2[rows], ssm[rows])
         heads = np.arange(Hv) != 1
-        assert np.array_equal(out2.reshape(T, Hv, dk)[:, heads], out.reshape(T, Hv, dk)[:, heads])
+        assert np.array_equal(out2[:, heads], out[:, heads])
+
+
+@pytest.mark.parametrize("dk,Hk,Hv,K,at", [(128, 2, 4, 4, 40), (128, 1, 3, 3, 27), (64, 2, 2, 4, 124)])
+@pytest.mark.parametrize("part", ["q", "k", "v"])
+@pytest.mark.parametrize("factor", [1e8, 1e13, np.inf, np.nan])
+def test_blocked_form_earlier_tokens_do_not_see_later_ones(mfa, dk, Hk, Hv, K, at, part, factor):
+    """One token whose q, k or v is 1e8 or 1e13 times the others', infinite or NaN, in the first block and late in the
+    second: what comes before it is the same bits.  (A product of 16 x 16 tiles multiplies the tokens ahead of a tile's
+    last by zeros, so a token that is not finite may reach the others of its own 16.)  A token's q is no other's business."""
+    case = GdnCase(500 + at + dk + K, Hk, Hv, dk, dk, K=K, T=150)
+    clean, _, _ = _run(mfa, case)
+    first = {"q": 0, "k": Hk * dk, "v": 2 * Hk * dk}[part]
+    last = {"q": Hk * dk, "k": 2 * Hk * dk, "v": case.C}[part]
+    case.qkv[at, first:last] *= np.float32(factor)
+    out, _, ssm = _run(mfa, case)
+    before = at if np.isfinite(factor) else at // 16 * 16
+    assert np.array_equal(out[:before], clean[:before])
+    if part == "q":
+        assert np.array_equal(out[at + K:], clean[at + K:])
+    if np.isfinite(factor):
+        ref_out, _, ref_ssm = case.oracle()
+        assert rel_err(out, ref_out) <= TOL_F32 and rel_err(ssm, ref_ssm) <= TOL_F32
+    else:
+        assert not np.isfinite(out[at]).all(axis=1).any()
+
+
+@pytest.mark.parametrize("dk,K,T", [(128, 4, 64), (128, 3, 64), (64, 4, 130), (128, 4, 256)])
+@pytest.mark.parametrize("logit", [-8.0, -16.0, -20.0, -40.0, -60.0])
+def test_blocked_form_of_barely_open_gates(mfa, dk, K, T, logit):
+    """beta of 3e-4 down to 9e-27 into an empty state under a decay of 0.99: T diag(beta) and W are as small as beta, and
+    state and outputs are held to their own size."""
+    case = GdnCase(11, 2, 4, dk, dk, K=K, T=T, zero_state=True, plain=True)
+    case.alpha[:] = -4.6
+    case.beta[:] = logit
+    ref_out, _, ref_ssm = case.oracle()
+    out, _, ssm = _run(mfa, case)
+    assert _own_scale_err(ssm, ref_ssm, dk) <= TOL_F32
+    assert _own_scale_err(out, ref_out, dk) <= TOL_F32
+
+
+@pytest.mark.parametrize("dk,K,T,alpha", [(128, 4, 64, -0.846), (128, 3, 65, 0.0), (64, 4, 130, -0.846), (128, 4, 200, -0.846)])
+def test_blocked_form_of_a_state_that_only_decays(mfa, dk, K, T, alpha):
+    """No values at all, beta = 0.5 and a decay of 0.7 or 0.5 a token: what is left of the state after the chunk, 1e-10 to 1e-32
+    of what it was, and the outputs read from it on the way keep their precision.  The decay, the same for every token, is
+    rounded by up to 2^-24 in the oracle and its logarithm as much here: T 2^-23 beside the usual bar."""
+    tol = TOL_F32 + T * 2.0 ** -23
+    case = GdnCase(12, 2, 4, dk, dk, K=K, T=T, plain=True)
+    v0 = 4 * dk
+    case.qkv[:, v0:] = 0.0
+    case.conv_state.reshape(K - 1, case.C)[:, v0:] = 0.0
+    case.alpha[:] = alpha
+    case.beta[:] = 0.0
+    ref_out, _, ref_ssm = case.oracle()
+    out, _, ssm = _run(mfa, case)
+    assert _own_scale_err(ssm, ref_ssm, dk) <= tol
+    assert _own_scale_err(out, ref_out, dk) <= tol
+
+
+@pytest.mark.parametrize("dk,K,T", [(128, 4, 64), (128, 3, 65), (64, 4, 130), (128, 4, 200)])
+def test_blocked_form_of_tokens_and_channels_of_every_size(mfa, dk, K, T):
+    """Values whose size changes by up to 2^24 from token to token under a decay of 0.5, and key channels of 2^-30 to 1: outputs
+    are held to their own row's size, the state's columns (a key channel each) to theirs.  The decay's logarithm runs up to
+    -45 in a block, in six additions that round by up to 2^-19 each, and a factor is e to the difference of two such sums:
+    2.3e-5 beside the usual bar."""
+    tol = TOL_F32 + 12 * 2.0 ** -19
+    case = GdnCase(13 + T, 2, 4, dk, dk, K=K, T=T, plain=True)
+    rng = np.random.default_rng(T)
+    v0, k0 = 4 * dk, 2 * dk
+    case.qkv[:, v0:] *= np.exp2(rng.integers(-12, 13, T)).astype(np.float32)[:, None]
+    case.alpha[:] = 0.0
+    col = np.exp2(rng.integers(-30, 1, 2 * dk)).astype(np.float32)
+    case.qkv[:, k0:v0] *= col
+    case.conv_state.reshape(K - 1, case.C)[:, k0:v0] *= col
+    state = case.ssm_state.reshape(2, 2, dk, dk)
+    state *= col.reshape(2, 1, 1, dk)
+    ref_out, _, ref_ssm = case.oracle()
+    out, _, ssm = _run(mfa, case)
+    cols = lambda s: s.reshape(4, dk, dk).transpose(0, 2, 1)  # noqa: E731
+    assert _own_scale_err(cols(ssm), cols(ref_ssm), dk) <= tol
+    assert _own_scale_err(out, ref_out, dk) <= tol
 
 
 def test_chunk_at_the_a17b_head_counts(mfa):
