@@ -333,11 +333,12 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
             const float inv_scale = 1.0f / sqrtf((float)DK);
             const float inv_rms = 1.0f / sqrtf(ss / (float)DK + 1e-6f);
             const float sc = is_q ? inv_scale * inv_scale : inv_scale;
+            wave_lds_order();   // a row's lanes are one wave's: all have read it
 #pragma unroll
             for (int i = 0; i < EPL / 4; i++) {
                 float4 y = {x[i].x * inv_rms, x[i].y * inv_rms, x[i].z * inv_rms, x[i].w * inv_rms};
                 y.x *= sc; y.y *= sc; y.z *= sc; y.w *= sc;
-                put4(row, 4 * (LPP * i + sub), y);   // (a row's lanes are one wave's: all have read it)
+                put4(row, 4 * (LPP * i + sub), y);
             }
         }
     } else {

@@ -82,11 +82,16 @@ __device__ inline void mla_operands(const f32x4 (&x)[4], float *buf, int lane, b
     const int n = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int r = 0; r < 4; r++) *reinterpret_cast<f32x4 *>(buf + (4 * r + g) * kMlaRow + 4 * n) = x[r];
+    wave_lds_order();
+    f32x4 y[2][2];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         const float *at = buf + n * kMlaRow + 32 * k + 8 * g;
-        mla_split8(mla_load4(at), mla_load4(at + 4), hi[k], lo[k]);
+        y[k][0] = mla_load4(at), y[k][1] = mla_load4(at + 4);
     }
+    wave_lds_order();   // ahead of the next call's writes
+#pragma unroll
+    for (int k = 0; k < 2; k++) mla_split8(y[k][0], y[k][1], hi[k], lo[k]);
 }
 
 // Workgroup id -> (split, head group).  Workgroups go to the 8 XCDs in turn; those of one split read the same rows and sit on

@@ -35,6 +35,9 @@ __device__ inline float rows_max(float v) {
     rows_swap32(a, b);
     return fmaxf(a, b);
 }
+// Between one lane's LDS accesses and another's of the same wave: LDS executes a wave's instructions in order, so nothing has to be
+// waited for; it is the compiler that has to keep the order.  Costs no instruction.
+__device__ inline void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
 __device__ inline float rows_sum(float v) {
     float a = v, b = v;
     rows_swap16(a, b);
