@@ -148,10 +148,10 @@ def test_mla_kernels_at_their_borders(mfa, H, L):
     assert rel_err(out, ref.reshape(-1)) <= TOL_F32
 
 
-def test_mla_not_a_number_and_infinity_stay_in_their_heads(mfa):
-    """A query row that is not finite spoils its own head and no other of its tile; a row of the cache past the end is
-    never read into a result."""
-    H, L = 20, 200
+@pytest.mark.parametrize("H,L", [(20, 200), (128, 4097), (128, 16385)])
+def test_mla_not_a_number_and_infinity_stay_in_their_heads(mfa, H, L):
+    """A query row that is not finite spoils its own head and no other of its tile: in rounds of 16 heads a workgroup, of
+    32, and streamed by 64."""
     qp, qe, lat, rk = _random(77, H, L)
     clean = mfa.mla_sdpa_folded(H, R, P, L, 0.07, qp, qe, lat, rk).reshape(H, R)
     qp[3, 5], qp[17, 0] = np.nan, np.inf
@@ -159,6 +159,29 @@ def test_mla_not_a_number_and_infinity_stay_in_their_heads(mfa):
     others = [h for h in range(H) if h not in (3, 17)]
     assert np.isnan(out[3]).all() and np.isnan(out[17]).all()
     assert np.array_equal(out[others], clean[others])
+
+
+@pytest.mark.parametrize("H,L", [(20, 200), (128, 4097), (128, 16385)])
+def test_mla_rows_past_the_end_reach_no_result(mfa, H, L):
+    """The same three kernels over arrays whose rows behind the cache's last position are NaN: the same bits as with
+    other rows there."""
+    from moeflux_amd import Config, ffi
+    from moeflux_amd.hip import DeviceArray
+    qp, qe, lat, rk = _random(78, H, L + 160)
+    q = [DeviceArray.from_host(a) for a in (qp, qe)]
+    outs = []
+    with mfa.Ctx(Config(num_layers=1, full_attn_interval=1, num_attn_heads=8, num_kv_heads=2, head_dim=64,
+                        kv_capacity=4)) as c:
+        for tail in (0.0, np.nan):
+            lat[L:], rk[L:] = tail, tail
+            kv = [DeviceArray.from_host(a) for a in (lat, rk)]
+            do = DeviceArray((H * R,), np.float32, zero=True)
+            rc = c.lib.mfa_mla_sdpa_folded_dev(c.h, H, R, P, L, C.c_float(0.07), q[0].ptr, q[1].ptr, kv[0].ptr,
+                                               kv[1].ptr, do.ptr)
+            assert rc == 0, ffi.last_error()
+            c.sync()
+            outs.append(do.to_host())
+    assert np.isfinite(outs[0]).all() and np.array_equal(outs[0], outs[1])
 
 
 def test_mla_errors(mfa):
