@@ -47,9 +47,8 @@
 //     parts of the 16 positions followed by their lo parts, so that with P = [p_hi | p_hi]
 //     one instruction adds x_hi p_hi + x_lo p_hi and a second with [p_lo | p_lo] adds x_hi p_lo
 //     (and x_lo p_lo, which comes for free).
-//     The value waves fetch and split 6 of a block's 16 latent rows (two channels per
-//     thread), the score waves the other 10 and the rotary keys: the split at which the call is
-//     fastest (12 / 4, which evens out the clocks the two roles spend per block, is 4 % slower).
+//     The value waves fetch and split 6 of a block's 16 latent rows (four channels of every second one per
+//     thread), the score waves the other 10 and the rotary keys (4 or 8 for the value waves are no faster).
 #include <algorithm>
 #include <type_traits>
 
@@ -317,7 +316,6 @@ __global__ __launch_bounds__(kMlaWaves * 64, 2) void mla_rounds_kernel(
     }
 }
 
-__device__ inline f32x2 mla_load2(const float *p) { return *reinterpret_cast<const f32x2 *>(p); }
 __device__ inline bf16x8 mla_lds8(const void *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
 typedef short mla_i16x4 __attribute__((ext_vector_type(4)));
@@ -603,13 +601,16 @@ bool mla_shape_supported(int kv_lora_rank, int qk_rope_head_dim) {
 // Partition of the heads and of the cache over workgroups, a workgroup per CU.  Which kernel (us a layer, one call after the
 // other / three sequences side by side, in brackets the streaming kernel with its queries read in operand order):
 //   rounds, 16 heads  where one round of 128 positions is enough: 128 heads over 200 positions 11.5 / 7.6 (17.0 / 8.4), 1500
-//                     14.8 / 11.1 (26.1 / 15.1), 4096 18.1 / 13.9 (27.7 / 20.9); 64 over 2000 14.5 / 10.8 (24.0 / 11.4), 8192 18.7 / 13.7
-//                     (28.8 / 22.6).  17 to 32 heads, whose two groups share an L2: up to three rounds, 32 over 32768 26.0 / 25.7
-//                     (33.8 / 28.9), 49000 33.9 / 36.0 (40.0 / 36.4).  Up to 16 heads, where nobody shares the second read of
-//                     the rows: up to 80 positions, 16 over 16384 19.9 / 15.2 (23.6 / 15.9), but 32768 32.0 / 24.8 (30.5 / 25.3)
-//   rounds, 32 heads  up to two rounds: 128 over 8192 24.3 / 18.5 (28.6 / 24.4), 16384 31.7 / 28.3 (34.0 / 32.6), but 24000
-//                     40.8 / 39.8 (41.5 / 39.4); 64 over 32768 33.8 / 31.3 (38.0 / 36.5)
-//   streaming, 64     beyond: 128 over 32768 43.7 / 44.5 (47.9 / 48.7), 65536 76.5 / 74.7 (79.5 / 79.8)
+//                     14.8 / 11.1 (26.1 / 15.1), 4096 17.9 / 13.7, where 32 heads take 20.8 / 13.9 and at 4600 22.2 / 15.3 against 21.3 / 16.7;
+//                     64 over 2000 14.5 / 10.8 (24.0 / 11.4), 8192 18.7 / 13.7
+//                     (28.8 / 22.6).  17 to 32 heads, whose two groups share an L2: up to three rounds, 30 over 24576 21.7 / 20.3 (the
+//                     present streaming kernel 29.1 / 24.4), 40000 29.2 / 30.6 (35.0 / 31.3), 49152 32.9 / 36.1 (39.4 / 35.0),
+//                     but 55000 39.3 / 40.2 (41.1 / 38.2).  Up to 16 heads, where nobody shares the second read of
+//                     the rows: up to 80 positions a CU, from where on it is a draw: 16 over 16384 19.3 / 15.3 (streaming 23.0 / 16.3), 18400 23.4 / 16.6 (23.6 /
+//                     16.5), 20480 25.8 / 17.8 (25.3 / 18.3), 22500 25.1 / 19.1 (24.8 / 20.2), but 32768 32.0 / 24.8 (30.5 / 25.3)
+//   rounds, 32 heads  up to two rounds: 128 over 8192 24.3 / 18.5 (28.6 / 24.4), 12000 26.6 / 23.2 (streaming 30.4 / 26.2), 16384 30.9 / 28.0 (31.7 / 31.0), 18000
+//                     34.8 / 32.4 (34.8 / 32.5), but 24000 40.8 / 39.8 (41.5 / 39.4); 64 over 32768 33.8 / 31.3 (38.0 / 36.5)
+//   streaming, 64     beyond: 128 over 32768 43.6 / 44.8 (47.9 / 48.7), 65536 76.5 / 74.7 (79.5 / 79.8)
 MlaPlan mla_plan(int H, int L, int num_cus, int forced_splits) {
     MlaPlan p;
     p.nhg = (H + 15) / 16;
