@@ -147,7 +147,7 @@ __global__ __launch_bounds__(DK * 4) void gdn_wy_kernel(
     u32x4 *__restrict__ Kt, float *__restrict__ eLc, WyInputs in) {
     constexpr int DV = DK;
     constexpr int NK = DK / 16, NS = DK / 32;
-    // row strides (4-byte units) chosen so that 16-byte row reads by 8 lanes hit all banks
+    // row strides (4-byte units) chosen so that 16-byte row reads by 8 lanes hit all banks (LDK 4 to 52 past the parts: within 0.5 % of each other)
     constexpr int LDK = 3 * DK / 2 + 20, LDC = kC + 4;
     constexpr int NW = NK;        // waves; wave c owns columns 16c .. 16c+15 of U
     constexpr int NTHR = 64 * NW;
